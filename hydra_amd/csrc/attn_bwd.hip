@@ -29,6 +29,16 @@
 // The MFMA B operand of the PV-type products is taken straight from the
 // score accumulator registers; the A operand is read from the transposed
 // LDS tile in the same (register-order) permutation of the summed index.
+// A key mask is a template form of both kernels: dK/dV lanes own one key
+// each, so masked lanes only store zeros; dQ tests one bit per key on tiles
+// that hold a masked key and skips tiles of padding.  Masked calls and
+// head_dim 16 (one MFMA k-step; half of the 32-row d tile unused) keep P and
+// dS in two bf16 planes, hi + residual: their products are as exact as with
+// fp32 P and dS on bf16 outputs (error against 64 bits unchanged), at one
+// more MFMA per fragment.  Measured against one thread per row in fp32:
+// B8 4/1 heads x 64, S 777, padded: 101.4 ms -> below 0.1; B2 28/4 heads x
+// 16, S 2048, causal: 60 ms -> below 0.3 (whole layer steps 102.5 -> 1.41
+// and 61.3 -> 1.40 ms, what remains is the rest of the layer).
 // Generic path (attn_bwd_generic_*): one thread per query / key row, fp32
 // math, any element type, head_dim <= 256.
 #include "common.h"
@@ -66,6 +76,19 @@ __device__ __forceinline__ f32x16_t zero16() {
 __device__ __forceinline__ uint4 pack_c8(const f32x16_t& x, int base) {
   return make_uint4(pack2<bf16>(x[base + 0], x[base + 1]), pack2<bf16>(x[base + 2], x[base + 3]),
                     pack2<bf16>(x[base + 4], x[base + 5]), pack2<bf16>(x[base + 6], x[base + 7]));
+}
+
+// The bf16 rounding residuals of the same 8 registers (x - float(hi) with
+// hi = pack_c8(x, base)), rounded to bf16: hi + lo carries 16 significant
+// bits, so a product taken with both planes keeps P and dS at ~2^-17.
+__device__ __forceinline__ uint4 pack_c8_lo(const f32x16_t& x, int base, const uint4& hi) {
+  const uint32_t w[4] = {hi.x, hi.y, hi.z, hi.w};
+  uint32_t o[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    o[i] = pack2<bf16>(x[base + 2 * i] - __uint_as_float(w[i] << 16),
+                       x[base + 2 * i + 1] - __uint_as_float(w[i] & 0xffff0000u));
+  return make_uint4(o[0], o[1], o[2], o[3]);
 }
 
 // A fragment from a transposed LDS tile t[row][col] (pitch in elements),
@@ -194,23 +217,29 @@ struct DkdvLayout {
   static constexpr int QP = HD + 8;          // row-major pitch (elements): 16-byte rows, 4-bank skew
   static constexpr int TP = 32 + 4;          // transposed pitch (elements)
   static constexpr int ROWS = 32 * QP;       // one row-major 32-row tile
-  static constexpr int TRS = HD * TP;        // one transposed tile
+  // one transposed tile; a head_dim-16 tile keeps 32 rows: the d tile of the
+  // MFMA reads all of them, and its rows past head_dim are never stored
+  static constexpr int TRS = (HD < 32 ? 32 : HD) * TP;
   static constexpr int HGE = 2 * ROWS + 2 * TRS + 2 * 32 * 2;  // Q, dO, Q^T, dO^T, lse2, D (elements)
 };
 
-template <int HD, bool CAUSAL, int KB, int HG>
+// MASK as in bwd_visible (2 comes with CAUSAL = false: it walks every query
+// tile); NP: bf16 planes of P and dS (2: hi + residual, see pack_c8_lo).
+template <int HD, bool CAUSAL, int KB, int HG, int MASK, int NP>
 __global__ __launch_bounds__(64 * KB * HG) void attn_bwd_dkdv_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k, const bf16* __restrict__ v,
     const bf16* __restrict__ dout, const float* __restrict__ dvec, const float* __restrict__ lse2,
-    bf16* __restrict__ dk, bf16* __restrict__ dv, float* __restrict__ part, int Hq, int Hkv,
+    const uint8_t* __restrict__ kmask, bf16* __restrict__ dk, bf16* __restrict__ dv, float* __restrict__ part, int Hq, int Hkv,
     int S, int G, int nwg, int ch, int maxch,
     int64_t qs0, int64_t qs1, int64_t qs2, int64_t ks0, int64_t ks1, int64_t ks2,
     int64_t vs0, int64_t vs1, int64_t vs2, int64_t ds0, int64_t ds1, int64_t ds2,
     int64_t dks0, int64_t dks1, int64_t dks2, int64_t dvs0, int64_t dvs1, int64_t dvs2,
     float scale_log2, float scale) {
   constexpr int NT = 64 * KB * HG;
+  static_assert(HD >= 32 || HG == 1, "a wave's staging units share one head group");
   constexpr int KS = HD / 16;   // k-steps over head_dim
-  constexpr int DT = HD / 32;   // 32-row d tiles of dK^T / dV^T
+  constexpr int DT = (HD + 31) / 32;  // 32-row d tiles of dK^T / dV^T
+  constexpr int JT = HD < 32 ? 2 : 4;  // 8-row groups of a d tile that hold rows of head_dim
   constexpr int DC = HD / 8;    // 16-byte chunks per row
   using L = DkdvLayout<HD>;
   constexpr int STAGE = HG * L::HGE;
@@ -281,6 +310,21 @@ __global__ __launch_bounds__(64 * KB * HG) void attn_bwd_dkdv_kernel(
   const int kw0 = kg0 + 32 * kbl;         // first key of this wave
   const int key = kw0 + n;
 
+  // Key mask: a lane owns one key, so key padding (MASK 1) needs no test in
+  // the tiles -- a column of the MFMA's B operand reaches its own column of
+  // the result only -- and the masked lanes store zeros at the end; waves
+  // (and workgroups) without a visible key skip the walk.  MASK 2: query s
+  // sees the key iff s < kbnd.
+  bool kvis = key < S;
+  int kbnd = key;
+  if constexpr (MASK != 0) {
+    const bool keep = kvis && kmask[static_cast<int64_t>(b) * S + key] != 0;
+    if constexpr (MASK == 1) kvis = keep;
+    else if (!keep) kbnd = 0x7fffffff;
+  }
+  const bool wave_any = MASK != 1 || __builtin_amdgcn_readfirstlane(__any(kvis)) != 0;
+  const bool wg_any = MASK != 1 || __syncthreads_or(kvis) != 0;
+
   // K and V fragments (B operands of S = Q K^T, dP = dO V^T).
   uint4 kf[KS], vf[KS];
   {
@@ -313,7 +357,7 @@ __global__ __launch_bounds__(64 * KB * HG) void attn_bwd_dkdv_kernel(
   const int dreg = CAUSAL ? max(0, min(KB * kg + KB - qt0, nq)) : 0;
   const int nd = dreg == KB ? KB : 0;
   const int nr = max(nq - nd, 1);
-  const int ediag = nd ? rounds * nd : (dreg > 0 ? nsteps : 0);
+  const int ediag = MASK == 2 ? nsteps : nd ? rounds * nd : (dreg > 0 ? nsteps : 0);
   auto locate = [&](int step, int& hr, int& qt) {
     if (step < rounds * nd) {
       hr = step / nd;
@@ -420,7 +464,8 @@ __global__ __launch_bounds__(64 * KB * HG) void attn_bwd_dkdv_kernel(
         for (int i = 0; i < 4; ++i) {
           const int r = 4 * j + i;
           float p = __builtin_amdgcn_exp2f(fmaf(s[r], scale_log2, -lj[i]));
-          if constexpr (DIAG) p = (key <= q0 + 8 * j + 4 * hf + i) ? p : 0.f;
+          if constexpr (DIAG && MASK == 2) p = (q0 + 8 * j + 4 * hf + i < kbnd) ? p : 0.f;
+          else if constexpr (DIAG) p = (key <= q0 + 8 * j + 4 * hf + i) ? p : 0.f;
           s[r] = p;
           dp[r] = p * (dp[r] - dj[i]);
         }
@@ -429,10 +474,19 @@ __global__ __launch_bounds__(64 * KB * HG) void attn_bwd_dkdv_kernel(
       for (int c = 0; c < 2; ++c) {
         const uint4 pb = pack_c8(s, 8 * c);
         const uint4 sb = pack_c8(dp, 8 * c);
+        uint4 pl, sl;
+        if constexpr (NP == 2) {
+          pl = pack_c8_lo(s, 8 * c, pb);
+          sl = pack_c8_lo(dp, 8 * c, sb);
+        }
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
-          dva[dt] = mfma(lds_a_perm(Dt, 32 * dt + n, L::TP, c, hf), pb, dva[dt]);
-          dka[dt] = mfma(lds_a_perm(Qt, 32 * dt + n, L::TP, c, hf), sb, dka[dt]);
+          const uint4 ad = lds_a_perm(Dt, 32 * dt + n, L::TP, c, hf);
+          dva[dt] = mfma(ad, pb, dva[dt]);
+          if constexpr (NP == 2) dva[dt] = mfma(ad, pl, dva[dt]);
+          const uint4 aq = lds_a_perm(Qt, 32 * dt + n, L::TP, c, hf);
+          dka[dt] = mfma(aq, sb, dka[dt]);
+          if constexpr (NP == 2) dka[dt] = mfma(aq, sl, dka[dt]);
         }
       }
     }
@@ -441,6 +495,12 @@ __global__ __launch_bounds__(64 * KB * HG) void attn_bwd_dkdv_kernel(
     int hr, qt;
     locate(step, hr, qt);
     const int q0 = 32 * qt;
+    if (!wave_any) return;
+    if constexpr (MASK == 2) {  // every key after every query of the tile: no test needed
+      if (q0 + 31 < kw0 && kw0 + 31 < S) tile(std::false_type{}, q0, buf);
+      else tile(std::true_type{}, q0, buf);
+      return;
+    }
     // Causal: the tile reaches this wave's keys iff q0 + 31 >= kw0; only
     // the diagonal tile q0 == kw0 needs the key <= query mask.
     if (CAUSAL && q0 == kw0) tile(std::true_type{}, q0, buf);
@@ -452,6 +512,7 @@ __global__ __launch_bounds__(64 * KB * HG) void attn_bwd_dkdv_kernel(
   // that every path issues the same loads and each land() waits only for
   // its own set.
   const int last = nsteps - 1;  // >= 0
+  if (wg_any) {
   fetch(0, ra);
   land(0, ra);
   fetch(min(1, last), rb);
@@ -461,7 +522,7 @@ __global__ __launch_bounds__(64 * KB * HG) void attn_bwd_dkdv_kernel(
   auto unmasked = [&](int step, int buf) {
     int hr, qt;
     locate(step, hr, qt);
-    tile(std::false_type{}, 32 * qt, buf);
+    if (wave_any) tile(std::false_type{}, 32 * qt, buf);
   };
   int step = 0;
   for (; step < last && step + 1 < ediag; step += 2) {  // ediag is even or nsteps
@@ -485,6 +546,7 @@ __global__ __launch_bounds__(64 * KB * HG) void attn_bwd_dkdv_kernel(
     __syncthreads();
   }
   if (step == last) compute(step, 0);  // odd count: the last tile is in buffer 0
+  }
   __syncthreads();  // the fold below reuses the staging buffers
 
   // Fold the head groups (fixed order: group 0 + group 1 + ...), then store.
@@ -515,6 +577,12 @@ __global__ __launch_bounds__(64 * KB * HG) void attn_bwd_dkdv_kernel(
       }
     }
   }
+  if constexpr (MASK == 1) {
+    if (!kvis) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) { dka[dt] = zero16(); dva[dt] = zero16(); }
+    }
+  }
   if (nch > 1) {
     // One of several chunks: fp32 partials, summed in chunk order by
     // attn_bwd_dkdv_reduce_kernel.
@@ -525,7 +593,7 @@ __global__ __launch_bounds__(64 * KB * HG) void attn_bwd_dkdv_kernel(
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < JT; ++j) {
           const int d = 32 * dt + 8 * j + 4 * hf;
           *reinterpret_cast<float4*>(pk + d) =
               make_float4(dka[dt][4 * j], dka[dt][4 * j + 1], dka[dt][4 * j + 2], dka[dt][4 * j + 3]);
@@ -539,7 +607,7 @@ __global__ __launch_bounds__(64 * KB * HG) void attn_bwd_dkdv_kernel(
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < JT; ++j) {
         const int d = 32 * dt + 8 * j + 4 * hf;
         const f32x16_t& a = dka[dt];
         const f32x16_t& c = dva[dt];
@@ -605,15 +673,16 @@ struct DqLayout {
   static constexpr int KP = HD + 8;          // row-major pitch (elements)
   static constexpr int TP = BN + 4;          // transposed pitch (elements)
   static constexpr int ROWS = BN * KP;
-  static constexpr int TRS = HD * TP;
+  static constexpr int TRS = (HD < 32 ? 32 : HD) * TP;  // see DkdvLayout
   static constexpr int STAGE = 2 * ROWS + TRS;  // K, V, K^T
 };
 
-template <int HD, bool CAUSAL, int NW>
+// MASK, NP as in attn_bwd_dkdv_kernel.
+template <int HD, bool CAUSAL, int NW, int MASK, int NP>
 __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k, const bf16* __restrict__ v,
     const bf16* __restrict__ dout, const float* __restrict__ dvec, const float* __restrict__ lse2,
-    bf16* __restrict__ dq, int Hq, int Hkv, int S, int G, int ntasks, int items,
+    const uint8_t* __restrict__ kmask, bf16* __restrict__ dq, int Hq, int Hkv, int S, int G, int ntasks, int items,
     int64_t qs0, int64_t qs1, int64_t qs2, int64_t ks0, int64_t ks1, int64_t ks2,
     int64_t vs0, int64_t vs1, int64_t vs2, int64_t ds0, int64_t ds1, int64_t ds2,
     int64_t dqs0, int64_t dqs1, int64_t dqs2, float scale_log2, float scale) {
@@ -621,7 +690,8 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(
   constexpr int BN = L::BN;
   constexpr int MT = BN / 32;
   constexpr int KS = HD / 16;
-  constexpr int DT = HD / 32;
+  constexpr int DT = (HD + 31) / 32;
+  constexpr int JT = HD < 32 ? 2 : 4;  // 8-row groups of a d tile that hold rows of head_dim
   constexpr int DC = HD / 8;
   constexpr int UNITS = (BN / 2) * DC;        // (key pair, chunk) staging units
   constexpr int NT = 64 * NW;
@@ -673,11 +743,18 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(
 
   const auto krs = rows_rsrc(k + b * ks0 + kvh * ks1, (S - 1) * ks2 * 2 + HD * 2);
   const auto vrs = rows_rsrc(v + b * vs0 + kvh * vs1, (S - 1) * vs2 * 2 + HD * 2);
+  // MASK: every wave loads the flags of the tile's 64 keys, one per lane
+  // (past S: 0), and keeps them as one 64-bit word per staged tile.
+  __amdgpu_buffer_rsrc_t mrs;
+  if constexpr (MASK != 0) mrs = rows_rsrc(kmask + static_cast<int64_t>(b) * S, S);
+  uint64_t keep[2] = {0, 0};
   struct Regs {
     uint4 k[UPT][2], v[UPT][2];
+    uint8_t m;
   };
   Regs ra, rb;
   auto fetch = [&](int kt, Regs& R) {
+    if constexpr (MASK != 0) R.m = __builtin_amdgcn_raw_buffer_load_b8(mrs, BN * kt + lane, 0, 0);
 #pragma unroll
     for (int u = 0; u < UPT; ++u) {
       const int unit = tid + NT * u;
@@ -695,6 +772,7 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(
   };
   auto land = [&](int buf, const Regs& R) {
     uint16_t* st = smem + buf * L::STAGE;
+    if constexpr (MASK != 0) keep[buf] = __ballot(R.m != 0);
 #pragma unroll
     for (int u = 0; u < UPT; ++u) {
       const int unit = tid + NT * u;
@@ -720,6 +798,14 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(
       // MASKED: key = key0 + 4 hf + off, off = 32 mt + 8 (r / 4) + r % 4 a
       // constant per register, visible iff off <= lim
       const int lim = (CAUSAL ? min(qi, S - 1) : S - 1) - key0 - 4 * hf;
+      // with a key mask: bit `off` of this word
+      uint64_t vis = 0;
+      if constexpr (MASKED && MASK != 0) {
+        auto upto = [](int l) { return l < 0 ? 0ull : l >= 63 ? ~0ull : (2ull << l) - 1; };
+        const uint64_t kw = keep[buf] >> (4 * hf);
+        if constexpr (MASK == 1) vis = kw & upto(lim);
+        else vis = (~kw | ~upto(qi - key0 - 4 * hf)) & upto(lim);
+      }
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) { st[mt] = zero16(); dp[mt] = zero16(); }
 #pragma unroll
@@ -735,23 +821,37 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           float p = __builtin_amdgcn_exp2f(fmaf(st[mt][r], scale_log2, -l2));
-          if constexpr (MASKED)  // keys past S, and after the query when causal: P = 0
+          if constexpr (MASKED && MASK != 0)
+            p = (vis >> (32 * mt + 8 * (r >> 2) + (r & 3))) & 1 ? p : 0.f;
+          else if constexpr (MASKED)  // keys past S, and after the query when causal: P = 0
             p = 32 * mt + 8 * (r >> 2) + (r & 3) <= lim ? p : 0.f;
           dp[mt][r] = p * (dp[mt][r] - dd);
         }
 #pragma unroll
       for (int c = 0; c < 2 * MT; ++c) {
         const uint4 sb = pack_c8(dp[c >> 1], 8 * (c & 1));
+        uint4 sl;
+        if constexpr (NP == 2) sl = pack_c8_lo(dp[c >> 1], 8 * (c & 1), sb);
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-          acc[dt] = mfma(lds_a_perm(Kt, 32 * dt + n, L::TP, c, hf), sb, acc[dt]);
+        for (int dt = 0; dt < DT; ++dt) {
+          const uint4 ak = lds_a_perm(Kt, 32 * dt + n, L::TP, c, hf);
+          acc[dt] = mfma(ak, sb, acc[dt]);
+          if constexpr (NP == 2) acc[dt] = mfma(ak, sl, acc[dt]);
+        }
       }
     }
   };
   auto compute = [&](int kt, int buf) {
     const int key0 = BN * kt;
     if (!active || key0 > my_last) return;
-    if (key0 + BN > S || (CAUSAL && key0 + BN - 1 > q0)) tile(std::true_type{}, key0, buf);
+    if constexpr (MASK == 1) {
+      if (keep[buf] == 0) return;  // a tile of padding
+      if (keep[buf] != ~0ull) {
+        tile(std::true_type{}, key0, buf);
+        return;
+      }
+    }
+    if (MASK == 2 || key0 + BN > S || (CAUSAL && key0 + BN - 1 > q0)) tile(std::true_type{}, key0, buf);
     else tile(std::false_type{}, key0, buf);
   };
 
@@ -765,7 +865,7 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(
   // before S, so every active wave takes the unmasked code there, in a loop
   // of its own (kt_u even keeps the two-step pipeline aligned).
   const int q0_first = 32 * ((NW * item) / G);
-  const int kt_u = (CAUSAL ? min((q0_first + 1) / BN, S / BN) : S / BN) & ~1;
+  const int kt_u = MASK != 0 ? 0 : (CAUSAL ? min((q0_first + 1) / BN, S / BN) : S / BN) & ~1;
   int kt = 0;
   for (; kt < last && kt + 1 < kt_u; kt += 2) {
     fetch(min(kt + 2, last), ra);
@@ -794,7 +894,7 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < JT; ++j) {
         const int d = 32 * dt + 8 * j + 4 * hf;
         const f32x16_t& a = acc[dt];
         *reinterpret_cast<uint2*>(orow + d) =
@@ -991,7 +1091,7 @@ DkdvPlan plan_dkdv(int hd, int S, int G, int BHkv, bool causal) {
   DkdvPlan p{};
   // two head groups at head_dim 128 spill 631 registers to scratch; one
   // runs that backward 1.75-2.2x faster
-  p.HG = G % 2 == 0 && hd <= 64 ? 2 : 1;
+  p.HG = G % 2 == 0 && (hd == 32 || hd == 64) ? 2 : 1;
   p.KB = 4;
   const int nkg = (S + 32 * p.KB - 1) / (32 * p.KB), nqt = (S + 31) / 32;
   p.ch = nqt;
@@ -1064,8 +1164,11 @@ struct SideStream {
   }
 };
 
-template <int HD, bool CAUSAL>
+template <int HD, bool CAUSAL, int MASK>
 int launch_mfma(const BwdArgs& a, const float* dvec, const float* lse2, float* part) {
+  // Planes of P and dS: head_dim 16 and masked calls keep them to ~16 bits
+  // (two bf16 planes), the others round them to bf16.
+  constexpr int NP = HD == 16 || MASK != 0 ? 2 : 1;
   const float sl2 = a.scale * kLog2e;
   const int BHkv = a.B * a.Hkv, G = a.Hq / a.Hkv;
   const bf16* q = static_cast<const bf16*>(a.q);
@@ -1084,8 +1187,8 @@ int launch_mfma(const BwdArgs& a, const float* dvec, const float* lse2, float* p
     constexpr int NW = kDqWaves;
     const int ntasks = ((a.S + 31) / 32) * G;
     const int items = (ntasks + NW - 1) / NW;
-    attn_bwd_dq_kernel<HD, CAUSAL, NW><<<dim3(static_cast<unsigned>(items * BHkv)), 64 * NW, 0, dq_st>>>(
-        q, k, v, d, dvec, lse2, static_cast<bf16*>(a.dq), a.Hq, a.Hkv, a.S, G, ntasks, items,
+    attn_bwd_dq_kernel<HD, CAUSAL, NW, MASK, NP><<<dim3(static_cast<unsigned>(items * BHkv)), 64 * NW, 0, dq_st>>>(
+        q, k, v, d, dvec, lse2, a.kmask, static_cast<bf16*>(a.dq), a.Hq, a.Hkv, a.S, G, ntasks, items,
         a.qs[0], a.qs[1], a.qs[2], a.ks[0], a.ks[1], a.ks[2], a.vs[0], a.vs[1], a.vs[2], a.dos[0],
         a.dos[1], a.dos[2], a.dqs[0], a.dqs[1], a.dqs[2], sl2, a.scale);
     return check_launch("attn_bwd: dq");
@@ -1094,8 +1197,8 @@ int launch_mfma(const BwdArgs& a, const float* dvec, const float* lse2, float* p
     const DkdvPlan pl = plan_dkdv(HD, a.S, G, BHkv, CAUSAL);
     const dim3 grid(static_cast<unsigned>(pl.nwg * BHkv));
 #define HYDRA_DKDV(KBV, HGV)                                                                     \
-  attn_bwd_dkdv_kernel<HD, CAUSAL, KBV, HGV><<<grid, 64 * KBV * HGV, 0, a.st>>>(                 \
-      q, k, v, d, dvec, lse2, static_cast<bf16*>(a.dk), static_cast<bf16*>(a.dv), part, a.Hq,   \
+  attn_bwd_dkdv_kernel<HD, CAUSAL, KBV, HGV, MASK, NP><<<grid, 64 * KBV * HGV, 0, a.st>>>(       \
+      q, k, v, d, dvec, lse2, a.kmask, static_cast<bf16*>(a.dk), static_cast<bf16*>(a.dv), part, a.Hq, \
       a.Hkv, a.S, G, pl.nwg, pl.ch, pl.maxch, a.qs[0], a.qs[1], a.qs[2], a.ks[0], a.ks[1],      \
       a.ks[2], a.vs[0], a.vs[1], a.vs[2], a.dos[0], a.dos[1], a.dos[2], a.dks[0], a.dks[1],     \
       a.dks[2], a.dvs[0], a.dvs[1], a.dvs[2], sl2, a.scale);                                     \
@@ -1109,7 +1212,7 @@ int launch_mfma(const BwdArgs& a, const float* dvec, const float* lse2, float* p
             pl.maxch, a.dks[0], a.dks[1], a.dks[2], a.dvs[0], a.dvs[1], a.dvs[2], a.scale);      \
     if (int rc = check_launch("attn_bwd: dkdv reduce")) return rc;                              \
   }
-    if constexpr (HD <= 64) {
+    if constexpr (HD == 32 || HD == 64) {
       if (pl.HG == 2) {
         HYDRA_DKDV(4, 2)
       }
@@ -1172,8 +1275,12 @@ int run_generic(const BwdArgs& a, float* dvec, float* lse2) {
 template <int HD>
 int run_mfma(const BwdArgs& a, float* dvec, float* lse2, float* part) {
   if (int rc = launch_rowdot<bf16>(a, dvec, lse2)) return rc;
-  return a.causal ? launch_mfma<HD, true>(a, dvec, lse2, part)
-                  : launch_mfma<HD, false>(a, dvec, lse2, part);
+  if (a.mask_mode == HYDRA_MASK_REFERENCE_SDPA) return launch_mfma<HD, false, 2>(a, dvec, lse2, part);
+  if (a.mask_mode == HYDRA_MASK_KEY_PADDING)
+    return a.causal ? launch_mfma<HD, true, 1>(a, dvec, lse2, part)
+                    : launch_mfma<HD, false, 1>(a, dvec, lse2, part);
+  return a.causal ? launch_mfma<HD, true, 0>(a, dvec, lse2, part)
+                  : launch_mfma<HD, false, 0>(a, dvec, lse2, part);
 }
 
 }  // namespace
@@ -1221,8 +1328,7 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
                   static_cast<int>(Hq), static_cast<int>(Hkv), static_cast<int>(S),
                   static_cast<int>(hd), qs, ks, vs, os, gos, gqs, gks, gvs, causal != 0, scale,
                   st, mask_mode != HYDRA_MASK_NONE ? key_mask : nullptr, mask_mode};
-  // a key mask takes the VALU kernels
-  bool mfma_ok = dtype == HYDRA_BF16 && (hd == 32 || hd == 64 || hd == 128) && mask_mode == HYDRA_MASK_NONE;
+  bool mfma_ok = dtype == HYDRA_BF16 && (hd == 16 || hd == 32 || hd == 64 || hd == 128);
   // Tiles are addressed with 32-bit byte offsets within one head's rows
   // (up to 64 rows past S).
   for (const int64_t* s : {qs, ks, vs, gos, gqs, gks, gvs})
@@ -1236,7 +1342,8 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
   const size_t rows_bytes = (static_cast<size_t>(rows) * 2 * sizeof(float) + 255) & ~size_t(255);
   const size_t part_bytes =
       mfma_ok ? plan_dkdv(static_cast<int>(hd), static_cast<int>(S), static_cast<int>(Hq / Hkv),
-                          static_cast<int>(B * Hkv), causal != 0).part_bytes
+                          static_cast<int>(B * Hkv), causal != 0 && mask_mode != HYDRA_MASK_REFERENCE_SDPA)
+                    .part_bytes
               : 0;
   if (need) {
     *need = rows_bytes + part_bytes;
@@ -1251,6 +1358,7 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
   float* part = reinterpret_cast<float*>(static_cast<char*>(ws) + rows_bytes);
   if (mfma_ok) {
     switch (hd) {
+      case 16: return run_mfma<16>(a, dvec, lse2, part);
       case 32: return run_mfma<32>(a, dvec, lse2, part);
       case 64: return run_mfma<64>(a, dvec, lse2, part);
       default: return run_mfma<128>(a, dvec, lse2, part);
