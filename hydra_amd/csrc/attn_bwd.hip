@@ -39,8 +39,10 @@
 // B8 4/1 heads x 64, S 777, padded: 101.4 ms -> below 0.1; B2 28/4 heads x
 // 16, S 2048, causal: 60 ms -> below 0.3 (whole layer steps 102.5 -> 1.41
 // and 61.3 -> 1.40 ms, what remains is the rest of the layer).
-// Generic path (attn_bwd_generic_*): one thread per query / key row, fp32
-// math, any element type, head_dim <= 256.
+// Other element types, head dims and strides: attn_f32.hip (fp32 matrix
+// instructions) up to head_dim 128, above it attn_bwd_generic_* (one thread
+// per query / key row, fp32 math, head_dim <= 256).
+#include "attn_f32.h"
 #include "common.h"
 
 #include <algorithm>
@@ -1254,22 +1256,19 @@ int launch_generic(const BwdArgs& a, const float* dvec, const float* lse2) {
   return check_launch("attn_bwd: generic dq");
 }
 
-template <typename T, bool CAUSAL, int MASK>
-int launch_generic_d(const BwdArgs& a, const float* dvec, const float* lse2) {
-  if (a.hd <= 32) return launch_generic<T, 32, CAUSAL, MASK>(a, dvec, lse2);
-  if (a.hd <= 64) return launch_generic<T, 64, CAUSAL, MASK>(a, dvec, lse2);
-  if (a.hd <= 128) return launch_generic<T, 128, CAUSAL, MASK>(a, dvec, lse2);
-  return launch_generic<T, 256, CAUSAL, MASK>(a, dvec, lse2);
-}
-
 template <typename T>
-int run_generic(const BwdArgs& a, float* dvec, float* lse2) {
+int run_other(const BwdArgs& a, int dtype, float* dvec, float* lse2, float* part, size_t part_bytes) {
   if (int rc = launch_rowdot<T>(a, dvec, lse2)) return rc;
-  if (a.mask_mode == HYDRA_MASK_REFERENCE_SDPA) return launch_generic_d<T, true, 2>(a, dvec, lse2);
+  if (a.hd <= kAttnF32MaxHd)
+    return attn_bwd_f32(AttnF32Args{a.q, a.k, a.v, a.dout, nullptr, a.dq, a.dk, a.dv, nullptr, dvec, lse2, a.kmask,
+                                    a.mask_mode, a.B, a.Hq, a.Hkv, a.S, a.hd, a.qs, a.ks, a.vs, a.os, a.dos, a.dqs,
+                                    a.dks, a.dvs, a.causal, a.scale, dtype, a.st},
+                        part, part_bytes);
+  if (a.mask_mode == HYDRA_MASK_REFERENCE_SDPA) return launch_generic<T, 256, true, 2>(a, dvec, lse2);
   if (a.mask_mode == HYDRA_MASK_KEY_PADDING)
-    return a.causal ? launch_generic_d<T, true, 1>(a, dvec, lse2) : launch_generic_d<T, false, 1>(a, dvec, lse2);
-  return a.causal ? launch_generic_d<T, true, 0>(a, dvec, lse2)
-                  : launch_generic_d<T, false, 0>(a, dvec, lse2);
+    return a.causal ? launch_generic<T, 256, true, 1>(a, dvec, lse2) : launch_generic<T, 256, false, 1>(a, dvec, lse2);
+  return a.causal ? launch_generic<T, 256, true, 0>(a, dvec, lse2)
+                  : launch_generic<T, 256, false, 0>(a, dvec, lse2);
 }
 
 template <int HD>
@@ -1328,23 +1327,28 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
                   static_cast<int>(Hq), static_cast<int>(Hkv), static_cast<int>(S),
                   static_cast<int>(hd), qs, ks, vs, os, gos, gqs, gks, gvs, causal != 0, scale,
                   st, mask_mode != HYDRA_MASK_NONE ? key_mask : nullptr, mask_mode};
-  bool mfma_ok = dtype == HYDRA_BF16 && (hd == 16 || hd == 32 || hd == 64 || hd == 128);
+  bool mfma_shape = dtype == HYDRA_BF16 && (hd == 16 || hd == 32 || hd == 64 || hd == 128);
   // Tiles are addressed with 32-bit byte offsets within one head's rows
   // (up to 64 rows past S).
   for (const int64_t* s : {qs, ks, vs, gos, gqs, gks, gvs})
-    mfma_ok = mfma_ok && s[0] % 8 == 0 && s[1] % 8 == 0 && s[2] % 8 == 0 && s[2] >= hd &&
+    mfma_shape = mfma_shape && s[0] % 8 == 0 && s[1] % 8 == 0 && s[2] % 8 == 0 && s[2] >= hd &&
               (S + 64) * s[2] * 2 < (int64_t(1) << 31);
+  bool mfma_ok = mfma_shape;
   if (!need)
     for (const void* p : {q, k, v, grad_o, static_cast<const void*>(grad_q),
                           static_cast<const void*>(grad_k), static_cast<const void*>(grad_v)})
       mfma_ok = mfma_ok && aligned16(p);
-  // Workspace: D and lse2 per query row, then the dK/dV chunk partials.
+  // Workspace: D and lse2 per query row, then the chunk partials.  Its size
+  // follows from the shapes alone (the query sees no pointers).
   const size_t rows_bytes = (static_cast<size_t>(rows) * 2 * sizeof(float) + 255) & ~size_t(255);
   const size_t part_bytes =
-      mfma_ok ? plan_dkdv(static_cast<int>(hd), static_cast<int>(S), static_cast<int>(Hq / Hkv),
+      mfma_shape ? plan_dkdv(static_cast<int>(hd), static_cast<int>(S), static_cast<int>(Hq / Hkv),
                           static_cast<int>(B * Hkv), causal != 0 && mask_mode != HYDRA_MASK_REFERENCE_SDPA)
                     .part_bytes
-              : 0;
+      : hd <= kAttnF32MaxHd
+          ? attn_bwd_f32_workspace(static_cast<int>(B), static_cast<int>(Hq), static_cast<int>(Hkv),
+                                   static_cast<int>(S), static_cast<int>(hd), causal != 0, mask_mode)
+          : 0;
   if (need) {
     *need = rows_bytes + part_bytes;
     return HYDRA_OK;
@@ -1356,6 +1360,7 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
   float* dvec = static_cast<float*>(ws);
   float* lse2 = dvec + rows;
   float* part = reinterpret_cast<float*>(static_cast<char*>(ws) + rows_bytes);
+  const size_t room = static_cast<size_t>(workspace_bytes) - rows_bytes;
   if (mfma_ok) {
     switch (hd) {
       case 16: return run_mfma<16>(a, dvec, lse2, part);
@@ -1365,9 +1370,9 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
     }
   }
   switch (dtype) {
-    case HYDRA_F32: return run_generic<float>(a, dvec, lse2);
-    case HYDRA_BF16: return run_generic<bf16>(a, dvec, lse2);
-    default: return run_generic<f16>(a, dvec, lse2);
+    case HYDRA_F32: return run_other<float>(a, dtype, dvec, lse2, part, room);
+    case HYDRA_BF16: return run_other<bf16>(a, dtype, dvec, lse2, part, room);
+    default: return run_other<f16>(a, dtype, dvec, lse2, part, room);
   }
 }
 

@@ -1,0 +1,716 @@
+// Attention in fp32 arithmetic on v_mfma_f32_16x16x4_f32, for any element
+// type, any strides, head_dim up to 128: o = softmax(scale * q k^T [+ masks]) v
+// and its gradients, with the semantics of attn_fwd.hip and attn_bwd.hip
+// (reference: fused_attention.py:14-110, 113-338, 706-823 and the masked SDPA
+// call attention.py:268-299).  fp32 and fp16 calls run here, and bf16 calls
+// whose head_dim or strides the bf16 MFMA kernels do not take.  Products and
+// sums are fp32 throughout, so results are as exact as one thread's fp32 sums.
+//
+// What bounds it: the fp32 matrix rate (256 FLOP per CU and cycle, a tenth of
+// bf16's measured rate); a 16x16x4 step takes 32 cycles of a SIMD, against one
+// 4-byte LDS read per lane, so LDS and the softmax's VALU work hide behind it.
+// The 16x16 tile (and not 32x32x2) because a wave then holds 16 rows: K and V
+// (or Q and dO) fragments and both accumulators of head_dim 128 fit the
+// registers without spills.
+//
+// Layouts.  A fragment of rows X[m][d] (m = lane % 16, g = lane / 16) takes the
+// summed index d in the order 16 j + 4 g + i over steps (j, i): one 16-byte LDS
+// read feeds four steps, and the resident side holds the same order.  A result
+// tile has row 4 g + r in register r and column lane % 16, so register r is the
+// B operand of the next product with the summed index in the order 4 g + r,
+// whose A operand is one 4-byte read of row 4 g + r of the staged tile: nothing
+// is transposed.  Staged rows are head_dim + 4 words apart, which puts the four
+// row groups of such a read into different banks.
+//
+// Every wave owns 16 rows (queries forward and for dQ, keys for dK/dV); a
+// workgroup's four waves share the staged 32-row tiles of the other side,
+// double-buffered, the next tile's loads in flight during the arithmetic.
+// dK/dV and dQ walks are cut into chunks of equally many tiles so that the
+// launch fills the device; their fp32 partials are summed in chunk order
+// (deterministic).
+//
+// Measured, forward + backward of one call, against what these calls took
+// before (16 lanes per query row forward, one thread per row backward, VALU):
+// fp16 B2 8/2 heads x 64, S 1500, causal 198.1 -> 0.36 ms; fp32 B4 8/2 x 64,
+// S 2048, causal 274 -> 1.21 ms; fp32 B1 4/1 x 128, S 1000 172.9 -> 0.26 ms;
+// fp32 B2 8/2 x 16, S 512, causal 8.7 -> 0.17 ms (launch-bound).  Errors
+// against 64 bits: fp32 1.8e-6 -> 6.9e-7, fp16 2.2e-4 (the output's rounding)
+// both.
+#include "attn_f32.h"
+
+#include <algorithm>
+#include <cmath>
+
+#include "common.h"
+
+namespace hydra {
+namespace {
+
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
+constexpr float kLog2eF = 1.4426950408889634f;
+constexpr float kLn2F = 0.6931471805599453f;
+constexpr int kWaves = 4;
+constexpr int kThreads = 64 * kWaves;
+constexpr int kTile = 32;  // staged rows per step
+
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+struct Strides3 {
+  int64_t b, h, s;
+};
+
+// One operand of the staged side: rows `row0 ..` of `base`, `rs` apart,
+// elements `es` apart; `vec`: 16-byte loads are allowed (hd == HDP, unit
+// element stride, aligned rows).
+template <typename T>
+struct Rows {
+  const T* base;
+  int64_t rs, es;
+};
+
+// Registers of one thread's share of a staged tile, and its way to LDS.
+template <typename T, int HDP>
+struct Stage {
+  static constexpr int P = HDP + 4;                 // words per staged row
+  static constexpr int E = 16 / int(sizeof(T));     // elements per 16-byte load
+  static constexpr int VU = (kTile * HDP / E + kThreads - 1) / kThreads;
+  static constexpr int SU = kTile * HDP / kThreads;  // scalar path: elements per thread
+  static constexpr int WORDS = kTile * P;
+  static constexpr bool WHOLE = (kTile * HDP / E) % kThreads == 0;
+
+  uint4 raw[VU];
+
+  __device__ __forceinline__ void fetch(const Rows<T>& r, int row0, int S) {
+#pragma unroll
+    for (int u = 0; u < VU; ++u) {
+      const int i = threadIdx.x + kThreads * u;
+      const int row = i / (HDP / E), c = i - row * (HDP / E);
+      const bool ok = (WHOLE || row < kTile) && row0 + row < S;
+      raw[u] = ok ? *reinterpret_cast<const uint4*>(r.base + static_cast<int64_t>(row0 + row) * r.rs + c * E)
+                  : make_uint4(0, 0, 0, 0);
+    }
+  }
+  __device__ __forceinline__ void land(float* dst) const {
+#pragma unroll
+    for (int u = 0; u < VU; ++u) {
+      const int i = threadIdx.x + kThreads * u;
+      const int row = i / (HDP / E), c = i - row * (HDP / E);
+      if (WHOLE || row < kTile) {
+        float f[E];
+        unpack16<T>(raw[u], f);
+#pragma unroll
+        for (int e = 0; e < E; e += 4)
+          *reinterpret_cast<float4*>(&dst[row * P + c * E + e]) = make_float4(f[e], f[e + 1], f[e + 2], f[e + 3]);
+      }
+    }
+  }
+  // Any strides and head_dim: element by element, straight to LDS.
+  static __device__ __forceinline__ void direct(const Rows<T>& r, int row0, int S, int hd, float* dst) {
+#pragma unroll 4
+    for (int u = 0; u < SU; ++u) {
+      const int i = threadIdx.x + kThreads * u;
+      const int row = i / HDP, d = i - row * HDP;
+      const bool ok = row0 + row < S && d < hd;
+      dst[row * P + d] = ok ? to_f32(r.base[static_cast<int64_t>(row0 + row) * r.rs + d * r.es]) : 0.f;
+    }
+  }
+};
+
+// The resident fragment of one row (column lane % 16 of B): elements
+// 16 j + 4 g + i of the row, zero past hd or for a row that is not there.
+template <typename T, int HDP>
+__device__ __forceinline__ void load_frag(float (&f)[HDP / 16][4], const T* row, int64_t es, int g, int hd, bool ok) {
+#pragma unroll
+  for (int j = 0; j < HDP / 16; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int d = 16 * j + 4 * g + i;
+      f[j][i] = ok && d < hd ? to_f32(row[d * es]) : 0.f;
+    }
+}
+
+// S and dP tiles (or S alone): rows of two staged operands times the
+// resident fragments.
+template <int HDP>
+__device__ __forceinline__ f32x4 row_product(const float* rows, const float (&f)[HDP / 16][4], int n, int g) {
+  f32x4 c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < HDP / 16; ++j) {
+    const float4 a = *reinterpret_cast<const float4*>(&rows[n * (HDP + 4) + 16 * j + 4 * g]);
+    c = mfma4(a.x, f[j][0], c);
+    c = mfma4(a.y, f[j][1], c);
+    c = mfma4(a.z, f[j][2], c);
+    c = mfma4(a.w, f[j][3], c);
+  }
+  return c;
+}
+
+// acc[d tile] += rows^T * x: x a result tile whose rows are 16 staged rows.
+template <int HDP>
+__device__ __forceinline__ void col_product(f32x4 (&acc)[HDP / 16], const float* rows, const f32x4& x, int n, int g) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int t = 0; t < HDP / 16; ++t) acc[t] = mfma4(rows[(4 * g + r) * (HDP + 4) + 16 * t + n], x[r], acc[t]);
+}
+
+// Writes a wave's 16 rows (column n) of accumulators, scaled.
+template <typename T, int HDP>
+__device__ __forceinline__ void store_rows(T* row, const f32x4 (&acc)[HDP / 16], float scale, int g, int hd) {
+#pragma unroll
+  for (int t = 0; t < HDP / 16; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int d = 16 * t + 4 * g + r;
+      if (d < hd) row[d] = from_f32<T>(acc[t][r] * scale);
+    }
+}
+template <int HDP>
+__device__ __forceinline__ void store_part(float* row, const f32x4 (&acc)[HDP / 16], int g) {
+#pragma unroll
+  for (int t = 0; t < HDP / 16; ++t)
+    *reinterpret_cast<float4*>(row + 16 * t + 4 * g) = make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
+}
+
+// Whether query s sees key t < S (keep: the key mask's flag of t).
+__device__ __forceinline__ bool sees(int s, int t, bool keep, bool causal, int mode) {
+  if (mode == HYDRA_MASK_REFERENCE_SDPA) return t > s || !keep;
+  return (!causal || t <= s) && (mode != HYDRA_MASK_KEY_PADDING || keep);
+}
+
+// Queries of a wave: task (16 rows of one query head of the group) of an
+// item of kWaves tasks, the group's heads first so that a workgroup's waves
+// share the key range.
+struct Task {
+  int h, q0;
+  bool active;
+};
+__device__ __forceinline__ Task task_of(int task, int ntasks, int kvh, int G) {
+  Task t;
+  t.active = task < ntasks;
+  const int c = t.active ? task : ntasks - 1;
+  t.q0 = 16 * (c / G);
+  t.h = kvh * G + c % G;
+  return t;
+}
+
+// ---------------------------------------------------------------- forward
+template <typename T, int HDP>
+__global__ __launch_bounds__(kThreads) void attn_fwd_f32_kernel(
+    const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, T* __restrict__ o,
+    float* __restrict__ lse, const uint8_t* __restrict__ kmask, int mode, int Hq, int Hkv, int S, int hd, int G,
+    int ntasks, int items, Strides3 qs, Strides3 ks, Strides3 vs, int64_t vs3, Strides3 os, int causal, int vec,
+    float scale_log2) {
+  using St = Stage<T, HDP>;
+  __shared__ __attribute__((aligned(16))) float smem[2][2 * St::WORDS];
+  __shared__ int keepv[2][kTile];
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int BHkv = gridDim.x / items;
+  const int bk = blockIdx.x % BHkv;
+  const int item = items - 1 - static_cast<int>(blockIdx.x / BHkv);  // longest key ranges first
+  const int b = bk / Hkv, kvh = bk - b * Hkv;
+  const Task tk = task_of(kWaves * item + wave, ntasks, kvh, G);
+  const int qi = tk.q0 + n;
+  const bool qok = tk.active && qi < S;
+  float qf[HDP / 16][4];
+  load_frag<T, HDP>(qf, q + b * qs.b + tk.h * qs.h + static_cast<int64_t>(qok ? qi : 0) * qs.s, 1, g, hd, qok);
+
+  const bool walk = causal && mode != HYDRA_MASK_REFERENCE_SDPA;
+  const int last_task = min(kWaves * item + kWaves - 1, ntasks - 1);
+  const int kend = walk ? min(16 * (last_task / G) + 16, S) : S;
+  const int nt = (kend + kTile - 1) / kTile;
+  const int my_end = !tk.active ? 0 : walk ? min(tk.q0 + 16, S) : S;  // keys this wave sees
+  const Rows<T> kr{k + b * ks.b + kvh * ks.h, ks.s, 1};
+  const Rows<T> vr{v + b * vs.b + kvh * vs.h, vs.s, vs3};
+
+  f32x4 acc[HDP / 16];
+#pragma unroll
+  for (int t = 0; t < HDP / 16; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+  St sk, sv;
+  int kp = 0;
+  auto fetch = [&](int t) {
+    if (vec) {
+      sk.fetch(kr, kTile * t, S);
+      sv.fetch(vr, kTile * t, S);
+    }
+    if (mode != HYDRA_MASK_NONE && tid < kTile) {
+      const int key = kTile * t + tid;
+      kp = key < S ? kmask[static_cast<int64_t>(b) * S + key] : 0;
+    }
+  };
+  auto land = [&](int t, int buf) {
+    if (vec) {
+      sk.land(smem[buf]);
+      sv.land(smem[buf] + St::WORDS);
+    } else {
+      St::direct(kr, kTile * t, S, hd, smem[buf]);
+      St::direct(vr, kTile * t, S, hd, smem[buf] + St::WORDS);
+    }
+    if (mode != HYDRA_MASK_NONE && tid < kTile) keepv[buf][tid] = kp;
+  };
+  fetch(0);
+  land(0, 0);
+  for (int t = 0; t < nt; ++t) {
+    __syncthreads();
+    const int buf = t & 1, t0 = kTile * t;
+    if (t + 1 < nt) fetch(t + 1);
+    if (t0 < my_end) {
+      const float* Ks = smem[buf];
+      const float* Vs = Ks + St::WORDS;
+      f32x4 x[2];
+      float mt = m;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) x[u] = row_product<HDP>(Ks + 16 * u * St::P, qf, n, g);
+      // whole tile visible to every row of the wave: no tests
+      const bool plain = mode == HYDRA_MASK_NONE && t0 + kTile - 1 <= (walk ? tk.q0 : S - 1) && t0 + kTile <= S;
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float xs = x[u][r] * scale_log2;
+          if (!plain) {
+            const int i = 16 * u + 4 * g + r, key = t0 + i;
+            const bool keep = mode == HYDRA_MASK_NONE || keepv[buf][i] != 0;
+            if (!(key < S && sees(qi, key, keep, causal, mode))) xs = -INFINITY;
+          }
+          x[u][r] = xs;
+          mt = fmaxf(mt, xs);
+        }
+      mt = fmaxf(mt, __shfl_xor(mt, 16));
+      mt = fmaxf(mt, __shfl_xor(mt, 32));
+      const float ms = mt == -INFINITY ? 0.f : mt;  // nothing visible yet: every p is exp2(-inf) = 0
+      if (__any(mt > m)) {
+        const float alpha = __builtin_amdgcn_exp2f(m - ms);  // m = -inf -> 0
+        l *= alpha;
+#pragma unroll
+        for (int d = 0; d < HDP / 16; ++d) acc[d] *= alpha;
+        m = mt;
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          x[u][r] = __builtin_amdgcn_exp2f(x[u][r] - ms);
+          l += x[u][r];
+        }
+        col_product<HDP>(acc, Vs + 16 * u * St::P, x[u], n, g);
+      }
+    }
+    if (t + 1 < nt) land(t + 1, buf ^ 1);
+  }
+  l += __shfl_xor(l, 16);
+  l += __shfl_xor(l, 32);
+  if (!qok) return;
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  store_rows<T, HDP>(o + b * os.b + tk.h * os.h + static_cast<int64_t>(qi) * os.s, acc, inv, g, hd);
+  if (lse && g == 0)
+    lse[(static_cast<int64_t>(b) * Hq + tk.h) * S + qi] = l > 0.f ? (m + __log2f(l)) * kLn2F : -INFINITY;
+}
+
+// --------------------------------------------------------------- backward
+// Tiles of 32 queries that reach key group kg (64 keys), per query head.
+__host__ __device__ inline int q_tiles(int kg, int S, bool walk) {
+  const int all = (S + kTile - 1) / kTile;
+  return walk ? all - 2 * kg : all;
+}
+
+// dK/dV: grid (chunk, key group, batch x kv head), the chunk fastest.
+template <typename T, int HDP>
+__global__ __launch_bounds__(kThreads) void attn_bwd_f32_dkdv_kernel(
+    const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, const T* __restrict__ dout,
+    const float* __restrict__ dvec, const float* __restrict__ lse2, const uint8_t* __restrict__ kmask, int mode,
+    T* __restrict__ dk, T* __restrict__ dv, float* __restrict__ part, int Hq, int Hkv, int S, int hd, int G,
+    int nkg, int ch, int maxch, Strides3 qs, Strides3 ks, Strides3 vs, Strides3 ds, Strides3 dks, Strides3 dvs,
+    int causal, int vec, float scale_log2, float scale) {
+  using St = Stage<T, HDP>;
+  __shared__ __attribute__((aligned(16))) float smem[2][2 * St::WORDS];
+  __shared__ __attribute__((aligned(16))) float rowv[2][2][kTile];  // lse2 and D of the tile's rows
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = blockIdx.x % maxch, rest = blockIdx.x / maxch;
+  const int kg = rest % nkg, bk = rest / nkg;
+  const int b = bk / Hkv, kvh = bk - b * Hkv;
+  const bool walk = causal && mode != HYDRA_MASK_REFERENCE_SDPA;
+  const int qt0 = walk ? 2 * kg : 0;
+  const int nq = q_tiles(kg, S, walk);
+  const int total = G * nq;
+  if (c * ch >= total) return;
+  const int kw0 = 64 * kg + 16 * wave, key = kw0 + n;
+  bool keep = key < S;
+  if (mode != HYDRA_MASK_NONE && keep) keep = kmask[static_cast<int64_t>(b) * S + key] != 0;
+  // Key padding: a lane's key is its own column of every product, so masked
+  // lanes store zeros at the end and waves without a key that counts rest.
+  const bool pad = mode == HYDRA_MASK_KEY_PADDING;
+  const bool wave_any = !pad || __builtin_amdgcn_readfirstlane(__any(keep)) != 0;
+  const bool wg_any = !pad || __syncthreads_or(keep) != 0;
+  const int kbnd = mode == HYDRA_MASK_REFERENCE_SDPA && !keep ? 0x7fffffff : key;
+
+  float kf[HDP / 16][4], vf[HDP / 16][4];
+  load_frag<T, HDP>(kf, k + b * ks.b + kvh * ks.h + static_cast<int64_t>(key < S ? key : 0) * ks.s, 1, g, hd, key < S);
+  load_frag<T, HDP>(vf, v + b * vs.b + kvh * vs.h + static_cast<int64_t>(key < S ? key : 0) * vs.s, 1, g, hd, key < S);
+  f32x4 dka[HDP / 16], dva[HDP / 16];
+#pragma unroll
+  for (int t = 0; t < HDP / 16; ++t) dka[t] = dva[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  St sq, sd;
+  float rv = 0.f;
+  auto fetch = [&](int step) {
+    const int hr = step / nq, row0 = kTile * (qt0 + step - hr * nq), h = kvh * G + hr;
+    if (vec) {
+      sq.fetch(Rows<T>{q + b * qs.b + h * qs.h, qs.s, 1}, row0, S);
+      sd.fetch(Rows<T>{dout + b * ds.b + h * ds.h, ds.s, 1}, row0, S);
+    }
+    if (tid < 2 * kTile) {  // rows past S: zero, with zero Q and dO they add nothing
+      const int row = row0 + (tid & (kTile - 1));
+      const float* src = tid < kTile ? lse2 : dvec;
+      rv = row < S ? src[(static_cast<int64_t>(b) * Hq + h) * S + row] : 0.f;
+    }
+  };
+  auto land = [&](int step, int buf) {
+    if (vec) {
+      sq.land(smem[buf]);
+      sd.land(smem[buf] + St::WORDS);
+    } else {
+      const int hr = step / nq, row0 = kTile * (qt0 + step - hr * nq), h = kvh * G + hr;
+      St::direct(Rows<T>{q + b * qs.b + h * qs.h, qs.s, 1}, row0, S, hd, smem[buf]);
+      St::direct(Rows<T>{dout + b * ds.b + h * ds.h, ds.s, 1}, row0, S, hd, smem[buf] + St::WORDS);
+    }
+    if (tid < 2 * kTile) rowv[buf][tid / kTile][tid & (kTile - 1)] = rv;
+  };
+  const int first = c * ch, end = wg_any ? min(first + ch, total) : first;
+  if (first < end) {
+    fetch(first);
+    land(first, 0);
+  }
+  for (int step = first; step < end; ++step) {
+    __syncthreads();
+    const int buf = (step - first) & 1;
+    if (step + 1 < end) fetch(step + 1);
+    const int q0 = kTile * (qt0 + step % nq);
+    // causal: a tile before the wave's keys holds nothing of theirs
+    if (wave_any && (!walk || q0 + kTile - 1 >= kw0)) {
+      const bool plain = walk ? q0 >= kw0 + 15 : mode != HYDRA_MASK_REFERENCE_SDPA;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const float* Qs = smem[buf] + 16 * u * St::P;
+        const float* Ds = Qs + St::WORDS;
+        f32x4 p = row_product<HDP>(Qs, kf, n, g), dp = row_product<HDP>(Ds, vf, n, g);
+        const float4 l4 = *reinterpret_cast<const float4*>(&rowv[buf][0][16 * u + 4 * g]);
+        const float4 d4 = *reinterpret_cast<const float4*>(&rowv[buf][1][16 * u + 4 * g]);
+        const float lr[4] = {l4.x, l4.y, l4.z, l4.w}, dr[4] = {d4.x, d4.y, d4.z, d4.w};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float e = __builtin_amdgcn_exp2f(fmaf(p[r], scale_log2, -lr[r]));
+          if (!plain) {
+            const int s = q0 + 16 * u + 4 * g + r;
+            const bool see = mode == HYDRA_MASK_REFERENCE_SDPA ? s < kbnd : key <= s;
+            e = see ? e : 0.f;
+          }
+          p[r] = e;
+          dp[r] = e * (dp[r] - dr[r]);
+        }
+        col_product<HDP>(dva, Ds, p, n, g);
+        col_product<HDP>(dka, Qs, dp, n, g);
+      }
+    }
+    if (step + 1 < end) land(step + 1, buf ^ 1);
+  }
+  if (pad && !keep) {
+#pragma unroll
+    for (int t = 0; t < HDP / 16; ++t) dka[t] = dva[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  if (maxch > 1) {  // summed by attn_bwd_f32_reduce_kernel
+    const int64_t rows = static_cast<int64_t>(gridDim.x) / maxch * 64;  // of one chunk's partial
+    float* pk = part + ((static_cast<int64_t>(c) * 2) * rows + (static_cast<int64_t>(rest) * 64 + 16 * wave + n)) * HDP;
+    store_part<HDP>(pk, dka, g);
+    store_part<HDP>(pk + rows * HDP, dva, g);
+  } else if (key < S) {
+    store_rows<T, HDP>(dk + b * dks.b + kvh * dks.h + static_cast<int64_t>(key) * dks.s, dka, scale, g, hd);
+    store_rows<T, HDP>(dv + b * dvs.b + kvh * dvs.h + static_cast<int64_t>(key) * dvs.s, dva, 1.f, g, hd);
+  }
+}
+
+// dQ: grid (chunk, item, batch x kv head).
+template <typename T, int HDP>
+__global__ __launch_bounds__(kThreads) void attn_bwd_f32_dq_kernel(
+    const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, const T* __restrict__ dout,
+    const float* __restrict__ dvec, const float* __restrict__ lse2, const uint8_t* __restrict__ kmask, int mode,
+    T* __restrict__ dq, float* __restrict__ part, int Hq, int Hkv, int S, int hd, int G, int ntasks, int items,
+    int ch, int maxch, Strides3 qs, Strides3 ks, Strides3 vs, Strides3 ds, Strides3 dqs, int causal, int vec,
+    float scale_log2, float scale) {
+  using St = Stage<T, HDP>;
+  __shared__ __attribute__((aligned(16))) float smem[2][2 * St::WORDS];
+  __shared__ int keepv[2][kTile];
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = blockIdx.x % maxch, rest = blockIdx.x / maxch;
+  const int item = items - 1 - rest % items, bk = rest / items;
+  const int b = bk / Hkv, kvh = bk - b * Hkv;
+  const bool walk = causal && mode != HYDRA_MASK_REFERENCE_SDPA;
+  const int last_task = min(kWaves * item + kWaves - 1, ntasks - 1);
+  const int kend = walk ? min(16 * (last_task / G) + 16, S) : S;
+  const int nt = (kend + kTile - 1) / kTile;
+  const int first = c * ch, end = min(first + ch, nt);
+  if (first >= nt) return;
+  const Task tk = task_of(kWaves * item + wave, ntasks, kvh, G);
+  const int qi = tk.q0 + n;
+  const bool qok = tk.active && qi < S;
+  const int my_end = !tk.active ? 0 : walk ? min(tk.q0 + 16, S) : S;
+  float qf[HDP / 16][4], of[HDP / 16][4];
+  const int64_t qr = qok ? qi : 0;
+  load_frag<T, HDP>(qf, q + b * qs.b + tk.h * qs.h + qr * qs.s, 1, g, hd, qok);
+  load_frag<T, HDP>(of, dout + b * ds.b + tk.h * ds.h + qr * ds.s, 1, g, hd, qok);
+  float l2 = 0.f, dd = 0.f;
+  if (qok) {
+    const int64_t ri = (static_cast<int64_t>(b) * Hq + tk.h) * S + qi;
+    l2 = lse2[ri];
+    dd = dvec[ri];
+  }
+  f32x4 acc[HDP / 16];
+#pragma unroll
+  for (int t = 0; t < HDP / 16; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const Rows<T> kr{k + b * ks.b + kvh * ks.h, ks.s, 1};
+  const Rows<T> vr{v + b * vs.b + kvh * vs.h, vs.s, 1};
+  St sk, sv;
+  int kp = 0;
+  auto fetch = [&](int t) {
+    if (vec) {
+      sk.fetch(kr, kTile * t, S);
+      sv.fetch(vr, kTile * t, S);
+    }
+    if (mode != HYDRA_MASK_NONE && tid < kTile) {
+      const int key = kTile * t + tid;
+      kp = key < S ? kmask[static_cast<int64_t>(b) * S + key] : 0;
+    }
+  };
+  auto land = [&](int t, int buf) {
+    if (vec) {
+      sk.land(smem[buf]);
+      sv.land(smem[buf] + St::WORDS);
+    } else {
+      St::direct(kr, kTile * t, S, hd, smem[buf]);
+      St::direct(vr, kTile * t, S, hd, smem[buf] + St::WORDS);
+    }
+    if (mode != HYDRA_MASK_NONE && tid < kTile) keepv[buf][tid] = kp;
+  };
+  fetch(first);
+  land(first, 0);
+  for (int t = first; t < end; ++t) {
+    __syncthreads();
+    const int buf = (t - first) & 1, t0 = kTile * t;
+    if (t + 1 < end) fetch(t + 1);
+    if (t0 < my_end) {
+      const bool plain = mode == HYDRA_MASK_NONE && t0 + kTile - 1 <= (walk ? tk.q0 : S - 1) && t0 + kTile <= S;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const float* Ks = smem[buf] + 16 * u * St::P;
+        const float* Vs = Ks + St::WORDS;
+        f32x4 p = row_product<HDP>(Ks, qf, n, g), dp = row_product<HDP>(Vs, of, n, g);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float e = __builtin_amdgcn_exp2f(fmaf(p[r], scale_log2, -l2));
+          if (!plain) {
+            const int i = 16 * u + 4 * g + r, key = t0 + i;
+            const bool keep = mode == HYDRA_MASK_NONE || keepv[buf][i] != 0;
+            e = key < S && sees(qi, key, keep, causal, mode) ? e : 0.f;
+          }
+          dp[r] = e * (dp[r] - dd);
+        }
+        col_product<HDP>(acc, Ks, dp, n, g);
+      }
+    }
+    if (t + 1 < end) land(t + 1, buf ^ 1);
+  }
+  if (maxch > 1) {
+    const int64_t rows = static_cast<int64_t>(gridDim.x) / maxch * 64;
+    store_part<HDP>(part + (static_cast<int64_t>(c) * rows + (static_cast<int64_t>(bk) * items + item) * 64 + 16 * wave + n) * HDP,
+                    acc, g);
+  } else if (qok) {
+    store_rows<T, HDP>(dq + b * dqs.b + tk.h * dqs.h + static_cast<int64_t>(qi) * dqs.s, acc, scale, g, hd);
+  }
+}
+
+// Chunk partials in chunk order -> one gradient row per thread group of
+// HDP / 4 threads.  which: 0 dk, 1 dv, 2 dq (blockIdx.y + first).
+struct ReduceArgs {
+  const float *pkv, *pq;
+  void *dk, *dv, *dq;
+  Strides3 dks, dvs, dqs;
+  int Hq, Hkv, S, hd, G, ntasks, items, nkg, BHkv;
+  int ch_kv, max_kv, ch_q, max_q;
+  int walk;
+  float scale;
+};
+template <typename T, int HDP>
+__global__ __launch_bounds__(256) void attn_bwd_f32_reduce_kernel(ReduceArgs a, int first) {
+  constexpr int TPR = HDP / 4;
+  const int which = first + blockIdx.y;
+  const int64_t i = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) / TPR;
+  const int d = 4 * (threadIdx.x % TPR);
+  const int64_t rows = static_cast<int64_t>(a.BHkv) * (which == 2 ? a.items : a.nkg) * 64;
+  if (i >= rows) return;
+  const int j = static_cast<int>(i / 64), w = static_cast<int>(i % 64);  // tile of 64 rows, row in it
+  T* out;
+  const float* p;
+  int nch;
+  int64_t step;
+  if (which == 2) {
+    const int item = j % a.items, bk = j / a.items, b = bk / a.Hkv, kvh = bk - b * a.Hkv;
+    const int task = kWaves * item + w / 16;
+    if (task >= a.ntasks) return;
+    const int row = 16 * (task / a.G) + w % 16, h = kvh * a.G + task % a.G;
+    if (row >= a.S) return;
+    const int last_task = min(kWaves * item + kWaves - 1, a.ntasks - 1);
+    const int kend = a.walk ? min(16 * (last_task / a.G) + 16, a.S) : a.S;
+    nch = ((kend + kTile - 1) / kTile + a.ch_q - 1) / a.ch_q;
+    p = a.pq + i * HDP + d;
+    step = rows * HDP;
+    out = static_cast<T*>(a.dq) + b * a.dqs.b + h * a.dqs.h + static_cast<int64_t>(row) * a.dqs.s;
+  } else {
+    const int kg = j % a.nkg, bk = j / a.nkg, b = bk / a.Hkv, kvh = bk - b * a.Hkv;
+    const int row = 64 * kg + w;
+    if (row >= a.S) return;
+    nch = (a.G * q_tiles(kg, a.S, a.walk) + a.ch_kv - 1) / a.ch_kv;
+    p = a.pkv + (which * rows + i) * HDP + d;
+    step = 2 * rows * HDP;
+    const Strides3& s = which ? a.dvs : a.dks;
+    out = static_cast<T*>(which ? a.dv : a.dk) + b * s.b + kvh * s.h + static_cast<int64_t>(row) * s.s;
+  }
+  float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int c = 0; c < nch; ++c) {
+    const float4 x = *reinterpret_cast<const float4*>(p + c * step);
+    sum.x += x.x; sum.y += x.y; sum.z += x.z; sum.w += x.w;
+  }
+  const float f = which == 1 ? 1.f : a.scale;
+  const float o[4] = {sum.x * f, sum.y * f, sum.z * f, sum.w * f};
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (d + r < a.hd) out[d + r] = from_f32<T>(o[r]);
+}
+
+// How the walks are cut: chunks of ch tiles, enough of them for kPerCu
+// workgroups on every CU, none shorter than kMinTiles.
+struct Plan {
+  int HDP, G, ntasks, items, nkg, BHkv;
+  int ch_kv, max_kv, ch_q, max_q;
+  size_t kv_floats, q_floats;
+};
+constexpr int kPerCu = 4, kMinTiles = 6;
+
+// split = false: every walk whole (no partials).
+Plan plan_of(int B, int Hq, int Hkv, int S, int hd, bool walk, bool split) {
+  Plan p{};
+  p.HDP = hd <= 16 ? 16 : hd <= 32 ? 32 : hd <= 64 ? 64 : 128;
+  p.G = Hq / Hkv;
+  p.BHkv = B * Hkv;
+  p.ntasks = p.G * ((S + 15) / 16);
+  p.items = (p.ntasks + kWaves - 1) / kWaves;
+  p.nkg = (S + 63) / 64;
+  const int all = (S + kTile - 1) / kTile;
+  auto cut = [&](int64_t tiles, int longest, int* ch, int* nch) {
+    const int64_t want = (tiles + kPerCu * device_cus() - 1) / (kPerCu * device_cus());
+    *ch = split ? static_cast<int>(std::max<int64_t>(want, kMinTiles)) : longest;
+    *nch = (longest + *ch - 1) / *ch;
+  };
+  int64_t tk = 0, tq = 0;
+  for (int g = 0; g < p.nkg; ++g) tk += p.G * q_tiles(g, S, walk);
+  for (int i = 0; i < p.items; ++i) {
+    const int lt = std::min(kWaves * i + kWaves - 1, p.ntasks - 1);
+    tq += ((walk ? std::min(16 * (lt / p.G) + 16, S) : S) + kTile - 1) / kTile;
+  }
+  cut(tk * p.BHkv, p.G * all, &p.ch_kv, &p.max_kv);
+  cut(tq * p.BHkv, all, &p.ch_q, &p.max_q);
+  p.kv_floats = p.max_kv > 1 ? size_t(p.BHkv) * p.nkg * 64 * p.HDP * 2 * p.max_kv : 0;
+  p.q_floats = p.max_q > 1 ? size_t(p.BHkv) * p.items * 64 * p.HDP * p.max_q : 0;
+  return p;
+}
+
+Strides3 s3(const int64_t* s) { return Strides3{s[0], s[1], s[2]}; }
+
+// 16-byte row loads: whole rows of HDP elements, aligned.
+bool vec_ok(const void* p, const int64_t* s, int E) {
+  return aligned16(p) && s[0] % E == 0 && s[1] % E == 0 && s[2] % E == 0 && s[3] == 1;
+}
+
+template <typename T, int HDP>
+int launch_fwd(const AttnF32Args& a) {
+  constexpr int E = 16 / int(sizeof(T));
+  const int G = a.Hq / a.Hkv, ntasks = G * ((a.S + 15) / 16), items = (ntasks + kWaves - 1) / kWaves;
+  const bool vec = a.hd == HDP && vec_ok(a.k, a.ks, E) && vec_ok(a.v, a.vs, E);
+  const int64_t blocks = static_cast<int64_t>(items) * a.B * a.Hkv;
+  if (blocks >= (int64_t(1) << 31)) return fail(HYDRA_ERR_ARG, "attn_fwd: too many rows");
+  attn_fwd_f32_kernel<T, HDP><<<dim3(static_cast<unsigned>(blocks)), kThreads, 0, a.st>>>(
+      static_cast<const T*>(a.q), static_cast<const T*>(a.k), static_cast<const T*>(a.v), static_cast<T*>(a.o),
+      a.lse, a.kmask, a.mask_mode, a.Hq, a.Hkv, a.S, a.hd, G, ntasks, items, s3(a.qs), s3(a.ks), s3(a.vs), a.vs[3],
+      s3(a.os), a.causal ? 1 : 0, vec ? 1 : 0, a.scale * kLog2eF);
+  return check_launch("attn_fwd_f32_kernel");
+}
+
+template <typename T, int HDP>
+int launch_bwd(const AttnF32Args& a, float* part, size_t part_bytes) {
+  constexpr int E = 16 / int(sizeof(T));
+  const bool walk = a.causal && a.mask_mode != HYDRA_MASK_REFERENCE_SDPA;
+  Plan p = plan_of(a.B, a.Hq, a.Hkv, a.S, a.hd, walk, true);
+  if ((p.kv_floats + p.q_floats) * sizeof(float) > part_bytes) p = plan_of(a.B, a.Hq, a.Hkv, a.S, a.hd, walk, false);
+  const bool whole = a.hd == HDP;
+  const float sl2 = a.scale * kLog2eF;
+  const int64_t bkv = static_cast<int64_t>(p.max_kv) * p.nkg * p.BHkv, bq = static_cast<int64_t>(p.max_q) * p.items * p.BHkv;
+  if (bkv >= (int64_t(1) << 31) || bq >= (int64_t(1) << 31)) return fail(HYDRA_ERR_ARG, "attn_bwd: problem too large");
+  const T* q = static_cast<const T*>(a.q);
+  const T* k = static_cast<const T*>(a.k);
+  const T* v = static_cast<const T*>(a.v);
+  const T* d = static_cast<const T*>(a.dout);
+  float* pq = part + p.kv_floats;
+  attn_bwd_f32_dkdv_kernel<T, HDP><<<dim3(static_cast<unsigned>(bkv)), kThreads, 0, a.st>>>(
+      q, k, v, d, a.dvec, a.lse2, a.kmask, a.mask_mode, static_cast<T*>(a.dk), static_cast<T*>(a.dv), part, a.Hq,
+      a.Hkv, a.S, a.hd, p.G, p.nkg, p.ch_kv, p.max_kv, s3(a.qs), s3(a.ks), s3(a.vs), s3(a.dos), s3(a.dks), s3(a.dvs),
+      a.causal ? 1 : 0, whole && vec_ok(a.q, a.qs, E) && vec_ok(a.dout, a.dos, E) ? 1 : 0, sl2, a.scale);
+  if (int rc = check_launch("attn_bwd: f32 dkdv")) return rc;
+  attn_bwd_f32_dq_kernel<T, HDP><<<dim3(static_cast<unsigned>(bq)), kThreads, 0, a.st>>>(
+      q, k, v, d, a.dvec, a.lse2, a.kmask, a.mask_mode, static_cast<T*>(a.dq), pq, a.Hq, a.Hkv, a.S, a.hd, p.G,
+      p.ntasks, p.items, p.ch_q, p.max_q, s3(a.qs), s3(a.ks), s3(a.vs), s3(a.dos), s3(a.dqs), a.causal ? 1 : 0,
+      whole && vec_ok(a.k, a.ks, E) && vec_ok(a.v, a.vs, E) ? 1 : 0, sl2, a.scale);
+  if (int rc = check_launch("attn_bwd: f32 dq")) return rc;
+  if (p.max_kv == 1 && p.max_q == 1) return HYDRA_OK;
+  const ReduceArgs r{part, pq, a.dk, a.dv, a.dq, s3(a.dks), s3(a.dvs), s3(a.dqs), a.Hq, a.Hkv, a.S, a.hd, p.G,
+                     p.ntasks, p.items, p.nkg, p.BHkv, p.ch_kv, p.max_kv, p.ch_q, p.max_q, walk ? 1 : 0, a.scale};
+  // one launch for the gradients that were cut: dk and dv, dq, or all three
+  const int first = p.max_kv > 1 ? 0 : 2, count = (p.max_kv > 1 ? 2 : 0) + (p.max_q > 1 ? 1 : 0);
+  const int64_t rows = static_cast<int64_t>(p.BHkv) * 64 * std::max(p.max_kv > 1 ? p.nkg : 0, p.max_q > 1 ? p.items : 0);
+  const int64_t blocks = (rows * (HDP / 4) + 255) / 256;
+  if (blocks >= (int64_t(1) << 31)) return fail(HYDRA_ERR_ARG, "attn_bwd: problem too large");
+  attn_bwd_f32_reduce_kernel<T, HDP><<<dim3(static_cast<unsigned>(blocks), count), 256, 0, a.st>>>(r, first);
+  return check_launch("attn_bwd: f32 reduce");
+}
+
+}  // namespace
+
+int attn_fwd_f32(const AttnF32Args& a) {
+  return HYDRA_DISPATCH_DTYPE(a.dtype, T, [&] {
+    if (a.hd <= 16) return launch_fwd<T, 16>(a);
+    if (a.hd <= 32) return launch_fwd<T, 32>(a);
+    if (a.hd <= 64) return launch_fwd<T, 64>(a);
+    return launch_fwd<T, 128>(a);
+  });
+}
+
+size_t attn_bwd_f32_workspace(int B, int Hq, int Hkv, int S, int hd, bool causal, int mask_mode) {
+  const Plan p = plan_of(B, Hq, Hkv, S, hd, causal && mask_mode != HYDRA_MASK_REFERENCE_SDPA, true);
+  return (p.kv_floats + p.q_floats) * sizeof(float);
+}
+
+int attn_bwd_f32(const AttnF32Args& a, float* part, size_t part_bytes) {
+  return HYDRA_DISPATCH_DTYPE(a.dtype, T, [&] {
+    if (a.hd <= 16) return launch_bwd<T, 16>(a, part, part_bytes);
+    if (a.hd <= 32) return launch_bwd<T, 32>(a, part, part_bytes);
+    if (a.hd <= 64) return launch_bwd<T, 64>(a, part, part_bytes);
+    return launch_bwd<T, 128>(a, part, part_bytes);
+  });
+}
+
+}  // namespace hydra

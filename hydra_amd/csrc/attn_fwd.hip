@@ -26,10 +26,10 @@
 //  * Schedule: stream-K (equal key-tile ranges over one resident wave of
 //    workgroups, split items folded by attn_merge_kernel) when items are
 //    few, else one workgroup per item, longest first.
-// VALU paths (fp32 math, any element type): attn_fwd_split_kernel for
-// head_dim in {8, 16, 32, 64, 128} (16 lanes per query row, key-split), and
-// attn_fwd_generic_kernel (one thread per query row) for any other
-// head_dim <= 256.
+// Other element types, head dims and strides: attn_f32.hip (fp32 matrix
+// instructions) up to head_dim 128, above it attn_fwd_generic_kernel (one
+// thread per query row, fp32 math, head_dim <= 256).
+#include "attn_f32.h"
 #include "common.h"
 #include "lds_dma.h"
 
@@ -1435,201 +1435,6 @@ static int launch_mfma(const void* q, const void* k, const void* v, void* o, flo
   return dev ? go(F_(), M0(), X2()) : use_fixed ? go(F_(), M0(), X1()) : go(F_(), M0(), X0());
 }
 
-// ---------------------------------------------------------------------------
-// Key-split VALU kernel (fp32 / fp16, and bf16 shapes the MFMA kernel does
-// not take), head_dim a compile-time HD in {8, 16, 32, 64, 128}: a
-// workgroup takes 16 consecutive query rows of one (batch, head) and stages
-// 64-key tiles of K and V (fp32, rows padded by one word so the 16 keys a
-// row's lanes read fall in distinct banks) in LDS; each row is split over 16
-// lanes, lane l taking keys l, l+16, .. of every tile with its own online
-// softmax (exp2 domain, one rescale per tile), and the 16 partial states are
-// merged by shuffles at the end.  Same semantics as attn_fwd_generic_kernel
-// (mask modes, lse), the rows spread over 16x the threads.
-// ---------------------------------------------------------------------------
-template <typename T, int HD>
-__global__ __launch_bounds__(256) void attn_fwd_split_kernel(
-    const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
-    T* __restrict__ o, float* __restrict__ lse, const uint8_t* __restrict__ kmask,
-    int B, int S, int Hq, int Hkv, int causal, int mask_mode,
-    int64_t qs0, int64_t qs1, int64_t qs2, int64_t ks0, int64_t ks1, int64_t ks2,
-    int64_t vs0, int64_t vs1, int64_t vs2, int64_t vs3, int64_t os0, int64_t os1, int64_t os2,
-    float scale) {
-  constexpr int KL = 16;            // lanes per query row
-  constexpr int RW = 256 / KL;      // query rows per workgroup
-  constexpr int TK = 64;            // keys per staged tile
-  constexpr int KPT = TK / KL;      // keys per lane per tile
-  constexpr int KP = HD + 1;        // padded LDS row (words)
-  __shared__ float Ks[TK * KP], Vs[TK * KP];
-  __shared__ int Vis[TK];           // key usable under the key mask (modes 1, 2)
-  const int BH = B * Hq;
-  const int nsb = (S + RW - 1) / RW;
-  // longest rows first: blocks of the last query rows are dispatched first
-  const int bh = blockIdx.x % BH;
-  const int sb = nsb - 1 - static_cast<int>(blockIdx.x / BH);
-  const int b = bh / Hq, h = bh - b * Hq;
-  const int j = h / (Hq / Hkv);
-  const int tid = threadIdx.x, row = tid / KL, kl = tid % KL;
-  // Above head_dim 64 a row's lanes also split the head dimension: lane
-  // pair (2i, 2i+1) takes keys i, i + KL/2, .. and the two halves of d, and
-  // adds its partial dot products with one shuffle (the whole q row and
-  // output accumulator per lane would not fit in registers).
-  constexpr int DS = HD > 64 ? 2 : 1;   // d-slices per row
-  constexpr int DH = HD / DS;           // dims per lane
-  constexpr int KLK = KL / DS;          // key lanes per row
-  const int dh = kl % DS, kln = kl / DS;
-  const int s = sb * RW + row;
-  const bool live = s < S;
-  const float qscale = scale * kLog2e;
-  float qv[DH], acc[DH];
-  {
-    const T* qr = q + b * qs0 + h * qs1 + static_cast<int64_t>(live ? s : 0) * qs2 + dh * DH;
-#pragma unroll
-    for (int d = 0; d < DH; ++d) {
-      qv[d] = to_f32(qr[d]) * qscale;
-      acc[d] = 0.f;
-    }
-  }
-  float m = -INFINITY, l = 0.f;
-  const bool walk = causal && mask_mode != HYDRA_MASK_REFERENCE_SDPA;
-  const int kend = walk ? min(S, sb * RW + RW) : S;
-  const T* kb = k + b * ks0 + j * ks1;
-  const T* vb = v + b * vs0 + j * vs1;
-  // Head dims up to 64: the next tile's K and V are loaded into registers
-  // before this tile's arithmetic, so the loads' latency hides behind it
-  // (one tile in flight; written to LDS after the next barrier).
-  constexpr bool PF = HD <= 64;
-  constexpr int PER = PF ? TK * HD / 256 : 1;  // elements per thread per tile
-  static_assert(!PF || TK * HD % 256 == 0, "whole tile per pass");
-  float kpre[PER], vpre[PER];
-  auto prefetch = [&](int t0) {
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int i = tid + 256 * u;
-      const int kk = i / HD, d = i - kk * HD;
-      const int t = t0 + kk;
-      const bool in = t < S;
-      kpre[u] = in ? to_f32(kb[static_cast<int64_t>(t) * ks2 + d]) : 0.f;
-      vpre[u] = in ? to_f32(vb[static_cast<int64_t>(t) * vs2 + d * vs3]) : 0.f;
-    }
-  };
-  if constexpr (PF) prefetch(0);
-  for (int t0 = 0; t0 < kend; t0 += TK) {
-    __syncthreads();
-    if constexpr (PF) {
-#pragma unroll
-      for (int u = 0; u < PER; ++u) {
-        const int i = tid + 256 * u;
-        const int kk = i / HD, d = i - kk * HD;
-        Ks[kk * KP + d] = kpre[u];
-        Vs[kk * KP + d] = vpre[u];
-      }
-    } else {
-      for (int i = tid; i < TK * HD; i += 256) {
-        const int kk = i / HD, d = i - kk * HD;
-        const int t = t0 + kk;
-        const bool in = t < S;
-        Ks[kk * KP + d] = in ? to_f32(kb[static_cast<int64_t>(t) * ks2 + d]) : 0.f;
-        Vs[kk * KP + d] = in ? to_f32(vb[static_cast<int64_t>(t) * vs2 + d * vs3]) : 0.f;
-      }
-    }
-    if (mask_mode != HYDRA_MASK_NONE && tid < TK) {
-      const int t = t0 + tid;
-      Vis[tid] = t < S ? (kmask[static_cast<int64_t>(b) * S + t] != 0) : 0;
-    }
-    __syncthreads();
-    if constexpr (PF) {
-      if (t0 + TK < kend) prefetch(t0 + TK);
-    }
-    float x[KPT * DS];
-    float mt = m;
-#pragma unroll
-    for (int u = 0; u < KPT * DS; ++u) {
-      const int kk = kln + KLK * u;
-      const int t = t0 + kk;
-      bool vis = live && t < S;
-      if (mask_mode == HYDRA_MASK_REFERENCE_SDPA) vis = vis && (t > s || Vis[kk] == 0);
-      else {
-        if (causal) vis = vis && t <= s;
-        if (mask_mode == HYDRA_MASK_KEY_PADDING) vis = vis && Vis[kk] != 0;
-      }
-      float dot = 0.f;
-      const float* kr = Ks + kk * KP + dh * DH;
-#pragma unroll
-      for (int d = 0; d < DH; ++d) dot = fmaf(qv[d], kr[d], dot);
-      if constexpr (DS == 2) dot += __shfl_xor(dot, 1, KL);
-      x[u] = vis ? dot : -INFINITY;
-      mt = fmaxf(mt, x[u]);
-    }
-    if (mt == -INFINITY) continue;  // nothing visible to this lane yet
-    if (mt > m) {
-      const float alpha = __builtin_amdgcn_exp2f(m - mt);  // m = -inf -> 0
-      l *= alpha;
-#pragma unroll
-      for (int d = 0; d < DH; ++d) acc[d] *= alpha;
-      m = mt;
-    }
-#pragma unroll
-    for (int u = 0; u < KPT * DS; ++u) {
-      const float pu = __builtin_amdgcn_exp2f(x[u] - m);  // -inf -> 0
-      l += pu;
-      const float* vr = Vs + (kln + KLK * u) * KP + dh * DH;
-#pragma unroll
-      for (int d = 0; d < DH; ++d) acc[d] = fmaf(pu, vr[d], acc[d]);
-    }
-  }
-  // merge the key lanes of the row (lanes of one d-slice: offsets >= DS)
-  float mg = m;
-#pragma unroll
-  for (int off = KL / 2; off >= DS; off >>= 1) mg = fmaxf(mg, __shfl_xor(mg, off, KL));
-  const float f = (m == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m - mg);
-  l *= f;
-#pragma unroll
-  for (int off = KL / 2; off >= DS; off >>= 1) l += __shfl_xor(l, off, KL);
-#pragma unroll
-  for (int d = 0; d < DH; ++d) {
-    float a = acc[d] * f;
-#pragma unroll
-    for (int off = KL / 2; off >= DS; off >>= 1) a += __shfl_xor(a, off, KL);
-    acc[d] = a;
-  }
-  if (!live) return;
-  const float inv = l > 0.f ? 1.f / l : 0.f;
-  T* orow = o + b * os0 + h * os1 + static_cast<int64_t>(s) * os2 + dh * DH;
-#pragma unroll
-  for (int d = 0; d < DH; ++d)
-    if (d % KLK == kln) orow[d] = from_f32<T>(acc[d] * inv);
-  if (lse && kl == 0)
-    lse[(static_cast<int64_t>(b) * Hq + h) * S + s] = l > 0.f ? (mg + __log2f(l)) * kLn2 : -INFINITY;
-}
-
-template <typename T>
-static int launch_split(const void* q, const void* k, const void* v, void* o, float* lse,
-                        const uint8_t* kmask, int mask_mode, int64_t B, int64_t Hq, int64_t Hkv,
-                        int64_t S, int64_t hd, const int64_t* qs, const int64_t* ks,
-                        const int64_t* vs, const int64_t* os, bool causal, float scale,
-                        hipStream_t st) {
-  const int64_t nblk = B * Hq * ((S + 15) / 16);
-  const dim3 grid(static_cast<unsigned>(nblk));
-  auto Q = static_cast<const T*>(q);
-  auto K = static_cast<const T*>(k);
-  auto V = static_cast<const T*>(v);
-  auto O = static_cast<T*>(o);
-#define HYDRA_SPLIT_LAUNCH(HD)                                                              \
-  attn_fwd_split_kernel<T, HD><<<grid, 256, 0, st>>>(                                       \
-      Q, K, V, O, lse, kmask, (int)B, (int)S, (int)Hq, (int)Hkv, causal ? 1 : 0, mask_mode, \
-      qs[0], qs[1], qs[2], ks[0], ks[1], ks[2], vs[0], vs[1], vs[2], vs[3], os[0], os[1],   \
-      os[2], scale)
-  switch (hd) {
-    case 8: HYDRA_SPLIT_LAUNCH(8); break;
-    case 16: HYDRA_SPLIT_LAUNCH(16); break;
-    case 32: HYDRA_SPLIT_LAUNCH(32); break;
-    case 64: HYDRA_SPLIT_LAUNCH(64); break;
-    default: HYDRA_SPLIT_LAUNCH(128); break;
-  }
-#undef HYDRA_SPLIT_LAUNCH
-  return check_launch("attn_fwd_split_kernel");
-}
-
 template <typename T>
 static int launch_generic(const void* q, const void* k, const void* v, void* o, float* lse,
                           const uint8_t* kmask, int mask_mode, int64_t B, int64_t Hq,
@@ -1647,10 +1452,7 @@ static int launch_generic(const void* q, const void* k, const void* v, void* o, 
       Q, K, V, O, lse, kmask, (int)B, (int)S, (int)Hq, (int)Hkv, (int)hd, causal ? 1 : 0, \
       mask_mode, qs[0], qs[1], qs[2], ks[0], ks[1], ks[2], vs[0], vs[1], vs[2], vs[3], os[0], \
       os[1], os[2], scale)
-  if (hd <= 32) HYDRA_GEN_LAUNCH(32);
-  else if (hd <= 64) HYDRA_GEN_LAUNCH(64);
-  else if (hd <= 128) HYDRA_GEN_LAUNCH(128);
-  else HYDRA_GEN_LAUNCH(256);
+  HYDRA_GEN_LAUNCH(256);
 #undef HYDRA_GEN_LAUNCH
   return check_launch("attn_fwd_generic_kernel");
 }
@@ -1728,12 +1530,15 @@ static int attn_fwd_impl(const void* q, const void* k, const void* v, void* o,
     }
   }
   HYDRA_REQUIRE(B * Hq * S / 256 < (int64_t(1) << 31), "attn_fwd: too many rows");
-  if (need) return HYDRA_OK;  // the VALU kernels take no scratch
-  const bool split_shape = hd == 8 || hd == 16 || hd == 32 || hd == 64 || hd == 128;
+  if (need) return HYDRA_OK;  // the other kernels take no scratch
+  if (hd <= kAttnF32MaxHd && getenv("HYDRA_ATTN_GENERIC") == nullptr) {
+    if (dtype != HYDRA_F32 && dtype != HYDRA_BF16 && dtype != HYDRA_F16)
+      return fail(HYDRA_ERR_ARG, "unknown dtype code");
+    return attn_fwd_f32(AttnF32Args{q, k, v, nullptr, o, nullptr, nullptr, nullptr, lse, nullptr, nullptr, km,
+                                    mask_mode, (int)B, (int)Hq, (int)Hkv, (int)S, (int)hd, qs, ks, vs, os, nullptr,
+                                    nullptr, nullptr, nullptr, causal != 0, scale, dtype, st});
+  }
   return HYDRA_DISPATCH_DTYPE(dtype, T, [&] {
-    if (split_shape && getenv("HYDRA_ATTN_GENERIC") == nullptr)
-      return launch_split<T>(q, k, v, o, lse, km, mask_mode, B, Hq, Hkv, S, hd, qs, ks, vs, os,
-                             causal != 0, scale, st);
     return launch_generic<T>(q, k, v, o, lse, km, mask_mode, B, Hq, Hkv, S, hd, qs, ks, vs,
                              os, causal != 0, scale, st);
   });
