@@ -61,6 +61,7 @@ SIGNATURES = {
                                  _I64P, _I64P, _I, _I, _I, _I64P],
     "hydra_linear_fwd": [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _I, _I, _P],
     "hydra_ce_rows": [_P, _I64, _I64, _I64, _P, _I64, _P, _P, _P, _I64, _P, _I, _P],
+    "hydra_ce_grad_planes": [_P, _I64, _I64, _I64, _P, _I64, _P, _I64, _I64, _P, _P],
     "hydra_ccgqa_prep_tiled_ok": [_I64, _I64, _I64, _I],
     "hydra_ccgqa_prep_faults": [_P],
     "hydra_ccgqa_prep_bwd": [_P, _I64, _P, _P, _P, _P, _P, _I64, _P, _P, _P, _P, _P, _I64, _P,

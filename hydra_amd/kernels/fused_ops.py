@@ -374,6 +374,21 @@ def _ce_rows(logits: torch.Tensor, targets: torch.Tensor, ignore_index: int,
     return loss
 
 
+def _ce_grad_planes(logits: torch.Tensor, targets: torch.Tensor, ignore_index: int,
+                    grad_scale: torch.Tensor) -> torch.Tensor:
+    """(softmax(x) - onehot(t)) * grad_scale[0] of fp32 logits [rows, V] as two
+    bf16 planes [2 * rows, V] (rounded values, then residuals; rows padded to
+    16 bytes)."""
+    rows, V = logits.shape
+    pitch = (V + 7) // 8 * 8
+    planes = torch.empty((2 * rows, pitch), dtype=torch.bfloat16, device=logits.device)
+    with torch.cuda.device(logits.device):
+        _lib.call("hydra_ce_grad_planes", logits.data_ptr(), rows, V, logits.stride(0), targets.data_ptr(),
+                  int(ignore_index), planes.data_ptr(), pitch, rows * pitch, _lib.ptr(grad_scale),
+                  _lib.stream(logits))
+    return planes[:, :V]
+
+
 class ChunkedCrossEntropyFunction(torch.autograd.Function):
     """fused_ops.py:1382-1531: mean token cross-entropy of hidden @ weight^T
     over tokens whose target is not ignore_index, computed chunk by chunk
@@ -410,11 +425,34 @@ class ChunkedCrossEntropyFunction(torch.autograd.Function):
         hidden_states, weight, t, n_valid = ctx.saved_tensors
         dim = hidden_states.shape[-1]
         h = hidden_states.reshape(-1, dim)
-        wf = weight.float()
         scale = (grad_output.float() / n_valid.clamp(min=1)).reshape(1).contiguous()
         grad_h = torch.empty(h.shape, dtype=torch.float32, device=h.device)
-        grad_w = torch.zeros(weight.shape, dtype=torch.float32, device=h.device)
         cs = ctx.chunk_size
+        if h.dtype == weight.dtype == torch.bfloat16:
+            # bf16 products are exact in fp32 accumulation, so the logits and
+            # both gradient GEMMs run on the bf16 matrix cores with fp32
+            # results, the logits' gradient as two bf16 planes.  Forward +
+            # backward, 8192 tokens x 768 x vocab 32000: 9.65 -> 3.16 ms
+            # (three fp32 GEMMs of 1.45 ms per 4096-token chunk before).
+            # Other dtypes keep the fp32 GEMMs: fp32 operands would need three
+            # planes each, six products, for no gain worth the name.
+            grad_w = None
+            for s in range(0, h.shape[0], cs):
+                hc = h[s:s + cs]
+                n = hc.shape[0]
+                planes = _ce_grad_planes(torch.mm(hc, weight.t(), out_dtype=torch.float32), t[s:s + cs],
+                                         ctx.ignore_index, scale)
+                gh = torch.mm(planes, weight, out_dtype=torch.float32)
+                torch.add(gh[:n], gh[n:], out=grad_h[s:s + cs])
+                both = torch.cat((hc, hc))
+                grad_w = (torch.mm(planes.t(), both, out_dtype=torch.float32) if grad_w is None else
+                          torch.addmm(grad_w, planes.t(), both, out_dtype=torch.float32))
+            if grad_w is None:
+                grad_w = torch.zeros(weight.shape, dtype=torch.float32, device=h.device)
+            return (grad_h.view_as(hidden_states).to(hidden_states.dtype), grad_w.to(weight.dtype),
+                    None, None, None)
+        grad_w = torch.zeros(weight.shape, dtype=torch.float32, device=h.device)
+        wf = weight.float()
         for s in range(0, h.shape[0], cs):
             hc = h[s:s + cs].float()
             g = F.linear(hc, wf).contiguous()  # logits, overwritten by their gradient

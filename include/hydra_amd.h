@@ -400,6 +400,16 @@ int hydra_ce_rows(const void* logits, int64_t rows, int64_t vocab, int64_t logit
                   void* grad, int64_t grad_rs, const float* grad_scale, int dtype,
                   void* stream);
 
+/* The same gradient of fp32 logits, g = (softmax(x[r]) - onehot(t)) *
+ * grad_scale[0], written as two bf16 planes instead of fp32: planes[0] the
+ * rounded value, planes[1] (plane_stride elements further) the residual
+ * g - planes[0] rounded, rows planes_rs elements apart.  For the bf16 GEMMs of
+ * ChunkedCrossEntropyFunction's backward (fused_ops.py:1459-1531). */
+int hydra_ce_grad_planes(const float* logits, int64_t rows, int64_t vocab, int64_t logits_rs,
+                         const int64_t* targets, int64_t ignore_index, void* planes,
+                         int64_t planes_rs, int64_t plane_stride, const float* grad_scale,
+                         void* stream);
+
 /* ---- block compositions (hydra/model/framework, hydra/layers) --------- */
 
 /* Token embedding: out[r, :] = table[clamp(ids[r], 0, vocab-1), :] * scale,

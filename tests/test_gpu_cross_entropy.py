@@ -121,3 +121,31 @@ def test_ce_rows_masked_logits(cuda, V, with_grad):
         assert torch.isfinite(gc).all()
         assert max_rel_err(gc, gr) < 1e-5
         assert (gc[torch.isinf(x)] == 0).all()
+
+
+@pytest.mark.parametrize("rows,V", [(3, 1), (5, 7), (4, 1000), (2, 8191), (3, 8192), (3, 16392), (2, 32768),
+                                    (2, 40008), (3, 50257)])
+def test_ce_grad_planes(cuda, rows, V):
+    """hydra_ce_grad_planes at the edges of its row forms (registers, read
+    twice, unaligned): both planes' sum against the fp64 gradient.  The planes
+    carry 16 significant bits (2^-17 per value) of an fp32 value whose exponent
+    argument is rounded at |x| 2^-24 (|x| <= 60 here): 2^-16 covers both."""
+    from hydra_amd.kernels.fused_ops import _ce_grad_planes
+
+    g = torch.Generator().manual_seed(V)
+    x = torch.randn(rows, V, generator=g) * 5
+    x[0, 0] = -float("inf") if V > 1 else 0.0
+    t = torch.randint(0, V, (rows,), generator=g)
+    t[-1] = -100
+    scale = torch.tensor([0.37])
+    got = _ce_grad_planes(x.to(cuda), t.to(cuda), -100, scale.to(cuda)).double().cpu()
+    ref = torch.softmax(x.double(), 1)
+    ref[torch.arange(rows), t.clamp(0)] -= 1
+    ref = ref * 0.37
+    ref[-1] = 0
+    got = got[:rows] + got[rows:]
+    assert got[-1].abs().max() == 0
+    if V > 1:
+        assert float((got - ref).norm() / ref.norm()) < 2.0 ** -16
+    else:
+        assert got.abs().max() < 1e-6
