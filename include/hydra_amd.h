@@ -521,6 +521,14 @@ int hydra_mod_scatter(void* out, const void* y, const int64_t* idx,
                       int64_t D, int64_t o_bs, int64_t o_ls, int mode,
                       int dtype, void* stream);
 
+/* Backward of the weighted ADD form: grad_y[b, j] = w[b, j] * g and grad_w[b,
+ * j] = <g, y[b, j]> (fp32 sums) with g = grad[b, idx[b, j]] (grad: [B, L, D],
+ * strides g_bs, g_ls; y, grad_y: contiguous [B, k, D]; w, grad_w: fp32 [B,
+ * k]).  grad_y or grad_w may be NULL.  Indices outside [0, L) give zeros. */
+int hydra_mod_scatter_bwd(const void* grad, const void* y, const int64_t* idx, const float* w,
+                          void* grad_y, float* grad_w, int64_t B, int64_t L, int64_t k,
+                          int64_t D, int64_t g_bs, int64_t g_ls, int dtype, void* stream);
+
 /* ---- measurement aid ----------------------------------------------------- */
 
 /* dst[0, bytes) = src[0, bytes): a plain device-to-device copy with

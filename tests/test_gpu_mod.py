@@ -362,3 +362,29 @@ def test_mod_mlp_ste_training_backward(cuda):
     assert max_rel_err(xd.grad.cpu(), xr.grad) < 1e-5
     for name, p in wrap.named_parameters():
         assert max_rel_err(p.grad.cpu(), ref[name].grad) < 1e-5, name
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [1, 7, 8, 520, 1280, 2056, 4100])
+def test_weighted_scatter_gradients(cuda, D, dtype):
+    """hydra_mod_scatter_bwd at row widths around its chunk rounds (and off
+    the 16-byte path): both gradients against fp64.  grad_values is one
+    product rounded once (unit roundoff of 8, 11 and 24 significant bits: 2^-8
+    bf16, 2^-11 fp16, 2^-24 fp32); grad_w an fp32 sum of D exact-ish products, sqrt(D) 2^-24
+    at most, bounded by 2^-17 of the products' 2-norm."""
+    from hydra_amd.routing import weighted_residual_scatter
+
+    g = torch.Generator().manual_seed(D)
+    B, L, k = 2, 9, 5
+    out = torch.randn(B, L, D, generator=g).to(dtype).to(cuda)
+    vals = torch.randn(B, k, D, generator=g).to(dtype).to(cuda).requires_grad_()
+    idx = torch.stack([torch.randperm(L, generator=g)[:k] for _ in range(B)]).to(cuda)
+    w = torch.rand(B, k, generator=g).to(cuda).requires_grad_()
+    go = torch.randn(B, L, D, generator=g).to(dtype).to(cuda)
+    res = weighted_residual_scatter(out.clone(), vals, idx, w)
+    gv, gw = torch.autograd.grad(res, [vals, w], go)
+    sel = go.double().gather(1, idx[..., None].expand(-1, -1, D))
+    ref_v, prod = sel * w.detach().double()[..., None], sel * vals.detach().double()
+    u = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24}[dtype]
+    assert ((gv.double() - ref_v).abs() <= u * ref_v.abs() + 2.0 ** -25).all()
+    assert ((gw.double() - prod.sum(-1)).abs() <= 2.0 ** -17 * prod.norm(dim=-1)).all()
