@@ -66,6 +66,9 @@ SIGNATURES = {
     "hydra_ccgqa_prep_faults": [_P],
     "hydra_ccgqa_prep_bwd": [_P, _I64, _P, _P, _P, _P, _P, _I64, _P, _P, _P, _P, _P, _I64, _P,
                              _I64, _I64, _I64, _I64, _I64, _I, _I, _P],
+    "hydra_ccgqa_prep_bwd_conv_workspace": [_I64, _I64, _I64, _I64, _I64, _I64, _I, _I],
+    "hydra_ccgqa_prep_bwd_conv": [_P, _I64, _P, _P, _P, _P, _P, _P, _P, _I64, _P, _P, _P, _P, _I64, _P, _P,
+                                  _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I, _I, _P, _I64, _P],
     "hydra_causal_im2col": [_P, _I64, _P, _I64, _I64, _I64, _I64, _I64, _I, _P],
     "hydra_causal_col2im": [_P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I, _I, _P],
     "hydra_embedding_fwd": [_P, _I64, _P, _I64, _I64, _I64, _F, _P, _I64, _I, _P],
@@ -83,7 +86,7 @@ SIGNATURES = {
 }
 
 # entry points that return a value (not a status) of type int64_t
-_RETURNS_INT64 = {"hydra_rms_norm_bwd_workspace"}
+_RETURNS_INT64 = {"hydra_rms_norm_bwd_workspace", "hydra_ccgqa_prep_bwd_conv_workspace"}
 
 _lib = None
 

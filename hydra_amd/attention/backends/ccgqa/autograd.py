@@ -4,7 +4,10 @@ which the reference trains through torch autograd).
 
 forward:  hydra_ccgqa_prep_fwd (the inference kernel), keeping only qkv, the
           conv weights and the temperature.
-backward: 1. the conv outputs y2 recomputed by the same kernel with the
+backward: bf16 with three-tap convs in one call (hydra_ccgqa_prep_bwd_conv:
+          implicit-GEMM convs, the pointwise chain and the weight gradients);
+          other dtypes, tap counts and widths:
+          1. the conv outputs y2 recomputed by the same kernel with the
              convs alone;
           2. hydra_ccgqa_prep_bwd: RoPE transpose, F.normalize backward
              (temperature gradient as per-token partials), QK-mean and
@@ -24,7 +27,7 @@ import torch
 
 from ...._lib import CCGQA_CONVS, CCGQA_QK_NORM, CCGQA_W_TILED
 from .ops import (causal_col2im, causal_im2col, ccgqa_prep, ccgqa_prep_backward,
-                  tiled_weights_ok)
+                  ccgqa_prep_backward_convs, tiled_weights_ok)
 
 
 def _conv_pair_backward(x0: torch.Tensor, dy2: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor,
@@ -87,6 +90,12 @@ class CCGQAPrepFunction(torch.autograd.Function):
         gk = z(Hkv) if gk is None else gk
         gv = z(Hkv) if gv is None else gv
         convs = bool(flags & CCGQA_CONVS)
+        if convs:
+            got = ccgqa_prep_backward_convs(qkv, Hq, Hkv, hd, flags, wq1, wq2, wk1, wk2, gq, gk, gv,
+                                            temperature=temp, cos=cos, sin=sin,
+                                            want_temperature=temp is not None and ctx.needs_input_grad[5])
+            if got is not None:
+                return (*got, None, None, None, None, None, None)
         y2q = y2k = None
         if convs:
             fl = CCGQA_CONVS | (CCGQA_W_TILED if tiled else 0)

@@ -357,3 +357,54 @@ def ccgqa_prep_backward(qkv: torch.Tensor, n_heads: int, n_kv_heads: int, head_d
                   n_heads, n_kv_heads, head_dim, flags & ~CCGQA_W_TILED, _lib.dtype_code(qkv),
                   _lib.stream(qkv))
     return dy, dqkv, dtemp
+
+
+def ccgqa_prep_backward_convs(qkv: torch.Tensor, n_heads: int, n_kv_heads: int, head_dim: int, flags: int,
+                              wq1, wq2, wk1, wk2, dq, dk, dv, temperature=None, cos=None, sin=None,
+                              want_temperature: bool = True):
+    """The whole backward of ccgqa_prep (hydra_ccgqa_prep_bwd_conv): (dqkv,
+    dwq1, dwq2, dwk1, dwk2, dtemperature or None), or None where the kernels
+    do not take the sizes, dtypes or strides (weights in qkv's dtype)."""
+    dt = qkv.dtype
+    B, S, W = qkv.shape
+    ks = wq1.shape[-1]
+    weights = (wq1, wq2, wk1, wk2)
+    norm = bool(flags & CCGQA_QK_NORM)
+    if dt != torch.bfloat16 or any(w.dtype != dt for w in weights) or \
+            (norm and (temperature.dtype != dt or temperature.numel() != 1)):
+        return None
+    flags &= ~CCGQA_W_TILED
+    need = _lib.query("hydra_ccgqa_prep_bwd_conv_workspace", B, S, n_heads, n_kv_heads, head_dim, ks, flags,
+                      _lib.dtype_code(qkv))
+    if need < 0:
+        return None
+    _lib.require_gpu("ccgqa_prep_backward", qkv, *weights, dq, dk, dv, temperature, cos, sin)
+    L, K = n_heads * head_dim, n_kv_heads * head_dim
+    if W != L + 2 * K:
+        raise ValueError(f"ccgqa_prep_backward: qkv width {W} != L + 2K = {L + 2 * K}")
+    if qkv.stride(-1) != 1 or (B > 1 and qkv.stride(0) != S * qkv.stride(1)):
+        qkv = qkv.contiguous()
+    dq, dk, dv = (t.to(dt).contiguous() for t in (dq, dk, dv))
+    weights = tuple(w.detach().contiguous() for w in weights)
+    if flags & CCGQA_ROPE:
+        if cos.dim() == 4:
+            cos, sin = cos[0, 0], sin[0, 0]
+        cos = cos[:S].float().contiguous()
+        sin = sin[:S].float().contiguous()
+    else:
+        cos = sin = None
+    dqkv = torch.empty((B, S, W), dtype=dt, device=qkv.device)
+    dws = tuple(torch.empty_like(w) for w in weights)
+    dtemp = torch.empty_like(temperature) if norm and want_temperature else None
+    ws = _lib.scratch(need, qkv)
+    with torch.cuda.device(qkv.device):
+        rc = _lib.call_status(
+            "hydra_ccgqa_prep_bwd_conv", qkv.data_ptr(), qkv.stride(1), *(w.data_ptr() for w in weights),
+            temperature.data_ptr() if norm else None, _lib.ptr(cos), _lib.ptr(sin),
+            head_dim // 2 if cos is None else cos.stride(0), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+            dqkv.data_ptr(), W, *(w.data_ptr() for w in dws), _lib.ptr(dtemp), B, S, n_heads, n_kv_heads,
+            head_dim, ks, flags, _lib.dtype_code(qkv), ws.data_ptr(), need, _lib.stream(qkv))
+    if rc == _lib.ERR_UNSUPPORTED:
+        return None
+    _lib.check(rc, "hydra_ccgqa_prep_bwd_conv")
+    return (dqkv, *dws, dtemp)

@@ -5,7 +5,7 @@
 // kernels/fused_conv.py:39-62, trained through autograd there).
 //
 // Split in three kinds of work:
-//   * hydra_ccgqa_prep_bwd: the pointwise chain, one token per wave --
+//   * hydra_ccgqa_prep_bwd: the pointwise chain (launch_prep_bwd) --
 //     RoPE transpose, F.normalize backward (with the temperature and its
 //     gradient), QK-mean backward, value-shift backward.  It reads the conv
 //     outputs (recomputed by the caller with the forward kernel) and the
@@ -16,6 +16,9 @@
 //     GEMM over [tap, channel] columns (per group), so the conv backward is
 //     plain library GEMMs: dX = col2im(dY W), dW = dY^T im2col(X).
 //   * the GEMMs themselves (hipBLASLt through the caller).
+// bf16 with three taps takes hydra_ccgqa_prep_bwd_conv (ccgqa_conv_bwd.hip)
+// instead of the last two.
+#include "ccgqa_prep_bwd.h"
 #include "common.h"
 
 #include <algorithm>
@@ -36,6 +39,179 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
+// The pointwise chain, 8 channels (16 bytes of a 16-bit type) per thread:
+// head_dim / 8 neighbouring threads hold a head, so its norm and projection
+// are shuffles among them, and the sums over heads (QK-mean, forward and
+// backward) go through one LDS row per token.  A workgroup takes
+// 256 / ((L + K) / 8) tokens.  Bound by HBM (every tensor is read or written
+// once, 16 bytes per lane); a lane per head walking its head_dim serially
+// through LDS took 34 us at 4096 tokens x 640 channels.
+template <typename T>
+__device__ __forceinline__ void load8(const T* p, float (&f)[8]) {
+  load16<T>(p, f);
+  if constexpr (sizeof(T) == 4) load16<T>(p + 4, f + 4);
+}
+template <typename T>
+__device__ __forceinline__ void store8(T* p, const float (&f)[8]) {
+  store16<T>(p, f);
+  if constexpr (sizeof(T) == 4) store16<T>(p + 4, f + 4);
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void ccgqa_prep_bwd_vec_kernel(PrepBwdArgs a, int tpb) {
+  __shared__ __attribute__((aligned(16))) float rows[256 * 8];  // [token][L + K]
+  __shared__ float dts[256];                                    // [token][k head]
+  const int Hq = a.Hq, Hkv = a.Hkv, hd = a.hd, G = Hq / Hkv;
+  const int L = Hq * hd, K = Hkv * hd, CW = L + K, nch = CW / 8, hc = hd / 8;
+  const bool convs = a.flags & HYDRA_CCGQA_CONVS;
+  const bool qk_mean = a.flags & HYDRA_CCGQA_QK_MEAN;
+  const bool vshift = a.flags & HYDRA_CCGQA_VALUE_SHIFT;
+  const bool qk_norm = a.flags & HYDRA_CCGQA_QK_NORM;
+  const bool rope = a.flags & HYDRA_CCGQA_ROPE;
+  const int tid = threadIdx.x;
+  const int64_t ntok = static_cast<int64_t>(a.B) * a.S, tok0 = static_cast<int64_t>(blockIdx.x) * tpb;
+  const int tl = tid / nch, ch = 8 * (tid - tl * nch);  // token of the workgroup, first channel
+  const int64_t tok = tok0 + tl;
+  const bool live = tl < tpb && tok < ntok;
+  const int b = live ? static_cast<int>(tok / a.S) : 0;
+  const int s = live ? static_cast<int>(tok - static_cast<int64_t>(b) * a.S) : 0;
+  const bool is_k = ch >= L;
+  const int kc = is_k ? ch - L : ch, h = kc / hd, d = kc - h * hd;
+  const T* xr = static_cast<const T*>(a.qkv) + tok * a.qkv_rs;
+  float* row = rows + tl * CW;
+  float x[8], g[8], x0[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x[e] = g[e] = x0[e] = 0.f;
+  if (live) {
+    load8<T>(xr + ch, x0);
+    if (convs) {
+      const T* y = is_k ? static_cast<const T*>(a.y2k) + b * a.yk_b : static_cast<const T*>(a.y2q) + b * a.yq_b;
+      load8<T>(y + h * a.y_h + s * a.y_s + d, x);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = x0[e];
+    }
+    const T* gs = is_k ? static_cast<const T*>(a.dk) + ((static_cast<int64_t>(b) * Hkv + h) * a.S + s) * hd + d
+                       : static_cast<const T*>(a.dq) + ((static_cast<int64_t>(b) * Hq + h) * a.S + s) * hd + d;
+    load8<T>(gs, g);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) row[ch + e] = x0[e];
+  }
+  __syncthreads();
+  // the pre-norm value, the working dtype's roundings as in the forward
+  if (live && qk_mean) {
+    float t[8];
+    if (G == 1) {  // (q0_h + k0_h) / 2 for q and k head h
+      const float* other = row + (is_k ? kc : L + kc);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) t[e] = rd<T>(0.5f * rd<T>(x0[e] + other[e]));
+    } else {  // q heads: mean of the k heads; k heads: mean of the q heads
+      const int nh = is_k ? Hq : Hkv;
+      const float* src = row + (is_k ? 0 : L) + d;
+      float sum[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sum[e] = 0.f;
+      for (int hx = 0; hx < nh; ++hx)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sum[e] += src[hx * hd + e];
+      const float inv = 1.f / static_cast<float>(nh);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) t[e] = rd<T>(0.5f * rd<T>(sum[e] * inv));
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = rd<T>(x[e] + t[e]);
+  }
+  if (live && rope) {  // forward (x0,x1) -> (x0 c - x1 s, x0 s + x1 c); its transpose
+    const float* cp = a.cs + static_cast<int64_t>(s) * a.cs_rs + d / 2;
+    const float* sp = a.sn + static_cast<int64_t>(s) * a.cs_rs + d / 2;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float c = cp[e], sv = sp[e];
+      const float g0 = g[2 * e] * c + g[2 * e + 1] * sv, g1 = g[2 * e + 1] * c - g[2 * e] * sv;
+      g[2 * e] = g0;
+      g[2 * e + 1] = g1;
+    }
+  }
+  if (qk_norm) {  // F.normalize backward (dead threads take part in the shuffles with zeros)
+    const float tval = a.temp ? to_f32(static_cast<const T*>(a.temp)[0]) : 1.f;
+    auto head_sum = [&](float v) {
+      for (int off = hc / 2; off > 0; off >>= 1) v += __shfl_xor(v, off);
+      return v;
+    };
+    float ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ss = fmaf(x[e], x[e], ss);
+    const float n = __builtin_sqrtf(head_sum(ss));
+    const float den = fmaxf(rd<T>(n), 1e-12f);  // x / max(n, 1e-12), the norm rounded
+    float dot = 0.f, dt = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float xh = x[e] / den;
+      dot = fmaf(xh, g[e], dot);
+      dt = fmaf(rd<T>(xh), g[e], dt);  // k = rd(x / den) * temperature
+    }
+    dot = head_sum(dot);
+    dt = head_sum(dt);
+    if (live && is_k && d == 0) dts[tl * Hkv + h] = dt;
+    if (is_k) dot *= tval;
+    const float rinv = 1.f / den, sc = is_k ? tval : 1.f;
+    const float proj = rd<T>(n) > 1e-12f ? dot : 0.f;  // below eps the divisor is constant
+#pragma unroll
+    for (int e = 0; e < 8; ++e) g[e] = (g[e] * sc - x[e] * rinv * proj) * rinv;
+  }
+  __syncthreads();  // readers of the q0/k0 rows are done
+  if (live) {
+    if (convs) store8<T>(static_cast<T*>(a.dy) + tok * CW + ch, g);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) row[ch + e] = g[e];
+  }
+  __syncthreads();
+  if (live) {
+    // q0/k0 parts of grad(qkv): QK-mean (+ the direct path without convs)
+    float m[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) m[e] = 0.f;
+    if (qk_mean && G == 1) {  // (q0 + k0) / 2 feeds q and k of head h
+      const float* other = row + (is_k ? kc : L + kc);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) m[e] = 0.5f * (g[e] + other[e]);
+    } else if (qk_mean) {
+      // q0 channel: through the q mean into every k head; k0 channel: through
+      // the k mean into every q head
+      const int nh = is_k ? Hq : Hkv;
+      const float* src = row + (is_k ? 0 : L) + d;
+      for (int hx = 0; hx < nh; ++hx)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) m[e] += src[hx * hd + e];
+      const float inv = 1.f / static_cast<float>(is_k ? Hkv : Hq);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) m[e] *= 0.5f * inv;
+    }
+    if (!convs) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) m[e] += g[e];
+    }
+    T* gr = static_cast<T*>(a.dqkv) + tok * a.dqkv_rs;
+    store8<T>(gr + ch, m);
+    if (ch == 0 && qk_norm && a.dtemp_tok) {
+      float dtemp = 0.f;
+      for (int hx = 0; hx < Hkv; ++hx) dtemp += dts[tl * Hkv + hx];
+      a.dtemp_tok[tok] = dtemp;
+    }
+    // v part, by the k channels' threads (value shift: the second half came
+    // from token s - 1)
+    if (is_k) {
+      const bool next = vshift && kc >= K / 2;
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = 0.f;
+      if (!next || s + 1 < a.S)
+        load8<T>(static_cast<const T*>(a.dv) + ((static_cast<int64_t>(b) * Hkv + h) * a.S + s + (next ? 1 : 0)) * hd + d, v);
+      store8<T>(gr + CW + kc, v);
+    }
+  }
+}
+
 // One token (b, s) per wave.  LDS per wave: xs[CW] (the pre-norm value
 // qc/kc), gs[CW] (incoming gradient after the RoPE transpose, then the
 // gradient of qc/kc), hs[2*NH] (per-head norm and projection).
@@ -46,7 +222,7 @@ __global__ __launch_bounds__(kPbThreads) void ccgqa_prep_bwd_kernel(
     const float* __restrict__ sn, int64_t cs_rs, const T* __restrict__ dq,
     const T* __restrict__ dk, const T* __restrict__ dv, T* __restrict__ dy,
     T* __restrict__ dqkv, int64_t dqkv_rs, float* __restrict__ dtemp_tok, int B, int S, int Hq,
-    int Hkv, int hd, int flags) {
+    int Hkv, int hd, int flags, int64_t yq_b, int64_t yk_b, int64_t y_h, int64_t y_s) {
   extern __shared__ float pb_smem[];
   const int L = Hq * hd, K = Hkv * hd, CW = L + K, NH = Hq + Hkv;
   const int G = Hq / Hkv;
@@ -74,8 +250,7 @@ __global__ __launch_bounds__(kPbThreads) void ccgqa_prep_bwd_kernel(
       const int h = (is_k ? ch - L : ch) / hd, d = (is_k ? ch - L : ch) - h * hd;
       float x0, x1;
       if (convs) {
-        const T* y = is_k ? y2k + ((static_cast<int64_t>(b) * Hkv + h) * S + s) * hd + d
-                          : y2q + ((static_cast<int64_t>(b) * Hq + h) * S + s) * hd + d;
+        const T* y = (is_k ? y2k + b * yk_b : y2q + b * yq_b) + h * y_h + s * y_s + d;
         x0 = to_f32(y[0]);
         x1 = to_f32(y[1]);
       } else {
@@ -262,6 +437,42 @@ __global__ __launch_bounds__(256) void causal_col2im_kernel(const T* __restrict_
   *o = from_f32<T>(acc);
 }
 
+int launch_prep_bwd(const PrepBwdArgs& a) {
+  const int L = a.Hq * a.hd, K = a.Hkv * a.hd, CW = L + K;
+  const int64_t ntok = static_cast<int64_t>(a.B) * a.S;
+  return HYDRA_DISPATCH_DTYPE(a.dtype, T, [&] {
+    // Whole 8-channel pieces everywhere: heads of 8, 16, .., 512 channels, one
+    // workgroup row of at most 2048, 16-byte rows; the halves of v on a piece
+    // boundary when shifted.
+    const bool hd_ok = a.hd % 8 == 0 && (a.hd & (a.hd - 1)) == 0 && a.hd <= 512;
+    const bool rows_ok = a.qkv_rs % 8 == 0 && a.dqkv_rs % 8 == 0 && a.yq_b % 8 == 0 && a.yk_b % 8 == 0 &&
+                         a.y_h % 8 == 0 && a.y_s % 8 == 0 && (!(a.flags & HYDRA_CCGQA_VALUE_SHIFT) || K % 16 == 0);
+    bool ptr_ok = true;
+    for (const void* p : {a.qkv, a.y2q, a.y2k, a.dq, a.dk, a.dv, static_cast<const void*>(a.dy),
+                          static_cast<const void*>(a.dqkv)})
+      ptr_ok = ptr_ok && aligned16(p);
+    if (hd_ok && rows_ok && ptr_ok && CW <= 2048) {
+      const int tpb = 256 / (CW / 8);
+      ccgqa_prep_bwd_vec_kernel<T><<<dim3(static_cast<unsigned>((ntok + tpb - 1) / tpb)), 256, 0, a.st>>>(a, tpb);
+      return check_launch("ccgqa_prep_bwd_vec_kernel");
+    }
+    const size_t lds = static_cast<size_t>(kPbThreads / 64) * (2 * CW + 2 * (a.Hq + a.Hkv)) * sizeof(float);
+    const unsigned grid = static_cast<unsigned>(std::min<int64_t>((ntok + 3) / 4, 8192));
+    auto kern = ccgqa_prep_bwd_kernel<T>;
+    if (lds > 64 * 1024 &&
+        hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)) != hipSuccess)
+      return fail(HYDRA_ERR_LAUNCH, "ccgqa_prep_bwd: cannot set the kernel's LDS size");
+    kern<<<grid, kPbThreads, lds, a.st>>>(
+        static_cast<const T*>(a.qkv), a.qkv_rs, static_cast<const T*>(a.y2q), static_cast<const T*>(a.y2k),
+        static_cast<const T*>(a.temp), a.cs, a.sn, a.cs_rs, static_cast<const T*>(a.dq),
+        static_cast<const T*>(a.dk), static_cast<const T*>(a.dv), static_cast<T*>(a.dy),
+        static_cast<T*>(a.dqkv), a.dqkv_rs, a.dtemp_tok, a.B, a.S, a.Hq, a.Hkv, a.hd, a.flags, a.yq_b, a.yk_b,
+        a.y_h, a.y_s);
+    return check_launch("ccgqa_prep_bwd_kernel");
+  });
+}
+
 }  // namespace hydra
 
 using namespace hydra;
@@ -288,23 +499,10 @@ extern "C" int hydra_ccgqa_prep_bwd(const void* qkv, int64_t qkv_rs, const void*
   HYDRA_REQUIRE(!(flags & HYDRA_CCGQA_ROPE) || (cos && sin && cs_rs >= hd / 2),
                 "ccgqa_prep_bwd: cos/sin [S, hd/2] required");
   HYDRA_REQUIRE(B * S < (int64_t(1) << 31), "ccgqa_prep_bwd: too many tokens");
-  auto st = static_cast<hipStream_t>(stream);
-  const size_t lds = static_cast<size_t>(kPbThreads / 64) * (2 * CW + 2 * (Hq + Hkv)) * sizeof(float);
-  const int64_t ntok = B * S;
-  const unsigned grid = static_cast<unsigned>(std::min<int64_t>((ntok + 3) / 4, 8192));
-  return HYDRA_DISPATCH_DTYPE(dtype, T, [&] {
-    auto kern = ccgqa_prep_bwd_kernel<T>;
-    if (lds > 64 * 1024 &&
-        hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)) != hipSuccess)
-      return fail(HYDRA_ERR_LAUNCH, "ccgqa_prep_bwd: cannot set the kernel's LDS size");
-    kern<<<grid, kPbThreads, lds, st>>>(
-        static_cast<const T*>(qkv), qkv_rs, static_cast<const T*>(y2q), static_cast<const T*>(y2k),
-        static_cast<const T*>(temp), cos, sin, cs_rs, static_cast<const T*>(dq),
-        static_cast<const T*>(dk), static_cast<const T*>(dv), static_cast<T*>(dy),
-        static_cast<T*>(dqkv), dqkv_rs, dtemp_tok, (int)B, (int)S, (int)Hq, (int)Hkv, (int)hd, flags);
-    return check_launch("ccgqa_prep_bwd_kernel");
-  });
+  return launch_prep_bwd(PrepBwdArgs{qkv, qkv_rs, y2q, y2k, Hq * S * hd, Hkv * S * hd, S * hd, hd, temp, cos, sin,
+                                     cs_rs, dq, dk, dv, dy, dqkv, dqkv_rs, dtemp_tok, static_cast<int>(B),
+                                     static_cast<int>(S), static_cast<int>(Hq), static_cast<int>(Hkv),
+                                     static_cast<int>(hd), flags, dtype, static_cast<hipStream_t>(stream)});
 }
 
 extern "C" int hydra_causal_im2col(const void* x, int64_t x_rs, void* out, int64_t B, int64_t S,

@@ -238,6 +238,28 @@ int hydra_ccgqa_prep_bwd(const void* qkv, int64_t qkv_rs, const void* y2q,
                          int64_t Hq, int64_t Hkv, int64_t hd, int flags, int dtype,
                          void* stream);
 
+/* The whole backward of the bf16 q/k/v preparation with three-tap convs: from
+ * qkv, the Conv1d weights (wq1 [L, hd, 3], wq2 [L, L, 3], wk1 [K, hd, 3], wk2
+ * [K, K, 3], contiguous), the temperature and RoPE tables of the forward, and
+ * dq/dk/dv [B, H, S, hd]: dqkv [B*S, L+2K] (row stride dqkv_rs), the weights'
+ * gradients in the weights' layouts and dtemp (one value; NULL: not wanted).
+ * Replaces autograd through attention.py:205-266 and fused_conv.py:39-62.
+ * hydra_ccgqa_prep_bwd_conv_workspace returns the scratch bytes, or -1 where
+ * the sizes or the type are not taken (head_dim other than 8 .. 128 by powers
+ * of two, K % 16 != 0, L + K > 2048, other dtypes or tap counts, no convs): the
+ * caller then composes hydra_ccgqa_prep_bwd, hydra_causal_im2col / _col2im and
+ * GEMMs.  Returns HYDRA_ERR_UNSUPPORTED for rows off 16-byte boundaries. */
+int64_t hydra_ccgqa_prep_bwd_conv_workspace(int64_t B, int64_t S, int64_t Hq, int64_t Hkv,
+                                            int64_t hd, int64_t conv_ks, int flags, int dtype);
+int hydra_ccgqa_prep_bwd_conv(const void* qkv, int64_t qkv_rs, const void* wq1, const void* wq2,
+                              const void* wk1, const void* wk2, const void* temp,
+                              const float* cos, const float* sin, int64_t cs_rs, const void* dq,
+                              const void* dk, const void* dv, void* dqkv, int64_t dqkv_rs,
+                              void* dwq1, void* dwq2, void* dwk1, void* dwk2, void* dtemp,
+                              int64_t B, int64_t S, int64_t Hq, int64_t Hkv, int64_t hd,
+                              int64_t conv_ks, int flags, int dtype, void* workspace,
+                              int64_t workspace_bytes, void* stream);
+
 /* The `taps`-tap causal conv of OptimizedConvSequence (kernels/fused_conv.py:
  * 52-57, left padding taps-1 per batch row) as a GEMM operand: x [B,S,G*cg]
  * (row stride x_rs) -> out [G][B*S][taps*cg] contiguous,

@@ -1,0 +1,72 @@
+"""GPU parity of the bf16 prep backward in one call (hydra_ccgqa_prep_bwd_conv)
+at the edges of its tiles: token counts around the 128-token conv tiles and
+64-token weight-gradient steps, channel counts off and on the 64-channel
+blocks, groups narrower than, as wide as and wider than a block, one and
+several heads, and head_dim 24, which stays on the composed path.
+
+Reference: fp64 autograd through the oracle's prep on the same bf16 inputs.
+Error: 2-norm of the difference over 2-norm of the gradient.  A gradient passes
+at most four bf16 roundings (y1, the pre-norm value, dy2, dy1) of 2^-8 each
+before its own: 2^-6 bounds them with the output's."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from oracle import ccgqa as occ
+
+pytestmark = pytest.mark.gpu
+
+NAMES = ("q_conv.conv1.weight", "q_conv.conv2.weight", "k_conv.conv1.weight", "k_conv.conv2.weight")
+
+
+def _grads(cuda, B, S, Hq, Hkv, hd, features):
+    from hydra_amd.attention.backends.ccgqa.autograd import ccgqa_prep_train
+    from hydra_amd.attention.backends.ccgqa.ops import prep_flags
+
+    use_mean, use_shift, use_norm, use_rope = features
+    cfg = occ.CCGQAConfig(dim=4 * Hq * hd, n_heads=Hq, n_kv_heads=Hkv, compression_factor=4, max_seq_len=512,
+                          use_qk_mean=use_mean, use_value_shift=use_shift, use_qk_norm=use_norm, use_rope=use_rope)
+    g = torch.Generator().manual_seed(S * 7 + hd + Hq)
+    L, K = Hq * hd, Hkv * hd
+    params = {k: v.to(torch.bfloat16) for k, v in occ.init_params(cfg, g, std=0.1, temperature=1.7).items()}
+    rand = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)  # noqa: E731
+    qkv, gq, gk, gv = rand(B, S, L + 2 * K), rand(B, Hq, S, hd), rand(B, Hkv, S, hd), rand(B, Hkv, S, hd)
+    cos, sin = occ.fused_ops.rope_cache(hd, S)
+    p64 = {k: v.double().requires_grad_() for k, v in params.items()}
+    x64 = qkv.double().requires_grad_()
+    q, k, v = occ.prep(p64, x64, cfg, cos.double(), sin.double())
+    wrt = [x64] + [p64[n] for n in NAMES] + ([p64["key_temperature"]] if use_norm else [])
+    ref = torch.autograd.grad((q * gq.double()).sum() + (k * gk.double()).sum() + (v * gv.double()).sum(), wrt)
+
+    dp = {k: v.to(cuda).requires_grad_() for k, v in params.items()}
+    xd = qkv.to(cuda).requires_grad_()
+    flags = prep_flags(True, use_mean, use_shift, use_norm, use_rope)
+    outs = ccgqa_prep_train(xd, Hq, Hkv, hd, flags, *(dp[n] for n in NAMES),
+                            temperature=dp["key_temperature"] if use_norm else None,
+                            cos=cos.to(cuda) if use_rope else None, sin=sin.to(cuda) if use_rope else None)
+    wrt = [xd] + [dp[n] for n in NAMES] + ([dp["key_temperature"]] if use_norm else [])
+    return torch.autograd.grad(outs, wrt, [t.to(cuda) for t in (gq, gk, gv)]), ref
+
+
+def _check(got, ref):
+    for i, (a, r) in enumerate(zip(got, ref)):
+        a = a.double().cpu()
+        assert a.shape == r.shape and torch.isfinite(a).all(), i
+        # the temperature's one value is a sum of signed terms: compare it on
+        # the scale of the terms' own rounding, not of what remains
+        err = float((a - r).norm() / r.norm()) if r.numel() > 1 else float((a - r).abs() / (1 + r.abs()))
+        assert err < 2.0 ** -6 if r.numel() > 1 else err < 0.1, f"output {i}: {err:.3g}"
+
+
+@pytest.mark.parametrize("heads", [(2, 2, 8), (4, 2, 16), (28, 4, 16), (3, 3, 32), (6, 2, 32), (8, 2, 64), (2, 1, 128),
+                                   (4, 2, 128), (2, 1, 24)])
+@pytest.mark.parametrize("B,S", [(1, 1), (2, 2), (1, 64), (1, 127), (3, 129), (2, 200)])
+def test_conv_backward_shapes(cuda, heads, B, S):
+    _check(*_grads(cuda, B, S, *heads, (True, True, True, True)))
+
+
+@pytest.mark.parametrize("features", [(False, False, False, False), (True, False, False, True),
+                                      (False, True, True, False)])
+def test_conv_backward_features(cuda, features):
+    _check(*_grads(cuda, 2, 70, 4, 2, 32, features))
