@@ -66,6 +66,7 @@ SIGNATURES = {
     "hydra_ccgqa_prep_faults": [_P],
     "hydra_ccgqa_prep_bwd": [_P, _I64, _P, _P, _P, _P, _P, _I64, _P, _P, _P, _P, _P, _I64, _P,
                              _I64, _I64, _I64, _I64, _I64, _I, _I, _P],
+    "hydra_ccgqa_pack_conv_tiled": [_P, _P, _P, _P, _P, _I64, _I64, _I64, _I, _P],
     "hydra_ccgqa_prep_bwd_conv_workspace": [_I64, _I64, _I64, _I64, _I64, _I64, _I, _I],
     "hydra_ccgqa_prep_bwd_conv": [_P, _I64, _P, _P, _P, _P, _P, _P, _P, _I64, _P, _P, _P, _P, _I64, _P, _P,
                                   _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I, _I, _P, _I64, _P],

@@ -35,6 +35,27 @@ def pack_conv_weight(w: torch.Tensor, dtype: torch.dtype, tiled: bool = False) -
     return t.reshape(k, O // 32, 32, I // 16, 2, 8).permute(0, 1, 3, 4, 2, 5).contiguous()
 
 
+def pack_conv_weights_tiled(ws, dtype: torch.dtype, n_heads: int, n_kv_heads: int, head_dim: int):
+    """The four conv weights (wq1, wq2, wk1, wk2) in MFMA-fragment order, as
+    pack_conv_weight(w, dtype, True) gives them, in one launch where they are
+    in `dtype` already (hydra_ccgqa_pack_conv_tiled)."""
+    ws = tuple(w.detach() for w in ws)
+    L, K = n_heads * head_dim, n_kv_heads * head_dim
+    shapes = ((L, head_dim), (L, L), (K, head_dim), (K, K))
+    if dtype not in (torch.bfloat16, torch.float16) or any(
+            w.dtype != dtype or not w.is_contiguous() or w.shape != (*s, 3) for w, s in zip(ws, shapes)):
+        return tuple(pack_conv_weight(w, dtype, True) for w in ws)
+    out = torch.empty(sum(w.numel() for w in ws), dtype=dtype, device=ws[0].device)
+    with torch.cuda.device(out.device):
+        _lib.call("hydra_ccgqa_pack_conv_tiled", *(w.data_ptr() for w in ws), out.data_ptr(), n_heads, n_kv_heads,
+                  head_dim, _lib.dtype_code(out), _lib.stream(out))
+    packed, at = [], 0
+    for (o, i), w in zip(shapes, ws):
+        packed.append(out[at:at + w.numel()].view(3, o // 32, i // 16, 2, 32, 8))
+        at += w.numel()
+    return tuple(packed)
+
+
 def tiled_weights_ok(n_heads: int, n_kv_heads: int, head_dim: int, dtype: torch.dtype) -> bool:
     """Whether the prep kernel takes its MFMA path for this head layout and
     dtype, i.e. accepts CCGQA_W_TILED weights."""
@@ -66,8 +87,10 @@ def ccgqa_prep(qkv: torch.Tensor, n_heads: int, n_kv_heads: int, head_dim: int, 
         tiled = bool(flags & CCGQA_W_TILED)
         if packed:
             ws = tuple(w.to(dt).contiguous() for w in ws)
+        elif tiled:
+            ws = pack_conv_weights_tiled(ws, dt, n_heads, n_kv_heads, head_dim)
         else:
-            ws = tuple(pack_conv_weight(w, dt, tiled) for w in ws)
+            ws = tuple(pack_conv_weight(w, dt) for w in ws)
         ks = conv_ks
         exp = [(ks, L, head_dim), (ks, L, L), (ks, K, head_dim), (ks, K, K)]
         if tiled:

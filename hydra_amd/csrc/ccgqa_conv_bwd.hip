@@ -26,12 +26,13 @@
 // that used to be a launch of its own (im2col, col2im, transposing copies,
 // ~45 launches in all) is part of one of eight.
 //
-// Measured at B4 x S1024, dim 2048, 8/2 heads x 64 (kernel trace): pack 12 us,
-// y1 10 and y2 26, pointwise 17 (34 as one token per wave), dy1 27, grad(x0)
-// 11, weight gradients 22 + 11; the composed form took ~430 us of kernels in
-// ~45 launches.  Whole layer steps: that shape 1.32 -> 0.84 ms, 28/4 heads x
-// 16 at B2 x S2048 1.40 -> 0.87, padded B8 x S777 4/1 x 64 1.41 -> 0.92 (all
-// bound by the host's launches now).
+// Measured at B4 x S1024, dim 2048, 8/2 heads x 64 (kernel trace): pack 6 us
+// (12 with one packed piece per thread), y1 7 and y2 14 (26 with the staged
+// pieces in scratch memory and four waves), pointwise 17 (34 as one token per
+// wave), dy1 14, grad(x0) 9, weight gradients 22 + 11; the composed form took
+// ~430 us of kernels in ~45 launches.  Whole layer steps: that shape 1.32 ->
+// 0.78 ms, padded B8 x S777 4/1 x 64 1.41 -> 0.85, 28/4 heads x 16 at B2 x
+// S2048 1.40 -> 0.87 (bound by the host's launches now).
 #include "ccgqa_prep_bwd.h"
 #include "common.h"
 
@@ -49,6 +50,7 @@ constexpr int kTaps = 3;
 constexpr int kWBlk = kTaps * kBlk * kBlk;      // one packed weight block
 constexpr int kPitch = kBlk + 8;                // LDS row pitch (elements): 16-byte rows, 4-bank skew
 constexpr int kTM = 128;                        // tokens per conv tile
+constexpr int kConvThreads = 512;
 constexpr int kWT = 64;                         // tokens per weight-gradient step
 
 __device__ __forceinline__ f32x16_t mfma(uint4 a, uint4 b, f32x16_t c) {
@@ -82,13 +84,17 @@ struct PackJob {
   uint16_t* out;
   Blocks b;
   int transposed;
-  int first;      // its first 8-element piece
+  int first;      // its first piece (8 input channels of an output channel)
 };
 struct PackArgs {
   PackJob job[8];
   int pieces;
 };
 
+// A thread takes 8 input channels of one output channel, all taps: forward its
+// 24 source values are one run (neighbouring threads: neighbouring runs);
+// transposed they lie in 8 source rows, and neighbouring threads take
+// neighbouring output channels, so that each row is still read in order.
 __global__ __launch_bounds__(256) void conv_pack_kernel(PackArgs a) {
   const int p = blockIdx.x * 256 + threadIdx.x;
   if (p >= a.pieces) return;
@@ -96,21 +102,31 @@ __global__ __launch_bounds__(256) void conv_pack_kernel(PackArgs a) {
 #pragma unroll
   for (int k = 1; k < 8; ++k) j = p >= a.job[k].first ? k : j;
   const PackJob& q = a.job[j];
-  const int e = (p - q.first) * 8;
-  const int blk = e / kWBlk, rem = e - blk * kWBlk;
-  const int t = rem / (kBlk * kBlk), o = rem / kBlk % kBlk, i = rem % kBlk;
+  const int e = p - q.first, blk = e / (kBlk * kBlk / 8), rem = e % (kBlk * kBlk / 8);
+  const int o = q.transposed ? rem % kBlk : rem / 8, i = 8 * (q.transposed ? rem / kBlk : rem % 8);
   const int ob = blk / q.b.span, ib = q.b.first(ob) + blk % q.b.span;
-  const int oc = kBlk * ob + o;
-  uint16_t v[8];
+  const int oc = kBlk * ob + o, ic = kBlk * ib + i;
+  uint32_t v[kTaps][8];
+  const bool ok = oc < q.b.C && ic < q.b.C && oc / q.b.cg == ic / q.b.cg;  // all 8: groups are of 8 k channels
+  if (!ok) {
 #pragma unroll
-  for (int u = 0; u < 8; ++u) {
-    const int ic = kBlk * ib + i + u;
-    const int row = q.transposed ? ic : oc, col = q.transposed ? oc : ic;
-    const bool ok = oc < q.b.C && ic < q.b.C && row / q.b.cg == col / q.b.cg;
-    v[u] = ok ? q.w[(static_cast<int64_t>(row) * q.b.cg + col % q.b.cg) * kTaps + t].bits : 0;
+    for (int t = 0; t < kTaps; ++t)
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[t][u] = 0;
+  } else {
+    const int row = q.transposed ? ic : oc, col = (q.transposed ? oc : ic) % q.b.cg;
+    const int64_t step = q.transposed ? static_cast<int64_t>(q.b.cg) * kTaps : kTaps;
+    const bf16* w = q.w + (static_cast<int64_t>(row) * q.b.cg + col) * kTaps;
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+      for (int t = 0; t < kTaps; ++t) v[t][u] = w[u * step + t].bits;
   }
-  *reinterpret_cast<uint4*>(q.out + e) =
-      make_uint4(v[0] | v[1] << 16, v[2] | v[3] << 16, v[4] | v[5] << 16, v[6] | v[7] << 16);
+  uint16_t* out = q.out + static_cast<int64_t>(blk) * kWBlk + o * kBlk + i;
+#pragma unroll
+  for (int t = 0; t < kTaps; ++t)
+    *reinterpret_cast<uint4*>(out + t * kBlk * kBlk) =
+        make_uint4(v[t][0] | v[t][1] << 16, v[t][2] | v[t][3] << 16, v[t][4] | v[t][5] << 16, v[t][6] | v[t][7] << 16);
 }
 
 // ------------------------------------------------------------------- conv
@@ -127,32 +143,40 @@ struct ConvArgs {
   int S, tiles, ntiles;  // token tiles per sequence, over all sequences
 };
 
-// job[second], field by field (an indexed copy of the argument struct would go
-// through scratch memory).
+// job[second], value by value (an indexed access, or a conditional that names
+// the fields, would go through a copy in scratch memory).
+template <typename V>
+__device__ __forceinline__ V pick(bool second, V q, V p) {
+  return second ? q : p;
+}
 __device__ __forceinline__ ConvJob conv_job(const ConvArgs& a, bool second) {
   const ConvJob &p = a.job[0], &q = a.job[1];
   ConvJob j;
-  j.x = second ? q.x : p.x;
-  j.y = second ? q.y : p.y;
-  j.w = second ? q.w : p.w;
-  j.xrs = second ? q.xrs : p.xrs;
-  j.yrs = second ? q.yrs : p.yrs;
-  j.b.C = second ? q.b.C : p.b.C;
-  j.b.cg = second ? q.b.cg : p.b.cg;
-  j.b.n = second ? q.b.n : p.b.n;
-  j.b.span = second ? q.b.span : p.b.span;
-  j.b.dense = second ? q.b.dense : p.b.dense;
-  j.first = second ? q.first : p.first;
+  j.x = pick(second, q.x, p.x);
+  j.y = pick(second, q.y, p.y);
+  j.w = pick(second, q.w, p.w);
+  j.xrs = pick(second, q.xrs, p.xrs);
+  j.yrs = pick(second, q.yrs, p.yrs);
+  j.b.C = pick(second, q.b.C, p.b.C);
+  j.b.cg = pick(second, q.b.cg, p.b.cg);
+  j.b.n = pick(second, q.b.n, p.b.n);
+  j.b.span = pick(second, q.b.span, p.b.span);
+  j.b.dense = pick(second, q.b.dense, p.b.dense);
+  j.first = pick(second, q.first, p.first);
   return j;
 }
 
 // BACK: tap t reads token s + 2 - t (a conv's transpose), else s - (2 - t).
 // ACC: adds to the output rows.
+// Eight waves, each 32 tokens x 32 output channels: two per SIMD, which hides
+// the LDS and L2 latency of a grid of about one workgroup per CU better than
+// four waves of 32 x 64 did (the reads per product go from 1.5 to 2 fragments).
 template <bool BACK, bool ACC>
-__global__ __launch_bounds__(256) void conv_kernel(ConvArgs a) {
+__global__ __launch_bounds__(kConvThreads) void conv_kernel(ConvArgs a) {
+  constexpr int NT = kConvThreads;
   constexpr int XR = kTM + kTaps - 1;                          // staged token rows
-  constexpr int XU = (XR * (kBlk / 8) + 255) / 256;            // 16-byte pieces per thread
-  constexpr int WU = kWBlk / 8 / 256;
+  constexpr int XU = (XR * (kBlk / 8) + NT - 1) / NT;          // 16-byte pieces per thread
+  constexpr int WU = kWBlk / 8 / NT;
   __shared__ __attribute__((aligned(16))) uint16_t xs[XR * kPitch], ws[kTaps * kBlk * kPitch];
   const ConvJob q = conv_job(a, static_cast<int>(blockIdx.x) >= a.job[1].first);
   const int idx = blockIdx.x - q.first;
@@ -162,6 +186,7 @@ __global__ __launch_bounds__(256) void conv_kernel(ConvArgs a) {
   const int b = tile / a.tiles, s0 = kTM * (tile - b * a.tiles);
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, hf = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wt = 32 * (wave & 3), wc = 32 * (wave >> 2);  // this wave's tokens and channels
   const int ib0 = q.b.first(ob);
   const uint16_t* x = q.x + static_cast<int64_t>(b) * a.S * q.xrs;
   uint4 rx[XU], rw[WU];
@@ -169,27 +194,27 @@ __global__ __launch_bounds__(256) void conv_kernel(ConvArgs a) {
     const int c0 = kBlk * (ib0 + it);
 #pragma unroll
     for (int u = 0; u < XU; ++u) {
-      const int i = tid + 256 * u, row = i >> 3, c = c0 + 8 * (i & 7);
+      const int i = tid + NT * u, row = i >> 3, c = c0 + 8 * (i & 7);
       const int s = s0 + row - (BACK ? 0 : kTaps - 1);
-      rx[u] = row < XR && s >= 0 && s < a.S && c < q.b.C
-                  ? *reinterpret_cast<const uint4*>(x + s * q.xrs + c) : make_uint4(0, 0, 0, 0);
+      rx[u] = make_uint4(0, 0, 0, 0);
+      if (row < XR && s >= 0 && s < a.S && c < q.b.C) rx[u] = ld16raw<false>(x + s * q.xrs + c);
     }
     const uint16_t* w = q.w + static_cast<int64_t>(ob * q.b.span + it) * kWBlk;
 #pragma unroll
-    for (int u = 0; u < WU; ++u) rw[u] = *reinterpret_cast<const uint4*>(w + 8 * (tid + 256 * u));
+    for (int u = 0; u < WU; ++u) rw[u] = ld16raw<false>(w + 8 * (tid + NT * u));
   };
-  f32x16_t acc[2] = {zero16(), zero16()};
+  f32x16_t acc = zero16();
   fetch(0);
   for (int it = 0; it < q.b.span; ++it) {
     if (it) __syncthreads();  // the previous tile's readers are done
 #pragma unroll
     for (int u = 0; u < XU; ++u) {
-      const int i = tid + 256 * u, row = i >> 3;
+      const int i = tid + NT * u, row = i >> 3;
       if (row < XR) *reinterpret_cast<uint4*>(&xs[row * kPitch + 8 * (i & 7)]) = rx[u];
     }
 #pragma unroll
     for (int u = 0; u < WU; ++u) {
-      const int i = tid + 256 * u;
+      const int i = tid + NT * u;
       *reinterpret_cast<uint4*>(&ws[(i >> 3) * kPitch + 8 * (i & 7)]) = rw[u];
     }
     __syncthreads();
@@ -198,39 +223,33 @@ __global__ __launch_bounds__(256) void conv_kernel(ConvArgs a) {
     for (int ks = 0; ks < kBlk / 16; ++ks)
 #pragma unroll
       for (int t = 0; t < kTaps; ++t) {
-        const int xrow = 32 * wave + n + (BACK ? kTaps - 1 - t : t);
+        const int xrow = wt + n + (BACK ? kTaps - 1 - t : t);
         const uint4 xf = *reinterpret_cast<const uint4*>(&xs[xrow * kPitch + 16 * ks + 8 * hf]);
-#pragma unroll
-        for (int m = 0; m < 2; ++m) {
-          const uint4 wf =
-              *reinterpret_cast<const uint4*>(&ws[(kBlk * t + 32 * m + n) * kPitch + 16 * ks + 8 * hf]);
-          acc[m] = mfma(wf, xf, acc[m]);
-        }
+        const uint4 wf = *reinterpret_cast<const uint4*>(&ws[(kBlk * t + wc + n) * kPitch + 16 * ks + 8 * hf]);
+        acc = mfma(wf, xf, acc);
       }
   }
   // a lane holds one token's channels, four consecutive ones per register group
-  const int s = s0 + 32 * wave + n;
+  const int s = s0 + wt + n;
   if (s >= a.S) return;
   uint16_t* y = q.y + (static_cast<int64_t>(b) * a.S + s) * q.yrs;
 #pragma unroll
-  for (int m = 0; m < 2; ++m)
+  for (int j = 0; j < 4; ++j) {
+    const int c = kBlk * ob + wc + 8 * j + 4 * hf;
+    if (c >= q.b.C) continue;
+    float f[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int c = kBlk * ob + 32 * m + 8 * j + 4 * hf;
-      if (c >= q.b.C) continue;
-      float f[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) f[r] = acc[m][4 * j + r];
-      uint2* dst = reinterpret_cast<uint2*>(y + c);
-      if constexpr (ACC) {
-        const uint2 old = *dst;
-        f[0] += __uint_as_float(old.x << 16);
-        f[1] += __uint_as_float(old.x & 0xffff0000u);
-        f[2] += __uint_as_float(old.y << 16);
-        f[3] += __uint_as_float(old.y & 0xffff0000u);
-      }
-      *dst = make_uint2(pack2<bf16>(f[0], f[1]), pack2<bf16>(f[2], f[3]));
+    for (int r = 0; r < 4; ++r) f[r] = acc[4 * j + r];
+    uint2* dst = reinterpret_cast<uint2*>(y + c);
+    if constexpr (ACC) {
+      const uint2 old = *dst;
+      f[0] += __uint_as_float(old.x << 16);
+      f[1] += __uint_as_float(old.x & 0xffff0000u);
+      f[2] += __uint_as_float(old.y << 16);
+      f[3] += __uint_as_float(old.y & 0xffff0000u);
     }
+    *dst = make_uint2(pack2<bf16>(f[0], f[1]), pack2<bf16>(f[2], f[3]));
+  }
 }
 
 // ------------------------------------------------------- weight gradients
@@ -422,7 +441,7 @@ int launch_conv(const ConvJob& jq, const ConvJob& jk, int64_t B, int64_t S, hipS
   a.ntiles = static_cast<int>(B) * a.tiles;
   a.job[0].first = 0;
   a.job[1].first = jq.b.n * a.ntiles;
-  conv_kernel<BACK, ACC><<<dim3(static_cast<unsigned>((jq.b.n + jk.b.n) * a.ntiles)), 256, 0, st>>>(a);
+  conv_kernel<BACK, ACC><<<dim3(static_cast<unsigned>((jq.b.n + jk.b.n) * a.ntiles)), kConvThreads, 0, st>>>(a);
   return check_launch("ccgqa_conv_bwd: conv");
 }
 
@@ -468,7 +487,7 @@ extern "C" int hydra_ccgqa_prep_bwd_conv(const void* qkv, int64_t qkv_rs, const 
   PackArgs pk{};
   for (int i = 0; i < 8; ++i) {
     pk.job[i] = PackJob{w[i & 3], reinterpret_cast<uint16_t*>(ws + p.pack[i]), p.b[i & 3], i >> 2, pk.pieces};
-    pk.pieces += p.b[i & 3].n * p.b[i & 3].span * (kWBlk / 8);
+    pk.pieces += p.b[i & 3].n * p.b[i & 3].span * (kBlk * kBlk / 8);
   }
   conv_pack_kernel<<<dim3(static_cast<unsigned>((pk.pieces + 255) / 256)), 256, 0, st>>>(pk);
   if (int rc = check_launch("ccgqa_conv_bwd: pack")) return rc;

@@ -1274,6 +1274,66 @@ extern "C" int hydra_ccgqa_prep_faults(unsigned int* count) {
   return HYDRA_OK;
 }
 
+namespace hydra {
+// Conv1d weights [O][I][3] -> the MFMA-fragment order of HYDRA_CCGQA_W_TILED,
+// [3][O/32][I/16][2][32][8], four weights in one launch.  A thread takes 8
+// input channels of one output channel, all taps: 24 consecutive values in,
+// three 16-byte pieces out (neighbouring threads: neighbouring output
+// channels, i.e. neighbouring pieces).
+struct TilePackArgs {
+  const uint16_t* w[4];
+  uint16_t* out[4];
+  int O[4], I[4], first[4];
+  int pieces;
+};
+__global__ __launch_bounds__(256) void conv_pack_tiled_kernel(TilePackArgs a) {
+  const int p = blockIdx.x * 256 + threadIdx.x;
+  if (p >= a.pieces) return;
+  int j = 0;
+#pragma unroll
+  for (int k = 1; k < 4; ++k) j = p >= a.first[k] ? k : j;
+  const int e = p - a.first[j], O = a.O[j], I = a.I[j];
+  const int o = e % O, i = 8 * (e / O);
+  const uint16_t* w = a.w[j] + (static_cast<int64_t>(o) * I + i) * 3;
+  uint32_t v[3][8];
+#pragma unroll
+  for (int u = 0; u < 8; ++u)
+#pragma unroll
+    for (int t = 0; t < 3; ++t) v[t][u] = w[3 * u + t];
+  uint16_t* out = a.out[j] + (((static_cast<int64_t>(o / 32) * (I / 16) + i / 16) * 2 + i / 8 % 2) * 32 + o % 32) * 8;
+#pragma unroll
+  for (int t = 0; t < 3; ++t)
+    *reinterpret_cast<uint4*>(out + static_cast<int64_t>(t) * O * I) =
+        make_uint4(v[t][0] | v[t][1] << 16, v[t][2] | v[t][3] << 16, v[t][4] | v[t][5] << 16, v[t][6] | v[t][7] << 16);
+}
+}  // namespace hydra
+
+extern "C" int hydra_ccgqa_pack_conv_tiled(const void* wq1, const void* wq2, const void* wk1, const void* wk2, void* out,
+                                           int64_t Hq, int64_t Hkv, int64_t hd, int dtype, void* stream) {
+  HYDRA_REQUIRE(Hq >= 1 && Hkv >= 1 && hd >= 1, "ccgqa_pack_conv_tiled: bad size");
+  const int64_t L = Hq * hd, K = Hkv * hd;
+  HYDRA_REQUIRE(dtype == HYDRA_BF16 || dtype == HYDRA_F16, "ccgqa_pack_conv_tiled: 16-bit weights only");
+  HYDRA_REQUIRE(hd % 16 == 0 && L % 32 == 0 && K % 32 == 0, "ccgqa_pack_conv_tiled: the order needs hd % 16, L % 32 and K % 32 == 0");
+  HYDRA_REQUIRE(L * L + K * K < (int64_t(1) << 28), "ccgqa_pack_conv_tiled: too large");
+  HYDRA_REQUIRE(wq1 && wq2 && wk1 && wk2 && out && hydra::aligned16(out), "ccgqa_pack_conv_tiled: null or unaligned pointer");
+  const void* w[4] = {wq1, wq2, wk1, wk2};
+  const int64_t O[4] = {L, L, K, K}, I[4] = {hd, L, hd, K};
+  hydra::TilePackArgs a{};
+  auto dst = static_cast<uint16_t*>(out);
+  for (int i = 0; i < 4; ++i) {
+    a.w[i] = static_cast<const uint16_t*>(w[i]);
+    a.out[i] = dst;
+    a.O[i] = static_cast<int>(O[i]);
+    a.I[i] = static_cast<int>(I[i]);
+    a.first[i] = a.pieces;
+    a.pieces += static_cast<int>(O[i] * I[i] / 8);
+    dst += 3 * O[i] * I[i];
+  }
+  hydra::conv_pack_tiled_kernel<<<dim3(static_cast<unsigned>((a.pieces + 255) / 256)), 256, 0,
+                                  static_cast<hipStream_t>(stream)>>>(a);
+  return hydra::check_launch("conv_pack_tiled_kernel");
+}
+
 extern "C" int hydra_ccgqa_prep_tiled_ok(int64_t Hq, int64_t Hkv, int64_t hd, int dtype) {
   if (Hq < 1 || Hkv < 1 || Hq % Hkv != 0) return 0;
   if (dtype != HYDRA_BF16 || !(hd == 16 || hd == 32 || hd == 64 || hd == 128)) return 0;

@@ -238,6 +238,13 @@ int hydra_ccgqa_prep_bwd(const void* qkv, int64_t qkv_rs, const void* y2q,
                          int64_t Hq, int64_t Hkv, int64_t hd, int flags, int dtype,
                          void* stream);
 
+/* The four conv weights (Conv1d layout, contiguous, 16-bit) into the order of
+ * HYDRA_CCGQA_W_TILED in one launch: out holds wq1's 3*L*hd elements, then
+ * wq2's 3*L*L, wk1's 3*K*hd and wk2's 3*K*K (hd % 16, L % 32, K % 32 == 0). */
+int hydra_ccgqa_pack_conv_tiled(const void* wq1, const void* wq2, const void* wk1,
+                                const void* wk2, void* out, int64_t Hq, int64_t Hkv, int64_t hd,
+                                int dtype, void* stream);
+
 /* The whole backward of the bf16 q/k/v preparation with three-tap convs: from
  * qkv, the Conv1d weights (wq1 [L, hd, 3], wq2 [L, L, 3], wk1 [K, hd, 3], wk2
  * [K, K, 3], contiguous), the temperature and RoPE tables of the forward, and
