@@ -9,7 +9,9 @@ the call raises.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
+import functools
 import os
 from pathlib import Path
 
@@ -23,6 +25,7 @@ F32, BF16, F16 = 0, 1, 2
 CCGQA_CONVS, CCGQA_QK_MEAN, CCGQA_VALUE_SHIFT, CCGQA_QK_NORM, CCGQA_ROPE = 1, 2, 4, 8, 16
 CCGQA_V_TRANSPOSED = 32
 CCGQA_W_TILED = 64
+CCGQA_ROPE_BF16 = 256
 MASK_NONE, MASK_KEY_PADDING, MASK_REFERENCE_SDPA = 0, 1, 2
 SCATTER_ADD, SCATTER_REPLACE, SCATTER_ADD_SEQ = 0, 1, 2
 NORM_NONE, NORM_RMS, NORM_ADA = 0, 1, 2
@@ -183,13 +186,38 @@ def ptr(t) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+@functools.lru_cache(maxsize=1024)
+def _stride_array(values):
+    return (ctypes.c_int64 * len(values))(*values)
+
+
 def strides(t: torch.Tensor):
-    arr = (ctypes.c_int64 * t.dim())(*t.stride())
-    return arr
+    """t's strides as a C array (shared by equal strides: the library only
+    reads it)."""
+    return _stride_array(t.stride())
 
 
 def stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """torch's current stream of t's device, as the raw handle."""
+    return _raw_stream(t.device.index)
+
+
+def _raw_stream_of(index: int) -> int:
+    return torch.cuda.current_stream(index).cuda_stream
+
+
+# torch's own accessor without the Stream object around the handle (~1 us
+# less per launch), where this torch has it
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", _raw_stream_of)
+
+_HERE = contextlib.nullcontext()
+
+
+def on_device(t: torch.Tensor):
+    """Context with t's device current: nothing to do when it already is,
+    which is every launch of a one-GPU process (switching costs ~4 us)."""
+    index = t.device.index
+    return _HERE if torch.cuda.current_device() == index else torch.cuda.device(index)
 
 
 def require_gpu(name: str, *tensors) -> None:

@@ -25,7 +25,7 @@ from __future__ import annotations
 
 import torch
 
-from ...._lib import CCGQA_CONVS, CCGQA_QK_NORM, CCGQA_ROPE, CCGQA_W_TILED
+from ...._lib import CCGQA_CONVS, CCGQA_QK_NORM, CCGQA_W_TILED
 from .ops import (causal_col2im, causal_im2col, ccgqa_prep, ccgqa_prep_backward,
                   ccgqa_prep_backward_convs, tiled_weights_ok)
 
@@ -71,10 +71,6 @@ class CCGQAPrepFunction(torch.autograd.Function):
         ks = wq1.shape[-1] if convs else 3
         tiled = convs and ks == 3 and tiled_weights_ok(n_heads, n_kv_heads, head_dim, qkv.dtype)
         fl = flags | (CCGQA_W_TILED if tiled else 0)
-        if flags & CCGQA_ROPE:
-            # in the kernels' form (fp32 [S, hd/2]) once, for the backward too
-            S = qkv.shape[1]
-            cos, sin = ((t[0, 0] if t.dim() == 4 else t)[:S].float().contiguous() for t in (cos, sin))
         q, k, v = ccgqa_prep(qkv, n_heads, n_kv_heads, head_dim, fl, wq1, wq2, wk1, wk2,
                              temperature=temperature, cos=cos, sin=sin, conv_ks=ks)
         ctx.save_for_backward(qkv, wq1, wq2, wk1, wk2, temperature)

@@ -10,7 +10,7 @@ from typing import Optional
 import torch
 import torch.nn.functional as F
 
-from ...._lib import (CCGQA_CONVS, CCGQA_QK_MEAN, CCGQA_QK_NORM, CCGQA_ROPE,
+from ...._lib import (CCGQA_CONVS, CCGQA_QK_MEAN, CCGQA_QK_NORM, CCGQA_ROPE, CCGQA_ROPE_BF16,
                       CCGQA_V_TRANSPOSED, CCGQA_VALUE_SHIFT, CCGQA_W_TILED, MASK_KEY_PADDING, MASK_NONE,
                       MASK_REFERENCE_SDPA)
 from .... import _lib
@@ -46,7 +46,7 @@ def pack_conv_weights_tiled(ws, dtype: torch.dtype, n_heads: int, n_kv_heads: in
             w.dtype != dtype or not w.is_contiguous() or w.shape != (*s, 3) for w, s in zip(ws, shapes)):
         return tuple(pack_conv_weight(w, dtype, True) for w in ws)
     out = torch.empty(sum(w.numel() for w in ws), dtype=dtype, device=ws[0].device)
-    with torch.cuda.device(out.device):
+    with _lib.on_device(out):
         _lib.call("hydra_ccgqa_pack_conv_tiled", *(w.data_ptr() for w in ws), out.data_ptr(), n_heads, n_kv_heads,
                   head_dim, _lib.dtype_code(out), _lib.stream(out))
     packed, at = [], 0
@@ -63,6 +63,22 @@ def tiled_weights_ok(n_heads: int, n_kv_heads: int, head_dim: int, dtype: torch.
         return False
     return _lib.query("hydra_ccgqa_prep_tiled_ok", n_heads, n_kv_heads, head_dim,
                       _lib._DTYPE_CODE[dtype]) == 1
+
+
+def _rope_tables(cos: torch.Tensor, sin: torch.Tensor, S: int, bf16_ok: bool):
+    """RoPE tables [.., Smax, hd/2] as the kernels take them: (cos, sin, row
+    stride, flag), read in place when they are fp32 -- or bf16, where the
+    kernel widens them itself (bf16_ok; flag CCGQA_ROPE_BF16) -- with rows one
+    stride apart; converted otherwise."""
+    if cos.shape[-2] < S:
+        raise ValueError(f"ccgqa_prep: RoPE cache covers {cos.shape[-2]} positions < S={S}")
+    half = bf16_ok and cos.dtype == sin.dtype == torch.bfloat16
+    if (half or cos.dtype == sin.dtype == torch.float32) and cos.stride(-1) == sin.stride(-1) == 1 and \
+            cos.stride(-2) == sin.stride(-2) and cos.stride(-2) % 4 == 0 and \
+            (cos.data_ptr() | sin.data_ptr()) % 16 == 0:
+        return cos, sin, cos.stride(-2), CCGQA_ROPE_BF16 if half else 0
+    cos, sin = ((t[0, 0] if t.dim() == 4 else t)[:S].float().contiguous() for t in (cos, sin))
+    return cos, sin, cos.stride(0), 0
 
 
 def ccgqa_prep(qkv: torch.Tensor, n_heads: int, n_kv_heads: int, head_dim: int, flags: int,
@@ -102,23 +118,20 @@ def ccgqa_prep(qkv: torch.Tensor, n_heads: int, n_kv_heads: int, head_dim: int, 
     else:
         wq1 = wq2 = wk1 = wk2 = None
     temp = None if temperature is None else temperature.detach().to(dt).contiguous()
+    rope_rs = head_dim // 2
     if flags & CCGQA_ROPE:
-        if cos.dim() == 4:
-            cos, sin = cos[0, 0], sin[0, 0]
-        if cos.shape[0] < S:
-            raise ValueError(f"ccgqa_prep: RoPE cache covers {cos.shape[0]} positions < S={S}")
-        cos = cos[:S].float().contiguous()
-        sin = sin[:S].float().contiguous()
+        # MFMA-tiled weights mean the MFMA path, which widens bf16 tables itself
+        cos, sin, rope_rs, rope16 = _rope_tables(cos, sin, S, bool(flags & CCGQA_W_TILED))
+        flags |= rope16
     q = torch.empty((B, n_heads, S, head_dim), dtype=dt, device=qkv.device)
     k = torch.empty((B, n_kv_heads, S, head_dim), dtype=dt, device=qkv.device)
     vt = bool(flags & CCGQA_V_TRANSPOSED)
     v = torch.empty((B, n_kv_heads, head_dim, S) if vt else (B, n_kv_heads, S, head_dim),
                     dtype=dt, device=qkv.device)
-    with torch.cuda.device(qkv.device):
+    with _lib.on_device(qkv):
         _lib.call("hydra_ccgqa_prep_fwd", qkv.data_ptr(), qkv.stride(1), _lib.ptr(wq1),
                   _lib.ptr(wq2), _lib.ptr(wk1), _lib.ptr(wk2), _lib.ptr(temp), _lib.ptr(cos),
-                  _lib.ptr(sin), head_dim // 2 if cos is None else cos.stride(0),
-                  q.data_ptr(), k.data_ptr(), v.data_ptr(), B, S, n_heads, n_kv_heads,
+                  _lib.ptr(sin), rope_rs, q.data_ptr(), k.data_ptr(), v.data_ptr(), B, S, n_heads, n_kv_heads,
                   head_dim, conv_ks, flags, _lib.dtype_code(qkv), _lib.stream(qkv))
     return q, k, (v.transpose(2, 3) if vt else v)
 
@@ -167,7 +180,7 @@ def attention_forward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, caus
             bt = bt.float()
         bt = bt.reshape(-1)[:1].contiguous()
         _lib.require_gpu("attention_forward", bt)
-    with torch.cuda.device(q.device):
+    with _lib.on_device(q):
         st = (_lib.strides(q), _lib.strides(k), _lib.strides(v), _lib.strides(out))
         need = ctypes.c_int64(0)
         _lib.call("hydra_attn_fwd_workspace", B, Hq, Hkv, S, hd, *st, 1 if causal else 0, mask_mode,
@@ -218,7 +231,7 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: t
             raise ValueError(f"attention_backward: key mask must be [B,S] = [{B},{S}]")
         _lib.require_gpu("attention_backward", key_mask)
         km = (key_mask != 0).to(torch.uint8).contiguous()
-    with torch.cuda.device(q.device):
+    with _lib.on_device(q):
         st = (_lib.strides(q), _lib.strides(k), _lib.strides(v), _lib.strides(out),
               _lib.strides(grad_out), _lib.strides(dq), _lib.strides(dk), _lib.strides(dv))
         need = ctypes.c_int64(0)
@@ -317,7 +330,7 @@ def causal_im2col(x: torch.Tensor, groups: int, taps: int = 3) -> torch.Tensor:
         x = x.contiguous()
     cg = C // groups
     out = torch.empty((groups, B * S, taps * cg), dtype=x.dtype, device=x.device)
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x):
         _lib.call("hydra_causal_im2col", x.data_ptr(), x.stride(1), out.data_ptr(), B, S, groups, cg,
                   taps, _lib.dtype_code(x), _lib.stream(x))
     return out
@@ -336,7 +349,7 @@ def causal_col2im(cols: torch.Tensor, out: torch.Tensor, accumulate: bool = Fals
     if out.stride(-1) != 1 or (B > 1 and out.stride(0) != S * out.stride(1)):
         raise ValueError("causal_col2im: out needs unit channel stride and uniform row stride")
     cols = cols.contiguous()
-    with torch.cuda.device(out.device):
+    with _lib.on_device(out):
         _lib.call("hydra_causal_col2im", cols.data_ptr(), out.data_ptr(), out.stride(1), B, S, G,
                   C // G, taps, 1 if accumulate else 0, _lib.dtype_code(out), _lib.stream(out))
     return out
@@ -372,7 +385,7 @@ def ccgqa_prep_backward(qkv: torch.Tensor, n_heads: int, n_kv_heads: int, head_d
             cos, sin = cos[0, 0], sin[0, 0]
         cos = cos[:S].float().contiguous()
         sin = sin[:S].float().contiguous()
-    with torch.cuda.device(qkv.device):
+    with _lib.on_device(qkv):
         _lib.call("hydra_ccgqa_prep_bwd", qkv.data_ptr(), qkv.stride(1), _lib.ptr(y2q), _lib.ptr(y2k),
                   _lib.ptr(temp), _lib.ptr(cos), _lib.ptr(sin),
                   head_dim // 2 if cos is None else cos.stride(0), dq.data_ptr(), dk.data_ptr(),
@@ -409,22 +422,20 @@ def ccgqa_prep_backward_convs(qkv: torch.Tensor, n_heads: int, n_kv_heads: int, 
         qkv = qkv.contiguous()
     dq, dk, dv = (t.to(dt).contiguous() for t in (dq, dk, dv))
     weights = tuple(w.detach().contiguous() for w in weights)
+    rope_rs = head_dim // 2
     if flags & CCGQA_ROPE:
-        if cos.dim() == 4:
-            cos, sin = cos[0, 0], sin[0, 0]
-        cos = cos[:S].float().contiguous()
-        sin = sin[:S].float().contiguous()
+        cos, sin, rope_rs, rope16 = _rope_tables(cos, sin, S, True)
+        flags |= rope16
     else:
         cos = sin = None
     dqkv = torch.empty((B, S, W), dtype=dt, device=qkv.device)
     dws = tuple(torch.empty_like(w) for w in weights)
     dtemp = torch.empty_like(temperature) if norm and want_temperature else None
     ws = _lib.scratch(need, qkv)
-    with torch.cuda.device(qkv.device):
+    with _lib.on_device(qkv):
         rc = _lib.call_status(
             "hydra_ccgqa_prep_bwd_conv", qkv.data_ptr(), qkv.stride(1), *(w.data_ptr() for w in weights),
-            temperature.data_ptr() if norm else None, _lib.ptr(cos), _lib.ptr(sin),
-            head_dim // 2 if cos is None else cos.stride(0), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+            temperature.data_ptr() if norm else None, _lib.ptr(cos), _lib.ptr(sin), rope_rs, dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
             dqkv.data_ptr(), W, *(w.data_ptr() for w in dws), _lib.ptr(dtemp), B, S, n_heads, n_kv_heads,
             head_dim, ks, flags, _lib.dtype_code(qkv), ws.data_ptr(), need, _lib.stream(qkv))
     if rc == _lib.ERR_UNSUPPORTED:

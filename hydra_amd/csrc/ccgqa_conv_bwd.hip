@@ -467,7 +467,7 @@ extern "C" int hydra_ccgqa_prep_bwd_conv(const void* qkv, int64_t qkv_rs, const 
   if (!supported(B, S, Hq, Hkv, hd, ks, flags, dtype))
     return fail(HYDRA_ERR_UNSUPPORTED, "ccgqa_prep_bwd_conv: sizes or type not taken");
   const int64_t L = Hq * hd, K = Hkv * hd, CW = L + K;
-  HYDRA_REQUIRE((flags & ~127) == 0 && !(flags & HYDRA_CCGQA_V_TRANSPOSED), "ccgqa_prep_bwd_conv: bad flags");
+  HYDRA_REQUIRE((flags & ~(127 | HYDRA_CCGQA_ROPE_BF16)) == 0 && !(flags & HYDRA_CCGQA_V_TRANSPOSED), "ccgqa_prep_bwd_conv: bad flags");
   HYDRA_REQUIRE(qkv && wq1 && wq2 && wk1 && wk2 && dq && dk && dv && dqkv && dwq1 && dwq2 && dwk1 && dwk2,
                 "ccgqa_prep_bwd_conv: null pointer");
   HYDRA_REQUIRE(qkv_rs >= CW + K && dqkv_rs >= CW + K, "ccgqa_prep_bwd_conv: row stride smaller than L + 2K");

@@ -744,8 +744,16 @@ __global__ __launch_bounds__(kPrepThreads) void ccgqa_prep_mfma_kernel(
         const int r = rem / Q4, c4 = (rem - r * Q4) * 4;
         const int s = s0 + r;
         cval[j] = make_uint4(0, 0, 0, 0);
-        if (i < nc && s < S)
-          cval[j] = *reinterpret_cast<const uint4*>((which ? sn : cs) + static_cast<int64_t>(s) * cs_rs + c4);
+        if (i < nc && s < S) {
+          const int64_t at = static_cast<int64_t>(s) * cs_rs + c4;
+          if (flags & HYDRA_CCGQA_ROPE_BF16) {  // 4 bf16 values, widened when they are stored
+            const uint2 h = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(which ? sn : cs) + at);
+            cval[j].x = h.x;
+            cval[j].y = h.y;
+          } else {
+            cval[j] = ld16raw<false>((which ? sn : cs) + at);
+          }
+        }
       }
 #pragma unroll
       for (int j = 0; j < KX; ++j)
@@ -762,6 +770,8 @@ __global__ __launch_bounds__(kPrepThreads) void ccgqa_prep_mfma_kernel(
           const int which = i / (TT * Q4), rem = i - which * (TT * Q4);
           const int r = rem / Q4, c4 = (rem - r * Q4) * 4;
           float* d = (which ? SNl : CSl) + r * CSR + c4;  // 8-byte aligned rows
+          if (flags & HYDRA_CCGQA_ROPE_BF16)
+            cval[j] = make_uint4(cval[j].x << 16, cval[j].x & 0xffff0000u, cval[j].y << 16, cval[j].y & 0xffff0000u);
           *reinterpret_cast<uint2*>(d) = make_uint2(cval[j].x, cval[j].y);
           *reinterpret_cast<uint2*>(d + 2) = make_uint2(cval[j].z, cval[j].w);
         }
@@ -1356,7 +1366,7 @@ extern "C" int hydra_ccgqa_prep_fwd(const void* qkv, int64_t qkv_rs, const void*
   HYDRA_REQUIRE(conv_ks >= 1 && conv_ks <= 16, "ccgqa_prep: conv kernel size must be in [1, 16]");
   HYDRA_REQUIRE(Hq % Hkv == 0, "ccgqa_prep: n_heads must be a multiple of n_kv_heads");
   HYDRA_REQUIRE(hd % 2 == 0, "ccgqa_prep: head_dim must be even");
-  HYDRA_REQUIRE((flags & ~127) == 0, "ccgqa_prep: unknown flag bits");
+  HYDRA_REQUIRE((flags & ~(127 | HYDRA_CCGQA_ROPE_BF16)) == 0, "ccgqa_prep: unknown flag bits");
   const int64_t L = Hq * hd, K = Hkv * hd;
   HYDRA_REQUIRE(!(flags & HYDRA_CCGQA_VALUE_SHIFT) || K % 2 == 0,
                 "ccgqa_prep: kv_dim must be even for the value shift");
@@ -1398,9 +1408,9 @@ extern "C" int hydra_ccgqa_prep_fwd(const void* qkv, int64_t qkv_rs, const void*
     }
     if (rc >= 0) return rc;
   }
-  if (flags & HYDRA_CCGQA_W_TILED)
+  if (flags & (HYDRA_CCGQA_W_TILED | HYDRA_CCGQA_ROPE_BF16))
     return fail(HYDRA_ERR_UNSUPPORTED,
-                "ccgqa_prep: MFMA-tiled conv weights need the MFMA path (bf16, head_dim 16/32/64/128, "
+                "ccgqa_prep: MFMA-tiled conv weights and bf16 tables need the MFMA path (bf16, head_dim 16/32/64/128, "
                 "16-byte aligned pointers, S % 8 == 0 with V_TRANSPOSED)");
   int dev = 0, max_lds = 65536;
   if (hipGetDevice(&dev) != hipSuccess ||

@@ -122,11 +122,12 @@ __global__ __launch_bounds__(256) void ccgqa_prep_bwd_vec_kernel(PrepBwdArgs a, 
     for (int e = 0; e < 8; ++e) x[e] = rd<T>(x[e] + t[e]);
   }
   if (live && rope) {  // forward (x0,x1) -> (x0 c - x1 s, x0 s + x1 c); its transpose
-    const float* cp = a.cs + static_cast<int64_t>(s) * a.cs_rs + d / 2;
-    const float* sp = a.sn + static_cast<int64_t>(s) * a.cs_rs + d / 2;
+    const int64_t at = static_cast<int64_t>(s) * a.cs_rs + d / 2;
+    const bool b16 = a.flags & HYDRA_CCGQA_ROPE_BF16;
+    const bf16 *c16 = reinterpret_cast<const bf16*>(a.cs) + at, *s16 = reinterpret_cast<const bf16*>(a.sn) + at;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const float c = cp[e], sv = sp[e];
+      const float c = b16 ? to_f32(c16[e]) : a.cs[at + e], sv = b16 ? to_f32(s16[e]) : a.sn[at + e];
       const float g0 = g[2 * e] * c + g[2 * e + 1] * sv, g1 = g[2 * e + 1] * c - g[2 * e] * sv;
       g[2 * e] = g0;
       g[2 * e + 1] = g1;
@@ -456,6 +457,8 @@ int launch_prep_bwd(const PrepBwdArgs& a) {
       ccgqa_prep_bwd_vec_kernel<T><<<dim3(static_cast<unsigned>((ntok + tpb - 1) / tpb)), 256, 0, a.st>>>(a, tpb);
       return check_launch("ccgqa_prep_bwd_vec_kernel");
     }
+    if (a.flags & HYDRA_CCGQA_ROPE_BF16)
+      return fail(HYDRA_ERR_UNSUPPORTED, "ccgqa_prep_bwd: bf16 tables need the vector path");
     const size_t lds = static_cast<size_t>(kPbThreads / 64) * (2 * CW + 2 * (a.Hq + a.Hkv)) * sizeof(float);
     const unsigned grid = static_cast<unsigned>(std::min<int64_t>((ntok + 3) / 4, 8192));
     auto kern = ccgqa_prep_bwd_kernel<T>;

@@ -128,7 +128,7 @@ def _rope_call(entry: str, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor
     if x.stride(-1) != 1:
         x = x.contiguous()
     out = torch.empty((B, H, S, D), dtype=x.dtype, device=x.device)
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x):
         _lib.call(entry, x.data_ptr(), cos.data_ptr(), sin.data_ptr(), out.data_ptr(),
                   B, H, S, D, _lib.strides(x), cos.stride(0), _lib.dtype_code(x),
                   _lib.dtype_code(cos), _lib.stream(x))
@@ -175,7 +175,7 @@ class _QKNormFunction(torch.autograd.Function):
         qc, kc = q.contiguous(), k.contiguous()
         qo, ko = torch.empty_like(qc), torch.empty_like(kc)
         hd = q.shape[-1]
-        with torch.cuda.device(q.device):
+        with _lib.on_device(q):
             _lib.call("hydra_qk_norm_fwd", qc.data_ptr(), kc.data_ptr(), qo.data_ptr(), ko.data_ptr(),
                       qc.numel() // hd, kc.numel() // hd, hd, float(scale), float(temperature),
                       _lib.dtype_code(q), _lib.stream(q))
@@ -191,7 +191,7 @@ class _QKNormFunction(torch.autograd.Function):
         gko = torch.zeros_like(k) if grad_k_out is None else grad_k_out.to(k.dtype).contiguous()
         gq, gk = torch.empty_like(q), torch.empty_like(k)
         hd = q.shape[-1]
-        with torch.cuda.device(q.device):
+        with _lib.on_device(q):
             _lib.call("hydra_qk_norm_bwd", q.data_ptr(), k.data_ptr(), gqo.data_ptr(), gko.data_ptr(),
                       gq.data_ptr(), gk.data_ptr(), q.numel() // hd, k.numel() // hd, hd, ctx.scale,
                       ctx.temperature, _lib.dtype_code(q), _lib.stream(q))
@@ -251,7 +251,7 @@ class _SwiGLUFunction(torch.autograd.Function):
         up, uv = _as_rows(up)
         hidden = gate.shape[-1] if gate.dim() else 1
         out = torch.empty(gate.shape, dtype=gate.dtype, device=gate.device)
-        with torch.cuda.device(gate.device):
+        with _lib.on_device(gate):
             _lib.call("hydra_swiglu_fwd", gate.data_ptr(), up.data_ptr(), out.data_ptr(),
                       gv[0], hidden, gv[1], uv[1], hidden, _lib.dtype_code(gate), _lib.stream(gate))
         ctx.save_for_backward(gate, up)
@@ -267,7 +267,7 @@ class _SwiGLUFunction(torch.autograd.Function):
         hidden = gate.shape[-1] if gate.dim() else 1
         gg = torch.empty(gate.shape, dtype=gate.dtype, device=gate.device)
         gu = torch.empty(up.shape, dtype=up.dtype, device=up.device)
-        with torch.cuda.device(gate.device):
+        with _lib.on_device(gate):
             _lib.call("hydra_swiglu_bwd", gate.data_ptr(), up.data_ptr(), go.data_ptr(), gg.data_ptr(),
                       gu.data_ptr(), gv[0], hidden, gv[1], uv[1], ov[1], hidden, hidden,
                       _lib.dtype_code(gate), _lib.stream(gate))
@@ -309,7 +309,7 @@ class _RMSNormFunction(torch.autograd.Function):
         w = _norm_weight(weight, x)
         x, xv = _as_rows(x)
         out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-        with torch.cuda.device(x.device):
+        with _lib.on_device(x):
             if w.dtype == x.dtype:
                 _lib.call("hydra_rms_norm_fwd", x.data_ptr(), w.data_ptr(), out.data_ptr(),
                           xv[0], dim, xv[1], dim, float(eps), _lib.dtype_code(x), _lib.stream(x))
@@ -331,7 +331,7 @@ class _RMSNormFunction(torch.autograd.Function):
         go, ov = _as_rows(grad_out.to(x.dtype))
         gx = torch.empty(x.shape, dtype=x.dtype, device=x.device)
         gw = torch.empty((dim,), dtype=w.dtype, device=x.device)
-        with torch.cuda.device(x.device):
+        with _lib.on_device(x):
             need = _lib.query("hydra_rms_norm_bwd_workspace", xv[0], dim)
             ws = _lib.scratch(need, x)
             _lib.call("hydra_rms_norm_bwd", x.data_ptr(), w.data_ptr(), go.data_ptr(), gx.data_ptr(),
@@ -382,7 +382,7 @@ def _ce_grad_planes(logits: torch.Tensor, targets: torch.Tensor, ignore_index: i
     rows, V = logits.shape
     pitch = (V + 7) // 8 * 8
     planes = torch.empty((2 * rows, pitch), dtype=torch.bfloat16, device=logits.device)
-    with torch.cuda.device(logits.device):
+    with _lib.on_device(logits):
         _lib.call("hydra_ce_grad_planes", logits.data_ptr(), rows, V, logits.stride(0), targets.data_ptr(),
                   int(ignore_index), planes.data_ptr(), pitch, rows * pitch, _lib.ptr(grad_scale),
                   _lib.stream(logits))

@@ -68,7 +68,7 @@ def residual_norm(x: torch.Tensor, *, r: Optional[torch.Tensor] = None, alpha: f
         w = w.contiguous()
     h = torch.empty((rows, dim), dtype=x.dtype, device=x.device) if (want_h or norm == _lib.NORM_NONE) else None
     y = torch.empty((rows, dim), dtype=x.dtype, device=x.device) if norm != _lib.NORM_NONE else None
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x):
         _lib.call("hydra_residual_norm_fwd", x2.data_ptr(), x2.stride(0), _lib.ptr(r2),
                   r2.stride(0) if r2 is not None else 0, float(alpha), _lib.ptr(vecs[0]),
                   _lib.ptr(vecs[1]), _lib.ptr(w), float(eps), int(norm), _lib.ptr(h), dim,

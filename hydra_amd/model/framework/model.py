@@ -28,7 +28,7 @@ def embedding_lookup(table: torch.Tensor, ids: torch.Tensor, scale: float = 1.0)
     idx = ids.reshape(-1).to(torch.int64).contiguous()
     t = table if table.stride(-1) == 1 else table.contiguous()
     out = torch.empty((idx.numel(), dim), dtype=table.dtype, device=table.device)
-    with torch.cuda.device(table.device):
+    with _lib.on_device(table):
         _lib.call("hydra_embedding_fwd", idx.data_ptr(), idx.numel(), t.data_ptr(), V, dim,
                   t.stride(0), float(scale), out.data_ptr(), dim, _lib.dtype_code(table),
                   _lib.stream(table))

@@ -87,7 +87,7 @@ def mor_route(logits: torch.Tensor, n_recursions: int, min_depth: int = 0):
     probs = torch.empty_like(lg)
     lout = torch.empty_like(lg)
     depths = torch.empty(lg.shape, dtype=torch.int64, device=lg.device)
-    with torch.cuda.device(lg.device):
+    with _lib.on_device(lg):
         _lib.call("hydra_mor_route", lg.data_ptr(), lg.numel(), probs.data_ptr(), lout.data_ptr(),
                   depths.data_ptr(), int(n_recursions), int(min_depth), _lib.dtype_code(lg),
                   _lib.stream(lg))
@@ -105,7 +105,7 @@ def mor_update(current: torch.Tensor, delta: torch.Tensor, output: torch.Tensor,
     if d2.stride(-1) != 1:
         d2 = d2.contiguous()
     dep = depths.reshape(-1).to(torch.int64).contiguous()
-    with torch.cuda.device(current.device):
+    with _lib.on_device(current):
         _lib.call("hydra_mor_update", c2.data_ptr(), c2.stride(0), d2.data_ptr(), d2.stride(0),
                   o2.data_ptr(), o2.stride(0), dep.data_ptr(), c2.shape[0], dim, int(recursion),
                   _lib.dtype_code(current), _lib.stream(current))

@@ -47,7 +47,7 @@ def mod_topk(scores: torch.Tensor, k: int, *, want_desc: bool = True, want_sorte
     srt = torch.empty((B, k), dtype=torch.int64, device=dev) if want_sorted else None
     mask = torch.empty((B, L), dtype=mask_dtype, device=dev) if mask_dtype is not None else None
     mcode = _lib.dtype_code(mask) if mask is not None else _lib.F32
-    with torch.cuda.device(dev):
+    with _lib.on_device(scores):
         _lib.call("hydra_mod_topk", scores.data_ptr(), B, L, scores.stride(0) if B > 0 else L, k,
                   _lib.ptr(desc), _lib.ptr(srt), _lib.ptr(mask), _lib.dtype_code(scores), mcode,
                   _lib.stream(scores))
@@ -68,7 +68,7 @@ def _gather(x: torch.Tensor, idx: torch.Tensor) -> torch.Tensor:
         x = x.contiguous()
         st = _bl_strides(x)
     out = torch.empty((B, k, D), dtype=x.dtype, device=x.device)
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x):
         _lib.call("hydra_mod_gather", x.data_ptr(), idx.data_ptr(), out.data_ptr(), B, L, k, D,
                   st[0], st[1], _lib.dtype_code(x), _lib.stream(x))
     return out
@@ -86,7 +86,7 @@ def _scatter_raw(output: torch.Tensor, values: Optional[torch.Tensor], idx: torc
         vals = values.to(output.dtype) if values.dtype != output.dtype else values
         vals = vals.contiguous()
     w = None if weights is None else weights.to(torch.float32).contiguous()
-    with torch.cuda.device(output.device):
+    with _lib.on_device(output):
         _lib.call("hydra_mod_scatter", output.data_ptr(), _lib.ptr(vals), idx.data_ptr(),
                   _lib.ptr(w), B, L, k, D, st[0], st[1], mode, _lib.dtype_code(output),
                   _lib.stream(output))
@@ -102,7 +102,7 @@ def _scatter_grads(grad, values, idx, weights, need_values, need_weights):
     g_vals = torch.empty(vals.shape, dtype=vals.dtype, device=vals.device) if need_values else None
     g_w = torch.empty(w.shape, dtype=torch.float32, device=w.device) if need_weights else None
     if need_values or need_weights:
-        with torch.cuda.device(grad.device):
+        with _lib.on_device(grad):
             _lib.call("hydra_mod_scatter_bwd", grad.data_ptr(), vals.data_ptr(), idx.data_ptr(), w.data_ptr(),
                       _lib.ptr(g_vals), _lib.ptr(g_w), B, L, idx.shape[1], D, grad.stride(0), grad.stride(1),
                       _lib.dtype_code(grad), _lib.stream(grad))

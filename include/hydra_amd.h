@@ -165,6 +165,7 @@ int hydra_qk_norm_bwd(const void* q, const void* k, const void* grad_qo, const v
 #define HYDRA_CCGQA_ROPE        16
 #define HYDRA_CCGQA_V_TRANSPOSED 32 /* write v as [B, Hkv, hd, S] */
 #define HYDRA_CCGQA_W_TILED     64  /* conv weights in MFMA-fragment order (below) */
+#define HYDRA_CCGQA_ROPE_BF16   256 /* cos/sin point to bf16 tables (MFMA path only) */
 
 /* Everything of CCGQAAttention.forward between the qkv GEMM and the attention
  * core, in one pass over token tiles: split of the fused projection, value

@@ -70,3 +70,29 @@ def test_conv_backward_shapes(cuda, heads, B, S):
                                       (False, True, True, False)])
 def test_conv_backward_features(cuda, features):
     _check(*_grads(cuda, 2, 70, 4, 2, 32, features))
+
+
+@pytest.mark.parametrize("hd,S", [(16, 70), (64, 33), (128, 129)])
+def test_bf16_rope_tables(cuda, hd, S):
+    """bf16 RoPE tables (a module cast to bf16) are widened inside the kernels:
+    the same bits as tables converted to fp32 before the call, forward and
+    backward, also from a longer [1, 1, Smax, hd/2] cache."""
+    from hydra_amd.attention.backends.ccgqa.autograd import ccgqa_prep_train
+    from hydra_amd.attention.backends.ccgqa.ops import prep_flags
+
+    Hq, Hkv = 4, 2
+    g = torch.Generator().manual_seed(hd + S)
+    L, K = Hq * hd, Hkv * hd
+    rand = lambda *s: (torch.randn(*s, generator=g) * 0.3).to(torch.bfloat16).to(cuda)  # noqa: E731
+    ws = [rand(L, hd, 3), rand(L, L, 3), rand(K, hd, 3), rand(K, K, 3)]
+    qkv, temp = rand(2, S, L + 2 * K), torch.ones(1, dtype=torch.bfloat16, device=cuda)
+    gos = [rand(2, h, S, hd) for h in (Hq, Hkv, Hkv)]
+    cos, sin = (t.to(torch.bfloat16).to(cuda)[None, None] for t in occ.fused_ops.rope_cache(hd, 200))
+    flags = prep_flags(True, True, True, True, True)
+    res = []
+    for c, s in ((cos, sin), (cos.float(), sin.float())):
+        leaves = [t.clone().requires_grad_() for t in (qkv, *ws, temp)]
+        outs = ccgqa_prep_train(leaves[0], Hq, Hkv, hd, flags, *leaves[1:5], temperature=leaves[5], cos=c, sin=s)
+        res.append([*outs, *torch.autograd.grad(outs, leaves, gos)])
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
