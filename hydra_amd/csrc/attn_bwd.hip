@@ -14,21 +14,26 @@
 //  * attn_bwd_rowdot_kernel: D and lse * log2(e) per query row (fp32).
 //  * attn_bwd_dkdv_kernel: lanes own keys.  A workgroup is KB key blocks of
 //    32 keys x HG head groups (one wave each); a step stages 32 query rows
-//    of Q and dO for HG heads in LDS, row-major (A operand of S = Q K^T and
-//    dP = dO V^T) and transposed (A operand of dV^T += dO^T P and
-//    dK^T += Q^T dS), so the KB waves of a head group share each staged
-//    tile.  K and V fragments stay in registers for the whole walk; at the
+//    of Q and dO for HG heads in LDS, read as rows (A operand of S = Q K^T
+//    and dP = dO V^T) and, through the transposing LDS read, as columns (A
+//    operand of dV^T += dO^T P and dK^T += Q^T dS); the KB waves of a head
+//    group share each staged tile.  K and V fragments stay in registers for the whole walk; at the
 //    end the head groups' partial dK/dV are summed through LDS in a fixed
 //    order.  Workgroups start with the lowest keys (the longest causal
 //    walks); with few key groups each one's query range is cut into
 //    chunks whose fp32 partials attn_bwd_dkdv_reduce_kernel sums in order.
+//    Against a second, transposed copy of each tile (written element pair by
+//    element pair) the transposing read halves the staging's LDS bytes and
+//    needs 25 registers less: dK/dV 200 -> 183 us and dQ 115 -> 104 at B4 4/1
+//    heads x 64, S 4096 (the two run side by side), dK/dV 274 -> 163 and dQ
+//    250 -> 225 at B2 16/4 x 16; bit for bit the same results.
 //  * attn_bwd_dq_kernel: lanes own queries, as in the forward: S^T = K Q^T,
-//    dP^T = V dO^T, dQ^T += K^T dS^T; a step stages 64 keys of K and V
-//    (row-major) and K^T in LDS, shared by the 4 query tasks of an item.
+//    dP^T = V dO^T, dQ^T += K^T dS^T; a step stages 64 keys of K and V in
+//    LDS, shared by the 4 query tasks of an item.
 //    It runs on a side stream, concurrently with dK/dV (see SideStream).
 // The MFMA B operand of the PV-type products is taken straight from the
-// score accumulator registers; the A operand is read from the transposed
-// LDS tile in the same (register-order) permutation of the summed index.
+// score accumulator registers; the A operand is read from the LDS tile in the
+// same (register-order) permutation of the summed index.
 // A key mask is a template form of both kernels: dK/dV lanes own one key
 // each, so masked lanes only store zeros; dQ tests one bit per key on tiles
 // that hold a masked key and skips tiles of padding.  Masked calls and
@@ -93,31 +98,25 @@ __device__ __forceinline__ uint4 pack_c8_lo(const f32x16_t& x, int base, const u
   return make_uint4(o[0], o[1], o[2], o[3]);
 }
 
-// A fragment from a transposed LDS tile t[row][col] (pitch in elements),
-// with the columns in the permutation pack_c8 gives the k index: lane
-// (n, hf) takes row `row`, columns 16c + 4hf + 0..3 and 16c + 8 + 4hf + 0..3.
-__device__ __forceinline__ uint4 lds_a_perm(const uint16_t* t, int row, int pitch, int c, int hf) {
-  const uint16_t* p = t + row * pitch + 16 * c + 4 * hf;
-  const uint2 lo = *reinterpret_cast<const uint2*>(p);
-  const uint2 hi = *reinterpret_cast<const uint2*>(p + 8);
+// A fragment of the transpose of a row-major LDS tile t[row][col]: 32 columns
+// from m0, the summed rows in the order pack_c8 gives them (lane half hf: rows
+// 16c + 4hf + 0..3 and 16c + 8 + 4hf + 0..3).  The transposing read takes 4
+// rows of 16 columns per 16 lanes (lane i: row i / 4, columns 4 (i % 4) ..) and
+// returns column i's four values.
+typedef __attribute__((ext_vector_type(4))) short s16x4_t;
+__device__ __forceinline__ uint4 lds_a_tr(const uint16_t* t, int pitch, int m0, int c, int lane) {
+  const uint16_t* p = t + (16 * c + 4 * (lane >> 5) + ((lane & 15) >> 2)) * pitch + m0 + 16 * ((lane >> 4) & 1) +
+                      4 * (lane & 3);
+  typedef __attribute__((address_space(3))) s16x4_t* lds_t;
+  const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_t)(p)));
+  const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_t)(p + 8 * pitch)));
   return make_uint4(lo.x, lo.y, hi.x, hi.y);
 }
 
-// Element i of two 16-byte rows a and b as one 32-bit word (a_i | b_i << 16).
-__device__ __forceinline__ uint32_t pair_word(const uint4& a, const uint4& b, int i) {
-  const uint32_t wa = i < 2 ? a.x : i < 4 ? a.y : i < 6 ? a.z : a.w;
-  const uint32_t wb = i < 2 ? b.x : i < 4 ? b.y : i < 6 ? b.z : b.w;
-  return (i & 1) ? (wa >> 16) | (wb & 0xffff0000u) : (wa & 0xffffu) | (wb << 16);
-}
-
-// Writes the 8 d-values of rows 2p and 2p+1 (chunk c) into a transposed tile
-// t[d][row] as 8 words.
-__device__ __forceinline__ void st_pair_t(uint16_t* t, int pitch, int c, int p, const uint4& a,
-                                          const uint4& b) {
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-    *reinterpret_cast<uint32_t*>(&t[(8 * c + i) * pitch + 2 * p]) = pair_word(a, b, i);
-}
+// Row pitch (elements) of a staged tile: 16-byte rows whose offsets keep both
+// the 16-byte row reads (8 rows at a time) and the transposing reads (4 rows of
+// 32 bytes) on distinct banks.
+constexpr int tile_pitch(int hd) { return hd == 32 || hd == 128 ? hd + 16 : hd + 8; }
 
 // Buffer resource over `bytes` bytes from `base`: loads past the end return
 // zero (hardware range check), so tiles that overhang S need no branches --
@@ -216,13 +215,11 @@ __global__ __launch_bounds__(256) void attn_bwd_rowdot_kernel(
 // dK/dV, lanes own keys (bf16, MFMA).
 template <int HD>
 struct DkdvLayout {
-  static constexpr int QP = HD + 8;          // row-major pitch (elements): 16-byte rows, 4-bank skew
-  static constexpr int TP = 32 + 4;          // transposed pitch (elements)
-  static constexpr int ROWS = 32 * QP;       // one row-major 32-row tile
-  // one transposed tile; a head_dim-16 tile keeps 32 rows: the d tile of the
-  // MFMA reads all of them, and its rows past head_dim are never stored
-  static constexpr int TRS = (HD < 32 ? 32 : HD) * TP;
-  static constexpr int HGE = 2 * ROWS + 2 * TRS + 2 * 32 * 2;  // Q, dO, Q^T, dO^T, lse2, D (elements)
+  static constexpr int QP = tile_pitch(HD);
+  static constexpr int ROWS = 32 * QP;       // one 32-row tile
+  // Q, dO, lse2, D (elements).  (At head_dim 16 the d tile's upper half reads
+  // up to 8 elements past a tile, into what follows it; it is never stored.)
+  static constexpr int HGE = 2 * ROWS + 2 * 32 * 2;
 };
 
 // MASK as in bwd_visible (2 comes with CAUSAL = false: it walks every query
@@ -245,7 +242,7 @@ __global__ __launch_bounds__(64 * KB * HG) void attn_bwd_dkdv_kernel(
   constexpr int DC = HD / 8;    // 16-byte chunks per row
   using L = DkdvLayout<HD>;
   constexpr int STAGE = HG * L::HGE;
-  constexpr int UNITS = HG * 16 * DC;         // (head group, row pair, chunk) staging units
+  constexpr int UNITS = HG * 32 * DC;         // (head group, row, chunk) staging units
   constexpr int UPT = (UNITS + NT - 1) / NT;
   constexpr int FOLD = (HG - 1) * KB * 64 * 2 * DT * 16;  // floats exchanged at the end
   constexpr int SMEM = 2 * STAGE > FOLD * 2 ? 2 * STAGE : FOLD * 2;
@@ -371,9 +368,10 @@ __global__ __launch_bounds__(64 * KB * HG) void attn_bwd_dkdv_kernel(
     }
   };
 
-  // Staging registers: per unit the chunk c of rows 2p, 2p+1 of Q and dO.
+  // Staging registers: per unit one 16-byte chunk of a row of Q and of dO
+  // (chunk fastest: whole rows per wave).
   struct Regs {
-    uint4 q[UPT][2], d[UPT][2];
+    uint4 q[UPT], d[UPT];
     float l, dv;  // lse2 / D of one row (threads < 32 * HG)
   };
   Regs ra, rb;
@@ -384,21 +382,16 @@ __global__ __launch_bounds__(64 * KB * HG) void attn_bwd_dkdv_kernel(
     for (int u = 0; u < UPT; ++u) {
       const int unit = tid + NT * u;
       if (UNITS % NT == 0 || unit < UNITS) {
-        // 16 * DC >= 64 units share a head group, so g is wave-uniform (and
+        // 32 * DC >= 64 units share a head group, so g is wave-uniform (and
         // the buffer resources below scalar).
-        const int g = __builtin_amdgcn_readfirstlane(unit / (16 * DC));
-        const int rem = unit - g * (16 * DC);
-        const int c = rem >> 4, p = rem & 15;  // p fastest: conflict-free transposed writes
+        const int g = __builtin_amdgcn_readfirstlane(unit / (32 * DC));
+        const int rem = unit - g * (32 * DC);
+        const int c = rem % DC, row = 32 * qt + rem / DC;  // rows >= S read as zero
         const int h = kvh * G + hr * HG + g;
-        const int r0 = 32 * qt + 2 * p;  // rows >= S read as zero
         const auto qr = rows_rsrc(q + b * qs0 + h * qs1, (S - 1) * qs2 * 2 + HD * 2);
         const auto dr = rows_rsrc(dout + b * ds0 + h * ds1, (S - 1) * ds2 * 2 + HD * 2);
-        const int qo = r0 * static_cast<int>(qs2) * 2 + 16 * c;
-        const int dof = r0 * static_cast<int>(ds2) * 2 + 16 * c;
-        R.q[u][0] = ld16_buf(qr, qo);
-        R.q[u][1] = ld16_buf(qr, qo + static_cast<int>(qs2) * 2);
-        R.d[u][0] = ld16_buf(dr, dof);
-        R.d[u][1] = ld16_buf(dr, dof + static_cast<int>(ds2) * 2);
+        R.q[u] = ld16_buf(qr, row * static_cast<int>(qs2) * 2 + 16 * c);
+        R.d[u] = ld16_buf(dr, row * static_cast<int>(ds2) * 2 + 16 * c);
       }
     }
     {
@@ -420,19 +413,14 @@ __global__ __launch_bounds__(64 * KB * HG) void attn_bwd_dkdv_kernel(
     for (int u = 0; u < UPT; ++u) {
       const int unit = tid + NT * u;
       if (UNITS % NT == 0 || unit < UNITS) {
-        const int g = unit / (16 * DC), rem = unit - g * (16 * DC);
-        const int c = rem >> 4, p = rem & 15;  // p fastest: conflict-free transposed writes
-        uint16_t* hb = st + g * L::HGE;
-        *reinterpret_cast<uint4*>(&hb[(2 * p) * L::QP + 8 * c]) = R.q[u][0];
-        *reinterpret_cast<uint4*>(&hb[(2 * p + 1) * L::QP + 8 * c]) = R.q[u][1];
-        *reinterpret_cast<uint4*>(&hb[L::ROWS + (2 * p) * L::QP + 8 * c]) = R.d[u][0];
-        *reinterpret_cast<uint4*>(&hb[L::ROWS + (2 * p + 1) * L::QP + 8 * c]) = R.d[u][1];
-        st_pair_t(hb + 2 * L::ROWS, L::TP, c, p, R.q[u][0], R.q[u][1]);
-        st_pair_t(hb + 2 * L::ROWS + L::TRS, L::TP, c, p, R.d[u][0], R.d[u][1]);
+        const int g = unit / (32 * DC), rem = unit - g * (32 * DC);
+        uint16_t* hb = st + g * L::HGE + rem / DC * L::QP + 8 * (rem % DC);
+        *reinterpret_cast<uint4*>(hb) = R.q[u];
+        *reinterpret_cast<uint4*>(hb + L::ROWS) = R.d[u];
       }
     }
     if (tid < 32 * HG) {
-      float* f = reinterpret_cast<float*>(st + (tid >> 5) * L::HGE + 2 * L::ROWS + 2 * L::TRS);
+      float* f = reinterpret_cast<float*>(st + (tid >> 5) * L::HGE + 2 * L::ROWS);
       f[tid & 31] = R.l;
       f[32 + (tid & 31)] = R.dv;
     }
@@ -445,9 +433,7 @@ __global__ __launch_bounds__(64 * KB * HG) void attn_bwd_dkdv_kernel(
       const uint16_t* hb = smem + buf * STAGE + hg * L::HGE;
       const uint16_t* Qs = hb;
       const uint16_t* Ds = hb + L::ROWS;
-      const uint16_t* Qt = hb + 2 * L::ROWS;
-      const uint16_t* Dt = Qt + L::TRS;
-      const float* lsv = reinterpret_cast<const float*>(Dt + L::TRS);
+      const float* lsv = reinterpret_cast<const float*>(Ds + L::ROWS);
       f32x16_t s = zero16(), dp = zero16();
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
@@ -483,10 +469,10 @@ __global__ __launch_bounds__(64 * KB * HG) void attn_bwd_dkdv_kernel(
         }
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
-          const uint4 ad = lds_a_perm(Dt, 32 * dt + n, L::TP, c, hf);
+          const uint4 ad = lds_a_tr(Ds, L::QP, 32 * dt, c, lane);
           dva[dt] = mfma(ad, pb, dva[dt]);
           if constexpr (NP == 2) dva[dt] = mfma(ad, pl, dva[dt]);
-          const uint4 aq = lds_a_perm(Qt, 32 * dt + n, L::TP, c, hf);
+          const uint4 aq = lds_a_tr(Qs, L::QP, 32 * dt, c, lane);
           dka[dt] = mfma(aq, sb, dka[dt]);
           if constexpr (NP == 2) dka[dt] = mfma(aq, sl, dka[dt]);
         }
@@ -672,11 +658,9 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_reduce_kernel(
 template <int HD>
 struct DqLayout {
   static constexpr int BN = 64;              // keys per step
-  static constexpr int KP = HD + 8;          // row-major pitch (elements)
-  static constexpr int TP = BN + 4;          // transposed pitch (elements)
+  static constexpr int KP = tile_pitch(HD);
   static constexpr int ROWS = BN * KP;
-  static constexpr int TRS = (HD < 32 ? 32 : HD) * TP;  // see DkdvLayout
-  static constexpr int STAGE = 2 * ROWS + TRS;  // K, V, K^T
+  static constexpr int STAGE = 2 * ROWS;     // K, V (head_dim 16: see DkdvLayout)
 };
 
 // MASK, NP as in attn_bwd_dkdv_kernel.
@@ -695,7 +679,7 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(
   constexpr int DT = (HD + 31) / 32;
   constexpr int JT = HD < 32 ? 2 : 4;  // 8-row groups of a d tile that hold rows of head_dim
   constexpr int DC = HD / 8;
-  constexpr int UNITS = (BN / 2) * DC;        // (key pair, chunk) staging units
+  constexpr int UNITS = BN * DC;              // (key, chunk) staging units
   constexpr int NT = 64 * NW;
   constexpr int UPT = (UNITS + NT - 1) / NT;
   __shared__ __attribute__((aligned(16))) uint16_t smem[2 * L::STAGE];
@@ -751,7 +735,7 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(
   if constexpr (MASK != 0) mrs = rows_rsrc(kmask + static_cast<int64_t>(b) * S, S);
   uint64_t keep[2] = {0, 0};
   struct Regs {
-    uint4 k[UPT][2], v[UPT][2];
+    uint4 k[UPT], v[UPT];
     uint8_t m;
   };
   Regs ra, rb;
@@ -761,14 +745,9 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(
     for (int u = 0; u < UPT; ++u) {
       const int unit = tid + NT * u;
       if (UNITS % NT == 0 || unit < UNITS) {
-        const int c = unit >> 5, p = unit & 31;  // p fastest: conflict-free transposed writes
-        const int k0 = BN * kt + 2 * p;  // keys >= S read as zero
-        const int ko = k0 * static_cast<int>(ks2) * 2 + 16 * c;
-        const int vo = k0 * static_cast<int>(vs2) * 2 + 16 * c;
-        R.k[u][0] = ld16_buf(krs, ko);
-        R.k[u][1] = ld16_buf(krs, ko + static_cast<int>(ks2) * 2);
-        R.v[u][0] = ld16_buf(vrs, vo);
-        R.v[u][1] = ld16_buf(vrs, vo + static_cast<int>(vs2) * 2);
+        const int c = unit % DC, key = BN * kt + unit / DC;  // keys >= S read as zero
+        R.k[u] = ld16_buf(krs, key * static_cast<int>(ks2) * 2 + 16 * c);
+        R.v[u] = ld16_buf(vrs, key * static_cast<int>(vs2) * 2 + 16 * c);
       }
     }
   };
@@ -779,12 +758,9 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(
     for (int u = 0; u < UPT; ++u) {
       const int unit = tid + NT * u;
       if (UNITS % NT == 0 || unit < UNITS) {
-        const int c = unit >> 5, p = unit & 31;  // p fastest: conflict-free transposed writes
-        *reinterpret_cast<uint4*>(&st[(2 * p) * L::KP + 8 * c]) = R.k[u][0];
-        *reinterpret_cast<uint4*>(&st[(2 * p + 1) * L::KP + 8 * c]) = R.k[u][1];
-        *reinterpret_cast<uint4*>(&st[L::ROWS + (2 * p) * L::KP + 8 * c]) = R.v[u][0];
-        *reinterpret_cast<uint4*>(&st[L::ROWS + (2 * p + 1) * L::KP + 8 * c]) = R.v[u][1];
-        st_pair_t(st + 2 * L::ROWS, L::TP, c, p, R.k[u][0], R.k[u][1]);
+        uint16_t* row = st + unit / DC * L::KP + 8 * (unit % DC);
+        *reinterpret_cast<uint4*>(row) = R.k[u];
+        *reinterpret_cast<uint4*>(row + L::ROWS) = R.v[u];
       }
     }
   };
@@ -795,7 +771,6 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(
     {
       const uint16_t* Ks = smem + buf * L::STAGE;
       const uint16_t* Vs = Ks + L::ROWS;
-      const uint16_t* Kt = Ks + 2 * L::ROWS;
       f32x16_t st[MT], dp[MT];
       // MASKED: key = key0 + 4 hf + off, off = 32 mt + 8 (r / 4) + r % 4 a
       // constant per register, visible iff off <= lim
@@ -836,7 +811,7 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(
         if constexpr (NP == 2) sl = pack_c8_lo(dp[c >> 1], 8 * (c & 1), sb);
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
-          const uint4 ak = lds_a_perm(Kt, 32 * dt + n, L::TP, c, hf);
+          const uint4 ak = lds_a_tr(Ks, L::KP, 32 * dt, c, lane);
           acc[dt] = mfma(ak, sb, acc[dt]);
           if constexpr (NP == 2) acc[dt] = mfma(ak, sl, acc[dt]);
         }
