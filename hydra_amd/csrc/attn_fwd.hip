@@ -848,8 +848,9 @@ __device__ __forceinline__ void attn_fwd_kp_body(
   };
 
   // The group's loads of tile kb of item `it` into its buffer buf.  Keys at
-  // or past S (last tile only; S % 8 == 0 on this path) load as zeros: K
-  // rows through num_records, V^T chunks through the lane's offset.
+  // or past S (last tile only) load as zeros: K rows through num_records, V^T
+  // chunks of 8 keys through the lane's offset (a chunk that reaches past S
+  // is whole and zero there: V^T rows are padded to a multiple of 8 keys).
   auto fetch = [&](const Item& it, int kb, int buf) {
     const int key0 = kb * BN;
     const int rows = min(BN, S - key0);
@@ -862,7 +863,8 @@ __device__ __forceinline__ void attn_fwd_kp_body(
       const int j = wq + NW * i;
       if (j < KINS) load16_to_lds(kr, ks_lds + 1024 * j, koffs[i]);
     }
-    const i32x4_t vr = raw_rsrc(it.vbase + key0, static_cast<int>((HD - 1) * vs2 * 2 + rows * 2));
+    const int vrows = min(BN, ((S + 7) & ~7) - key0);
+    const i32x4_t vr = raw_rsrc(it.vbase + key0, static_cast<int>((HD - 1) * vs2 * 2 + vrows * 2));
     if (key0 + BN <= S) {
 #pragma unroll
       for (int i = 0; i < VIPW; ++i) {
@@ -1212,6 +1214,40 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(
     lse[(static_cast<int64_t>(b) * Hq + h) * S + qi] = L > 0.f ? (M + __log2f(L)) * kLn2 : -INFINITY;
 }
 
+// Row-major V [S][HD] -> V^T rows [HD][Sp], Sp = S rounded up to 8 keys (zeros
+// past S), so that calls with few items can take the key-split kernel: a
+// workgroup turns 64 keys of one (batch, kv head) through LDS, the transposing
+// read giving each lane four keys of a column.
+template <int HD>
+__global__ __launch_bounds__(256) void attn_v_transpose_kernel(const bf16* __restrict__ v, bf16* __restrict__ vt, int S,
+                                                               int Sp, int Hkv, int64_t vs0, int64_t vs1, int64_t vs2) {
+  constexpr int PITCH = HD + 8, DC = HD / 8;
+  __shared__ __attribute__((aligned(16))) uint16_t t[64 * PITCH];
+  const int ntile = (Sp + 63) / 64;
+  const int tile = blockIdx.x % ntile, bk = blockIdx.x / ntile, b = bk / Hkv, kvh = bk - b * Hkv;
+  const int key0 = 64 * tile, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const bf16* src = v + b * vs0 + kvh * vs1;
+  for (int i = tid; i < 64 * DC; i += 256) {
+    const int row = i / DC, c = i - row * DC;
+    uint4 x = make_uint4(0, 0, 0, 0);
+    if (key0 + row < S) x = ld16raw<false>(src + static_cast<int64_t>(key0 + row) * vs2 + 8 * c);
+    *reinterpret_cast<uint4*>(&t[row * PITCH + 8 * c]) = x;
+  }
+  __syncthreads();
+  typedef __attribute__((ext_vector_type(4))) short s16x4_t;
+  typedef __attribute__((address_space(3))) s16x4_t* lds_t;
+  uint16_t* dst = reinterpret_cast<uint16_t*>(vt) + static_cast<int64_t>(bk) * HD * Sp;
+  // 16 lanes read 4 keys x 16 columns: (column block, key quad) per 16 lanes
+  for (int g = wave * 4 + (lane >> 4); g < (HD / 16) * 16; g += 16) {
+    const int kq = g % 16, cb = g / 16, i = lane & 15;
+    const s16x4_t r =
+        __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_t)(&t[(4 * kq + (i >> 2)) * PITCH + 16 * cb + 4 * (i & 3)]));
+    const int key = key0 + 4 * kq;
+    if (key < Sp)
+      *reinterpret_cast<uint2*>(dst + static_cast<int64_t>(16 * cb + i) * Sp + key) = __builtin_bit_cast(uint2, r);
+  }
+}
+
 // ---- generic path ---------------------------------------------------------
 template <typename T, int MAXHD>
 __global__ __launch_bounds__(256) void attn_fwd_generic_kernel(
@@ -1340,10 +1376,31 @@ static int launch_mfma(const void* q, const void* k, const void* v, void* o, flo
     if (sched && strcmp(sched, "streamk") == 0) kp = false;
     if (sched && strcmp(sched, "kp") == 0) kp = vt && s32;
     if (getenv("HYDRA_ATTN_WGS")) kp = false;
-    if (kp) {
+    // Row-major V where stream-K would cut items: V is transposed first and
+    // the key-split kernel runs, which replaces the merge launch (and keeps
+    // partial sums in fp32).  Core forward at B4 4/1 heads x 64, S 4096: 67 us
+    // of stream-K + merge -> 60 with the transpose; up to one key tile
+    // no item is cut, so stream-K is one launch and stays.
+    const int Sp = static_cast<int>((S + 7) & ~int64_t(7));
+    const int64_t vt_elems = int64_t(BH) * HD * Sp;
+    const bool turn = !vt && s32 && items < 2 * slots && !sched && !getenv("HYDRA_ATTN_WGS") &&
+                      S > kAttnBN && vt_elems < (int64_t(1) << 31);
+    if (kp || turn) {
+      const bf16* Vk = V;
+      const int64_t tvs[4] = {int64_t(Hkv) * HD * Sp, int64_t(HD) * Sp, 1, Sp};
+      const int64_t* vk = turn ? tvs : vs;
       if (need) {
-        *need = 0;
+        *need = turn ? static_cast<size_t>(vt_elems) * sizeof(bf16) : 0;
         return HYDRA_OK;
+      }
+      if (turn) {
+        if (ws_ptr == nullptr || ws_bytes < static_cast<size_t>(vt_elems) * sizeof(bf16))
+          return fail(HYDRA_ERR_ARG, "attn_fwd: workspace of " + std::to_string(vt_elems * sizeof(bf16)) +
+                                         " bytes required (hydra_attn_fwd_workspace)");
+        attn_v_transpose_kernel<HD><<<dim3(static_cast<unsigned>(BH * ((Sp + 63) / 64))), 256, 0, st>>>(
+            V, static_cast<bf16*>(ws_ptr), iS, Sp, (int)Hkv, vs[0], vs[1], vs[2]);
+        if (int rc = check_launch("attn_v_transpose_kernel")) return rc;
+        Vk = static_cast<const bf16*>(ws_ptr);
       }
       constexpr int KP = HD == 128 ? 2 : 3;  // key groups (LDS: KP double-buffered K/V^T tiles)
       auto kkern = attn_fwd_kp_kernel<HD, C, M, NW, KP, FX>;
@@ -1354,7 +1411,7 @@ static int launch_mfma(const void* q, const void* k, const void* v, void* o, flo
       const int Pk = static_cast<int>(std::min<int64_t>(items, std::max<int64_t>(kslots, (items + 1) / 2)));
       const int32_t qs32[3] = {(int32_t)qs[0], (int32_t)qs[1], (int32_t)qs[2]};
       const int32_t ks32[3] = {(int32_t)ks[0], (int32_t)ks[1], (int32_t)ks[2]};
-      const int32_t vs32[3] = {(int32_t)vs[0], (int32_t)vs[1], (int32_t)vs[3]};
+      const int32_t vs32[3] = {(int32_t)vk[0], (int32_t)vk[1], (int32_t)vk[3]};
       const int32_t os32[3] = {(int32_t)os[0], (int32_t)os[1], (int32_t)os[2]};
       // 16-byte aligned output rows take whole-row stores through LDS (hd
       // 64); others the 8-byte stores (the workspace query cannot see the
@@ -1362,7 +1419,7 @@ static int launch_mfma(const void* q, const void* k, const void* v, void* o, flo
       const bool o16 = (reinterpret_cast<uintptr_t>(O) & 15) == 0 && os[0] % 8 == 0 && os[1] % 8 == 0 &&
                        os[2] % 8 == 0;
       kkern<<<dim3(static_cast<unsigned>(Pk)), 64 * NW * KP, 0, st>>>(
-          Q, K, V, O, lse, kmask, iS, (int)Hq, (int)Hkv, G, ntasks, nwg, BH, Pk, qs32[0], qs32[1], qs32[2],
+          Q, K, Vk, O, lse, kmask, iS, (int)Hq, (int)Hkv, G, ntasks, nwg, BH, Pk, qs32[0], qs32[1], qs32[2],
           ks32[0], ks32[1], ks32[2], vs32[0], vs32[1], vs32[2], os32[0], os32[1], os32[2], sl2, tau, tau_bf16,
           o16 ? 1 : 0, Pk <= g_clock_stamp_cap ? g_clock_stamps : nullptr);
       return check_launch("attn_fwd_kp_kernel");
