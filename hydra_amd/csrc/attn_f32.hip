@@ -31,10 +31,10 @@
 //
 // Measured, forward + backward of one call, against what these calls took
 // before (16 lanes per query row forward, one thread per row backward, VALU):
-// fp16 B2 8/2 heads x 64, S 1500, causal 198.1 -> 0.36 ms; fp32 B4 8/2 x 64,
-// S 2048, causal 274 -> 1.21 ms; fp32 B1 4/1 x 128, S 1000 172.9 -> 0.26 ms;
+// fp16 B2 8/2 heads x 64, S 1500, causal 198.1 -> 0.27 ms; fp32 B4 8/2 x 64,
+// S 2048, causal 274 -> 0.82 ms; fp32 B1 4/1 x 128, S 1000 172.9 -> 0.26 ms;
 // fp32 B2 8/2 x 16, S 512, causal 8.7 -> 0.17 ms (launch-bound).  Errors
-// against 64 bits: fp32 1.8e-6 -> 6.9e-7, fp16 2.2e-4 (the output's rounding)
+// against 64 bits: fp32 1.8e-6 -> 5.9e-7, fp16 2.2e-4 (the output's rounding)
 // both.
 #include "attn_f32.h"
 
@@ -71,7 +71,8 @@ struct Rows {
   int64_t rs, es;
 };
 
-// Registers of one thread's share of a staged tile, and its way to LDS.
+// Registers of one thread's share of a staged tile, and its way to LDS (t:
+// the thread's index among the kThreads that stage it).
 template <typename T, int HDP>
 struct Stage {
   static constexpr int P = HDP + 4;                 // words per staged row
@@ -83,20 +84,20 @@ struct Stage {
 
   uint4 raw[VU];
 
-  __device__ __forceinline__ void fetch(const Rows<T>& r, int row0, int S) {
+  __device__ __forceinline__ void fetch(const Rows<T>& r, int row0, int S, int t) {
 #pragma unroll
     for (int u = 0; u < VU; ++u) {
-      const int i = threadIdx.x + kThreads * u;
+      const int i = t + kThreads * u;
       const int row = i / (HDP / E), c = i - row * (HDP / E);
       const bool ok = (WHOLE || row < kTile) && row0 + row < S;
       raw[u] = ok ? *reinterpret_cast<const uint4*>(r.base + static_cast<int64_t>(row0 + row) * r.rs + c * E)
                   : make_uint4(0, 0, 0, 0);
     }
   }
-  __device__ __forceinline__ void land(float* dst) const {
+  __device__ __forceinline__ void land(float* dst, int t) const {
 #pragma unroll
     for (int u = 0; u < VU; ++u) {
-      const int i = threadIdx.x + kThreads * u;
+      const int i = t + kThreads * u;
       const int row = i / (HDP / E), c = i - row * (HDP / E);
       if (WHOLE || row < kTile) {
         float f[E];
@@ -108,10 +109,10 @@ struct Stage {
     }
   }
   // Any strides and head_dim: element by element, straight to LDS.
-  static __device__ __forceinline__ void direct(const Rows<T>& r, int row0, int S, int hd, float* dst) {
+  static __device__ __forceinline__ void direct(const Rows<T>& r, int row0, int S, int hd, float* dst, int t) {
 #pragma unroll 4
     for (int u = 0; u < SU; ++u) {
-      const int i = threadIdx.x + kThreads * u;
+      const int i = t + kThreads * u;
       const int row = i / HDP, d = i - row * HDP;
       const bool ok = row0 + row < S && d < hd;
       dst[row * P + d] = ok ? to_f32(r.base[static_cast<int64_t>(row0 + row) * r.rs + d * r.es]) : 0.f;
@@ -121,15 +122,32 @@ struct Stage {
 
 // The resident fragment of one row (column lane % 16 of B): elements
 // 16 j + 4 g + i of the row, zero past hd or for a row that is not there.
+// vec: rows of HDP elements, aligned to four of them.
 template <typename T, int HDP>
-__device__ __forceinline__ void load_frag(float (&f)[HDP / 16][4], const T* row, int64_t es, int g, int hd, bool ok) {
+__device__ __forceinline__ void load_frag(float (&f)[HDP / 16][4], const T* row, int g, int hd, bool ok, bool vec) {
 #pragma unroll
   for (int j = 0; j < HDP / 16; ++j)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int d = 16 * j + 4 * g + i;
-      f[j][i] = ok && d < hd ? to_f32(row[d * es]) : 0.f;
-    }
+    for (int i = 0; i < 4; ++i) f[j][i] = 0.f;
+  if (!ok) return;
+  if (vec) {
+    struct alignas(4 * sizeof(T)) Four { T v[4]; };
+    Four raw[HDP / 16];
+#pragma unroll
+    for (int j = 0; j < HDP / 16; ++j) raw[j] = *reinterpret_cast<const Four*>(row + 16 * j + 4 * g);
+#pragma unroll
+    for (int j = 0; j < HDP / 16; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) f[j][i] = to_f32(raw[j].v[i]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < HDP / 16; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int d = 16 * j + 4 * g + i;
+        if (d < hd) f[j][i] = to_f32(row[d]);
+      }
+  }
 }
 
 // S and dP tiles (or S alone): rows of two staged operands times the
@@ -198,17 +216,24 @@ __device__ __forceinline__ Task task_of(int task, int ntasks, int kvh, int G) {
 }
 
 // ---------------------------------------------------------------- forward
-template <typename T, int HDP>
-__global__ __launch_bounds__(kThreads) void attn_fwd_f32_kernel(
+// KG key groups of four waves share an item: group kg walks key tiles kg, kg +
+// KG, .. with its own staged tiles, and group 0 folds the others' (O, m, l) in
+// group order at the end.  KG > 1 where there are too few items to fill the
+// device: their walks are then KG times shorter (see launch_fwd).
+template <typename T, int HDP, int KG>
+__global__ __launch_bounds__(kThreads * KG) void attn_fwd_f32_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, T* __restrict__ o,
     float* __restrict__ lse, const uint8_t* __restrict__ kmask, int mode, int Hq, int Hkv, int S, int hd, int G,
     int ntasks, int items, Strides3 qs, Strides3 ks, Strides3 vs, int64_t vs3, Strides3 os, int causal, int vec,
     float scale_log2) {
   using St = Stage<T, HDP>;
-  __shared__ __attribute__((aligned(16))) float smem[2][2 * St::WORDS];
-  __shared__ int keepv[2][kTile];
-  const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
+  __shared__ __attribute__((aligned(16))) float smem_all[KG][2][2 * St::WORDS];
+  __shared__ int keep_all[KG][2][kTile];
+  const int kg = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / kThreads) : 0;
+  const int tid = threadIdx.x - kg * kThreads, lane = tid & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  auto& smem = smem_all[kg];
+  auto& keepv = keep_all[kg];
   const int BHkv = gridDim.x / items;
   const int bk = blockIdx.x % BHkv;
   const int item = items - 1 - static_cast<int>(blockIdx.x / BHkv);  // longest key ranges first
@@ -217,7 +242,7 @@ __global__ __launch_bounds__(kThreads) void attn_fwd_f32_kernel(
   const int qi = tk.q0 + n;
   const bool qok = tk.active && qi < S;
   float qf[HDP / 16][4];
-  load_frag<T, HDP>(qf, q + b * qs.b + tk.h * qs.h + static_cast<int64_t>(qok ? qi : 0) * qs.s, 1, g, hd, qok);
+  load_frag<T, HDP>(qf, q + b * qs.b + tk.h * qs.h + static_cast<int64_t>(qok ? qi : 0) * qs.s, g, hd, qok, vec & 2);
 
   const bool walk = causal && mode != HYDRA_MASK_REFERENCE_SDPA;
   const int last_task = min(kWaves * item + kWaves - 1, ntasks - 1);
@@ -234,9 +259,9 @@ __global__ __launch_bounds__(kThreads) void attn_fwd_f32_kernel(
   St sk, sv;
   int kp = 0;
   auto fetch = [&](int t) {
-    if (vec) {
-      sk.fetch(kr, kTile * t, S);
-      sv.fetch(vr, kTile * t, S);
+    if (vec & 1) {
+      sk.fetch(kr, kTile * t, S, tid);
+      sv.fetch(vr, kTile * t, S, tid);
     }
     if (mode != HYDRA_MASK_NONE && tid < kTile) {
       const int key = kTile * t + tid;
@@ -244,21 +269,24 @@ __global__ __launch_bounds__(kThreads) void attn_fwd_f32_kernel(
     }
   };
   auto land = [&](int t, int buf) {
-    if (vec) {
-      sk.land(smem[buf]);
-      sv.land(smem[buf] + St::WORDS);
+    if (vec & 1) {
+      sk.land(smem[buf], tid);
+      sv.land(smem[buf] + St::WORDS, tid);
     } else {
-      St::direct(kr, kTile * t, S, hd, smem[buf]);
-      St::direct(vr, kTile * t, S, hd, smem[buf] + St::WORDS);
+      St::direct(kr, kTile * t, S, hd, smem[buf], tid);
+      St::direct(vr, kTile * t, S, hd, smem[buf] + St::WORDS, tid);
     }
     if (mode != HYDRA_MASK_NONE && tid < kTile) keepv[buf][tid] = kp;
   };
-  fetch(0);
-  land(0, 0);
-  for (int t = 0; t < nt; ++t) {
+  if (kg < nt) {
+    fetch(kg);
+    land(kg, 0);
+  }
+  const int steps = (nt + KG - 1) / KG;
+  for (int st = 0; st < steps; ++st) {
     __syncthreads();
-    const int buf = t & 1, t0 = kTile * t;
-    if (t + 1 < nt) fetch(t + 1);
+    const int t = KG * st + kg, buf = st & 1, t0 = kTile * t;
+    if (t + KG < nt) fetch(t + KG);
     if (t0 < my_end) {
       const float* Ks = smem[buf];
       const float* Vs = Ks + St::WORDS;
@@ -301,7 +329,37 @@ __global__ __launch_bounds__(kThreads) void attn_fwd_f32_kernel(
         col_product<HDP>(acc, Vs + 16 * u * St::P, x[u], n, g);
       }
     }
-    if (t + 1 < nt) land(t + 1, buf ^ 1);
+    if (t + KG < nt) land(t + KG, buf ^ 1);
+  }
+  if constexpr (KG > 1) {
+    constexpr int NA = HDP / 16, XF = 4 * NA + 2;  // floats a lane hands over
+    static_assert(kThreads * XF <= 4 * St::WORDS, "the exchange fits a group's tiles");
+    __syncthreads();  // every group is done with its tiles
+    float* mine = &smem_all[kg][0][0];
+    if (kg > 0) {
+#pragma unroll
+      for (int d = 0; d < NA; ++d)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) mine[(4 * d + r) * kThreads + tid] = acc[d][r];
+      mine[4 * NA * kThreads + tid] = m;
+      mine[(4 * NA + 1) * kThreads + tid] = l;
+    }
+    __syncthreads();
+    if (kg > 0) return;
+#pragma unroll
+    for (int o2 = 1; o2 < KG; ++o2) {
+      const float* x = &smem_all[o2][0][0];
+      const float m2 = x[4 * NA * kThreads + tid], l2 = x[(4 * NA + 1) * kThreads + tid];
+      if (m2 == -INFINITY) continue;  // saw no key of this row
+      const float mn = fmaxf(m, m2);
+      const float s1 = __builtin_amdgcn_exp2f(m - mn), s2 = __builtin_amdgcn_exp2f(m2 - mn);
+      l = l * s1 + l2 * s2;
+#pragma unroll
+      for (int d = 0; d < NA; ++d)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[d][r] = acc[d][r] * s1 + x[(4 * d + r) * kThreads + tid] * s2;
+      m = mn;
+    }
   }
   l += __shfl_xor(l, 16);
   l += __shfl_xor(l, 32);
@@ -319,27 +377,70 @@ __host__ __device__ inline int q_tiles(int kg, int S, bool walk) {
   return walk ? all - 2 * kg : all;
 }
 
-// dK/dV: grid (chunk, key group, batch x kv head), the chunk fastest.
+// Key tiles that item `i`'s queries (kWaves tasks of 16 rows) reach.
+__host__ __device__ inline int k_tiles(int i, int ntasks, int G, int S, bool walk) {
+  const int last = kWaves * i + kWaves - 1 < ntasks ? kWaves * i + kWaves - 1 : ntasks - 1;
+  const int end = walk && 16 * (last / G) + 16 < S ? 16 * (last / G) + 16 : S;
+  return (end + kTile - 1) / kTile;
+}
+
+// Workgroup id -> (batch x kv head, part i, chunk c of it): the parts' chunks
+// of one (batch, head) in a row, the (batch, head) fastest.  Workgroups go to
+// the 8 XCDs in turn, so each XCD gets every 8th of equally long chunks (grids
+// with empty chunks in them left some XCDs idle: dK/dV 588 us with the chunk
+// slowest, 397 with it fastest, 363 so, fp32 B4 8/2 heads x 64, S 2048),
+// and with 8 (batch, head) pairs one pair's rows per L2.  64 parts at a time.
+template <typename F>
+__device__ __forceinline__ bool locate(int id, int BHkv, int n, int ch, F tiles, int& bk, int& i, int& c) {
+  bk = id % BHkv;
+  int j = id / BHkv;
+  const int lane = threadIdx.x & 63;
+  for (int base = 0; base < n; base += 64) {
+    const int p = base + lane;
+    int cum = p < n ? (tiles(p) + ch - 1) / ch : 0;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int up = __shfl_up(cum, off);
+      if (lane >= off) cum += up;
+    }
+    const int all = __builtin_amdgcn_readlane(cum, 63);
+    if (j < all) {
+      const int at = __popcll(__ballot(cum <= j));  // the first part whose running count passes j
+      const int before = at ? __builtin_amdgcn_readlane(cum, at - 1) : 0;
+      i = base + at;
+      c = j - before;
+      return true;
+    }
+    j -= all;
+  }
+  return false;
+}
+
+// dK/dV: a workgroup takes 64 keys of one (batch, kv head) and a chunk of the
+// (head of the group, query tile) walk.
 template <typename T, int HDP>
 __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dkdv_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, const T* __restrict__ dout,
     const float* __restrict__ dvec, const float* __restrict__ lse2, const uint8_t* __restrict__ kmask, int mode,
     T* __restrict__ dk, T* __restrict__ dv, float* __restrict__ part, int Hq, int Hkv, int S, int hd, int G,
-    int nkg, int ch, int maxch, Strides3 qs, Strides3 ks, Strides3 vs, Strides3 ds, Strides3 dks, Strides3 dvs,
+    int BHkv, int nkg, int ch, int maxch, Strides3 qs, Strides3 ks, Strides3 vs, Strides3 ds, Strides3 dks, Strides3 dvs,
     int causal, int vec, float scale_log2, float scale) {
   using St = Stage<T, HDP>;
   __shared__ __attribute__((aligned(16))) float smem[2][2 * St::WORDS];
   __shared__ __attribute__((aligned(16))) float rowv[2][2][kTile];  // lse2 and D of the tile's rows
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int c = blockIdx.x % maxch, rest = blockIdx.x / maxch;
-  const int kg = rest % nkg, bk = rest / nkg;
-  const int b = bk / Hkv, kvh = bk - b * Hkv;
   const bool walk = causal && mode != HYDRA_MASK_REFERENCE_SDPA;
+  int bk, kg, c;
+  if (!locate(blockIdx.x, BHkv, nkg, ch, [&](int i) { return G * q_tiles(i, S, walk); }, bk, kg, c)) return;
+  bk = __builtin_amdgcn_readfirstlane(bk);
+  kg = __builtin_amdgcn_readfirstlane(kg);
+  c = __builtin_amdgcn_readfirstlane(c);
+  const int rest = bk * nkg + kg, parts = BHkv * nkg;
+  const int b = bk / Hkv, kvh = bk - b * Hkv;
   const int qt0 = walk ? 2 * kg : 0;
   const int nq = q_tiles(kg, S, walk);
   const int total = G * nq;
-  if (c * ch >= total) return;
   const int kw0 = 64 * kg + 16 * wave, key = kw0 + n;
   bool keep = key < S;
   if (mode != HYDRA_MASK_NONE && keep) keep = kmask[static_cast<int64_t>(b) * S + key] != 0;
@@ -351,8 +452,8 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dkdv_kernel(
   const int kbnd = mode == HYDRA_MASK_REFERENCE_SDPA && !keep ? 0x7fffffff : key;
 
   float kf[HDP / 16][4], vf[HDP / 16][4];
-  load_frag<T, HDP>(kf, k + b * ks.b + kvh * ks.h + static_cast<int64_t>(key < S ? key : 0) * ks.s, 1, g, hd, key < S);
-  load_frag<T, HDP>(vf, v + b * vs.b + kvh * vs.h + static_cast<int64_t>(key < S ? key : 0) * vs.s, 1, g, hd, key < S);
+  load_frag<T, HDP>(kf, k + b * ks.b + kvh * ks.h + static_cast<int64_t>(key < S ? key : 0) * ks.s, g, hd, key < S, vec & 2);
+  load_frag<T, HDP>(vf, v + b * vs.b + kvh * vs.h + static_cast<int64_t>(key < S ? key : 0) * vs.s, g, hd, key < S, vec & 2);
   f32x4 dka[HDP / 16], dva[HDP / 16];
 #pragma unroll
   for (int t = 0; t < HDP / 16; ++t) dka[t] = dva[t] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -361,9 +462,9 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dkdv_kernel(
   float rv = 0.f;
   auto fetch = [&](int step) {
     const int hr = step / nq, row0 = kTile * (qt0 + step - hr * nq), h = kvh * G + hr;
-    if (vec) {
-      sq.fetch(Rows<T>{q + b * qs.b + h * qs.h, qs.s, 1}, row0, S);
-      sd.fetch(Rows<T>{dout + b * ds.b + h * ds.h, ds.s, 1}, row0, S);
+    if (vec & 1) {
+      sq.fetch(Rows<T>{q + b * qs.b + h * qs.h, qs.s, 1}, row0, S, tid);
+      sd.fetch(Rows<T>{dout + b * ds.b + h * ds.h, ds.s, 1}, row0, S, tid);
     }
     if (tid < 2 * kTile) {  // rows past S: zero, with zero Q and dO they add nothing
       const int row = row0 + (tid & (kTile - 1));
@@ -372,13 +473,13 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dkdv_kernel(
     }
   };
   auto land = [&](int step, int buf) {
-    if (vec) {
-      sq.land(smem[buf]);
-      sd.land(smem[buf] + St::WORDS);
+    if (vec & 1) {
+      sq.land(smem[buf], tid);
+      sd.land(smem[buf] + St::WORDS, tid);
     } else {
       const int hr = step / nq, row0 = kTile * (qt0 + step - hr * nq), h = kvh * G + hr;
-      St::direct(Rows<T>{q + b * qs.b + h * qs.h, qs.s, 1}, row0, S, hd, smem[buf]);
-      St::direct(Rows<T>{dout + b * ds.b + h * ds.h, ds.s, 1}, row0, S, hd, smem[buf] + St::WORDS);
+      St::direct(Rows<T>{q + b * qs.b + h * qs.h, qs.s, 1}, row0, S, hd, smem[buf], tid);
+      St::direct(Rows<T>{dout + b * ds.b + h * ds.h, ds.s, 1}, row0, S, hd, smem[buf] + St::WORDS, tid);
     }
     if (tid < 2 * kTile) rowv[buf][tid / kTile][tid & (kTile - 1)] = rv;
   };
@@ -425,7 +526,7 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dkdv_kernel(
     for (int t = 0; t < HDP / 16; ++t) dka[t] = dva[t] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   if (maxch > 1) {  // summed by attn_bwd_f32_reduce_kernel
-    const int64_t rows = static_cast<int64_t>(gridDim.x) / maxch * 64;  // of one chunk's partial
+    const int64_t rows = static_cast<int64_t>(parts) * 64;  // of one chunk's partial
     float* pk = part + ((static_cast<int64_t>(c) * 2) * rows + (static_cast<int64_t>(rest) * 64 + 16 * wave + n)) * HDP;
     store_part<HDP>(pk, dka, g);
     store_part<HDP>(pk + rows * HDP, dva, g);
@@ -435,36 +536,37 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dkdv_kernel(
   }
 }
 
-// dQ: grid (chunk, item, batch x kv head).
+// dQ: a workgroup takes an item and a chunk of its key tiles.
 template <typename T, int HDP>
 __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dq_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, const T* __restrict__ dout,
     const float* __restrict__ dvec, const float* __restrict__ lse2, const uint8_t* __restrict__ kmask, int mode,
-    T* __restrict__ dq, float* __restrict__ part, int Hq, int Hkv, int S, int hd, int G, int ntasks, int items,
-    int ch, int maxch, Strides3 qs, Strides3 ks, Strides3 vs, Strides3 ds, Strides3 dqs, int causal, int vec,
+    T* __restrict__ dq, float* __restrict__ part, int Hq, int Hkv, int S, int hd, int G, int BHkv, int ntasks,
+    int items, int ch, int maxch, Strides3 qs, Strides3 ks, Strides3 vs, Strides3 ds, Strides3 dqs, int causal, int vec,
     float scale_log2, float scale) {
   using St = Stage<T, HDP>;
   __shared__ __attribute__((aligned(16))) float smem[2][2 * St::WORDS];
   __shared__ int keepv[2][kTile];
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int c = blockIdx.x % maxch, rest = blockIdx.x / maxch;
-  const int item = items - 1 - rest % items, bk = rest / items;
-  const int b = bk / Hkv, kvh = bk - b * Hkv;
   const bool walk = causal && mode != HYDRA_MASK_REFERENCE_SDPA;
-  const int last_task = min(kWaves * item + kWaves - 1, ntasks - 1);
-  const int kend = walk ? min(16 * (last_task / G) + 16, S) : S;
-  const int nt = (kend + kTile - 1) / kTile;
+  int bk, item, c;
+  if (!locate(blockIdx.x, BHkv, items, ch, [&](int i) { return k_tiles(i, ntasks, G, S, walk); }, bk, item, c)) return;
+  bk = __builtin_amdgcn_readfirstlane(bk);
+  item = __builtin_amdgcn_readfirstlane(item);
+  c = __builtin_amdgcn_readfirstlane(c);
+  const int parts = BHkv * items;
+  const int b = bk / Hkv, kvh = bk - b * Hkv;
+  const int nt = k_tiles(item, ntasks, G, S, walk);
   const int first = c * ch, end = min(first + ch, nt);
-  if (first >= nt) return;
   const Task tk = task_of(kWaves * item + wave, ntasks, kvh, G);
   const int qi = tk.q0 + n;
   const bool qok = tk.active && qi < S;
   const int my_end = !tk.active ? 0 : walk ? min(tk.q0 + 16, S) : S;
   float qf[HDP / 16][4], of[HDP / 16][4];
   const int64_t qr = qok ? qi : 0;
-  load_frag<T, HDP>(qf, q + b * qs.b + tk.h * qs.h + qr * qs.s, 1, g, hd, qok);
-  load_frag<T, HDP>(of, dout + b * ds.b + tk.h * ds.h + qr * ds.s, 1, g, hd, qok);
+  load_frag<T, HDP>(qf, q + b * qs.b + tk.h * qs.h + qr * qs.s, g, hd, qok, vec & 2);
+  load_frag<T, HDP>(of, dout + b * ds.b + tk.h * ds.h + qr * ds.s, g, hd, qok, vec & 2);
   float l2 = 0.f, dd = 0.f;
   if (qok) {
     const int64_t ri = (static_cast<int64_t>(b) * Hq + tk.h) * S + qi;
@@ -479,9 +581,9 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dq_kernel(
   St sk, sv;
   int kp = 0;
   auto fetch = [&](int t) {
-    if (vec) {
-      sk.fetch(kr, kTile * t, S);
-      sv.fetch(vr, kTile * t, S);
+    if (vec & 1) {
+      sk.fetch(kr, kTile * t, S, tid);
+      sv.fetch(vr, kTile * t, S, tid);
     }
     if (mode != HYDRA_MASK_NONE && tid < kTile) {
       const int key = kTile * t + tid;
@@ -489,12 +591,12 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dq_kernel(
     }
   };
   auto land = [&](int t, int buf) {
-    if (vec) {
-      sk.land(smem[buf]);
-      sv.land(smem[buf] + St::WORDS);
+    if (vec & 1) {
+      sk.land(smem[buf], tid);
+      sv.land(smem[buf] + St::WORDS, tid);
     } else {
-      St::direct(kr, kTile * t, S, hd, smem[buf]);
-      St::direct(vr, kTile * t, S, hd, smem[buf] + St::WORDS);
+      St::direct(kr, kTile * t, S, hd, smem[buf], tid);
+      St::direct(vr, kTile * t, S, hd, smem[buf] + St::WORDS, tid);
     }
     if (mode != HYDRA_MASK_NONE && tid < kTile) keepv[buf][tid] = kp;
   };
@@ -527,7 +629,7 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dq_kernel(
     if (t + 1 < end) land(t + 1, buf ^ 1);
   }
   if (maxch > 1) {
-    const int64_t rows = static_cast<int64_t>(gridDim.x) / maxch * 64;
+    const int64_t rows = static_cast<int64_t>(parts) * 64;
     store_part<HDP>(part + (static_cast<int64_t>(c) * rows + (static_cast<int64_t>(bk) * items + item) * 64 + 16 * wave + n) * HDP,
                     acc, g);
   } else if (qok) {
@@ -565,9 +667,7 @@ __global__ __launch_bounds__(256) void attn_bwd_f32_reduce_kernel(ReduceArgs a, 
     if (task >= a.ntasks) return;
     const int row = 16 * (task / a.G) + w % 16, h = kvh * a.G + task % a.G;
     if (row >= a.S) return;
-    const int last_task = min(kWaves * item + kWaves - 1, a.ntasks - 1);
-    const int kend = a.walk ? min(16 * (last_task / a.G) + 16, a.S) : a.S;
-    nch = ((kend + kTile - 1) / kTile + a.ch_q - 1) / a.ch_q;
+    nch = (k_tiles(item, a.ntasks, a.G, a.S, a.walk) + a.ch_q - 1) / a.ch_q;
     p = a.pq + i * HDP + d;
     step = rows * HDP;
     out = static_cast<T*>(a.dq) + b * a.dqs.b + h * a.dqs.h + static_cast<int64_t>(row) * a.dqs.s;
@@ -582,6 +682,7 @@ __global__ __launch_bounds__(256) void attn_bwd_f32_reduce_kernel(ReduceArgs a, 
     out = static_cast<T*>(which ? a.dv : a.dk) + b * s.b + kvh * s.h + static_cast<int64_t>(row) * s.s;
   }
   float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
   for (int c = 0; c < nch; ++c) {
     const float4 x = *reinterpret_cast<const float4*>(p + c * step);
     sum.x += x.x; sum.y += x.y; sum.z += x.z; sum.w += x.w;
@@ -593,14 +694,22 @@ __global__ __launch_bounds__(256) void attn_bwd_f32_reduce_kernel(ReduceArgs a, 
     if (d + r < a.hd) out[d + r] = from_f32<T>(o[r]);
 }
 
-// How the walks are cut: chunks of ch tiles, enough of them for kPerCu
-// workgroups on every CU, none shorter than kMinTiles.
+// How the walks are cut: chunks of equally many tiles, about kRounds times as
+// many workgroups as are resident at once (none shorter than kMinTiles), so
+// that the dispatcher evens out what causality and partial chunks leave uneven.
+// One exact round left the CUs idle 30% (dK/dV) to 50% (dQ) of the launch at
+// fp32 B4 8/2 heads x 64, S 2048; the partials of three rounds cost ~30 us of
+// HBM there (dK/dV 481 -> 363 us, dQ 499 -> 296).
 struct Plan {
   int HDP, G, ntasks, items, nkg, BHkv;
   int ch_kv, max_kv, ch_q, max_q;
+  int64_t wg_kv, wg_q;  // workgroups
   size_t kv_floats, q_floats;
 };
-constexpr int kPerCu = 4, kMinTiles = 6;
+constexpr int kMinTiles = 6, kRounds = 3;
+// Workgroups of each backward kernel resident on a CU (registers; 142 / 125 at
+// head_dim 64), by head_dim 16, 32, 64, 128.
+constexpr int kKvPerCu[4] = {6, 5, 3, 2}, kQPerCu[4] = {7, 5, 3, 2};
 
 // split = false: every walk whole (no partials).
 Plan plan_of(int B, int Hq, int Hkv, int S, int hd, bool walk, bool split) {
@@ -612,19 +721,21 @@ Plan plan_of(int B, int Hq, int Hkv, int S, int hd, bool walk, bool split) {
   p.items = (p.ntasks + kWaves - 1) / kWaves;
   p.nkg = (S + 63) / 64;
   const int all = (S + kTile - 1) / kTile;
-  auto cut = [&](int64_t tiles, int longest, int* ch, int* nch) {
-    const int64_t want = (tiles + kPerCu * device_cus() - 1) / (kPerCu * device_cus());
-    *ch = split ? static_cast<int>(std::max<int64_t>(want, kMinTiles)) : longest;
+  const int hi = p.HDP == 16 ? 0 : p.HDP == 32 ? 1 : p.HDP == 64 ? 2 : 3;
+  // tiles(i): the walk of part i of n, the same in every (batch, kv head)
+  auto cut = [&](int n, auto tiles, int longest, int per_cu, int* ch, int* nch, int64_t* wgs) {
+    const int64_t slots = static_cast<int64_t>(per_cu) * device_cus();
+    int64_t total = 0;
+    for (int i = 0; i < n; ++i) total += tiles(i);
+    const int64_t c = std::max<int64_t>((total * p.BHkv + kRounds * slots - 1) / (kRounds * slots), kMinTiles);
+    *ch = split ? static_cast<int>(std::min<int64_t>(c, longest)) : longest;
     *nch = (longest + *ch - 1) / *ch;
+    *wgs = 0;
+    for (int i = 0; i < n; ++i) *wgs += (tiles(i) + *ch - 1) / *ch;
+    *wgs *= p.BHkv;
   };
-  int64_t tk = 0, tq = 0;
-  for (int g = 0; g < p.nkg; ++g) tk += p.G * q_tiles(g, S, walk);
-  for (int i = 0; i < p.items; ++i) {
-    const int lt = std::min(kWaves * i + kWaves - 1, p.ntasks - 1);
-    tq += ((walk ? std::min(16 * (lt / p.G) + 16, S) : S) + kTile - 1) / kTile;
-  }
-  cut(tk * p.BHkv, p.G * all, &p.ch_kv, &p.max_kv);
-  cut(tq * p.BHkv, all, &p.ch_q, &p.max_q);
+  cut(p.nkg, [&](int g) { return p.G * q_tiles(g, S, walk); }, p.G * all, kKvPerCu[hi], &p.ch_kv, &p.max_kv, &p.wg_kv);
+  cut(p.items, [&](int i) { return k_tiles(i, p.ntasks, p.G, S, walk); }, all, kQPerCu[hi], &p.ch_q, &p.max_q, &p.wg_q);
   p.kv_floats = p.max_kv > 1 ? size_t(p.BHkv) * p.nkg * 64 * p.HDP * 2 * p.max_kv : 0;
   p.q_floats = p.max_q > 1 ? size_t(p.BHkv) * p.items * 64 * p.HDP * p.max_q : 0;
   return p;
@@ -641,13 +752,22 @@ template <typename T, int HDP>
 int launch_fwd(const AttnF32Args& a) {
   constexpr int E = 16 / int(sizeof(T));
   const int G = a.Hq / a.Hkv, ntasks = G * ((a.S + 15) / 16), items = (ntasks + kWaves - 1) / kWaves;
-  const bool vec = a.hd == HDP && vec_ok(a.k, a.ks, E) && vec_ok(a.v, a.vs, E);
+  const int vec = (a.hd == HDP && vec_ok(a.k, a.ks, E) && vec_ok(a.v, a.vs, E) ? 1 : 0) |
+                  (a.hd == HDP && vec_ok(a.q, a.qs, E) ? 2 : 0);
   const int64_t blocks = static_cast<int64_t>(items) * a.B * a.Hkv;
   if (blocks >= (int64_t(1) << 31)) return fail(HYDRA_ERR_ARG, "attn_fwd: too many rows");
-  attn_fwd_f32_kernel<T, HDP><<<dim3(static_cast<unsigned>(blocks)), kThreads, 0, a.st>>>(
+  // Key groups when the items are fewer than two per resident workgroup
+  // (registers: 3 per CU at head_dim 64): the longest walk sets the time then.
+  // Two groups at head_dim 128 (LDS), else four.  fp16 B2 8/2 x 64, S 1500
+  // (376 items): 104 -> 71 us.
+  constexpr int KG = HDP == 128 ? 2 : 4;
+  constexpr int per_cu = HDP <= 32 ? 5 : HDP == 64 ? 3 : 2;
+  const bool groups = blocks < 2 * int64_t(per_cu) * device_cus();
+  auto kern = groups ? attn_fwd_f32_kernel<T, HDP, KG> : attn_fwd_f32_kernel<T, HDP, 1>;
+  kern<<<dim3(static_cast<unsigned>(blocks)), kThreads * (groups ? KG : 1), 0, a.st>>>(
       static_cast<const T*>(a.q), static_cast<const T*>(a.k), static_cast<const T*>(a.v), static_cast<T*>(a.o),
       a.lse, a.kmask, a.mask_mode, a.Hq, a.Hkv, a.S, a.hd, G, ntasks, items, s3(a.qs), s3(a.ks), s3(a.vs), a.vs[3],
-      s3(a.os), a.causal ? 1 : 0, vec ? 1 : 0, a.scale * kLog2eF);
+      s3(a.os), a.causal ? 1 : 0, vec, a.scale * kLog2eF);
   return check_launch("attn_fwd_f32_kernel");
 }
 
@@ -657,24 +777,24 @@ int launch_bwd(const AttnF32Args& a, float* part, size_t part_bytes) {
   const bool walk = a.causal && a.mask_mode != HYDRA_MASK_REFERENCE_SDPA;
   Plan p = plan_of(a.B, a.Hq, a.Hkv, a.S, a.hd, walk, true);
   if ((p.kv_floats + p.q_floats) * sizeof(float) > part_bytes) p = plan_of(a.B, a.Hq, a.Hkv, a.S, a.hd, walk, false);
-  const bool whole = a.hd == HDP;
+  const bool qv = a.hd == HDP && vec_ok(a.q, a.qs, E) && vec_ok(a.dout, a.dos, E);
+  const bool kv = a.hd == HDP && vec_ok(a.k, a.ks, E) && vec_ok(a.v, a.vs, E);
   const float sl2 = a.scale * kLog2eF;
-  const int64_t bkv = static_cast<int64_t>(p.max_kv) * p.nkg * p.BHkv, bq = static_cast<int64_t>(p.max_q) * p.items * p.BHkv;
-  if (bkv >= (int64_t(1) << 31) || bq >= (int64_t(1) << 31)) return fail(HYDRA_ERR_ARG, "attn_bwd: problem too large");
+  if (p.wg_kv >= (int64_t(1) << 31) || p.wg_q >= (int64_t(1) << 31)) return fail(HYDRA_ERR_ARG, "attn_bwd: problem too large");
   const T* q = static_cast<const T*>(a.q);
   const T* k = static_cast<const T*>(a.k);
   const T* v = static_cast<const T*>(a.v);
   const T* d = static_cast<const T*>(a.dout);
   float* pq = part + p.kv_floats;
-  attn_bwd_f32_dkdv_kernel<T, HDP><<<dim3(static_cast<unsigned>(bkv)), kThreads, 0, a.st>>>(
+  attn_bwd_f32_dkdv_kernel<T, HDP><<<dim3(static_cast<unsigned>(p.wg_kv)), kThreads, 0, a.st>>>(
       q, k, v, d, a.dvec, a.lse2, a.kmask, a.mask_mode, static_cast<T*>(a.dk), static_cast<T*>(a.dv), part, a.Hq,
-      a.Hkv, a.S, a.hd, p.G, p.nkg, p.ch_kv, p.max_kv, s3(a.qs), s3(a.ks), s3(a.vs), s3(a.dos), s3(a.dks), s3(a.dvs),
-      a.causal ? 1 : 0, whole && vec_ok(a.q, a.qs, E) && vec_ok(a.dout, a.dos, E) ? 1 : 0, sl2, a.scale);
+      a.Hkv, a.S, a.hd, p.G, p.BHkv, p.nkg, p.ch_kv, p.max_kv, s3(a.qs), s3(a.ks), s3(a.vs), s3(a.dos), s3(a.dks), s3(a.dvs),
+      a.causal ? 1 : 0, (qv ? 1 : 0) | (kv ? 2 : 0), sl2, a.scale);
   if (int rc = check_launch("attn_bwd: f32 dkdv")) return rc;
-  attn_bwd_f32_dq_kernel<T, HDP><<<dim3(static_cast<unsigned>(bq)), kThreads, 0, a.st>>>(
+  attn_bwd_f32_dq_kernel<T, HDP><<<dim3(static_cast<unsigned>(p.wg_q)), kThreads, 0, a.st>>>(
       q, k, v, d, a.dvec, a.lse2, a.kmask, a.mask_mode, static_cast<T*>(a.dq), pq, a.Hq, a.Hkv, a.S, a.hd, p.G,
-      p.ntasks, p.items, p.ch_q, p.max_q, s3(a.qs), s3(a.ks), s3(a.vs), s3(a.dos), s3(a.dqs), a.causal ? 1 : 0,
-      whole && vec_ok(a.k, a.ks, E) && vec_ok(a.v, a.vs, E) ? 1 : 0, sl2, a.scale);
+      p.BHkv, p.ntasks, p.items, p.ch_q, p.max_q, s3(a.qs), s3(a.ks), s3(a.vs), s3(a.dos), s3(a.dqs), a.causal ? 1 : 0,
+      (kv ? 1 : 0) | (qv ? 2 : 0), sl2, a.scale);
   if (int rc = check_launch("attn_bwd: f32 dq")) return rc;
   if (p.max_kv == 1 && p.max_q == 1) return HYDRA_OK;
   const ReduceArgs r{part, pq, a.dk, a.dv, a.dq, s3(a.dks), s3(a.dvs), s3(a.dqs), a.Hq, a.Hkv, a.S, a.hd, p.G,
