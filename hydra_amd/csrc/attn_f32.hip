@@ -1,26 +1,36 @@
-// Attention in fp32 arithmetic on v_mfma_f32_16x16x4_f32, for any element
+// Attention in fp32 arithmetic on 16x16 matrix instructions, for any element
 // type, any strides, head_dim up to 128: o = softmax(scale * q k^T [+ masks]) v
 // and its gradients, with the semantics of attn_fwd.hip and attn_bwd.hip
 // (reference: fused_attention.py:14-110, 113-338, 706-823 and the masked SDPA
 // call attention.py:268-299).  fp32 and fp16 calls run here, and bf16 calls
-// whose head_dim or strides the bf16 MFMA kernels do not take.  Products and
-// sums are fp32 throughout, so results are as exact as one thread's fp32 sums.
+// whose head_dim or strides the bf16 MFMA kernels do not take.
 //
-// What bounds it: the fp32 matrix rate (256 FLOP per CU and cycle, a tenth of
-// bf16's measured rate); a 16x16x4 step takes 32 cycles of a SIMD, against one
-// 4-byte LDS read per lane, so LDS and the softmax's VALU work hide behind it.
-// The 16x16 tile (and not 32x32x2) because a wave then holds 16 rows: K and V
-// (or Q and dO) fragments and both accumulators of head_dim 128 fit the
-// registers without spills.
+// Arithmetic.  fp32 elements: v_mfma_f32_16x16x4_f32 throughout.  16-bit
+// elements: q k^T and dO v^T go to the 16-bit instructions as they are (their
+// products are exact in fp32), and the fp32 probabilities and score gradients
+// go there as two or three 16-bit planes that add up to them to fp32's own
+// precision (prob_product, grad_product), so nothing is held to 16 bits.  A
+// tile with an infinity or NaN in it, a score gradient that overflowed or a
+// probability past kPMax takes the fp32 instruction instead (col_product):
+// planes would make inf - inf of it.
+//
+// What bounds it.  fp32: the fp32 matrix rate (256 FLOP per CU and cycle, a
+// tenth of bf16's measured rate); a 16x16x4 step takes 32 cycles of a SIMD,
+// against one 4-byte LDS read per lane, so LDS and the softmax's VALU work hide
+// behind it.  16 bits: VALU (exponentials, splits) and LDS reads.  The 16x16
+// tile (and not 32x32) because a wave then holds 16 rows: K and V (or Q and dO)
+// fragments and both accumulators of head_dim 128 fit the registers without
+// spills.
 //
 // Layouts.  A fragment of rows X[m][d] (m = lane % 16, g = lane / 16) takes the
-// summed index d in the order 16 j + 4 g + i over steps (j, i): one 16-byte LDS
-// read feeds four steps, and the resident side holds the same order.  A result
-// tile has row 4 g + r in register r and column lane % 16, so register r is the
-// B operand of the next product with the summed index in the order 4 g + r,
-// whose A operand is one 4-byte read of row 4 g + r of the staged tile: nothing
-// is transposed.  Staged rows are head_dim + 4 words apart, which puts the four
-// row groups of such a read into different banks.
+// summed index d in runs of R = 4 (fp32, or head_dim 16) or 8 elements, 4 R j +
+// R g + i over steps (j, i): one 16-byte LDS read feeds a step, and the resident
+// side holds the same order.  A result tile has row 4 g + r in register r and
+// column lane % 16, so its registers are the B operand of the next product with
+// the summed index in the order 4 g + r, whose A operand is a 4-byte read of
+// row 4 g + r of the staged tile (fp32) or a transposing read (16 bits):
+// nothing is transposed.  Staged rows are 16 bytes longer than head_dim, which
+// puts the row groups of such reads into different banks.
 //
 // Every wave owns 16 rows (queries forward and for dQ, keys for dK/dV); a
 // workgroup's four waves share the staged 32-row tiles of the other side,
@@ -31,11 +41,14 @@
 //
 // Measured, forward + backward of one call, against what these calls took
 // before (16 lanes per query row forward, one thread per row backward, VALU):
-// fp16 B2 8/2 heads x 64, S 1500, causal 198.1 -> 0.27 ms; fp32 B4 8/2 x 64,
-// S 2048, causal 274 -> 0.82 ms; fp32 B1 4/1 x 128, S 1000 172.9 -> 0.26 ms;
-// fp32 B2 8/2 x 16, S 512, causal 8.7 -> 0.17 ms (launch-bound).  Errors
-// against 64 bits: fp32 1.8e-6 -> 5.9e-7, fp16 2.2e-4 (the output's rounding)
-// both.
+// fp16 B2 8/2 heads x 64, S 1500, causal 198.1 -> 0.15 ms (launch-bound); fp32
+// B4 8/2 x 64, S 2048, causal 274 -> 0.81 ms; fp32 B1 4/1 x 128, S 1000 172.9 ->
+// 0.26 ms; fp32 B2 8/2 x 16, S 512, causal 8.7 -> 0.17 ms (launch-bound).
+// Errors against 64 bits: fp32 1.8e-6 -> 5.8e-7, fp16 2.3e-4 (the output's
+// rounding) both.  16-bit planes against the fp32 instruction on the converted
+// rows, fp16: the first of these calls' kernels forward 71 -> 33, dK/dV 115 ->
+// 54, dQ 88 -> 40 us; B8 8/2 x 64, S 2048 1516 -> 616 us; B2 8/2 x 128, S 2048
+// 841 -> 352 us; B4 8/2 x 16, S 2048 270 -> 208 us.
 #include "attn_f32.h"
 
 #include <algorithm>
@@ -71,15 +84,32 @@ struct Rows {
   int64_t rs, es;
 };
 
+// How many consecutive elements of a row a lane holds per step of a row
+// product, and a row's steps.
+template <typename T, int HDP>
+struct Row16 {
+  static constexpr int R = sizeof(T) == 2 && HDP >= 32 ? 8 : 4;
+  static constexpr int N = HDP / (4 * R);
+  struct __attribute__((aligned(R * sizeof(T)))) Run {
+    T v[R];
+  };
+};
+
+// fp16's gradient products read the staged rows as two bf16 planes (hi + lo,
+// exact), tiles of their own after the staged pair.
+template <typename T>
+constexpr bool kPlaneTiles = std::is_same<T, f16>::value;
+
 // Registers of one thread's share of a staged tile, and its way to LDS (t:
-// the thread's index among the kThreads that stage it).
+// the thread's index among the kThreads that stage it).  land and direct
+// return whether an infinity or NaN was among the elements (16-bit types).
 template <typename T, int HDP>
 struct Stage {
-  static constexpr int P = HDP + 4;                 // words per staged row
   static constexpr int E = 16 / int(sizeof(T));     // elements per 16-byte load
+  static constexpr int P = HDP + E;                 // elements per staged row
   static constexpr int VU = (kTile * HDP / E + kThreads - 1) / kThreads;
   static constexpr int SU = kTile * HDP / kThreads;  // scalar path: elements per thread
-  static constexpr int WORDS = kTile * P;
+  static constexpr int N = kTile * P;                // elements per tile
   static constexpr bool WHOLE = (kTile * HDP / E) % kThreads == 0;
 
   uint4 raw[VU];
@@ -90,89 +120,241 @@ struct Stage {
       const int i = t + kThreads * u;
       const int row = i / (HDP / E), c = i - row * (HDP / E);
       const bool ok = (WHOLE || row < kTile) && row0 + row < S;
-      raw[u] = ok ? *reinterpret_cast<const uint4*>(r.base + static_cast<int64_t>(row0 + row) * r.rs + c * E)
-                  : make_uint4(0, 0, 0, 0);
+      raw[u] = make_uint4(0, 0, 0, 0);
+      if (ok) raw[u] = ld16raw<false>(r.base + static_cast<int64_t>(row0 + row) * r.rs + c * E);
     }
   }
-  __device__ __forceinline__ void land(float* dst, int t) const {
+  // planes: where the bf16 planes go (kPlaneTiles), or null
+  __device__ __forceinline__ bool land(T* dst, T* planes, int t) const {
+    uint32_t odd = 0;
 #pragma unroll
     for (int u = 0; u < VU; ++u) {
       const int i = t + kThreads * u;
       const int row = i / (HDP / E), c = i - row * (HDP / E);
       if (WHOLE || row < kTile) {
-        float f[E];
-        unpack16<T>(raw[u], f);
+        *reinterpret_cast<uint4*>(&dst[row * P + c * E]) = raw[u];
+        if constexpr (sizeof(T) == 2) odd |= exponent_full(raw[u].x) | exponent_full(raw[u].y) |
+                                             exponent_full(raw[u].z) | exponent_full(raw[u].w);
+        if constexpr (kPlaneTiles<T>) {
+          if (planes) {
+            float f[8], lo[8];
+            unpack16<f16>(raw[u], f);
+            const uint4 h = pack16<bf16>(f);
+            unpack16<bf16>(h, lo);
 #pragma unroll
-        for (int e = 0; e < E; e += 4)
-          *reinterpret_cast<float4*>(&dst[row * P + c * E + e]) = make_float4(f[e], f[e + 1], f[e + 2], f[e + 3]);
+            for (int e = 0; e < 8; ++e) lo[e] = f[e] - lo[e];
+            *reinterpret_cast<uint4*>(&planes[row * P + c * E]) = h;
+            *reinterpret_cast<uint4*>(&planes[N + row * P + c * E]) = pack16<bf16>(lo);
+          }
+        }
       }
     }
+    return odd != 0;
   }
   // Any strides and head_dim: element by element, straight to LDS.
-  static __device__ __forceinline__ void direct(const Rows<T>& r, int row0, int S, int hd, float* dst, int t) {
+  static __device__ __forceinline__ bool direct(const Rows<T>& r, int row0, int S, int hd, T* dst, T* planes, int t) {
+    bool odd = false;
 #pragma unroll 4
     for (int u = 0; u < SU; ++u) {
       const int i = t + kThreads * u;
       const int row = i / HDP, d = i - row * HDP;
       const bool ok = row0 + row < S && d < hd;
-      dst[row * P + d] = ok ? to_f32(r.base[static_cast<int64_t>(row0 + row) * r.rs + d * r.es]) : 0.f;
+      T x = from_f32<T>(0.f);
+      if (ok) x = r.base[static_cast<int64_t>(row0 + row) * r.rs + d * r.es];
+      dst[row * P + d] = x;
+      if constexpr (sizeof(T) == 2) odd |= exponent_full(x.bits) != 0;
+      if constexpr (kPlaneTiles<T>) {
+        if (planes) {
+          const float f = to_f32(x);
+          const bf16 h = from_f32<bf16>(f);
+          planes[row * P + d].bits = h.bits;
+          planes[N + row * P + d].bits = from_f32<bf16>(f - to_f32(h)).bits;
+        }
+      }
     }
+    return odd;
+  }
+  // nonzero: one of the two packed elements is an infinity or NaN
+  static __device__ __forceinline__ uint32_t exponent_full(uint32_t w) {
+    constexpr uint32_t M = std::is_same<T, f16>::value ? 0x7c007c00u : 0x7f807f80u;
+    constexpr uint32_t ONE = std::is_same<T, f16>::value ? 0x04000400u : 0x00800080u;
+    return ((w & M) + ONE) & 0x80008000u;
   }
 };
 
 // The resident fragment of one row (column lane % 16 of B): elements
-// 16 j + 4 g + i of the row, zero past hd or for a row that is not there.
-// vec: rows of HDP elements, aligned to four of them.
+// 4 R j + R g + i of the row (R = Row16::R), zero past hd or for a row that is not
+// there.  vec: rows of HDP elements, aligned to R of them.
 template <typename T, int HDP>
-__device__ __forceinline__ void load_frag(float (&f)[HDP / 16][4], const T* row, int g, int hd, bool ok, bool vec) {
+__device__ __forceinline__ void load_frag(const T* row, typename Row16<T, HDP>::Run (&f)[Row16<T, HDP>::N], int g, int hd,
+                                          bool ok, bool vec) {
+  constexpr int R = Row16<T, HDP>::R;
 #pragma unroll
-  for (int j = 0; j < HDP / 16; ++j)
+  for (int j = 0; j < Row16<T, HDP>::N; ++j)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) f[j][i] = 0.f;
+    for (int i = 0; i < R; ++i) f[j].v[i] = from_f32<T>(0.f);
   if (!ok) return;
   if (vec) {
-    struct alignas(4 * sizeof(T)) Four { T v[4]; };
-    Four raw[HDP / 16];
 #pragma unroll
-    for (int j = 0; j < HDP / 16; ++j) raw[j] = *reinterpret_cast<const Four*>(row + 16 * j + 4 * g);
-#pragma unroll
-    for (int j = 0; j < HDP / 16; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) f[j][i] = to_f32(raw[j].v[i]);
+    for (int j = 0; j < Row16<T, HDP>::N; ++j) f[j] = *reinterpret_cast<const typename Row16<T, HDP>::Run*>(row + 4 * R * j + R * g);
   } else {
 #pragma unroll
-    for (int j = 0; j < HDP / 16; ++j)
+    for (int j = 0; j < Row16<T, HDP>::N; ++j)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int d = 16 * j + 4 * g + i;
-        if (d < hd) f[j][i] = to_f32(row[d]);
+      for (int i = 0; i < R; ++i) {
+        const int d = 4 * R * j + R * g + i;
+        if (d < hd) f[j].v[i] = row[d];
       }
   }
 }
 
-// S and dP tiles (or S alone): rows of two staged operands times the
-// resident fragments.
-template <int HDP>
-__device__ __forceinline__ f32x4 row_product(const float* rows, const float (&f)[HDP / 16][4], int n, int g) {
+typedef __attribute__((ext_vector_type(4))) short s16x4;
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(4))) _Float16 f16x4;
+typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
+
+__device__ __forceinline__ f32x4 mfma16(f16, uint2 a, uint2 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(f16x4, a), __builtin_bit_cast(f16x4, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4 mfma16(bf16, uint2 a, uint2 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), c, 0, 0,
+                                                   0);
+}
+__device__ __forceinline__ f32x4 mfma32(f16, uint4 a, uint4 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4 mfma32(bf16, uint4 a, uint4 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0,
+                                                 0);
+}
+
+// S and dP tiles (or S alone): 16 staged rows times the resident fragment.
+// 16-bit elements go to the 16-bit matrix instructions as they are: their
+// products are exact there and the sums fp32.
+template <typename T, int HDP>
+__device__ __forceinline__ f32x4 row_product(const T* rows, const typename Row16<T, HDP>::Run (&f)[Row16<T, HDP>::N], int n, int g) {
+  constexpr int R = Row16<T, HDP>::R;
   f32x4 c = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int j = 0; j < HDP / 16; ++j) {
-    const float4 a = *reinterpret_cast<const float4*>(&rows[n * (HDP + 4) + 16 * j + 4 * g]);
-    c = mfma4(a.x, f[j][0], c);
-    c = mfma4(a.y, f[j][1], c);
-    c = mfma4(a.z, f[j][2], c);
-    c = mfma4(a.w, f[j][3], c);
+  for (int j = 0; j < Row16<T, HDP>::N; ++j) {
+    const auto a = *reinterpret_cast<const typename Row16<T, HDP>::Run*>(&rows[n * Stage<T, HDP>::P + 4 * R * j + R * g]);
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) c = mfma4(a.v[i], f[j].v[i], c);
+    } else if constexpr (R == 4) {
+      c = mfma16(T{}, __builtin_bit_cast(uint2, a), __builtin_bit_cast(uint2, f[j]), c);
+    } else {
+      c = mfma32(T{}, __builtin_bit_cast(uint4, a), __builtin_bit_cast(uint4, f[j]), c);
+    }
   }
   return c;
 }
 
-// acc[d tile] += rows^T * x: x a result tile whose rows are 16 staged rows.
-template <int HDP>
-__device__ __forceinline__ void col_product(f32x4 (&acc)[HDP / 16], const float* rows, const f32x4& x, int n, int g) {
+// acc[d tile] += rows^T * x in fp32: x a result tile whose rows are 16 staged
+// rows.  fp32 elements; 16-bit ones where a tile holds an infinity or NaN.
+template <typename T, int HDP>
+__device__ __forceinline__ void col_product(f32x4 (&acc)[HDP / 16], const T* rows, const f32x4& x, int n, int g) {
 #pragma unroll
   for (int r = 0; r < 4; ++r)
 #pragma unroll
-    for (int t = 0; t < HDP / 16; ++t) acc[t] = mfma4(rows[(4 * g + r) * (HDP + 4) + 16 * t + n], x[r], acc[t]);
+    for (int t = 0; t < HDP / 16; ++t)
+      acc[t] = mfma4(to_f32(rows[(4 * g + r) * Stage<T, HDP>::P + 16 * t + n]), x[r], acc[t]);
+}
+
+// The same over a whole staged tile of a 16-bit type, x as planes of 16-bit
+// values that add up to it.  The summed index: slot i < 4 of lane group g is
+// row 4 g + i, slot 4 + i row 16 + 4 g + i, which is the order the two result
+// tiles hold; the transposing LDS read gives the same (16 lanes read 4 rows of
+// 16 columns, lane j gets column j's four values).
+template <typename T, int HDP>
+__device__ __forceinline__ uint4 tile_cols(const T* tile, int t, int n, int g) {
+  typedef __attribute__((address_space(3))) s16x4* lds_t;
+  constexpr int P = Stage<T, HDP>::P;
+  const T* p = tile + (4 * g + (n >> 2)) * P + 16 * t + 4 * (n & 3);
+  const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_t)(p)));
+  const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_t)(p + 16 * P)));
+  return make_uint4(lo.x, lo.y, hi.x, hi.y);
+}
+
+// x as three bf16 planes, exactly (each takes the next 8 bits; x finite).
+__device__ __forceinline__ void split3(const f32x4 (&x)[2], uint4 (&p)[3]) {
+  uint32_t w[3][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    uint32_t b[2], m[2], l[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const float v = x[i >> 1][2 * (i & 1) + e];
+      b[e] = __float_as_uint(v);
+      const float r = v - __uint_as_float(b[e] & 0xffff0000u);
+      m[e] = __float_as_uint(r);
+      l[e] = __float_as_uint(r - __uint_as_float(m[e] & 0xffff0000u));
+    }
+    w[0][i] = __builtin_amdgcn_perm(b[1], b[0], 0x07060302);
+    w[1][i] = __builtin_amdgcn_perm(m[1], m[0], 0x07060302);
+    w[2][i] = __builtin_amdgcn_perm(l[1], l[0], 0x07060302);
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) p[k] = make_uint4(w[k][0], w[k][1], w[k][2], w[k][3]);
+}
+
+// Probabilities (0 .. 1): three bf16 planes beside bf16 rows; beside fp16 rows
+// two fp16 planes of x * kPScale, whose remainder is under half an fp32 ulp of
+// x (under 2^-39 for x below 2^-16, where the second plane goes subnormal).
+// Accumulators of either come out times kPScale.
+template <typename T>
+constexpr float kPScale = std::is_same<T, f16>::value ? 16384.f : 1.f;
+constexpr float kPMax = 3.5f;  // above: x * kPScale nears fp16's largest value
+
+template <typename T, int HDP>
+__device__ __forceinline__ void prob_product(f32x4 (&acc)[HDP / 16], const T* tile, const f32x4 (&x)[2], int n, int g) {
+  if constexpr (std::is_same<T, f16>::value) {
+    uint32_t h[4], l[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float a = x[i >> 1][2 * (i & 1)] * kPScale<T>, b = x[i >> 1][2 * (i & 1) + 1] * kPScale<T>;
+      const f16 ha = from_f32<f16>(a), hb = from_f32<f16>(b);
+      h[i] = static_cast<uint32_t>(ha.bits) | (static_cast<uint32_t>(hb.bits) << 16);
+      l[i] = pack2<f16>(a - to_f32(ha), b - to_f32(hb));
+    }
+    const uint4 ph = make_uint4(h[0], h[1], h[2], h[3]), pl = make_uint4(l[0], l[1], l[2], l[3]);
+#pragma unroll
+    for (int t = 0; t < HDP / 16; ++t) {
+      const uint4 a = tile_cols<T, HDP>(tile, t, n, g);
+      acc[t] = mfma32(f16{}, a, pl, acc[t]);
+      acc[t] = mfma32(f16{}, a, ph, acc[t]);
+    }
+  } else {
+    uint4 p[3];
+    split3(x, p);
+#pragma unroll
+    for (int t = 0; t < HDP / 16; ++t) {
+      const uint4 a = tile_cols<T, HDP>(tile, t, n, g);
+#pragma unroll
+      for (int k = 2; k >= 0; --k) acc[t] = mfma32(bf16{}, a, p[k], acc[t]);
+    }
+  }
+}
+
+// dS of any size: three bf16 planes times bf16 rows, or times the two bf16
+// planes of fp16 rows (the product of the two smallest, 2^-24 of the sum's
+// terms or less, left out).
+template <typename T, int HDP>
+__device__ __forceinline__ void grad_product(f32x4 (&acc)[HDP / 16], const T* tile, const T* planes,
+                                             const f32x4 (&x)[2], int n, int g) {
+  uint4 p[3];
+  split3(x, p);
+#pragma unroll
+  for (int t = 0; t < HDP / 16; ++t) {
+    const uint4 a = tile_cols<T, HDP>(kPlaneTiles<T> ? planes : tile, t, n, g);
+    if constexpr (kPlaneTiles<T>) {
+      const uint4 b = tile_cols<T, HDP>(planes + Stage<T, HDP>::N, t, n, g);
+      acc[t] = mfma32(bf16{}, b, p[1], acc[t]);
+      acc[t] = mfma32(bf16{}, b, p[0], acc[t]);
+    }
+#pragma unroll
+    for (int k = 2; k >= 0; --k) acc[t] = mfma32(bf16{}, a, p[k], acc[t]);
+  }
 }
 
 // Writes a wave's 16 rows (column n) of accumulators, scaled.
@@ -187,10 +369,16 @@ __device__ __forceinline__ void store_rows(T* row, const f32x4 (&acc)[HDP / 16],
     }
 }
 template <int HDP>
-__device__ __forceinline__ void store_part(float* row, const f32x4 (&acc)[HDP / 16], int g) {
+__device__ __forceinline__ void store_part(float* row, const f32x4 (&acc)[HDP / 16], float f, int g) {
 #pragma unroll
   for (int t = 0; t < HDP / 16; ++t)
-    *reinterpret_cast<float4*>(row + 16 * t + 4 * g) = make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
+    *reinterpret_cast<float4*>(row + 16 * t + 4 * g) = make_float4(acc[t][0] * f, acc[t][1] * f, acc[t][2] * f, acc[t][3] * f);
+}
+
+// The running maximum of |ds| with p's own limit folded in: infinite once the
+// planes of p or ds would not hold them.
+__device__ __forceinline__ float max_of(float big, float p, float ds) {
+  return fmaxf(fmaxf(big, fabsf(ds)), p > kPMax ? INFINITY : 0.f);
 }
 
 // Whether query s sees key t < S (keep: the key mask's flag of t).
@@ -227,13 +415,15 @@ __global__ __launch_bounds__(kThreads * KG) void attn_fwd_f32_kernel(
     int ntasks, int items, Strides3 qs, Strides3 ks, Strides3 vs, int64_t vs3, Strides3 os, int causal, int vec,
     float scale_log2) {
   using St = Stage<T, HDP>;
-  __shared__ __attribute__((aligned(16))) float smem_all[KG][2][2 * St::WORDS];
+  __shared__ __attribute__((aligned(16))) T smem_all[KG][2][2 * St::N];
   __shared__ int keep_all[KG][2][kTile];
+  __shared__ int odd_all[KG][2];  // the last tile landed there with an infinity or NaN in it (16-bit types)
   const int kg = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / kThreads) : 0;
   const int tid = threadIdx.x - kg * kThreads, lane = tid & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   auto& smem = smem_all[kg];
   auto& keepv = keep_all[kg];
+  auto& odd = odd_all[kg];
   const int BHkv = gridDim.x / items;
   const int bk = blockIdx.x % BHkv;
   const int item = items - 1 - static_cast<int>(blockIdx.x / BHkv);  // longest key ranges first
@@ -241,8 +431,8 @@ __global__ __launch_bounds__(kThreads * KG) void attn_fwd_f32_kernel(
   const Task tk = task_of(kWaves * item + wave, ntasks, kvh, G);
   const int qi = tk.q0 + n;
   const bool qok = tk.active && qi < S;
-  float qf[HDP / 16][4];
-  load_frag<T, HDP>(qf, q + b * qs.b + tk.h * qs.h + static_cast<int64_t>(qok ? qi : 0) * qs.s, g, hd, qok, vec & 2);
+  typename Row16<T, HDP>::Run qf[Row16<T, HDP>::N];
+  load_frag<T, HDP>(q + b * qs.b + tk.h * qs.h + static_cast<int64_t>(qok ? qi : 0) * qs.s, qf, g, hd, qok, vec & 2);
 
   const bool walk = causal && mode != HYDRA_MASK_REFERENCE_SDPA;
   const int last_task = min(kWaves * item + kWaves - 1, ntasks - 1);
@@ -269,15 +459,21 @@ __global__ __launch_bounds__(kThreads * KG) void attn_fwd_f32_kernel(
     }
   };
   auto land = [&](int t, int buf) {
+    bool o1, o2;
     if (vec & 1) {
-      sk.land(smem[buf], tid);
-      sv.land(smem[buf] + St::WORDS, tid);
+      o1 = sk.land(smem[buf], nullptr, tid);
+      o2 = sv.land(smem[buf] + St::N, nullptr, tid);
     } else {
-      St::direct(kr, kTile * t, S, hd, smem[buf], tid);
-      St::direct(vr, kTile * t, S, hd, smem[buf] + St::WORDS, tid);
+      o1 = St::direct(kr, kTile * t, S, hd, smem[buf], nullptr, tid);
+      o2 = St::direct(vr, kTile * t, S, hd, smem[buf] + St::N, nullptr, tid);
     }
+    if (sizeof(T) == 2 && (o1 || o2)) odd[buf] = t;
     if (mode != HYDRA_MASK_NONE && tid < kTile) keepv[buf][tid] = kp;
   };
+  if (sizeof(T) == 2) {
+    if (tid < 2) odd[tid] = -1;
+    __syncthreads();
+  }
   if (kg < nt) {
     fetch(kg);
     land(kg, 0);
@@ -288,12 +484,12 @@ __global__ __launch_bounds__(kThreads * KG) void attn_fwd_f32_kernel(
     const int t = KG * st + kg, buf = st & 1, t0 = kTile * t;
     if (t + KG < nt) fetch(t + KG);
     if (t0 < my_end) {
-      const float* Ks = smem[buf];
-      const float* Vs = Ks + St::WORDS;
+      const T* Ks = smem[buf];
+      const T* Vs = Ks + St::N;
       f32x4 x[2];
       float mt = m;
 #pragma unroll
-      for (int u = 0; u < 2; ++u) x[u] = row_product<HDP>(Ks + 16 * u * St::P, qf, n, g);
+      for (int u = 0; u < 2; ++u) x[u] = row_product<T, HDP>(Ks + 16 * u * St::P, qf, n, g);
       // whole tile visible to every row of the wave: no tests
       const bool plain = mode == HYDRA_MASK_NONE && t0 + kTile - 1 <= (walk ? tk.q0 : S - 1) && t0 + kTile <= S;
 #pragma unroll
@@ -326,16 +522,24 @@ __global__ __launch_bounds__(kThreads * KG) void attn_fwd_f32_kernel(
           x[u][r] = __builtin_amdgcn_exp2f(x[u][r] - ms);
           l += x[u][r];
         }
-        col_product<HDP>(acc, Vs + 16 * u * St::P, x[u], n, g);
+        if constexpr (sizeof(T) == 4) col_product<T, HDP>(acc, Vs + 16 * u * St::P, x[u], n, g);
+      }
+      if constexpr (sizeof(T) == 2) {
+        if (__builtin_amdgcn_readfirstlane(odd[buf]) != t) {
+          prob_product<T, HDP>(acc, Vs, x, n, g);
+        } else {  // planes would turn an infinity into inf - inf
+#pragma unroll
+          for (int u = 0; u < 2; ++u) col_product<T, HDP>(acc, Vs + 16 * u * St::P, x[u] * kPScale<T>, n, g);
+        }
       }
     }
     if (t + KG < nt) land(t + KG, buf ^ 1);
   }
   if constexpr (KG > 1) {
     constexpr int NA = HDP / 16, XF = 4 * NA + 2;  // floats a lane hands over
-    static_assert(kThreads * XF <= 4 * St::WORDS, "the exchange fits a group's tiles");
+    static_assert(kThreads * XF * sizeof(float) <= 4 * St::N * sizeof(T), "the exchange fits a group's tiles");
     __syncthreads();  // every group is done with its tiles
-    float* mine = &smem_all[kg][0][0];
+    float* mine = reinterpret_cast<float*>(&smem_all[kg][0][0]);
     if (kg > 0) {
 #pragma unroll
       for (int d = 0; d < NA; ++d)
@@ -348,7 +552,7 @@ __global__ __launch_bounds__(kThreads * KG) void attn_fwd_f32_kernel(
     if (kg > 0) return;
 #pragma unroll
     for (int o2 = 1; o2 < KG; ++o2) {
-      const float* x = &smem_all[o2][0][0];
+      const float* x = reinterpret_cast<const float*>(&smem_all[o2][0][0]);
       const float m2 = x[4 * NA * kThreads + tid], l2 = x[(4 * NA + 1) * kThreads + tid];
       if (m2 == -INFINITY) continue;  // saw no key of this row
       const float mn = fmaxf(m, m2);
@@ -364,7 +568,7 @@ __global__ __launch_bounds__(kThreads * KG) void attn_fwd_f32_kernel(
   l += __shfl_xor(l, 16);
   l += __shfl_xor(l, 32);
   if (!qok) return;
-  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const float inv = l > 0.f ? (1.f / kPScale<T>) / l : 0.f;
   store_rows<T, HDP>(o + b * os.b + tk.h * os.h + static_cast<int64_t>(qi) * os.s, acc, inv, g, hd);
   if (lse && g == 0)
     lse[(static_cast<int64_t>(b) * Hq + tk.h) * S + qi] = l > 0.f ? (m + __log2f(l)) * kLn2F : -INFINITY;
@@ -426,7 +630,9 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dkdv_kernel(
     int BHkv, int nkg, int ch, int maxch, Strides3 qs, Strides3 ks, Strides3 vs, Strides3 ds, Strides3 dks, Strides3 dvs,
     int causal, int vec, float scale_log2, float scale) {
   using St = Stage<T, HDP>;
-  __shared__ __attribute__((aligned(16))) float smem[2][2 * St::WORDS];
+  constexpr int NT = kPlaneTiles<T> ? 4 : 2;  // Q, dO, Q's planes
+  __shared__ __attribute__((aligned(16))) T smem[2][NT * St::N];
+  __shared__ int odd[2];  // the last step landed there with an infinity or NaN in it (16-bit types)
   __shared__ __attribute__((aligned(16))) float rowv[2][2][kTile];  // lse2 and D of the tile's rows
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -451,9 +657,9 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dkdv_kernel(
   const bool wg_any = !pad || __syncthreads_or(keep) != 0;
   const int kbnd = mode == HYDRA_MASK_REFERENCE_SDPA && !keep ? 0x7fffffff : key;
 
-  float kf[HDP / 16][4], vf[HDP / 16][4];
-  load_frag<T, HDP>(kf, k + b * ks.b + kvh * ks.h + static_cast<int64_t>(key < S ? key : 0) * ks.s, g, hd, key < S, vec & 2);
-  load_frag<T, HDP>(vf, v + b * vs.b + kvh * vs.h + static_cast<int64_t>(key < S ? key : 0) * vs.s, g, hd, key < S, vec & 2);
+  typename Row16<T, HDP>::Run kf[Row16<T, HDP>::N], vf[Row16<T, HDP>::N];
+  load_frag<T, HDP>(k + b * ks.b + kvh * ks.h + static_cast<int64_t>(key < S ? key : 0) * ks.s, kf, g, hd, key < S, vec & 2);
+  load_frag<T, HDP>(v + b * vs.b + kvh * vs.h + static_cast<int64_t>(key < S ? key : 0) * vs.s, vf, g, hd, key < S, vec & 2);
   f32x4 dka[HDP / 16], dva[HDP / 16];
 #pragma unroll
   for (int t = 0; t < HDP / 16; ++t) dka[t] = dva[t] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -473,17 +679,24 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dkdv_kernel(
     }
   };
   auto land = [&](int step, int buf) {
+    bool o1, o2;
+    T* planes = kPlaneTiles<T> ? smem[buf] + 2 * St::N : nullptr;
     if (vec & 1) {
-      sq.land(smem[buf], tid);
-      sd.land(smem[buf] + St::WORDS, tid);
+      o1 = sq.land(smem[buf], planes, tid);
+      o2 = sd.land(smem[buf] + St::N, nullptr, tid);
     } else {
       const int hr = step / nq, row0 = kTile * (qt0 + step - hr * nq), h = kvh * G + hr;
-      St::direct(Rows<T>{q + b * qs.b + h * qs.h, qs.s, 1}, row0, S, hd, smem[buf], tid);
-      St::direct(Rows<T>{dout + b * ds.b + h * ds.h, ds.s, 1}, row0, S, hd, smem[buf] + St::WORDS, tid);
+      o1 = St::direct(Rows<T>{q + b * qs.b + h * qs.h, qs.s, 1}, row0, S, hd, smem[buf], planes, tid);
+      o2 = St::direct(Rows<T>{dout + b * ds.b + h * ds.h, ds.s, 1}, row0, S, hd, smem[buf] + St::N, nullptr, tid);
     }
+    if (sizeof(T) == 2 && (o1 || o2)) odd[buf] = step;
     if (tid < 2 * kTile) rowv[buf][tid / kTile][tid & (kTile - 1)] = rv;
   };
   const int first = c * ch, end = wg_any ? min(first + ch, total) : first;
+  if (sizeof(T) == 2) {
+    if (tid < 2) odd[tid] = -1;
+    __syncthreads();
+  }
   if (first < end) {
     fetch(first);
     land(first, 0);
@@ -496,27 +709,46 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dkdv_kernel(
     // causal: a tile before the wave's keys holds nothing of theirs
     if (wave_any && (!walk || q0 + kTile - 1 >= kw0)) {
       const bool plain = walk ? q0 >= kw0 + 15 : mode != HYDRA_MASK_REFERENCE_SDPA;
+      f32x4 p[2], dp[2];
+      float big = 0.f;
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
-        const float* Qs = smem[buf] + 16 * u * St::P;
-        const float* Ds = Qs + St::WORDS;
-        f32x4 p = row_product<HDP>(Qs, kf, n, g), dp = row_product<HDP>(Ds, vf, n, g);
+        const T* Qs = smem[buf] + 16 * u * St::P;
+        const T* Ds = Qs + St::N;
+        p[u] = row_product<T, HDP>(Qs, kf, n, g);
+        dp[u] = row_product<T, HDP>(Ds, vf, n, g);
         const float4 l4 = *reinterpret_cast<const float4*>(&rowv[buf][0][16 * u + 4 * g]);
         const float4 d4 = *reinterpret_cast<const float4*>(&rowv[buf][1][16 * u + 4 * g]);
         const float lr[4] = {l4.x, l4.y, l4.z, l4.w}, dr[4] = {d4.x, d4.y, d4.z, d4.w};
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          float e = __builtin_amdgcn_exp2f(fmaf(p[r], scale_log2, -lr[r]));
+          float e = __builtin_amdgcn_exp2f(fmaf(p[u][r], scale_log2, -lr[r]));
           if (!plain) {
             const int s = q0 + 16 * u + 4 * g + r;
             const bool see = mode == HYDRA_MASK_REFERENCE_SDPA ? s < kbnd : key <= s;
             e = see ? e : 0.f;
           }
-          p[r] = e;
-          dp[r] = e * (dp[r] - dr[r]);
+          p[u][r] = e;
+          dp[u][r] = e * (dp[u][r] - dr[r]);
+          if constexpr (sizeof(T) == 2) big = max_of(big, e, dp[u][r]);
         }
-        col_product<HDP>(dva, Ds, p, n, g);
-        col_product<HDP>(dka, Qs, dp, n, g);
+        if constexpr (sizeof(T) == 4) {
+          col_product<T, HDP>(dva, Ds, p[u], n, g);
+          col_product<T, HDP>(dka, Qs, dp[u], n, g);
+        }
+      }
+      if constexpr (sizeof(T) == 2) {
+        const T* Qs = smem[buf];
+        if (!__any(big == INFINITY) && __builtin_amdgcn_readfirstlane(odd[buf]) != step) {
+          prob_product<T, HDP>(dva, Qs + St::N, p, n, g);
+          grad_product<T, HDP>(dka, Qs, Qs + 2 * St::N, dp, n, g);
+        } else {  // planes would turn an infinity into inf - inf
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            col_product<T, HDP>(dva, Qs + St::N + 16 * u * St::P, p[u] * kPScale<T>, n, g);
+            col_product<T, HDP>(dka, Qs + 16 * u * St::P, dp[u], n, g);
+          }
+        }
       }
     }
     if (step + 1 < end) land(step + 1, buf ^ 1);
@@ -528,11 +760,11 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dkdv_kernel(
   if (maxch > 1) {  // summed by attn_bwd_f32_reduce_kernel
     const int64_t rows = static_cast<int64_t>(parts) * 64;  // of one chunk's partial
     float* pk = part + ((static_cast<int64_t>(c) * 2) * rows + (static_cast<int64_t>(rest) * 64 + 16 * wave + n)) * HDP;
-    store_part<HDP>(pk, dka, g);
-    store_part<HDP>(pk + rows * HDP, dva, g);
+    store_part<HDP>(pk, dka, 1.f, g);
+    store_part<HDP>(pk + rows * HDP, dva, 1.f / kPScale<T>, g);
   } else if (key < S) {
     store_rows<T, HDP>(dk + b * dks.b + kvh * dks.h + static_cast<int64_t>(key) * dks.s, dka, scale, g, hd);
-    store_rows<T, HDP>(dv + b * dvs.b + kvh * dvs.h + static_cast<int64_t>(key) * dvs.s, dva, 1.f, g, hd);
+    store_rows<T, HDP>(dv + b * dvs.b + kvh * dvs.h + static_cast<int64_t>(key) * dvs.s, dva, 1.f / kPScale<T>, g, hd);
   }
 }
 
@@ -545,7 +777,9 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dq_kernel(
     int items, int ch, int maxch, Strides3 qs, Strides3 ks, Strides3 vs, Strides3 ds, Strides3 dqs, int causal, int vec,
     float scale_log2, float scale) {
   using St = Stage<T, HDP>;
-  __shared__ __attribute__((aligned(16))) float smem[2][2 * St::WORDS];
+  constexpr int NT = kPlaneTiles<T> ? 4 : 2;  // K, V, K's planes
+  __shared__ __attribute__((aligned(16))) T smem[2][NT * St::N];
+  __shared__ int odd[2];  // the last tile landed there with an infinity or NaN in it (16-bit types)
   __shared__ int keepv[2][kTile];
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -563,10 +797,10 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dq_kernel(
   const int qi = tk.q0 + n;
   const bool qok = tk.active && qi < S;
   const int my_end = !tk.active ? 0 : walk ? min(tk.q0 + 16, S) : S;
-  float qf[HDP / 16][4], of[HDP / 16][4];
+  typename Row16<T, HDP>::Run qf[Row16<T, HDP>::N], of[Row16<T, HDP>::N];
   const int64_t qr = qok ? qi : 0;
-  load_frag<T, HDP>(qf, q + b * qs.b + tk.h * qs.h + qr * qs.s, g, hd, qok, vec & 2);
-  load_frag<T, HDP>(of, dout + b * ds.b + tk.h * ds.h + qr * ds.s, g, hd, qok, vec & 2);
+  load_frag<T, HDP>(q + b * qs.b + tk.h * qs.h + qr * qs.s, qf, g, hd, qok, vec & 2);
+  load_frag<T, HDP>(dout + b * ds.b + tk.h * ds.h + qr * ds.s, of, g, hd, qok, vec & 2);
   float l2 = 0.f, dd = 0.f;
   if (qok) {
     const int64_t ri = (static_cast<int64_t>(b) * Hq + tk.h) * S + qi;
@@ -591,15 +825,22 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dq_kernel(
     }
   };
   auto land = [&](int t, int buf) {
+    bool o1, o2;
+    T* planes = kPlaneTiles<T> ? smem[buf] + 2 * St::N : nullptr;
     if (vec & 1) {
-      sk.land(smem[buf], tid);
-      sv.land(smem[buf] + St::WORDS, tid);
+      o1 = sk.land(smem[buf], planes, tid);
+      o2 = sv.land(smem[buf] + St::N, nullptr, tid);
     } else {
-      St::direct(kr, kTile * t, S, hd, smem[buf], tid);
-      St::direct(vr, kTile * t, S, hd, smem[buf] + St::WORDS, tid);
+      o1 = St::direct(kr, kTile * t, S, hd, smem[buf], planes, tid);
+      o2 = St::direct(vr, kTile * t, S, hd, smem[buf] + St::N, nullptr, tid);
     }
+    if (sizeof(T) == 2 && (o1 || o2)) odd[buf] = t;
     if (mode != HYDRA_MASK_NONE && tid < kTile) keepv[buf][tid] = kp;
   };
+  if (sizeof(T) == 2) {
+    if (tid < 2) odd[tid] = -1;
+    __syncthreads();
+  }
   fetch(first);
   land(first, 0);
   for (int t = first; t < end; ++t) {
@@ -608,11 +849,14 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dq_kernel(
     if (t + 1 < end) fetch(t + 1);
     if (t0 < my_end) {
       const bool plain = mode == HYDRA_MASK_NONE && t0 + kTile - 1 <= (walk ? tk.q0 : S - 1) && t0 + kTile <= S;
+      f32x4 dp[2];
+      float big = 0.f;
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
-        const float* Ks = smem[buf] + 16 * u * St::P;
-        const float* Vs = Ks + St::WORDS;
-        f32x4 p = row_product<HDP>(Ks, qf, n, g), dp = row_product<HDP>(Vs, of, n, g);
+        const T* Ks = smem[buf] + 16 * u * St::P;
+        const T* Vs = Ks + St::N;
+        const f32x4 p = row_product<T, HDP>(Ks, qf, n, g);
+        dp[u] = row_product<T, HDP>(Vs, of, n, g);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           float e = __builtin_amdgcn_exp2f(fmaf(p[r], scale_log2, -l2));
@@ -621,9 +865,19 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dq_kernel(
             const bool keep = mode == HYDRA_MASK_NONE || keepv[buf][i] != 0;
             e = key < S && sees(qi, key, keep, causal, mode) ? e : 0.f;
           }
-          dp[r] = e * (dp[r] - dd);
+          dp[u][r] = e * (dp[u][r] - dd);
+          if constexpr (sizeof(T) == 2) big = fmaxf(big, fabsf(dp[u][r]));
         }
-        col_product<HDP>(acc, Ks, dp, n, g);
+        if constexpr (sizeof(T) == 4) col_product<T, HDP>(acc, Ks, dp[u], n, g);
+      }
+      if constexpr (sizeof(T) == 2) {
+        const T* Ks = smem[buf];
+        if (!__any(big == INFINITY) && __builtin_amdgcn_readfirstlane(odd[buf]) != t) {
+          grad_product<T, HDP>(acc, Ks, Ks + 2 * St::N, dp, n, g);
+        } else {  // planes would turn an infinity into inf - inf
+#pragma unroll
+          for (int u = 0; u < 2; ++u) col_product<T, HDP>(acc, Ks + 16 * u * St::P, dp[u], n, g);
+        }
       }
     }
     if (t + 1 < end) land(t + 1, buf ^ 1);
@@ -631,7 +885,7 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dq_kernel(
   if (maxch > 1) {
     const int64_t rows = static_cast<int64_t>(parts) * 64;
     store_part<HDP>(part + (static_cast<int64_t>(c) * rows + (static_cast<int64_t>(bk) * items + item) * 64 + 16 * wave + n) * HDP,
-                    acc, g);
+                    acc, 1.f, g);
   } else if (qok) {
     store_rows<T, HDP>(dq + b * dqs.b + tk.h * dqs.h + static_cast<int64_t>(qi) * dqs.s, acc, scale, g, hd);
   }
@@ -759,7 +1013,7 @@ int launch_fwd(const AttnF32Args& a) {
   // Key groups when the items are fewer than two per resident workgroup
   // (registers: 3 per CU at head_dim 64): the longest walk sets the time then.
   // Two groups at head_dim 128 (LDS), else four.  fp16 B2 8/2 x 64, S 1500
-  // (376 items): 104 -> 71 us.
+  // (376 items): 104 -> 71 us (33 with the 16-bit rows).
   constexpr int KG = HDP == 128 ? 2 : 4;
   constexpr int per_cu = HDP <= 32 ? 5 : HDP == 64 ? 3 : 2;
   const bool groups = blocks < 2 * int64_t(per_cu) * device_cus();
