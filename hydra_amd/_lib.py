@@ -84,6 +84,7 @@ SIGNATURES = {
     "hydra_mod_gather": [_P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I, _P],
     "hydra_mod_scatter": [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I, _I, _P],
     "hydra_mod_scatter_bwd": [_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I, _P],
+    "hydra_router_probe": [_P, _I64, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I, _P],
     "hydra_stream_copy": [_P, _P, _I64, _P],
     "hydra_clock_probe": [_P, _I, _I, _I64P, _P],
     "hydra_attn_clock_stamps": [_P, _I64],

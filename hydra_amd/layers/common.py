@@ -125,12 +125,17 @@ class SwiGLUMLPFused(nn.Module):
         gate, up = F.linear(x, self.gate_up.weight).chunk(2, dim=-1)
         return F.linear(fused_swiglu(gate, up), self.down.weight)
 
-    def forward_residual(self, h: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+    def forward_residual(self, h: torch.Tensor, x: torch.Tensor, *, own: bool = False) -> torch.Tensor:
         """h + forward(x), with the residual add in the down projection's
-        GEMM epilogue (one rounding instead of two)."""
+        GEMM epilogue (one rounding instead of two).  own: h is the caller's
+        to give up, and may become the result (the GEMM then needs no copy of
+        it first: 7 us at 4096 x 1792 bf16)."""
         gate, up = F.linear(x, self.gate_up.weight).chunk(2, dim=-1)
         act = fused_swiglu(gate, up)
         dim = h.shape[-1]
+        if (own and h.is_contiguous() and not torch.is_autocast_enabled()
+                and not (torch.is_grad_enabled() and any(t.requires_grad for t in (h, act, self.down.weight)))):
+            return h.view(-1, dim).addmm_(act.reshape(-1, act.shape[-1]), self.down.weight.t()).view(h.shape)
         out = torch.addmm(h.reshape(-1, dim), act.reshape(-1, act.shape[-1]), self.down.weight.t())
         return out.view(h.shape)
 

@@ -17,7 +17,7 @@ from ... import _lib
 from ...attention.backends.ccgqa.attention import CCGQAAttention
 from ...attention.factory import build_hybrid_attention_module
 from ...layers import AdaRMSNorm, RMSNorm, SwiGLUMLPFused, residual_norm
-from ...routing.mixture_of_depths import MoDMLPWrapper
+from ...routing.mixture_of_depths import MoDMLPWrapper, _plain
 from ...routing.mixture_of_recursions import (MoRConfig, MoRExecutor, MoRRouter,
                                                dim_to_depth_scale)
 
@@ -29,9 +29,15 @@ def _recording(*tensors) -> bool:
 
 
 def _mlp_residual(mlp: nn.Module, h: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
-    """h + mlp(y), the add in the GEMM epilogue for the SwiGLU MLP."""
+    """h + mlp(y), the add in the GEMM epilogue for the SwiGLU MLP (also under
+    a MoD wrapper that does not route yet and that nobody hooks into).  h is a
+    fresh tensor of the caller's: its storage may hold the result."""
+    if (isinstance(mlp, MoDMLPWrapper) and type(mlp).forward is MoDMLPWrapper.forward and mlp._dense()
+            and isinstance(mlp.mlp, SwiGLUMLPFused) and _plain(mlp, mlp.mlp)):
+        mlp._note_dense(y)
+        mlp = mlp.mlp
     if isinstance(mlp, SwiGLUMLPFused):
-        return mlp.forward_residual(h, y)
+        return mlp.forward_residual(h, y, own=True)
     return h + mlp(y)
 
 
@@ -162,10 +168,7 @@ class HydraMoRBlock(nn.Module):
         for i in range(self.max_recursions):
             y = ex._pre(h, i, self.norm2)
             mlp = self._mlp()
-            if isinstance(mlp, SwiGLUMLPFused) and not _recording(h, y):
-                h = mlp.forward_residual(h, y)
-            else:
-                h = h + mlp(y)
+            h = h + mlp(y) if _recording(h, y) else _mlp_residual(mlp, h, y)
         return self.final_norm(h)
 
     def _forward_mor(self, x: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:

@@ -16,7 +16,17 @@ import torch.nn.functional as F
 
 from .base import BaseRouter
 from .ops import (gather_by_indices, mod_topk, router_k, scatter_replace,
-                  weighted_residual_scatter)
+                  weighted_residual_scatter, router_probe)
+
+
+def _recording(*tensors) -> bool:
+    return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
+
+
+def _plain(*modules) -> bool:
+    """Whether calling these modules is calling their forward: no hooks."""
+    return not any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                   for m in modules)
 
 
 def _aux_terms(scores: torch.Tensor, capacity_ratio: float) -> torch.Tensor:
@@ -164,6 +174,31 @@ class MoDMLPWrapper(nn.Module):
         self._last_probs_std_t = probs.std().detach()
         return probs
 
+    def _dense_scores(self, x: torch.Tensor) -> torch.Tensor:
+        """The router's scores of x, their probabilities' mean and deviation
+        noted: two launches where no gradient is recorded (six otherwise)."""
+        router, lin = self.mod_router, self.mod_router.router
+        if (type(lin) is nn.Linear and type(router).forward_logits is BaseRouter.forward_logits
+                and _plain(router, lin) and x.is_cuda and x.dtype in (torch.bfloat16, torch.float16, torch.float32)
+                and x.dtype == lin.weight.dtype and x.shape[-1] == lin.in_features
+                and 0 < x.numel() < (x.shape[-1] << 24) and not _recording(x, lin.weight, lin.bias)
+                and not torch.is_autocast_enabled() and not (router.training and router.jitter_noise > 0)):
+            scores, stats = router_probe(x, lin.weight, lin.bias)
+            self._last_scores = scores
+            self._last_probs_mean_t, self._last_probs_std_t = stats.unbind(0)
+            return scores
+        scores = router.forward_logits(x)
+        self._note_probs(scores)
+        return scores
+
+    def _note_dense(self, x: torch.Tensor) -> None:
+        self._routing_mode = "disabled"
+        self._tokens_total = self._tokens_processed = x.shape[1]
+        self._dense_aux(self._dense_scores(x))
+
+    def _dense(self) -> bool:
+        return not self.static_routing_mode and not getattr(self, "_mod_enabled", False)
+
     def _dense_aux(self, scores: torch.Tensor) -> None:
         if self.training and self.aux_loss_weight > 0:
             self._aux_loss = self.aux_loss_weight * _aux_terms(scores, self.capacity_ratio)
@@ -174,12 +209,8 @@ class MoDMLPWrapper(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self.static_routing_mode:
             return self._forward_static(x)
-        if not getattr(self, "_mod_enabled", False):
-            self._routing_mode = "disabled"
-            self._tokens_total = self._tokens_processed = x.shape[1]
-            scores = self.mod_router.forward_logits(x)
-            self._note_probs(scores)
-            self._dense_aux(scores)
+        if self._dense():
+            self._note_dense(x)
             return self.mlp(x)
         if not self.training:
             return self._forward_hard(x)

@@ -54,6 +54,34 @@ def mod_topk(scores: torch.Tensor, k: int, *, want_desc: bool = True, want_sorte
     return desc, srt, mask
 
 
+ROUTER_PROBE_BYTES = 12288  # HYDRA_ROUTER_PROBE_BYTES
+
+
+def router_probe(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]
+                 ) -> Tuple[torch.Tensor, torch.Tensor]:
+    """(scores, stats) of a router Linear(dim, 1) over x [..., dim]: scores
+    [...] and stats = [mean, std] of sigmoid(clamp(scores, -10, 10)), in x's
+    dtype, in two launches (hydra_router_probe).  Not differentiable."""
+    _lib.require_gpu("router_probe", x, weight, bias)
+    dim = x.shape[-1]
+    if weight.numel() != dim or (bias is not None and bias.numel() != 1):
+        raise ValueError("router_probe: weight must have dim elements and bias one")
+    if weight.dtype != x.dtype or (bias is not None and bias.dtype != x.dtype):
+        raise ValueError("router_probe: x, weight and bias must have one dtype")
+    x2 = x.reshape(-1, dim)
+    if x2.stride(-1) != 1 or (x2.shape[0] > 1 and x2.stride(0) < dim):
+        x2 = x2.contiguous()
+    scores = torch.empty(x.shape[:-1], dtype=x.dtype, device=x.device)
+    stats = torch.empty(2, dtype=x.dtype, device=x.device)
+    w = weight.reshape(-1).contiguous()
+    ws = _lib.scratch(ROUTER_PROBE_BYTES, x)
+    with _lib.on_device(x):
+        _lib.call("hydra_router_probe", x2.data_ptr(), x2.stride(0), w.data_ptr(), _lib.ptr(bias), scores.data_ptr(),
+                  stats.data_ptr(), ws.data_ptr(), ROUTER_PROBE_BYTES, x2.shape[0], dim, _lib.dtype_code(x),
+                  _lib.stream(x))
+    return scores, stats
+
+
 def _bl_strides(x: torch.Tensor):
     if x.stride(-1) != 1:
         return None

@@ -559,6 +559,18 @@ int hydra_mod_scatter_bwd(const void* grad, const void* y, const int64_t* idx, c
                           void* grad_y, float* grad_w, int64_t B, int64_t L, int64_t k,
                           int64_t D, int64_t g_bs, int64_t g_ls, int dtype, void* stream);
 
+/* Router scores (BaseRouter.forward_logits, hydra/routing/base.py:9-28) and
+ * what the dense path of MoDMLPWrapper notes of them (blocks.py:163-171):
+ * scores[r] = <x[r], w> + bias, p = sigmoid(clamp(scores, -10, 10)), stats =
+ * {mean(p), unbiased std(p)}; fp32 sums, tensors rounded to the dtype.  x:
+ * [rows, D], rows x_stride apart, 0 < rows < 2^24; w: [D]; bias: [1] or NULL;
+ * scores: [rows]; stats: [2]; workspace: HYDRA_ROUTER_PROBE_BYTES.  All of
+ * one dtype. */
+#define HYDRA_ROUTER_PROBE_BYTES 12288
+int hydra_router_probe(const void* x, int64_t x_stride, const void* w, const void* bias,
+                       void* scores, void* stats, void* workspace, int64_t workspace_bytes,
+                       int64_t rows, int64_t D, int dtype, void* stream);
+
 /* ---- measurement aid ----------------------------------------------------- */
 
 /* dst[0, bytes) = src[0, bytes): a plain device-to-device copy with
