@@ -218,9 +218,9 @@ class CCGQAAttention(nn.Module):
             cos=self.cos_cached if self.use_rope else None,
             sin=self.sin_cached if self.use_rope else None)
         if mask is None:
-            o = CCGQAAttentionFused.apply(q, k, v, True, True)
+            o = CCGQAAttentionFused.apply(q, k, v, True, True, True)
         else:
-            o = MaskedAttentionFunction.apply(q, k, v, mask.to(q.device), _mask_mode(), True)
+            o = MaskedAttentionFunction.apply(q, k, v, mask.to(q.device), _mask_mode(), True, True)
         out = F.linear(o.transpose(1, 2).reshape(B, S, self.latent_dim), self.o_proj.weight)
         if self.output_scale != 1.0:
             out = out * self.output_scale

@@ -136,6 +136,12 @@ def ccgqa_prep(qkv: torch.Tensor, n_heads: int, n_kv_heads: int, head_dim: int, 
     return q, k, (v.transpose(2, 3) if vt else v)
 
 
+def _mask_bytes(key_mask: torch.Tensor) -> torch.Tensor:
+    """The mask as 0/1 bytes: a bool mask's own, without a launch."""
+    kept = key_mask if key_mask.dtype == torch.bool else key_mask != 0
+    return kept.contiguous().view(torch.uint8)
+
+
 def attention_forward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: bool,
                       scale: Optional[float] = None, key_mask: Optional[torch.Tensor] = None,
                       mask_mode: int = MASK_NONE, out: Optional[torch.Tensor] = None,
@@ -171,7 +177,7 @@ def attention_forward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, caus
     if mask_mode != MASK_NONE:
         if key_mask is None or key_mask.shape != (B, S):
             raise ValueError(f"attention_forward: key mask must be [B,S] = [{B},{S}]")
-        km = (key_mask != 0).to(torch.uint8).contiguous()
+        km = _mask_bytes(key_mask)
     sc = float(hd ** -0.5) if scale is None else float(scale)
     bt = None
     if bound_temperature is not None:
@@ -230,7 +236,7 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: t
         if key_mask is None or key_mask.shape != (B, S):
             raise ValueError(f"attention_backward: key mask must be [B,S] = [{B},{S}]")
         _lib.require_gpu("attention_backward", key_mask)
-        km = (key_mask != 0).to(torch.uint8).contiguous()
+        km = _mask_bytes(key_mask)
     with _lib.on_device(q):
         st = (_lib.strides(q), _lib.strides(k), _lib.strides(v), _lib.strides(out),
               _lib.strides(grad_out), _lib.strides(dq), _lib.strides(dk), _lib.strides(dv))
