@@ -13,6 +13,7 @@ from typing import Optional, Tuple
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.nn.modules.module import _has_any_global_hook
 
 from .base import BaseRouter
 from .ops import (gather_by_indices, mod_topk, router_k, scatter_replace,
@@ -24,9 +25,11 @@ def _recording(*tensors) -> bool:
 
 
 def _plain(*modules) -> bool:
-    """Whether calling these modules is calling their forward: no hooks."""
-    return not any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
-                   for m in modules)
+    """Whether calling these modules is calling their class's forward: no
+    hooks, on them or on every module, and no forward set on the instance."""
+    return not _has_any_global_hook() and not any(
+        m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+        or "forward" in m.__dict__ for m in modules)
 
 
 def _aux_terms(scores: torch.Tensor, capacity_ratio: float) -> torch.Tensor:
