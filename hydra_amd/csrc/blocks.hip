@@ -41,6 +41,13 @@ __device__ __forceinline__ void load_elems(const W* p, float* out) {
   for (int i = 0; i < E / PER; ++i) load16<W>(p + i * PER, out + i * PER);
 }
 
+// The E values of f rounded to T and back (identity for fp32): one conversion
+// per pair for bf16.
+template <typename T>
+__device__ __forceinline__ void rnd_all(float* f) {
+  if constexpr (sizeof(T) != 4) unpack16<T>(pack16<T>(f), f);
+}
+
 enum NormMode { kNormNone = 0, kNormRms = 1, kNormAda = 2 };
 
 // ---------------------------------------------------------------------------
@@ -88,7 +95,13 @@ __global__ __launch_bounds__(kBlk) void embed_scalar_kernel(
 //        m = rnd(sum(rnd(v^2)) / dim), s = rnd(rsqrt(rnd(m + eps))),
 //        y = rnd(rnd(v * s) * w).
 // LPR lanes per row, CPL 16-byte chunks per lane, RI row groups per wave,
-// all loads of a wave's row groups issued before its reductions.
+// all loads of a wave's row groups issued before its reductions, and with them
+// those of the vectors where they fit the registers (16-bit elements): a wave
+// has few rows, so the vectors' L2 latency would follow x's.
+// What bounds it at a model's sizes is that latency and the waves in flight,
+// not bandwidth: 4096 x 1792 bf16, ADA with both vectors 14.0 -> 10.6 us (2.8
+// TB/s) from 32 lanes x 8 chunks with the vectors loaded after the rows;
+// residual add alone 12.0 -> 10.9.
 // ---------------------------------------------------------------------------
 struct ResNormArgs {
   const void* x; int64_t x_rs;
@@ -124,6 +137,19 @@ __global__ __launch_bounds__(kBlk) void resnorm_vec_kernel(ResNormArgs a) {
       }
     }
   }
+  constexpr bool kAhead = CPL <= 4 && sizeof(T) == 2 && sizeof(WT) == 2;
+  uint4 br[kAhead ? 2 : 1][kAhead ? CPL : 1], wr[kAhead ? CPL : 1];
+  if constexpr (kAhead) {
+#pragma unroll
+    for (int v = 0; v < CPL; ++v) {
+      const int vi = l + LPR * v;
+      br[0][v] = br[1][v] = wr[v] = make_uint4(0, 0, 0, 0);
+      if (vi >= a.nvec) continue;
+      if (a.b1) br[0][v] = ld16raw<false>(static_cast<const T*>(a.b1) + vi * E);
+      if (a.b2) br[1][v] = ld16raw<false>(static_cast<const T*>(a.b2) + vi * E);
+      if (NORM != kNormNone) wr[v] = ld16raw<false>(static_cast<const WT*>(a.w) + vi * E);
+    }
+  }
 #pragma unroll
   for (int g = 0; g < RI; ++g) {
     const int64_t row = row0 + g * RPW;
@@ -137,30 +163,43 @@ __global__ __launch_bounds__(kBlk) void resnorm_vec_kernel(ResNormArgs a) {
         float rf[E];
         unpack16<T>(rr[g][v], rf);
 #pragma unroll
-        for (int e = 0; e < E; ++e)
-          f[v][e] = rnd<T>(f[v][e] + (a.alpha == 1.f ? rf[e] : rnd<T>(a.alpha * rf[e])));
+        for (int e = 0; e < E; ++e) rf[e] = a.alpha == 1.f ? rf[e] : a.alpha * rf[e];
+        rnd_all<T>(rf);
+#pragma unroll
+        for (int e = 0; e < E; ++e) f[v][e] += rf[e];
+        rnd_all<T>(f[v]);
       }
       if (vi < a.nvec) {
         if (a.b1) {
           float bf[E];
-          load16<T>(static_cast<const T*>(a.b1) + vi * E, bf);
+          if constexpr (kAhead) unpack16<T>(br[0][v], bf);
+          else load16<T>(static_cast<const T*>(a.b1) + vi * E, bf);
 #pragma unroll
-          for (int e = 0; e < E; ++e) f[v][e] = rnd<T>(f[v][e] + bf[e]);
+          for (int e = 0; e < E; ++e) f[v][e] += bf[e];
+          rnd_all<T>(f[v]);
         }
         if (a.b2) {
           float bf[E];
-          load16<T>(static_cast<const T*>(a.b2) + vi * E, bf);
+          if constexpr (kAhead) unpack16<T>(br[1][v], bf);
+          else load16<T>(static_cast<const T*>(a.b2) + vi * E, bf);
 #pragma unroll
-          for (int e = 0; e < E; ++e) f[v][e] = rnd<T>(f[v][e] + bf[e]);
+          for (int e = 0; e < E; ++e) f[v][e] += bf[e];
+          rnd_all<T>(f[v]);
         }
       } else {
 #pragma unroll
         for (int e = 0; e < E; ++e) f[v][e] = 0.f;
       }
+      if constexpr (NORM == kNormAda) {
+        float sq[E];
 #pragma unroll
-      for (int e = 0; e < E; ++e) {
-        if constexpr (NORM == kNormAda) ss += rnd<T>(f[v][e] * f[v][e]);
-        else ss = fmaf(f[v][e], f[v][e], ss);
+        for (int e = 0; e < E; ++e) sq[e] = f[v][e] * f[v][e];
+        rnd_all<T>(sq);
+#pragma unroll
+        for (int e = 0; e < E; ++e) ss += sq[e];
+      } else {
+#pragma unroll
+        for (int e = 0; e < E; ++e) ss = fmaf(f[v][e], f[v][e], ss);
       }
     }
     if (a.h && row < a.rows) {
@@ -185,12 +224,13 @@ __global__ __launch_bounds__(kBlk) void resnorm_vec_kernel(ResNormArgs a) {
         const int vi = l + LPR * v;
         if (vi >= a.nvec) continue;
         float wf[E];
-        load_elems<WT, E>(static_cast<const WT*>(a.w) + vi * E, wf);
+        if constexpr (kAhead) unpack16<WT>(wr[v], wf);
+        else load_elems<WT, E>(static_cast<const WT*>(a.w) + vi * E, wf);
 #pragma unroll
-        for (int e = 0; e < E; ++e) {
-          if constexpr (NORM == kNormAda) f[v][e] = rnd<T>(rnd<T>(f[v][e] * s) * wf[e]);
-          else f[v][e] = f[v][e] * s * wf[e];
-        }
+        for (int e = 0; e < E; ++e) f[v][e] *= s;
+        if constexpr (NORM == kNormAda) rnd_all<T>(f[v]);
+#pragma unroll
+        for (int e = 0; e < E; ++e) f[v][e] *= wf[e];  // rounded by the store
         store16<T, true>(static_cast<T*>(a.y) + row * a.y_rs + vi * E, f[v]);
       }
     }
@@ -246,7 +286,7 @@ __global__ __launch_bounds__(kBlk) void resnorm_scalar_kernel(ResNormArgs a) {
 
 template <typename T, typename WT, int LPR, int CPL, int NORM>
 int launch_resnorm_vec(const ResNormArgs& a, hipStream_t st) {
-  constexpr int RI = CPL >= 4 ? 1 : (CPL >= 2 ? 2 : 4);
+  constexpr int RI = CPL >= 3 ? 1 : (CPL >= 2 ? 2 : 4);
   constexpr int RPB = (kBlk / 64) * (64 / LPR) * RI;
   const dim3 grid(static_cast<unsigned>((a.rows + RPB - 1) / RPB));
   resnorm_vec_kernel<T, WT, LPR, CPL, RI, NORM><<<grid, kBlk, 0, st>>>(a);
@@ -257,16 +297,21 @@ template <typename T, typename WT, int NORM>
 int launch_resnorm(ResNormArgs a, bool vec_ok, hipStream_t st) {
   constexpr int E = Vec<T>::N;
   if (vec_ok && a.nvec <= 64 * 8) {
-    int lpr = 64;
+    // up to 4 chunks per lane: the most lanes that divide the row evenly, else
+    // the fewest that hold it (1792 = 224 chunks: 64 x 4, half a chunk idle,
+    // instead of 32 x 7, where a wave held two rows and the launch half the waves)
+    int lpr = 0;
     for (int cand : {64, 32, 16, 8, 4})
-      if (a.nvec % cand == 0 && a.nvec / cand <= 8) { lpr = cand; break; }
+      if (lpr == 0 && a.nvec % cand == 0 && a.nvec / cand <= 4) lpr = cand;
+    for (int cand : {4, 8, 16, 32, 64})
+      if (lpr == 0 && ((a.nvec + cand - 1) / cand <= 4 || cand == 64)) lpr = cand;
     const int cpl = (a.nvec + lpr - 1) / lpr;
 #define HYDRA_RN_CASE(LP, CP) \
   if (lpr == LP && cpl <= CP) return launch_resnorm_vec<T, WT, LP, CP, NORM>(a, st);
-    HYDRA_RN_CASE(4, 1) HYDRA_RN_CASE(4, 2) HYDRA_RN_CASE(4, 4) HYDRA_RN_CASE(4, 8)
-    HYDRA_RN_CASE(8, 1) HYDRA_RN_CASE(8, 2) HYDRA_RN_CASE(8, 4) HYDRA_RN_CASE(8, 8)
-    HYDRA_RN_CASE(16, 1) HYDRA_RN_CASE(16, 2) HYDRA_RN_CASE(16, 4) HYDRA_RN_CASE(16, 8)
-    HYDRA_RN_CASE(32, 1) HYDRA_RN_CASE(32, 2) HYDRA_RN_CASE(32, 4) HYDRA_RN_CASE(32, 8)
+    HYDRA_RN_CASE(4, 1) HYDRA_RN_CASE(4, 2) HYDRA_RN_CASE(4, 4)
+    HYDRA_RN_CASE(8, 1) HYDRA_RN_CASE(8, 2) HYDRA_RN_CASE(8, 4)
+    HYDRA_RN_CASE(16, 1) HYDRA_RN_CASE(16, 2) HYDRA_RN_CASE(16, 4)
+    HYDRA_RN_CASE(32, 1) HYDRA_RN_CASE(32, 2) HYDRA_RN_CASE(32, 4)
     HYDRA_RN_CASE(64, 1) HYDRA_RN_CASE(64, 2) HYDRA_RN_CASE(64, 3) HYDRA_RN_CASE(64, 4)
     HYDRA_RN_CASE(64, 6) HYDRA_RN_CASE(64, 8)
 #undef HYDRA_RN_CASE
