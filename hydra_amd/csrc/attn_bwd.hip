@@ -30,7 +30,8 @@
 //  * attn_bwd_dq_kernel: lanes own queries, as in the forward: S^T = K Q^T,
 //    dP^T = V dO^T, dQ^T += K^T dS^T; a step stages 64 keys of K and V in
 //    LDS, shared by the 4 query tasks of an item.
-//    It runs on a side stream, concurrently with dK/dV (see SideStream).
+//    In long calls it runs on a side stream, concurrently with dK/dV (see
+//    overlap_dq).
 // The MFMA B operand of the PV-type products is taken straight from the
 // score accumulator registers; the A operand is read from the LDS tile in the
 // same (register-order) permutation of the summed index.
@@ -1083,6 +1084,24 @@ DkdvPlan plan_dkdv(int hd, int S, int G, int BHkv, bool causal) {
   return p;
 }
 
+// Whether dQ goes to the side stream.  The two events and waits cost the host
+// ~35 us (and the GPU a few), so they pay where the launches they overlap are
+// longer: at head_dim 128, past 2048 keys (the longest walk sets the time of
+// both launches) or past 6 G products of q k^T (head_dim 16 counts as 32: its
+// launches are bound by the exponentials).  Forward + backward, a call among
+// others / alone, one stream against two:
+//   below the line: B4 8/2 heads x 64, S 1024 144 / 190 against 180 / 204 us;
+//   B4 8/2 x 64, S 2048 (4.3 G) 153 / 235 against 175 / 236; B4 16/4 x 16, S
+//   2048 (4.3 G so counted) 172 / 252 against 195 / 265; a layer's training
+//   step B4 x S1024, 8/2 x 64 620 against 708, padded B8 x S777 649 against 743;
+//   above it: B4 4/1 x 64, S 4096 (8.6 G) 254 / 328 against 241 / 323; B1 4/1 x
+//   64, S 4096 152 / 236 against 189 / 226; B2 8/2 x 128, S 2048 238 / 324
+//   against 191 / 267.
+bool overlap_dq(int hd, bool causal, const BwdArgs& a) {
+  const double pairs = double(a.B) * a.Hq * a.S * a.S * (causal ? 0.5 : 1.0);
+  return hd >= 128 || a.S > 2048 || pairs * std::max(hd, 32) >= 6e9;
+}
+
 // A side stream per device (default priority, non-blocking) with a fork and
 // a join event.  fork() makes the side stream wait for everything queued on
 // the caller's stream so far; finish() makes the caller's stream wait for
@@ -1152,12 +1171,12 @@ int launch_mfma(const BwdArgs& a, const float* dvec, const float* lse2, float* p
   const bf16* k = static_cast<const bf16*>(a.k);
   const bf16* v = static_cast<const bf16*>(a.v);
   const bf16* d = static_cast<const bf16*>(a.dout);
-  // dQ needs only the row-dot's outputs, so it runs on a side stream,
-  // concurrently with dK/dV: the two launches' causal tails (CUs whose
-  // workgroups are done while others still walk the longest key ranges)
-  // take each other's workgroups.
+  // dQ needs only the row-dot's outputs, so where overlap_dq says so it runs
+  // on a side stream, concurrently with dK/dV: the two launches' causal tails
+  // (CUs whose workgroups are done while others still walk the longest key
+  // ranges) take each other's workgroups.
   SideStream side;
-  const hipStream_t dq_st = side.fork(a.st) ? side.stream : a.st;
+  const hipStream_t dq_st = overlap_dq(HD, CAUSAL, a) && side.fork(a.st) ? side.stream : a.st;
   auto launch_dq = [&]() {
     // An item is NW query tasks (32 query rows of one head) sharing each
     // staged K/V tile.
