@@ -68,13 +68,16 @@ def tiled_weights_ok(n_heads: int, n_kv_heads: int, head_dim: int, dtype: torch.
 def _rope_tables(cos: torch.Tensor, sin: torch.Tensor, S: int, bf16_ok: bool):
     """RoPE tables [.., Smax, hd/2] as the kernels take them: (cos, sin, row
     stride, flag), read in place when they are fp32 -- or bf16, where the
-    kernel widens them itself (bf16_ok; flag CCGQA_ROPE_BF16) -- with rows one
-    stride apart; converted otherwise."""
-    if cos.shape[-2] < S:
-        raise ValueError(f"ccgqa_prep: RoPE cache covers {cos.shape[-2]} positions < S={S}")
+    kernel widens them itself (bf16_ok; flag CCGQA_ROPE_BF16) -- with whole
+    rows one after the other; converted otherwise (an expanded table, a slice
+    of a wider one)."""
+    rows = cos.shape[-2] if cos.dim() == 4 else cos.shape[0]
+    if rows < S:
+        raise ValueError(f"ccgqa_prep: RoPE cache covers {rows} positions < S={S}")
     half = bf16_ok and cos.dtype == sin.dtype == torch.bfloat16
     if (half or cos.dtype == sin.dtype == torch.float32) and cos.stride(-1) == sin.stride(-1) == 1 and \
-            cos.stride(-2) == sin.stride(-2) and cos.stride(-2) % 4 == 0 and \
+            cos.dim() == sin.dim() and cos.dim() in (2, 4) and \
+            cos.stride(-2) == sin.stride(-2) == cos.shape[-1] == sin.shape[-1] and cos.shape[-1] % 4 == 0 and \
             (cos.data_ptr() | sin.data_ptr()) % 16 == 0:
         return cos, sin, cos.stride(-2), CCGQA_ROPE_BF16 if half else 0
     cos, sin = ((t[0, 0] if t.dim() == 4 else t)[:S].float().contiguous() for t in (cos, sin))
