@@ -17,7 +17,7 @@ from ... import _lib
 from ...attention.backends.ccgqa.attention import CCGQAAttention
 from ...attention.factory import build_hybrid_attention_module
 from ...layers import AdaRMSNorm, RMSNorm, SwiGLUMLPFused, residual_norm
-from ...routing.mixture_of_depths import MoDMLPWrapper, _plain
+from ...routing.mixture_of_depths import MoDMLPWrapper, _own, _plain
 from ...routing.mixture_of_recursions import (MoRConfig, MoRExecutor, MoRRouter,
                                                dim_to_depth_scale)
 
@@ -32,8 +32,9 @@ def _mlp_residual(mlp: nn.Module, h: torch.Tensor, y: torch.Tensor) -> torch.Ten
     """h + mlp(y), the add in the GEMM epilogue for the SwiGLU MLP (also under
     a MoD wrapper that does not route yet and that nobody hooks into).  h is a
     fresh tensor of the caller's: its storage may hold the result."""
-    if (isinstance(mlp, MoDMLPWrapper) and type(mlp).forward is MoDMLPWrapper.forward and mlp._dense()
-            and isinstance(mlp.mlp, SwiGLUMLPFused) and _plain(mlp, mlp.mlp)):
+    if (isinstance(mlp, MoDMLPWrapper) and _own(mlp, MoDMLPWrapper, "forward") and mlp._dense()
+            and isinstance(mlp.mlp, SwiGLUMLPFused) and _own(mlp.mlp, SwiGLUMLPFused, "forward")
+            and _plain(mlp, mlp.mlp)):
         mlp._note_dense(y)
         mlp = mlp.mlp
     if isinstance(mlp, SwiGLUMLPFused):

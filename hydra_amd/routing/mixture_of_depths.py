@@ -13,6 +13,7 @@ from typing import Optional, Tuple
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 from torch.nn.modules.module import _has_any_global_hook
 
 from .base import BaseRouter
@@ -30,6 +31,19 @@ def _plain(*modules) -> bool:
     return not _has_any_global_hook() and not any(
         m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
         or "forward" in m.__dict__ for m in modules)
+
+
+def _own(obj: nn.Module, base: type, *methods: str) -> bool:
+    """Whether obj's methods are base's: not overridden by its class, not set
+    on the instance."""
+    return all(getattr(type(obj), m) is getattr(base, m) and m not in obj.__dict__ for m in methods)
+
+
+def _plain_tensor(x: torch.Tensor) -> bool:
+    """Whether x has memory that a kernel may read in its place and no
+    transform follows the operations on it (forward-mode, vmap, tracing)."""
+    return (type(x) in (torch.Tensor, nn.Parameter) and forward_ad._current_level < 0
+            and torch._C._functorch.peek_interpreter_stack() is None and not torch.jit.is_tracing())
 
 
 def _aux_terms(scores: torch.Tensor, capacity_ratio: float) -> torch.Tensor:
@@ -181,8 +195,9 @@ class MoDMLPWrapper(nn.Module):
         """The router's scores of x, their probabilities' mean and deviation
         noted: two launches where no gradient is recorded (six otherwise)."""
         router, lin = self.mod_router, self.mod_router.router
-        if (type(lin) is nn.Linear and type(router).forward_logits is BaseRouter.forward_logits
-                and _plain(router, lin) and x.is_cuda and x.dtype in (torch.bfloat16, torch.float16, torch.float32)
+        if (type(lin) is nn.Linear and _own(router, BaseRouter, "forward_logits", "_apply_jitter")
+                and _own(self, MoDMLPWrapper, "_note_probs") and _plain(lin) and _plain_tensor(x)
+                and x.is_cuda and x.dtype in (torch.bfloat16, torch.float16, torch.float32)
                 and x.dtype == lin.weight.dtype and x.shape[-1] == lin.in_features
                 and 0 < x.numel() < (x.shape[-1] << 24) and not _recording(x, lin.weight, lin.bias)
                 and not torch.is_autocast_enabled() and not (router.training and router.jitter_noise > 0)):

@@ -3,6 +3,7 @@ nothing hooks into the call."""
 from __future__ import annotations
 
 import pytest
+import torch
 import torch.nn as nn
 from torch.nn.modules import module as nn_module
 
@@ -26,3 +27,53 @@ def test_hooked_modules_are_called(kind):
     finally:
         handle.remove()
     assert _plain(a, b)
+
+
+def test_an_overridden_mlp_forward_is_called():
+    """A wrapped SwiGLU MLP whose forward is another (by its class or on the
+    instance) runs that forward, not the parts of the parent's."""
+    from hydra_amd.layers import SwiGLUMLPFused
+    from hydra_amd.model.framework.blocks import _mlp_residual
+    from hydra_amd.routing.mixture_of_depths import MoDMLPWrapper
+
+    class Doubling(SwiGLUMLPFused):
+        def forward(self, x):
+            return 2 * x
+
+    on_instance = SwiGLUMLPFused(8, 16)
+    on_instance.forward = lambda x: 2 * x
+    h, y = torch.randn(2, 3, 8), torch.randn(2, 3, 8)
+    for mlp in (Doubling(8, 16), on_instance):
+        with torch.no_grad():
+            assert torch.equal(_mlp_residual(MoDMLPWrapper(mlp, 8).eval(), h, y), h + 2 * y)
+
+
+def test_methods_of_their_own():
+    from hydra_amd.routing.base import BaseRouter
+    from hydra_amd.routing.mixture_of_depths import MoDRouter, _own
+
+    class Noisy(MoDRouter):
+        def _apply_jitter(self, logits):
+            return logits + 1
+
+    names = ("forward_logits", "_apply_jitter")
+    router = MoDRouter(8)
+    assert _own(router, BaseRouter, *names) and not _own(Noisy(8), BaseRouter, *names)
+    router.forward_logits = lambda x: x[..., 0]
+    assert not _own(router, BaseRouter, *names)
+
+
+def test_tensors_under_a_transform_are_not_read_in_place():
+    from hydra_amd.routing.mixture_of_depths import _plain_tensor
+
+    seen = []
+    look = lambda x: (seen.append(_plain_tensor(x)), x * 1)[1]
+    x = torch.randn(3, 4)
+    look(x)
+    torch.func.vmap(look)(x)
+    torch.func.jvp(look, (x,), (x,))
+    with torch.autograd.forward_ad.dual_level():
+        look(torch.autograd.forward_ad.make_dual(x, x))
+    torch.jit.trace(look, (x,), check_trace=False)
+    look(x)
+    assert seen == [True, False, False, False, False, True]
