@@ -428,14 +428,15 @@ class ChunkedCrossEntropyFunction(torch.autograd.Function):
         scale = (grad_output.float() / n_valid.clamp(min=1)).reshape(1).contiguous()
         grad_h = torch.empty(h.shape, dtype=torch.float32, device=h.device)
         cs = ctx.chunk_size
-        if h.dtype == weight.dtype == torch.bfloat16:
+        if h.dtype == weight.dtype == torch.bfloat16 and not torch.is_grad_enabled():
             # bf16 products are exact in fp32 accumulation, so the logits and
             # both gradient GEMMs run on the bf16 matrix cores with fp32
             # results, the logits' gradient as two bf16 planes.  Forward +
             # backward, 8192 tokens x 768 x vocab 32000: 9.65 -> 3.16 ms
             # (three fp32 GEMMs of 1.45 ms per 4096-token chunk before).
             # Other dtypes keep the fp32 GEMMs: fp32 operands would need three
-            # planes each, six products, for no gain worth the name.
+            # planes each, six products, for no gain worth the name.  So does
+            # create_graph, which products with an `out` cannot record.
             grad_w = None
             for s in range(0, h.shape[0], cs):
                 hc = h[s:s + cs]

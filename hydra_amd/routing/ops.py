@@ -185,7 +185,9 @@ class _ScatterRows(torch.autograd.Function):
     def backward(ctx, grad):
         values, idx, weights = ctx.saved_tensors
         grad = grad.contiguous()
-        if weights is not None and values.dtype == grad.dtype and values.shape[-1] > 0:
+        # one kernel, except where create_graph records the products below
+        if (weights is not None and values.dtype == grad.dtype and values.shape[-1] > 0
+                and not torch.is_grad_enabled()):
             g_vals, g_w = _scatter_grads(grad, values, idx, weights, ctx.needs_input_grad[1],
                                          ctx.needs_input_grad[3])
             return (grad if ctx.needs_input_grad[0] else None), g_vals, None, g_w, None
