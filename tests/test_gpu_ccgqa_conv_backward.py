@@ -87,7 +87,7 @@ def test_bf16_rope_tables(cuda, hd, S):
     ws = [rand(L, hd, 3), rand(L, L, 3), rand(K, hd, 3), rand(K, K, 3)]
     qkv, temp = rand(2, S, L + 2 * K), torch.ones(1, dtype=torch.bfloat16, device=cuda)
     gos = [rand(2, h, S, hd) for h in (Hq, Hkv, Hkv)]
-    cos, sin = (t.to(torch.bfloat16).to(cuda)[None, None] for t in occ.fused_ops.rope_cache(hd, 200))
+    cos, sin = (t.to(torch.bfloat16).to(cuda) for t in occ.fused_ops.rope_cache(hd, 200))
     flags = prep_flags(True, True, True, True, True)
     res = []
     for c, s in ((cos, sin), (cos.float(), sin.float())):
