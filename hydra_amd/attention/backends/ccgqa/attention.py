@@ -37,7 +37,7 @@ from .autograd import ccgqa_prep_train
 from .kernels.fused_attention import CCGQAAttentionFused, MaskedAttentionFunction
 from .kernels.fused_conv import OptimizedConvSequence
 from .ops import (attention_forward, ccgqa_prep, linear_weight_ok, output_projection, pack_conv_weight,
-                  pack_linear_weight, prep_flags, tiled_weights_ok)
+                  pack_conv_weights_tiled, pack_linear_weight, prep_flags, tiled_weights_ok)
 
 # Kept for callers that probe these names (attention.py:13-28).
 FUSED_KERNELS_AVAILABLE = True
@@ -233,7 +233,9 @@ class CCGQAAttention(nn.Module):
         key = tuple((w.data_ptr(), w._version, w.device, dtype, tiled) for w in convw)
         cache = getattr(self, "_packed_cache", None)
         if cache is None or cache[0] != key:
-            cache = (key, tuple(pack_conv_weight(w, dtype, tiled) for w in convw))
+            # tiled: one launch for the four
+            cache = (key, pack_conv_weights_tiled(convw, dtype, self.n_heads, self.n_kv_heads, self.head_dim)
+                     if tiled else tuple(pack_conv_weight(w, dtype) for w in convw))
             self._packed_cache = cache
         return cache[1]
 
