@@ -45,6 +45,13 @@
 // B8 4/1 heads x 64, S 777, padded: 101.4 ms -> below 0.1; B2 28/4 heads x
 // 16, S 2048, causal: 60 ms -> below 0.3 (whole layer steps 102.5 -> 1.41
 // and 61.3 -> 1.40 ms, what remains is the rest of the layer).
+// In the same two forms rows that a query does not see stay out of its sums
+// whatever they hold: with an infinity or NaN in a staged row the weight 0 of
+// an unseen one gives NaN, so a wave that ends with a NaN in its accumulators
+// walks its range a second time, row by row in fp32 over the seen rows only
+// (bwd_row_dot, bwd_add_row).  Where no wave does, the test and the registers
+// cost 1% (B8 4/1 heads x 64, S 2048, key padding: 165 -> 167 us) to 4%
+// (head_dim 128, or the reference mask).
 // Other element types, head dims and strides: attn_f32.hip (fp32 matrix
 // instructions) up to head_dim 128, above it attn_bwd_generic_* (one thread
 // per query / key row, fp32 math, head_dim <= 256).
@@ -137,6 +144,62 @@ __device__ __forceinline__ float ld4_buf(__amdgpu_buffer_rsrc_t r, int off) {
 
 __device__ __forceinline__ uint4 ld16_or0(const bf16* p, bool ok) {
   return ok ? *reinterpret_cast<const uint4*>(p) : make_uint4(0, 0, 0, 0);
+}
+
+// Whether query s sees key t (t < S): causality, then the key mask
+// (MASK 1: key padding on top of causality; MASK 2: the forward's
+// reference-SDPA mode, key t > s or t padded, whatever `CAUSAL`).
+template <bool CAUSAL, int MASK>
+__device__ __forceinline__ bool bwd_visible(int s, int t, const uint8_t* kmrow) {
+  if constexpr (MASK == 2) return t > s || kmrow[t] == 0;
+  const bool c = !CAUSAL || t <= s;
+  if constexpr (MASK == 1) return c && kmrow[t] != 0;
+  return c;
+}
+
+// The second walk's steps (see the top of the file).  The forms that take it.
+template <int HD, int MASK>
+constexpr bool kSecondWalk = HD == 16 || MASK != 0;
+
+// The dot product of a row with each lane's resident row, f[s] its elements
+// 16 s + 8 hf ..
+template <int KS>
+__device__ __forceinline__ float bwd_row_dot(const bf16* row, const uint4 (&f)[KS], int hf) {
+  asm volatile("" : "+v"(hf));  // offsets made here, row by row, and not kept in registers
+  float s = 0.f;
+#pragma unroll
+  for (int k = 0; k < KS; ++k) {
+    float a[8], b[8];
+    load16<bf16>(row + 16 * k + 8 * hf, a);
+    unpack16<bf16>(f[k], b);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s = fmaf(a[e], b[e], s);
+  }
+  return s + __shfl_xor(s, 32);
+}
+// acc^T += w * row: register 4 j + i of tile dt is element 32 dt + 8 j + 4 hf + i.
+template <int DT, int JT>
+__device__ __forceinline__ void bwd_add_row(f32x16_t (&acc)[DT], const bf16* row, float w, int hf) {
+  asm volatile("" : "+v"(hf));
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int j = 0; j < JT; ++j) {
+      const uint2 x = *reinterpret_cast<const uint2*>(row + 32 * dt + 8 * j + 4 * hf);
+      acc[dt][4 * j] = fmaf(w, __uint_as_float(x.x << 16), acc[dt][4 * j]);
+      acc[dt][4 * j + 1] = fmaf(w, __uint_as_float(x.x & 0xffff0000u), acc[dt][4 * j + 1]);
+      acc[dt][4 * j + 2] = fmaf(w, __uint_as_float(x.y << 16), acc[dt][4 * j + 2]);
+      acc[dt][4 * j + 3] = fmaf(w, __uint_as_float(x.y & 0xffff0000u), acc[dt][4 * j + 3]);
+    }
+}
+template <int DT, int JT>
+__device__ __forceinline__ bool bwd_any_nan(const f32x16_t (&acc)[DT]) {
+  bool nan = false;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int r = 0; r < 4 * JT; ++r) nan |= acc[dt][r] != acc[dt][r];
+  return nan;
 }
 
 // ---------------------------------------------------------------------------
@@ -536,6 +599,32 @@ __global__ __launch_bounds__(64 * KB * HG) void attn_bwd_dkdv_kernel(
   }
   if (step == last) compute(step, 0);  // odd count: the last tile is in buffer 0
   }
+  if constexpr (kSecondWalk<HD, MASK>) {
+    // kvis: keys that are stored as zeros do not count (a query that sees no
+    // key gives them infinite weights)
+    if (__any(kvis && (bwd_any_nan<DT, JT>(dka) || bwd_any_nan<DT, JT>(dva)))) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) { dka[dt] = zero16(); dva[dt] = zero16(); }
+      for (int step = 0; step < nsteps; ++step) {
+        int hr, qt;
+        locate(step, hr, qt);
+        const int h = kvh * G + hr * HG + hg;
+#pragma unroll 1
+        for (int s = 32 * qt; s < min(32 * qt + 32, S); ++s) {
+          const bool sees = kvis && (MASK == 2 ? s < kbnd : !CAUSAL || key <= s);
+          if (!__any(sees)) continue;
+          const bf16* qr = q + b * qs0 + h * qs1 + s * qs2;
+          const bf16* dr = dout + b * ds0 + h * ds1 + s * ds2;
+          const int64_t ri = (static_cast<int64_t>(b) * Hq + h) * S + s;
+          const float p = __builtin_amdgcn_exp2f(fmaf(bwd_row_dot<KS>(qr, kf, hf), scale_log2, -lse2[ri]));
+          const float grad = p * (bwd_row_dot<KS>(dr, vf, hf) - dvec[ri]);
+          if (!sees) continue;
+          bwd_add_row<DT, JT>(dva, dr, p, hf);
+          bwd_add_row<DT, JT>(dka, qr, grad, hf);
+        }
+      }
+    }
+  }
   __syncthreads();  // the fold below reuses the staging buffers
 
   // Fold the head groups (fixed order: group 0 + group 1 + ...), then store.
@@ -867,6 +956,23 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(
   }
   if (kt == last) compute(kt, 0);  // odd count: the last tile is in buffer 0
 
+  if constexpr (kSecondWalk<HD, MASK>) {
+    if (__any(qok && bwd_any_nan<DT, JT>(acc))) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) acc[dt] = zero16();
+      const uint8_t* kmrow = MASK != 0 ? kmask + static_cast<int64_t>(b) * S : nullptr;
+#pragma unroll 1
+      for (int t = 0; t <= my_last; ++t) {
+        const bool sees = qok && bwd_visible<CAUSAL, MASK>(qi, t, kmrow);
+        if (!__any(sees)) continue;
+        const bf16* krow = k + b * ks0 + kvh * ks1 + t * ks2;
+        const bf16* vrow = v + b * vs0 + kvh * vs1 + t * vs2;
+        const float p = __builtin_amdgcn_exp2f(fmaf(bwd_row_dot<KS>(krow, qf, hf), scale_log2, -l2));
+        const float grad = p * (bwd_row_dot<KS>(vrow, of, hf) - dd);
+        if (sees) bwd_add_row<DT, JT>(acc, krow, grad, hf);
+      }
+    }
+  }
   if (qok) {
     bf16* orow = dq + b * dqs0 + h * dqs1 + static_cast<int64_t>(qi) * dqs2;
 #pragma unroll
@@ -885,17 +991,6 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(
 // ---------------------------------------------------------------------------
 // Generic path: fp32 math, one thread per query row (dQ) or key row (dK, dV).
 // Rows of up to MAXD elements are accumulated in registers.
-// Whether query s sees key t (t < S): causality, then the key mask
-// (MASK 1: key padding on top of causality; MASK 2: the forward's
-// reference-SDPA mode, key t > s or t padded, whatever `CAUSAL`).
-template <bool CAUSAL, int MASK>
-__device__ __forceinline__ bool bwd_visible(int s, int t, const uint8_t* kmrow) {
-  if constexpr (MASK == 2) return t > s || kmrow[t] == 0;
-  const bool c = !CAUSAL || t <= s;
-  if constexpr (MASK == 1) return c && kmrow[t] != 0;
-  return c;
-}
-
 template <typename T, int MAXD, bool CAUSAL, int MASK>
 __global__ __launch_bounds__(128) void attn_bwd_generic_dq_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,

@@ -9,10 +9,20 @@
 // elements: q k^T and dO v^T go to the 16-bit instructions as they are (their
 // products are exact in fp32), and the fp32 probabilities and score gradients
 // go there as two or three 16-bit planes that add up to them to fp32's own
-// precision (prob_product, grad_product), so nothing is held to 16 bits.  A
-// tile with an infinity or NaN in it, a score gradient that overflowed or a
-// probability past kPMax takes the fp32 instruction instead (col_product):
-// planes would make inf - inf of it.
+// precision (prob_product, grad_product), so nothing is held to 16 bits.
+//
+// Rows that a query does not see stay out of its sums whatever they hold, an
+// infinity or NaN included, but a product over a whole tile gives them the
+// weight 0, and 0 * inf is NaN; so are the planes of an infinity (inf - inf),
+// of a score gradient that overflowed and of a probability past what fp16's
+// planes hold.  All of these leave a NaN in the accumulators, so a wave that
+// ends with one walks its tiles a second time, row by row in fp32, each row
+// meeting only the columns that see it (row_dot, add_row).  It is a loop of its
+// own after the other: inside that one it would cost 30 to 70 registers there.
+// Forward / backward, against a test of every staged tile that 16-bit types
+// made before (for overflow alone; fp32 made none): fp16 B8 8/2 heads x 64, S
+// 2048 157 / 532 -> 134 / 463 us, fp32 B4 8/2 x 64, S 2048 192 / 615 -> 197 /
+// 616.
 //
 // What bounds it.  fp32: the fp32 matrix rate (256 FLOP per CU and cycle, a
 // tenth of bf16's measured rate); a 16x16x4 step takes 32 cycles of a SIMD,
@@ -101,8 +111,7 @@ template <typename T>
 constexpr bool kPlaneTiles = std::is_same<T, f16>::value;
 
 // Registers of one thread's share of a staged tile, and its way to LDS (t:
-// the thread's index among the kThreads that stage it).  land and direct
-// return whether an infinity or NaN was among the elements (16-bit types).
+// the thread's index among the kThreads that stage it).
 template <typename T, int HDP>
 struct Stage {
   static constexpr int E = 16 / int(sizeof(T));     // elements per 16-byte load
@@ -125,16 +134,13 @@ struct Stage {
     }
   }
   // planes: where the bf16 planes go (kPlaneTiles), or null
-  __device__ __forceinline__ bool land(T* dst, T* planes, int t) const {
-    uint32_t odd = 0;
+  __device__ __forceinline__ void land(T* dst, T* planes, int t) const {
 #pragma unroll
     for (int u = 0; u < VU; ++u) {
       const int i = t + kThreads * u;
       const int row = i / (HDP / E), c = i - row * (HDP / E);
       if (WHOLE || row < kTile) {
         *reinterpret_cast<uint4*>(&dst[row * P + c * E]) = raw[u];
-        if constexpr (sizeof(T) == 2) odd |= exponent_full(raw[u].x) | exponent_full(raw[u].y) |
-                                             exponent_full(raw[u].z) | exponent_full(raw[u].w);
         if constexpr (kPlaneTiles<T>) {
           if (planes) {
             float f[8], lo[8];
@@ -149,11 +155,9 @@ struct Stage {
         }
       }
     }
-    return odd != 0;
   }
   // Any strides and head_dim: element by element, straight to LDS.
-  static __device__ __forceinline__ bool direct(const Rows<T>& r, int row0, int S, int hd, T* dst, T* planes, int t) {
-    bool odd = false;
+  static __device__ __forceinline__ void direct(const Rows<T>& r, int row0, int S, int hd, T* dst, T* planes, int t) {
 #pragma unroll 4
     for (int u = 0; u < SU; ++u) {
       const int i = t + kThreads * u;
@@ -162,7 +166,6 @@ struct Stage {
       T x = from_f32<T>(0.f);
       if (ok) x = r.base[static_cast<int64_t>(row0 + row) * r.rs + d * r.es];
       dst[row * P + d] = x;
-      if constexpr (sizeof(T) == 2) odd |= exponent_full(x.bits) != 0;
       if constexpr (kPlaneTiles<T>) {
         if (planes) {
           const float f = to_f32(x);
@@ -172,13 +175,6 @@ struct Stage {
         }
       }
     }
-    return odd;
-  }
-  // nonzero: one of the two packed elements is an infinity or NaN
-  static __device__ __forceinline__ uint32_t exponent_full(uint32_t w) {
-    constexpr uint32_t M = std::is_same<T, f16>::value ? 0x7c007c00u : 0x7f807f80u;
-    constexpr uint32_t ONE = std::is_same<T, f16>::value ? 0x04000400u : 0x00800080u;
-    return ((w & M) + ONE) & 0x80008000u;
   }
 };
 
@@ -251,14 +247,58 @@ __device__ __forceinline__ f32x4 row_product(const T* rows, const typename Row16
 }
 
 // acc[d tile] += rows^T * x in fp32: x a result tile whose rows are 16 staged
-// rows.  fp32 elements; 16-bit ones where a tile holds an infinity or NaN.
-template <typename T, int HDP>
-__device__ __forceinline__ void col_product(f32x4 (&acc)[HDP / 16], const T* rows, const f32x4& x, int n, int g) {
+// rows of fp32 elements.
+template <int HDP>
+__device__ __forceinline__ void col_product(f32x4 (&acc)[HDP / 16], const float* rows, const f32x4& x, int n, int g) {
 #pragma unroll
   for (int r = 0; r < 4; ++r)
 #pragma unroll
     for (int t = 0; t < HDP / 16; ++t)
-      acc[t] = mfma4(to_f32(rows[(4 * g + r) * Stage<T, HDP>::P + 16 * t + n]), x[r], acc[t]);
+      acc[t] = mfma4(rows[(4 * g + r) * Stage<float, HDP>::P + 16 * t + n], x[r], acc[t]);
+}
+
+// What follows serves the second walk (see the top of the file): one row at a
+// time, straight from memory, any type and strides, plain fp32.
+// The dot product of a row with the resident fragment of each column.
+template <typename T, int HDP>
+__device__ __forceinline__ float row_dot(const T* row, const typename Row16<T, HDP>::Run (&f)[Row16<T, HDP>::N], int g,
+                                         int hd) {
+  constexpr int R = Row16<T, HDP>::R;
+  float s = 0.f;
+  asm volatile("" : "+v"(g));  // offsets and bounds made here, row by row: kept, they would take 60 registers
+#pragma unroll
+  for (int j = 0; j < Row16<T, HDP>::N; ++j) {
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int d = 4 * R * j + R * g + i;
+      if (d < hd) s = fmaf(to_f32(f[j].v[i]), to_f32(row[d]), s);
+    }
+  }
+  s += __shfl_xor(s, 16);
+  return s + __shfl_xor(s, 32);
+}
+// acc += w * row, elements es apart.
+template <typename T, int HDP>
+__device__ __forceinline__ void add_row(f32x4 (&acc)[HDP / 16], const T* row, int64_t es, float w, int g, int hd) {
+  asm volatile("" : "+v"(g));
+#pragma unroll
+  for (int t = 0; t < HDP / 16; ++t) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int d = 16 * t + 4 * g + r;
+      if (d < hd) acc[t][r] = fmaf(w, to_f32(row[d * es]), acc[t][r]);
+    }
+  }
+}
+
+template <int N>
+__device__ __forceinline__ bool any_nan(const f32x4 (&a)[N]) {
+  bool nan = false;
+#pragma unroll
+  for (int t = 0; t < N; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) nan |= a[t][r] != a[t][r];
+  return nan;
 }
 
 // The same over a whole staged tile of a 16-bit type, x as planes of 16-bit
@@ -304,7 +344,6 @@ __device__ __forceinline__ void split3(const f32x4 (&x)[2], uint4 (&p)[3]) {
 // Accumulators of either come out times kPScale.
 template <typename T>
 constexpr float kPScale = std::is_same<T, f16>::value ? 16384.f : 1.f;
-constexpr float kPMax = 3.5f;  // above: x * kPScale nears fp16's largest value
 
 template <typename T, int HDP>
 __device__ __forceinline__ void prob_product(f32x4 (&acc)[HDP / 16], const T* tile, const f32x4 (&x)[2], int n, int g) {
@@ -375,12 +414,6 @@ __device__ __forceinline__ void store_part(float* row, const f32x4 (&acc)[HDP / 
     *reinterpret_cast<float4*>(row + 16 * t + 4 * g) = make_float4(acc[t][0] * f, acc[t][1] * f, acc[t][2] * f, acc[t][3] * f);
 }
 
-// The running maximum of |ds| with p's own limit folded in: infinite once the
-// planes of p or ds would not hold them.
-__device__ __forceinline__ float max_of(float big, float p, float ds) {
-  return fmaxf(fmaxf(big, fabsf(ds)), p > kPMax ? INFINITY : 0.f);
-}
-
 // Whether query s sees key t < S (keep: the key mask's flag of t).
 __device__ __forceinline__ bool sees(int s, int t, bool keep, bool causal, int mode) {
   if (mode == HYDRA_MASK_REFERENCE_SDPA) return t > s || !keep;
@@ -417,13 +450,11 @@ __global__ __launch_bounds__(kThreads * KG) void attn_fwd_f32_kernel(
   using St = Stage<T, HDP>;
   __shared__ __attribute__((aligned(16))) T smem_all[KG][2][2 * St::N];
   __shared__ int keep_all[KG][2][kTile];
-  __shared__ int odd_all[KG][2];  // the last tile landed there with an infinity or NaN in it (16-bit types)
   const int kg = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / kThreads) : 0;
   const int tid = threadIdx.x - kg * kThreads, lane = tid & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   auto& smem = smem_all[kg];
   auto& keepv = keep_all[kg];
-  auto& odd = odd_all[kg];
   const int BHkv = gridDim.x / items;
   const int bk = blockIdx.x % BHkv;
   const int item = items - 1 - static_cast<int>(blockIdx.x / BHkv);  // longest key ranges first
@@ -459,21 +490,15 @@ __global__ __launch_bounds__(kThreads * KG) void attn_fwd_f32_kernel(
     }
   };
   auto land = [&](int t, int buf) {
-    bool o1, o2;
     if (vec & 1) {
-      o1 = sk.land(smem[buf], nullptr, tid);
-      o2 = sv.land(smem[buf] + St::N, nullptr, tid);
+      sk.land(smem[buf], nullptr, tid);
+      sv.land(smem[buf] + St::N, nullptr, tid);
     } else {
-      o1 = St::direct(kr, kTile * t, S, hd, smem[buf], nullptr, tid);
-      o2 = St::direct(vr, kTile * t, S, hd, smem[buf] + St::N, nullptr, tid);
+      St::direct(kr, kTile * t, S, hd, smem[buf], nullptr, tid);
+      St::direct(vr, kTile * t, S, hd, smem[buf] + St::N, nullptr, tid);
     }
-    if (sizeof(T) == 2 && (o1 || o2)) odd[buf] = t;
     if (mode != HYDRA_MASK_NONE && tid < kTile) keepv[buf][tid] = kp;
   };
-  if (sizeof(T) == 2) {
-    if (tid < 2) odd[tid] = -1;
-    __syncthreads();
-  }
   if (kg < nt) {
     fetch(kg);
     land(kg, 0);
@@ -522,18 +547,36 @@ __global__ __launch_bounds__(kThreads * KG) void attn_fwd_f32_kernel(
           x[u][r] = __builtin_amdgcn_exp2f(x[u][r] - ms);
           l += x[u][r];
         }
-        if constexpr (sizeof(T) == 4) col_product<T, HDP>(acc, Vs + 16 * u * St::P, x[u], n, g);
+        if constexpr (sizeof(T) == 4) col_product<HDP>(acc, Vs + 16 * u * St::P, x[u], n, g);
       }
-      if constexpr (sizeof(T) == 2) {
-        if (__builtin_amdgcn_readfirstlane(odd[buf]) != t) {
-          prob_product<T, HDP>(acc, Vs, x, n, g);
-        } else {  // planes would turn an infinity into inf - inf
-#pragma unroll
-          for (int u = 0; u < 2; ++u) col_product<T, HDP>(acc, Vs + 16 * u * St::P, x[u] * kPScale<T>, n, g);
-        }
-      }
+      if constexpr (sizeof(T) == 2) prob_product<T, HDP>(acc, Vs, x, n, g);
     }
     if (t + KG < nt) land(t + KG, buf ^ 1);
+  }
+  if (__any(qok && any_nan(acc))) {  // the second walk
+    m = -INFINITY;
+    l = 0.f;
+#pragma unroll
+    for (int d = 0; d < HDP / 16; ++d) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int t = kg; t < nt; t += KG)
+#pragma unroll 1
+      for (int key = kTile * t; key < min(kTile * t + kTile, S); ++key) {
+        const bool keep = mode == HYDRA_MASK_NONE || kmask[static_cast<int64_t>(b) * S + key] != 0;
+        const bool see = qok && sees(qi, key, keep, causal, mode);
+        if (!__any(see)) continue;
+        const float x = row_dot<T, HDP>(kr.base + key * kr.rs, qf, g, hd) * scale_log2;
+        if (!see) continue;
+        if (x > m) {
+          const float alpha = __builtin_amdgcn_exp2f(m - x);  // m = -inf -> 0
+          l *= alpha;
+#pragma unroll
+          for (int d = 0; d < HDP / 16; ++d) acc[d] *= alpha;
+          m = x;
+        }
+        const float p = __builtin_amdgcn_exp2f(x - (m == -INFINITY ? 0.f : m));
+        if (g == 0) l += p;  // the row's sum over its four lanes follows
+        add_row<T, HDP>(acc, vr.base + key * vr.rs, vr.es, p * kPScale<T>, g, hd);
+      }
   }
   if constexpr (KG > 1) {
     constexpr int NA = HDP / 16, XF = 4 * NA + 2;  // floats a lane hands over
@@ -632,7 +675,6 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dkdv_kernel(
   using St = Stage<T, HDP>;
   constexpr int NT = kPlaneTiles<T> ? 4 : 2;  // Q, dO, Q's planes
   __shared__ __attribute__((aligned(16))) T smem[2][NT * St::N];
-  __shared__ int odd[2];  // the last step landed there with an infinity or NaN in it (16-bit types)
   __shared__ __attribute__((aligned(16))) float rowv[2][2][kTile];  // lse2 and D of the tile's rows
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -679,24 +721,18 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dkdv_kernel(
     }
   };
   auto land = [&](int step, int buf) {
-    bool o1, o2;
     T* planes = kPlaneTiles<T> ? smem[buf] + 2 * St::N : nullptr;
     if (vec & 1) {
-      o1 = sq.land(smem[buf], planes, tid);
-      o2 = sd.land(smem[buf] + St::N, nullptr, tid);
+      sq.land(smem[buf], planes, tid);
+      sd.land(smem[buf] + St::N, nullptr, tid);
     } else {
       const int hr = step / nq, row0 = kTile * (qt0 + step - hr * nq), h = kvh * G + hr;
-      o1 = St::direct(Rows<T>{q + b * qs.b + h * qs.h, qs.s, 1}, row0, S, hd, smem[buf], planes, tid);
-      o2 = St::direct(Rows<T>{dout + b * ds.b + h * ds.h, ds.s, 1}, row0, S, hd, smem[buf] + St::N, nullptr, tid);
+      St::direct(Rows<T>{q + b * qs.b + h * qs.h, qs.s, 1}, row0, S, hd, smem[buf], planes, tid);
+      St::direct(Rows<T>{dout + b * ds.b + h * ds.h, ds.s, 1}, row0, S, hd, smem[buf] + St::N, nullptr, tid);
     }
-    if (sizeof(T) == 2 && (o1 || o2)) odd[buf] = step;
     if (tid < 2 * kTile) rowv[buf][tid / kTile][tid & (kTile - 1)] = rv;
   };
   const int first = c * ch, end = wg_any ? min(first + ch, total) : first;
-  if (sizeof(T) == 2) {
-    if (tid < 2) odd[tid] = -1;
-    __syncthreads();
-  }
   if (first < end) {
     fetch(first);
     land(first, 0);
@@ -710,7 +746,6 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dkdv_kernel(
     if (wave_any && (!walk || q0 + kTile - 1 >= kw0)) {
       const bool plain = walk ? q0 >= kw0 + 15 : mode != HYDRA_MASK_REFERENCE_SDPA;
       f32x4 p[2], dp[2];
-      float big = 0.f;
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         const T* Qs = smem[buf] + 16 * u * St::P;
@@ -730,28 +765,41 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dkdv_kernel(
           }
           p[u][r] = e;
           dp[u][r] = e * (dp[u][r] - dr[r]);
-          if constexpr (sizeof(T) == 2) big = max_of(big, e, dp[u][r]);
         }
         if constexpr (sizeof(T) == 4) {
-          col_product<T, HDP>(dva, Ds, p[u], n, g);
-          col_product<T, HDP>(dka, Qs, dp[u], n, g);
+          col_product<HDP>(dva, Ds, p[u], n, g);
+          col_product<HDP>(dka, Qs, dp[u], n, g);
         }
       }
       if constexpr (sizeof(T) == 2) {
         const T* Qs = smem[buf];
-        if (!__any(big == INFINITY) && __builtin_amdgcn_readfirstlane(odd[buf]) != step) {
-          prob_product<T, HDP>(dva, Qs + St::N, p, n, g);
-          grad_product<T, HDP>(dka, Qs, Qs + 2 * St::N, dp, n, g);
-        } else {  // planes would turn an infinity into inf - inf
-#pragma unroll
-          for (int u = 0; u < 2; ++u) {
-            col_product<T, HDP>(dva, Qs + St::N + 16 * u * St::P, p[u] * kPScale<T>, n, g);
-            col_product<T, HDP>(dka, Qs + 16 * u * St::P, dp[u], n, g);
-          }
-        }
+        prob_product<T, HDP>(dva, Qs + St::N, p, n, g);
+        grad_product<T, HDP>(dka, Qs, Qs + 2 * St::N, dp, n, g);
       }
     }
     if (step + 1 < end) land(step + 1, buf ^ 1);
+  }
+  // The second walk.  Keys that are stored as zeros (padding) or not at all do
+  // not count: their weights overflow where a query sees no key.
+  if (__any(key < S && (!pad || keep) && (any_nan(dka) || any_nan(dva)))) {
+#pragma unroll
+    for (int t = 0; t < HDP / 16; ++t) dka[t] = dva[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int step = first; step < end; ++step) {
+      const int hr = step / nq, row0 = kTile * (qt0 + step - hr * nq), h = kvh * G + hr;
+#pragma unroll 1
+      for (int s = row0; s < min(row0 + kTile, S); ++s) {
+        const bool see = key < S && (mode == HYDRA_MASK_REFERENCE_SDPA ? s < kbnd : !walk || key <= s);
+        if (!__any(see)) continue;
+        const T* qr = q + b * qs.b + h * qs.h + s * qs.s;
+        const T* dr = dout + b * ds.b + h * ds.h + s * ds.s;
+        const int64_t ri = (static_cast<int64_t>(b) * Hq + h) * S + s;
+        const float e = __builtin_amdgcn_exp2f(fmaf(row_dot<T, HDP>(qr, kf, g, hd), scale_log2, -lse2[ri]));
+        const float grad = e * (row_dot<T, HDP>(dr, vf, g, hd) - dvec[ri]);
+        if (!see) continue;
+        add_row<T, HDP>(dva, dr, 1, e * kPScale<T>, g, hd);
+        add_row<T, HDP>(dka, qr, 1, grad, g, hd);
+      }
+    }
   }
   if (pad && !keep) {
 #pragma unroll
@@ -779,7 +827,6 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dq_kernel(
   using St = Stage<T, HDP>;
   constexpr int NT = kPlaneTiles<T> ? 4 : 2;  // K, V, K's planes
   __shared__ __attribute__((aligned(16))) T smem[2][NT * St::N];
-  __shared__ int odd[2];  // the last tile landed there with an infinity or NaN in it (16-bit types)
   __shared__ int keepv[2][kTile];
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -825,22 +872,16 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dq_kernel(
     }
   };
   auto land = [&](int t, int buf) {
-    bool o1, o2;
     T* planes = kPlaneTiles<T> ? smem[buf] + 2 * St::N : nullptr;
     if (vec & 1) {
-      o1 = sk.land(smem[buf], planes, tid);
-      o2 = sv.land(smem[buf] + St::N, nullptr, tid);
+      sk.land(smem[buf], planes, tid);
+      sv.land(smem[buf] + St::N, nullptr, tid);
     } else {
-      o1 = St::direct(kr, kTile * t, S, hd, smem[buf], planes, tid);
-      o2 = St::direct(vr, kTile * t, S, hd, smem[buf] + St::N, nullptr, tid);
+      St::direct(kr, kTile * t, S, hd, smem[buf], planes, tid);
+      St::direct(vr, kTile * t, S, hd, smem[buf] + St::N, nullptr, tid);
     }
-    if (sizeof(T) == 2 && (o1 || o2)) odd[buf] = t;
     if (mode != HYDRA_MASK_NONE && tid < kTile) keepv[buf][tid] = kp;
   };
-  if (sizeof(T) == 2) {
-    if (tid < 2) odd[tid] = -1;
-    __syncthreads();
-  }
   fetch(first);
   land(first, 0);
   for (int t = first; t < end; ++t) {
@@ -850,7 +891,6 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dq_kernel(
     if (t0 < my_end) {
       const bool plain = mode == HYDRA_MASK_NONE && t0 + kTile - 1 <= (walk ? tk.q0 : S - 1) && t0 + kTile <= S;
       f32x4 dp[2];
-      float big = 0.f;
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         const T* Ks = smem[buf] + 16 * u * St::P;
@@ -866,21 +906,29 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_f32_dq_kernel(
             e = key < S && sees(qi, key, keep, causal, mode) ? e : 0.f;
           }
           dp[u][r] = e * (dp[u][r] - dd);
-          if constexpr (sizeof(T) == 2) big = fmaxf(big, fabsf(dp[u][r]));
         }
-        if constexpr (sizeof(T) == 4) col_product<T, HDP>(acc, Ks, dp[u], n, g);
+        if constexpr (sizeof(T) == 4) col_product<HDP>(acc, Ks, dp[u], n, g);
       }
       if constexpr (sizeof(T) == 2) {
         const T* Ks = smem[buf];
-        if (!__any(big == INFINITY) && __builtin_amdgcn_readfirstlane(odd[buf]) != t) {
-          grad_product<T, HDP>(acc, Ks, Ks + 2 * St::N, dp, n, g);
-        } else {  // planes would turn an infinity into inf - inf
-#pragma unroll
-          for (int u = 0; u < 2; ++u) col_product<T, HDP>(acc, Ks + 16 * u * St::P, dp[u], n, g);
-        }
+        grad_product<T, HDP>(acc, Ks, Ks + 2 * St::N, dp, n, g);
       }
     }
     if (t + 1 < end) land(t + 1, buf ^ 1);
+  }
+  if (__any(qok && any_nan(acc))) {  // the second walk
+#pragma unroll
+    for (int t = 0; t < HDP / 16; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int key = kTile * first; key < min(kTile * end, S); ++key) {
+      const bool keep = mode == HYDRA_MASK_NONE || kmask[static_cast<int64_t>(b) * S + key] != 0;
+      const bool see = qok && sees(qi, key, keep, causal, mode);
+      if (!__any(see)) continue;
+      const T* krow = kr.base + key * kr.rs;
+      const float e = __builtin_amdgcn_exp2f(fmaf(row_dot<T, HDP>(krow, qf, g, hd), scale_log2, -l2));
+      const float grad = e * (row_dot<T, HDP>(vr.base + key * vr.rs, of, g, hd) - dd);
+      if (see) add_row<T, HDP>(acc, krow, 1, grad, g, hd);
+    }
   }
   if (maxch > 1) {
     const int64_t rows = static_cast<int64_t>(parts) * 64;

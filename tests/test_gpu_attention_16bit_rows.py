@@ -95,12 +95,14 @@ def test_infinities(cuda, dtype, hd):
     v2[0, 0, 70, 5] = float("inf")
     out = _run(cuda, q, k, v2, go, True)[0]
     assert (out[0, :, 70:, 5] == float("inf")).all()
-    assert torch.equal(out[0, :, :64], base[0][0, :, :64])  # tiles of 32 keys
+    before = (out[0, :, :70] - base[0][0, :, :70]).norm() / base[0][0, :, :70].norm()
+    assert float(before) < U[dtype]  # NaN fails
     keep = [d for d in range(hd) if d != 5]
     assert float((out[..., keep] - base[0][..., keep]).norm() / base[0].norm()) < U[dtype]
     go2 = go.clone()
     go2[0, 1, 70, 5] = float("-inf")
     dv = _run(cuda, q, k, v, go2, True)[3]
     assert (dv[0, 0, :71, 5] == float("-inf")).all()
-    assert torch.equal(dv[0, 0, 128:], base[3][0, 0, 128:])
+    after = (dv[0, 0, 71:] - base[3][0, 0, 71:]).norm() / base[3][0, 0, 71:].norm()
+    assert float(after) < 2 * U[dtype]
     assert float((dv[..., keep] - base[3][..., keep]).norm() / base[3].norm()) < 2 * U[dtype]
