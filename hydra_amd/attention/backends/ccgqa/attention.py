@@ -36,7 +36,7 @@ from ...._lib import CCGQA_V_TRANSPOSED, CCGQA_W_TILED, MASK_KEY_PADDING, MASK_R
 from .autograd import ccgqa_prep_train
 from .kernels.fused_attention import CCGQAAttentionFused, MaskedAttentionFunction
 from .kernels.fused_conv import OptimizedConvSequence
-from .ops import (attention_forward, ccgqa_prep, linear_weight_ok, output_projection, pack_conv_weight,
+from .ops import (PackedWeights, attention_forward, ccgqa_prep, linear_weight_ok, output_projection, pack_conv_weight,
                   pack_conv_weights_tiled, pack_linear_weight, prep_flags, tiled_weights_ok)
 
 # Kept for callers that probe these names (attention.py:13-28).
@@ -184,7 +184,7 @@ class CCGQAAttention(nn.Module):
         if tiled:
             flags |= CCGQA_W_TILED  # conv weights in MFMA-fragment order
         with torch.no_grad():
-            packed = self._packed_conv_weights(convw, x.dtype, tiled) if self.use_convs else (None,) * 4
+            packed, packed_o = self._packed(convw, x.dtype, tiled)
             q, k, v = ccgqa_prep(
                 qkv.detach(), self.n_heads, self.n_kv_heads, self.head_dim, flags, *packed,
                 temperature=self.key_temperature if self.use_qk_norm else None,
@@ -197,8 +197,7 @@ class CCGQAAttention(nn.Module):
                               key_mask=mask, mask_mode=_mask_mode() if mask is not None else 0,
                               out=o_view,
                               bound_temperature=self.key_temperature if self.use_qk_norm else None)
-        w_o = self.o_proj.weight
-        out = output_projection(out, w_o, self._packed_o_proj() if linear_weight_ok(w_o) else None)
+        out = output_projection(out, self.o_proj.weight, packed_o)
         if self.output_scale != 1.0:
             out = out * self.output_scale
         return out
@@ -226,29 +225,35 @@ class CCGQAAttention(nn.Module):
             out = out * self.output_scale
         return out
 
+    def _packed(self, convw, dtype, tiled):
+        """The four conv weights packed in `dtype` (tap-major, or MFMA-tiled;
+        None without convs), and o_proj's weight in hydra_linear_fwd's fragment
+        order (None where that kernel does not take it); rebuilt only when a
+        weight changes."""
+        w_o = self.o_proj.weight
+        o_ok = linear_weight_ok(w_o)
+        ws = (*convw, w_o) if o_ok else convw
+        if not ws:
+            return (None,) * 4, None
+
+        packs = self.__dict__.get("_packs")  # made here: modules pickled without it work
+        if packs is None:
+            packs = self.__dict__.setdefault("_packs", PackedWeights())
+        tag = (len(convw), dtype, tiled)
+        packed = packs.get(ws, tag)
+        if packed is None:
+            if tiled:  # one launch for the four
+                packed = pack_conv_weights_tiled(convw, dtype, self.n_heads, self.n_kv_heads, self.head_dim)
+            else:
+                packed = tuple(pack_conv_weight(w, dtype) for w in convw)
+            packed = packs.put(ws, tag, (*packed, pack_linear_weight(w_o)) if o_ok else packed)
+        return (packed[:4] if convw else (None,) * 4), (packed[-1] if o_ok else None)
+
     def _packed_conv_weights(self, convw, dtype, tiled=False):
-        """Packed copies (tap-major, or MFMA-tiled) of the four conv weights in
-        `dtype`, rebuilt only when a weight changes (tensor version counter)
-        or moves."""
-        key = tuple((w.data_ptr(), w._version, w.device, dtype, tiled) for w in convw)
-        cache = getattr(self, "_packed_cache", None)
-        if cache is None or cache[0] != key:
-            # tiled: one launch for the four
-            cache = (key, pack_conv_weights_tiled(convw, dtype, self.n_heads, self.n_kv_heads, self.head_dim)
-                     if tiled else tuple(pack_conv_weight(w, dtype) for w in convw))
-            self._packed_cache = cache
-        return cache[1]
+        return self._packed(convw, dtype, tiled)[0]
 
     def _packed_o_proj(self):
-        """o_proj's weight in hydra_linear_fwd's fragment order, rebuilt only
-        when the weight changes (tensor version counter) or moves."""
-        w = self.o_proj.weight
-        key = (w.data_ptr(), w._version, w.device, w.dtype)
-        cache = getattr(self, "_packed_o_cache", None)
-        if cache is None or cache[0] != key:
-            cache = (key, pack_linear_weight(w))
-            self._packed_o_cache = cache
-        return cache[1]
+        return self._packed((), self.o_proj.weight.dtype, False)[1]
 
     def _load_from_state_dict(self, state_dict, prefix, local_metadata, strict, missing_keys,
                               unexpected_keys, error_msgs):

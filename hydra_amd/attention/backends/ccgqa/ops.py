@@ -4,7 +4,8 @@ here; strides, pointers and the current stream go to the library."""
 from __future__ import annotations
 
 import ctypes
-
+import threading
+import weakref
 from typing import Optional
 
 import torch
@@ -54,6 +55,100 @@ def pack_conv_weights_tiled(ws, dtype: torch.dtype, n_heads: int, n_kv_heads: in
         packed.append(out[at:at + w.numel()].view(3, o // 32, i // 16, 2, 32, 8))
         at += w.numel()
     return tuple(packed)
+
+
+class _Pack:
+    __slots__ = ("refs", "versions", "ptrs", "tensors", "event", "streams", "captured")
+
+    def same(self, ws) -> bool:
+        return len(ws) == len(self.refs) and all(r() is w for r, w in zip(self.refs, ws))
+
+    def holds(self, ws) -> bool:
+        for r, v, a, w in zip(self.refs, self.versions, self.ptrs, ws):
+            if r() is not w or w._version != v or w.data_ptr() != a:
+                return False
+        return True
+
+    def note(self, ws, tensors) -> None:
+        self.versions, self.ptrs = [w._version for w in ws], [w.data_ptr() for w in ws]
+        self.tensors = tensors
+
+
+class PackedWeights:
+    """Weights in a kernel's order, packed when first asked for and again when
+    one of them changes (tensor version counter), moves or is replaced (they
+    are compared as objects: another tensor may come to lie at a freed one's
+    address).
+
+    Streams: a call on another stream than the packing one waits for it, once.
+    Graphs: what is packed while a stream is being captured exists only once
+    the graph replays, so it is not kept (each replay packs again).  Tensors
+    that a capture read keep their memory as long as this object lives, and a
+    change of their weights is packed into that memory, between two
+    synchronisations with the device since replays are not tracked; it reaches
+    the replays with the next call outside the graph.
+
+    Copies and pickles are empty."""
+
+    def __init__(self):
+        self._last = {}        # tag -> _Pack
+        self._captured = []    # (tag, _Pack) that a capture read
+        self._lock = threading.Lock()
+
+    def __deepcopy__(self, memo):
+        return PackedWeights()
+
+    def __reduce__(self):
+        return PackedWeights, ()
+
+    def get(self, ws, tag):
+        """The tensors that the weights ws (a tuple) were last packed to, or
+        None; `tag` tells apart what ws may be packed to."""
+        p = self._last.get(tag)
+        if p is None or not p.holds(ws):
+            p = self._seen(ws, tag)
+            if p is None or not p.holds(ws):
+                return None
+        if ws[0].is_cuda:
+            if torch.cuda.is_current_stream_capturing():
+                if not p.captured:
+                    p.captured = True
+                    self._captured.append((tag, p))
+            elif _lib.stream(ws[0]) not in p.streams:
+                here = torch.cuda.current_stream(ws[0].device)
+                here.wait_event(p.event)
+                for t in p.tensors:
+                    t.record_stream(here)
+                p.streams.add(here.cuda_stream)
+        return p.tensors
+
+    def put(self, ws, tag, tensors):
+        """Keeps what ws was just packed to on the current stream; returns the
+        tensors to use."""
+        if ws[0].is_cuda and torch.cuda.is_current_stream_capturing():
+            return tensors
+        with self._lock:
+            p = self._seen(ws, tag)
+            if p is not None:
+                torch.cuda.synchronize(ws[0].device)  # replays that read them are done
+                for old, new in zip(p.tensors, tensors):
+                    old.copy_(new)
+                torch.cuda.synchronize(ws[0].device)  # replays to come read the new values
+                p.note(ws, p.tensors)
+            else:
+                p = _Pack()
+                p.refs, p.captured, p.event, p.streams = [weakref.ref(w) for w in ws], False, None, set()
+                # a layout that is the weight's own: a copy, or a later pack would write to the weight
+                p.note(ws, tuple(t.clone() if t.data_ptr() == w.data_ptr() else t for t, w in zip(tensors, ws)))
+                if ws[0].is_cuda:
+                    here = torch.cuda.current_stream(ws[0].device)
+                    p.event = here.record_event()
+                    p.streams.add(here.cuda_stream)
+            self._last[tag] = p
+        return p.tensors
+
+    def _seen(self, ws, tag):
+        return next((p for t, p in self._captured if t == tag and p.same(ws)), None)
 
 
 def tiled_weights_ok(n_heads: int, n_kv_heads: int, head_dim: int, dtype: torch.dtype) -> bool:

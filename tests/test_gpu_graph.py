@@ -94,3 +94,93 @@ def test_hydra_model_forward_graph_replays_match_eager(cuda):
     torch.cuda.synchronize()
     assert torch.equal(y, want2)
     del graph
+
+
+def _layer(cuda, seed=3):
+    from hydra_amd.attention import CCGQAAttention
+
+    torch.manual_seed(seed)
+    m = CCGQAAttention(dim=1024, n_heads=4, n_kv_heads=1, compression_factor=4, max_seq_len=512)
+    with torch.no_grad():
+        for p in m.parameters():
+            p.copy_(torch.randn(p.shape) * 0.02)
+        m.key_temperature.fill_(1.0)
+    return m.to(cuda, torch.bfloat16).eval()
+
+
+def _input(cuda):
+    g = torch.Generator(device=cuda).manual_seed(4)
+    return torch.randn(2, 512, 1024, device=cuda, generator=g).to(torch.bfloat16)
+
+
+def _captured(m, x):
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):  # the libraries' own first calls
+        _layer(x.device)(x)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = m(x)
+    return graph, y
+
+
+def test_first_call_in_a_capture(cuda):
+    """Weights packed inside the capture exist once the graph replays: an
+    eager call before that packs its own."""
+    x = _input(cuda)
+    with torch.no_grad():
+        want = _layer(cuda)(x).clone()
+        m = _layer(cuda)
+        graph, y = _captured(m, x)
+        assert torch.equal(m(x), want)
+        for _ in range(3):
+            y.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, want)
+            assert torch.equal(m(x), want)
+    del graph
+
+
+def test_weights_changed_after_a_capture(cuda):
+    """Replays read the packed weights that the last eager call left, in the
+    memory that the capture saw."""
+    x = _input(cuda)
+    with torch.no_grad():
+        m = _layer(cuda)
+        m(x)
+        graph, y = _captured(m, x)
+        for seed in (5, 6):
+            for p, q in zip(m.parameters(), _layer(cuda, seed).parameters()):
+                p.copy_(q)
+            want = m(x).clone()
+            other = torch.full((1 << 24,), 7.0, device=cuda)  # what a freed pack's memory would hold
+            for _ in range(3):
+                y.zero_()
+                graph.replay()
+                torch.cuda.synchronize()
+                assert torch.equal(y, want)
+            del other
+        assert torch.equal(want, _layer(cuda, 6)(x))
+    del graph
+
+
+def test_first_call_on_another_stream(cuda):
+    """A call on the default stream right after the packing one on a busy
+    stream."""
+    x = _input(cuda)
+    with torch.no_grad():
+        want = _layer(cuda)(x).clone()
+        a = torch.randn(8192, 8192, device=cuda).to(torch.bfloat16)
+        a @ a
+        m = _layer(cuda)
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            for _ in range(8):
+                a @ a
+            y = m(x)
+        got = m(x)
+        torch.cuda.synchronize()
+        assert torch.equal(y, want) and torch.equal(got, want)
