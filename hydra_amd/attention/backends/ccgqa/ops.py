@@ -43,8 +43,10 @@ def pack_conv_weights_tiled(ws, dtype: torch.dtype, n_heads: int, n_kv_heads: in
     ws = tuple(w.detach() for w in ws)
     L, K = n_heads * head_dim, n_kv_heads * head_dim
     shapes = ((L, head_dim), (L, L), (K, head_dim), (K, K))
-    if dtype not in (torch.bfloat16, torch.float16) or any(
-            w.dtype != dtype or not w.is_contiguous() or w.shape != (*s, 3) for w, s in zip(ws, shapes)):
+    # the launch takes addresses: weights on one GPU only
+    if dtype not in (torch.bfloat16, torch.float16) or not ws[0].is_cuda or any(
+            w.dtype != dtype or w.device != ws[0].device or not w.is_contiguous() or w.shape != (*s, 3)
+            for w, s in zip(ws, shapes)):
         return tuple(pack_conv_weight(w, dtype, True) for w in ws)
     out = torch.empty(sum(w.numel() for w in ws), dtype=dtype, device=ws[0].device)
     with _lib.on_device(out):

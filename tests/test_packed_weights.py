@@ -72,3 +72,18 @@ def test_a_copied_module_packs_its_own(how):
         n.q_conv.conv1.weight.fill_(3)
     assert (n._packed_conv_weights(convs(n), torch.float32)[0] == 3).all()
     assert not (m._packed_conv_weights(convs(m), torch.float32)[0] == 3).any()
+
+
+def test_packing_in_one_launch_refuses_host_memory(monkeypatch):
+    """The one-launch packing hands addresses to a kernel: weights that are not
+    all on one GPU take the torch operations, after which the caller's own
+    device check speaks."""
+    from hydra_amd import _lib
+    from hydra_amd.attention.backends.ccgqa.ops import ccgqa_prep, pack_conv_weight, pack_conv_weights_tiled
+
+    monkeypatch.setattr(_lib, "call", lambda *a: pytest.fail("a launch on host memory"))
+    ws = [torch.randn(*s, 3).to(torch.bfloat16) for s in ((128, 64), (128, 128), (64, 64), (64, 64))]
+    for got, w in zip(pack_conv_weights_tiled(ws, torch.bfloat16, 2, 1, 64), ws):
+        assert torch.equal(got, pack_conv_weight(w, torch.bfloat16, True))
+    with pytest.raises(RuntimeError, match="GPU tensors only"):
+        ccgqa_prep(torch.zeros(1, 8, 256, dtype=torch.bfloat16), 2, 1, 64, 1 | 64, *ws)
