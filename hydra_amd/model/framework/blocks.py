@@ -29,16 +29,20 @@ def _recording(*tensors) -> bool:
 
 
 def _mlp_residual(mlp: nn.Module, h: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
-    """h + mlp(y), the add in the GEMM epilogue for the SwiGLU MLP (also under
-    a MoD wrapper that does not route yet and that nobody hooks into).  h is a
-    fresh tensor of the caller's: its storage may hold the result."""
-    if (isinstance(mlp, MoDMLPWrapper) and _own(mlp, MoDMLPWrapper, "forward") and mlp._dense()
-            and isinstance(mlp.mlp, SwiGLUMLPFused) and _own(mlp.mlp, SwiGLUMLPFused, "forward")
-            and _plain(mlp, mlp.mlp)):
+    """h + mlp(y), the add in the GEMM epilogue for the SwiGLU MLP that nobody
+    changes or hooks into (also under such a MoD wrapper that does not route
+    yet).  h is a fresh tensor of the caller's: its storage may hold the
+    result."""
+    if isinstance(mlp, SwiGLUMLPFused) and _plain(mlp):
+        if not _own(mlp, SwiGLUMLPFused, "forward_residual"):
+            return mlp.forward_residual(h, y)
+        if _own(mlp, SwiGLUMLPFused, "forward"):
+            return mlp.forward_residual(h, y, own=True)
+    elif (isinstance(mlp, MoDMLPWrapper) and _own(mlp, MoDMLPWrapper, "forward") and mlp._dense()
+            and isinstance(mlp.mlp, SwiGLUMLPFused)
+            and _own(mlp.mlp, SwiGLUMLPFused, "forward", "forward_residual") and _plain(mlp, mlp.mlp)):
         mlp._note_dense(y)
-        mlp = mlp.mlp
-    if isinstance(mlp, SwiGLUMLPFused):
-        return mlp.forward_residual(h, y, own=True)
+        return mlp.mlp.forward_residual(h, y, own=True)
     return h + mlp(y)
 
 

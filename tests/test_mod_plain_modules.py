@@ -48,6 +48,41 @@ def test_an_overridden_mlp_forward_is_called():
             assert torch.equal(_mlp_residual(MoDMLPWrapper(mlp, 8).eval(), h, y), h + 2 * y)
 
 
+@pytest.mark.parametrize("wrapped", [False, True])
+@pytest.mark.parametrize("how", ["class", "instance", "hook", "residual"])
+def test_a_changed_mlp_is_used_as_it_is(how, wrapped):
+    """Alone as under a wrapper, an MLP with another forward (by its class or
+    on the instance) or with hooks is called; one whose class has its own
+    forward_residual(h, x) gets the two arguments that it takes."""
+    from hydra_amd.layers import SwiGLUMLPFused
+    from hydra_amd.model.framework.blocks import _mlp_residual
+    from hydra_amd.routing.mixture_of_depths import MoDMLPWrapper
+
+    class Doubling(SwiGLUMLPFused):
+        def forward(self, x):
+            return 2 * x
+
+    class Residual(Doubling):
+        def forward_residual(self, h, x):
+            return h + 2 * x
+
+    mlp = {"class": Doubling, "residual": Residual}.get(how, SwiGLUMLPFused)(8, 16)
+    if how == "instance":
+        mlp.forward = lambda x: 2 * x
+    elif how == "hook":  # the parent's forward needs a GPU: the hook must come before it
+        def hook(module, args):
+            raise KeyError("called")
+        mlp.register_forward_pre_hook(hook)
+    h, y = torch.randn(2, 3, 8), torch.randn(2, 3, 8)
+    block = MoDMLPWrapper(mlp, 8).eval() if wrapped else mlp
+    with torch.no_grad():
+        if how == "hook":
+            with pytest.raises(KeyError, match="called"):
+                _mlp_residual(block, h, y)
+        else:
+            assert torch.equal(_mlp_residual(block, h, y), h + 2 * y)
+
+
 def test_methods_of_their_own():
     from hydra_amd.routing.base import BaseRouter
     from hydra_amd.routing.mixture_of_depths import MoDRouter, _own
