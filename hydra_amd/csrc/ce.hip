@@ -18,7 +18,8 @@
 // For 16-bit hidden states and weights the backward's two GEMMs run on the
 // bf16 matrix cores: ce_planes kernels write the gradient of the fp32 logits
 // as two bf16 planes, hi and residual (16 significant bits together), instead
-// of one fp32 row -- the same bytes.  Products of bf16 values are exact in the
+// of one fp32 row -- the same bytes, and in the logits' own memory where a row
+// fits the registers.  Products of bf16 values are exact in the
 // GEMMs' fp32 accumulation, so the error of the 16-bit gradients against 64
 // bits stays at their rounding (1.7e-3 both), and the three fp32 GEMMs of a
 // chunk (4096 tokens x 32000 x 768: 4.4 ms at 140 TFLOP/s) become 1.3 ms of
@@ -223,6 +224,19 @@ __device__ __forceinline__ void chunk_stats(const float* v, float& m, float& s) 
   lse_merge(m, s, cm, cs);
 }
 
+// What bf16 leaves of g; an infinity is whole without it.
+__device__ __forceinline__ float plane_rest(float g, bf16 hi) {
+  const float h = to_f32(hi);
+  return fabsf(h) == INFINITY ? 0.f : g - h;
+}
+
+// Columns from V on hold nothing.
+__device__ __forceinline__ void mask_tail(float* v, int e, int V) {
+  if (e + 8 > V)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = e + i < V ? v[i] : -INFINITY;
+}
+
 // (softmax - onehot(t)) * scale of 8 logits at column e, as bf16 hi and
 // residual vectors.
 __device__ __forceinline__ void planes8(const float* v, int e, int t, float lse2, float sc, uint4& hi, uint4& lo) {
@@ -231,7 +245,7 @@ __device__ __forceinline__ void planes8(const float* v, int e, int t, float lse2
   for (int i = 0; i < 8; ++i) {
     const float p = __builtin_amdgcn_exp2f(fmaf(v[i], kLog2e, -lse2));
     g[i] = (p - (e + i == t ? 1.f : 0.f)) * sc;
-    r[i] = g[i] - to_f32(from_f32<bf16>(g[i]));
+    r[i] = plane_rest(g[i], from_f32<bf16>(g[i]));
   }
   hi = pack16<bf16>(g);
   lo = pack16<bf16>(r);
@@ -248,8 +262,10 @@ struct PlanesArgs {
   int64_t ignore_index;
 };
 
-// NCH > 0: the row stays in registers (V <= 2048 NCH, V % 8 == 0, aligned
-// rows); NCH = 0: read twice, VEC with 8 columns per thread, else one.
+// NCH > 0: the row stays in registers (V <= 2048 NCH, aligned rows of whole
+// 8-column pieces), and the planes may take the logits' memory: every thread
+// has read its columns before the barrier of row_lse2.  NCH = 0: read twice,
+// VEC with 8 columns per thread, else one.
 template <int NCH, bool VEC>
 __global__ __launch_bounds__(256) void ce_planes_kernel(PlanesArgs a) {
   __shared__ float red_m[4], red_s[4];
@@ -279,6 +295,7 @@ __global__ __launch_bounds__(256) void ce_planes_kernel(PlanesArgs a) {
         float v[8];
         unpack16<float>(raw[c][0], v);
         unpack16<float>(raw[c][1], v + 4);
+        mask_tail(v, (c * 256 + tid) * 8, V);
         chunk_stats<8>(v, m, s);
       }
     const float lse2 = row_lse2(m, s, red_m, red_s);
@@ -289,6 +306,7 @@ __global__ __launch_bounds__(256) void ce_planes_kernel(PlanesArgs a) {
         float v[8];
         unpack16<float>(raw[c][0], v);
         unpack16<float>(raw[c][1], v + 4);
+        mask_tail(v, e, V);
         uint4 h, l;
         planes8(v, e, t, lse2, sc, h, l);
         st16raw<true>(hi + e, h);
@@ -320,7 +338,7 @@ __global__ __launch_bounds__(256) void ce_planes_kernel(PlanesArgs a) {
       const float g = (p - (e == t ? 1.f : 0.f)) * sc;
       const bf16 h = from_f32<bf16>(g);
       hi[e] = h.bits;
-      lo[e] = from_f32<bf16>(g - to_f32(h)).bits;
+      lo[e] = from_f32<bf16>(plane_rest(g, h)).bits;
     }
   }
 }
@@ -394,17 +412,26 @@ extern "C" int hydra_ce_grad_planes(const float* logits, int64_t rows, int64_t v
   HYDRA_REQUIRE(rows >= 0 && vocab >= 1, "ce_grad_planes: bad size");
   HYDRA_REQUIRE(vocab < (int64_t(1) << 31) && rows < (int64_t(1) << 31), "ce_grad_planes: too large");
   HYDRA_REQUIRE(logits_rs >= vocab && planes_rs >= vocab, "ce_grad_planes: row stride < vocab");
-  HYDRA_REQUIRE(rows <= 1 || plane_stride >= (rows - 1) * planes_rs + vocab, "ce_grad_planes: planes overlap");
+  const bool in_place = planes == logits;
+  if (in_place)
+    HYDRA_REQUIRE(planes_rs == 2 * logits_rs && plane_stride == logits_rs,
+                  "ce_grad_planes: in place, a row's planes take the two halves of its bytes");
+  else
+    HYDRA_REQUIRE(rows <= 1 || plane_stride >= (rows - 1) * planes_rs + vocab, "ce_grad_planes: planes overlap");
   if (rows == 0) return HYDRA_OK;
   HYDRA_REQUIRE(logits && targets && planes && grad_scale, "ce_grad_planes: null pointer");
   const int V = static_cast<int>(vocab);
   const PlanesArgs a{logits, logits_rs, targets, static_cast<uint16_t*>(planes), planes_rs, plane_stride,
                      grad_scale, V, ignore_index};
-  const bool vec = V % 8 == 0 && logits_rs % 4 == 0 && planes_rs % 8 == 0 && plane_stride % 8 == 0 &&
-                   aligned16(logits) && aligned16(planes);
+  // In place the padding of a row up to 8 columns is the row's own.
+  const bool vec = (V % 8 == 0 || (in_place && logits_rs >= (vocab + 7) / 8 * 8)) && logits_rs % 4 == 0 &&
+                   planes_rs % 8 == 0 && plane_stride % 8 == 0 && aligned16(logits) && aligned16(planes);
   const dim3 grid(static_cast<unsigned>(rows));
   auto st = static_cast<hipStream_t>(stream);
-  const int nch = (V / 8 + 255) / 256;
+  const int64_t nch = ((vocab + 7) / 8 + 255) / 256;
+  if (in_place && (!vec || vocab > HYDRA_CE_IN_PLACE_VOCAB))
+    return fail(HYDRA_ERR_UNSUPPORTED, "ce_grad_planes: in place takes aligned rows of up to 32768 columns");
+  static_assert(HYDRA_CE_IN_PLACE_VOCAB == 16 * 256 * 8, "the longest rows that stay in registers");
   if (!vec) ce_planes_kernel<0, false><<<grid, 256, 0, st>>>(a);
   else if (nch <= 4) ce_planes_kernel<4, true><<<grid, 256, 0, st>>>(a);
   else if (nch <= 8) ce_planes_kernel<8, true><<<grid, 256, 0, st>>>(a);

@@ -389,6 +389,21 @@ def _ce_grad_planes(logits: torch.Tensor, targets: torch.Tensor, ignore_index: i
     return planes[:, :V]
 
 
+CE_IN_PLACE_VOCAB = 32768  # HYDRA_CE_IN_PLACE_VOCAB
+
+
+def _ce_grad_planes_in_place(logits: torch.Tensor, V: int, targets: torch.Tensor, ignore_index: int,
+                             grad_scale: torch.Tensor) -> torch.Tensor:
+    """The same planes in the memory of logits [rows, pitch] (pitch: V rounded
+    up to 8, V <= CE_IN_PLACE_VOCAB): [2 * rows, V], a row's rounded values,
+    then its residuals."""
+    rows, pitch = logits.shape
+    with _lib.on_device(logits):
+        _lib.call("hydra_ce_grad_planes", logits.data_ptr(), rows, V, pitch, targets.data_ptr(), int(ignore_index),
+                  logits.data_ptr(), 2 * pitch, pitch, _lib.ptr(grad_scale), _lib.stream(logits))
+    return logits.view(torch.bfloat16).view(2 * rows, pitch)[:, :V]
+
+
 class ChunkedCrossEntropyFunction(torch.autograd.Function):
     """fused_ops.py:1382-1531: mean token cross-entropy of hidden @ weight^T
     over tokens whose target is not ignore_index, computed chunk by chunk
@@ -437,17 +452,32 @@ class ChunkedCrossEntropyFunction(torch.autograd.Function):
             # Other dtypes keep the fp32 GEMMs: fp32 operands would need three
             # planes each, six products, for no gain worth the name.  So does
             # create_graph, which products with an `out` cannot record.
+            V = weight.shape[0]
+            in_place = V <= CE_IN_PLACE_VOCAB
+            # longer rows: the planes lie beside the logits, of half a chunk each
+            step = cs if in_place else max(1, (min(cs, h.shape[0]) + 1) // 2)
             grad_w = None
-            for s in range(0, h.shape[0], cs):
-                hc = h[s:s + cs]
+            for s in range(0, h.shape[0], step):
+                hc = h[s:s + step]
                 n = hc.shape[0]
-                planes = _ce_grad_planes(torch.mm(hc, weight.t(), out_dtype=torch.float32), t[s:s + cs],
-                                         ctx.ignore_index, scale)
-                gh = torch.mm(planes, weight, out_dtype=torch.float32)
-                torch.add(gh[:n], gh[n:], out=grad_h[s:s + cs])
-                both = torch.cat((hc, hc))
-                grad_w = (torch.mm(planes.t(), both, out_dtype=torch.float32) if grad_w is None else
-                          torch.addmm(grad_w, planes.t(), both, out_dtype=torch.float32))
+                logits = torch.empty((n, (V + 7) // 8 * 8), dtype=torch.float32, device=h.device)
+                torch.mm(hc, weight.t(), out_dtype=torch.float32, out=logits[:, :V])
+                if in_place:
+                    planes = _ce_grad_planes_in_place(logits, V, t[s:s + step], ctx.ignore_index, scale)
+                    pair = (n, 2)  # a token's two rows, one after the other
+                else:
+                    planes = _ce_grad_planes(logits[:, :V], t[s:s + step], ctx.ignore_index, scale)
+                    pair = (2, n)
+                del logits
+                side = pair.index(2)
+                gh = torch.mm(planes, weight, out_dtype=torch.float32).view(*pair, dim)
+                torch.add(gh.select(side, 0), gh.select(side, 1), out=grad_h[s:s + step])
+                both = hc.unsqueeze(side).expand(*pair, dim).reshape(2 * n, dim)
+                if grad_w is None:
+                    grad_w = torch.mm(planes.t(), both, out_dtype=torch.float32)
+                else:
+                    torch.addmm(grad_w, planes.t(), both, out_dtype=torch.float32, out=grad_w)
+                del planes
             if grad_w is None:
                 grad_w = torch.zeros(weight.shape, dtype=torch.float32, device=h.device)
             return (grad_h.view_as(hidden_states).to(hidden_states.dtype), grad_w.to(weight.dtype),

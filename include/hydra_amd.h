@@ -433,8 +433,13 @@ int hydra_ce_rows(const void* logits, int64_t rows, int64_t vocab, int64_t logit
 /* The same gradient of fp32 logits, g = (softmax(x[r]) - onehot(t)) *
  * grad_scale[0], written as two bf16 planes instead of fp32: planes[0] the
  * rounded value, planes[1] (plane_stride elements further) the residual
- * g - planes[0] rounded, rows planes_rs elements apart.  For the bf16 GEMMs of
- * ChunkedCrossEntropyFunction's backward (fused_ops.py:1459-1531). */
+ * g - planes[0] rounded (0 beside an infinity), rows planes_rs elements apart.
+ * In place (planes == logits, planes_rs == 2 * logits_rs, plane_stride ==
+ * logits_rs): a row's planes take the two halves of its bytes, padding up to a
+ * multiple of 8 columns included; 16-byte aligned rows of at most
+ * HYDRA_CE_IN_PLACE_VOCAB columns, others HYDRA_ERR_UNSUPPORTED.  For the bf16
+ * GEMMs of ChunkedCrossEntropyFunction's backward (fused_ops.py:1459-1531). */
+#define HYDRA_CE_IN_PLACE_VOCAB 32768
 int hydra_ce_grad_planes(const float* logits, int64_t rows, int64_t vocab, int64_t logits_rs,
                          const int64_t* targets, int64_t ignore_index, void* planes,
                          int64_t planes_rs, int64_t plane_stride, const float* grad_scale,

@@ -149,3 +149,87 @@ def test_ce_grad_planes(cuda, rows, V):
         assert float((got - ref).norm() / ref.norm()) < 2.0 ** -16
     else:
         assert got.abs().max() < 1e-6
+
+
+@pytest.mark.parametrize("rows,V", [(3, 1), (5, 7), (4, 1000), (2, 4099), (2, 8191), (3, 8193), (2, 16392), (2, 32767),
+                                    (2, 32768)])
+def test_ce_grad_planes_in_place(cuda, rows, V):
+    """The planes in the logits' own memory, rows of whole 8-column pieces and
+    ragged ones (whose padding holds NaNs beforehand); bound as above."""
+    from hydra_amd.kernels.fused_ops import _ce_grad_planes_in_place
+
+    g = torch.Generator().manual_seed(V)
+    x = torch.randn(rows, V, generator=g) * 5
+    t = torch.randint(0, V, (rows,), generator=g)
+    t[-1] = -100
+    logits = torch.full((rows, (V + 7) // 8 * 8), float("nan"), device=cuda)
+    logits[:, :V] = x.to(cuda)
+    got = _ce_grad_planes_in_place(logits, V, t.to(cuda), -100, torch.tensor([0.37], device=cuda)).double().cpu()
+    ref = torch.softmax(x.double(), 1)
+    ref[torch.arange(rows), t.clamp(0)] -= 1
+    ref = ref * 0.37
+    ref[-1] = 0
+    got = got[0::2] + got[1::2]
+    assert got[-1].abs().max() == 0
+    if V > 1:
+        assert float((got - ref).norm() / ref.norm()) < 2.0 ** -16
+    else:
+        assert got.abs().max() < 1e-6
+
+
+@pytest.mark.parametrize("V", [1000, 1003])
+def test_ce_grad_planes_of_infinite_gradients(cuda, V):
+    """An infinite gradient is its first plane; inf - inf beside it would make
+    NaN of the sum."""
+    from hydra_amd.kernels.fused_ops import _ce_grad_planes
+
+    x = torch.randn(2, V, generator=torch.Generator().manual_seed(1)).to(cuda)
+    t = torch.tensor([3, 5], device=cuda)
+    got = _ce_grad_planes(x, t, -100, torch.tensor([float("inf")], device=cuda)).float()
+    want = torch.full((2, V), float("inf"), device=cuda)
+    want[torch.arange(2, device=cuda), t] = -float("inf")
+    assert torch.equal(got[:2] + got[2:], want)
+
+
+@pytest.mark.parametrize("n,dim,V", [(70, 64, 33000), (33, 8, 4099), (1, 64, 40)])
+def test_backward_of_odd_sizes(cuda, n, dim, V):
+    """bf16 gradients over several chunks, rows longer than registers hold and
+    ragged vocabularies, against fp64 of the same inputs: half an ulp of
+    bf16, 2^-9, and the fp32 sums' rounding beside it."""
+    from hydra_amd.kernels import chunked_cross_entropy
+
+    g = torch.Generator().manual_seed(n)
+    h, w = torch.randn(n, dim, generator=g).to(torch.bfloat16), (torch.randn(V, dim, generator=g) * 0.3).to(torch.bfloat16)
+    t = torch.randint(0, V, (n,), generator=g)
+    hd, wd = h.to(cuda).requires_grad_(), w.to(cuda).requires_grad_()
+    chunked_cross_entropy(hd, wd, t.to(cuda), chunk_size=32).backward()
+    h64, w64 = h.double().requires_grad_(), w.double().requires_grad_()
+    torch.nn.functional.cross_entropy(h64 @ w64.t(), t).backward()
+    for a, r in ((hd.grad, h64.grad), (wd.grad, w64.grad)):
+        assert a.shape == r.shape
+        assert float((a.double().cpu() - r).norm() / r.norm()) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("V", [32000, 4099, 40000])
+def test_backward_holds_one_chunk_of_logits(cuda, V):
+    """The bf16 backward's scratch at its peak: one chunk of fp32 logits (the
+    gradient's planes in the same memory), the fp32 gradients and the product
+    that is added to one of them, 16 bytes of [rows, dim] and 8 of [V, dim], and
+    the returned gradients."""
+    from hydra_amd.kernels import chunked_cross_entropy
+
+    n, dim = 2048, 64
+    g = torch.Generator(device=cuda).manual_seed(V)
+    h = torch.randn(n, dim, device=cuda, generator=g).to(torch.bfloat16).requires_grad_()
+    w = (torch.randn(V, dim, device=cuda, generator=g) * 0.05).to(torch.bfloat16).requires_grad_()
+    t = torch.randint(0, V, (n,), device=cuda, generator=g)
+    for _ in range(2):  # the GEMM library's own workspace comes with the first pass
+        h.grad = w.grad = None
+        loss = chunked_cross_entropy(h, w, t)
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        loss.backward()
+        peak = torch.cuda.max_memory_allocated() - before
+    logits = n * ((V + 7) // 8 * 8) * 4
+    assert peak <= logits + 32 * n * dim + 10 * V * dim + (4 << 20), f"{peak / logits:.2f} chunks of logits"
