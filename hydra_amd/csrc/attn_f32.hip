@@ -21,8 +21,8 @@
 // own after the other: inside that one it would cost 30 to 70 registers there.
 // Forward / backward, against a test of every staged tile that 16-bit types
 // made before (for overflow alone; fp32 made none): fp16 B8 8/2 heads x 64, S
-// 2048 157 / 532 -> 134 / 463 us, fp32 B4 8/2 x 64, S 2048 192 / 615 -> 197 /
-// 616.
+// 2048 157 / 532 -> 129 / 467 us, fp32 B4 8/2 x 64, S 2048 192 / 615 -> 198 /
+// 617.
 //
 // What bounds it.  fp32: the fp32 matrix rate (256 FLOP per CU and cycle, a
 // tenth of bf16's measured rate); a 16x16x4 step takes 32 cycles of a SIMD,
@@ -316,23 +316,20 @@ __device__ __forceinline__ uint4 tile_cols(const T* tile, int t, int n, int g) {
   return make_uint4(lo.x, lo.y, hi.x, hi.y);
 }
 
-// x as three bf16 planes, exactly (each takes the next 8 bits; x finite).
+// x as three bf16 planes, exactly: each takes the next 8 bits, rounded to
+// nearest, so what is left after it is at most 2^-9 of it (truncation would
+// leave 2^-7).  A value past bf16's largest overflows to inf - inf.
 __device__ __forceinline__ void split3(const f32x4 (&x)[2], uint4 (&p)[3]) {
   uint32_t w[3][4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    uint32_t b[2], m[2], l[2];
+    float a = x[i >> 1][2 * (i & 1)], b = x[i >> 1][2 * (i & 1) + 1];
 #pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      const float v = x[i >> 1][2 * (i & 1) + e];
-      b[e] = __float_as_uint(v);
-      const float r = v - __uint_as_float(b[e] & 0xffff0000u);
-      m[e] = __float_as_uint(r);
-      l[e] = __float_as_uint(r - __uint_as_float(m[e] & 0xffff0000u));
+    for (int k = 0; k < 3; ++k) {
+      w[k][i] = pack2<bf16>(a, b);
+      a -= __uint_as_float(w[k][i] << 16);
+      b -= __uint_as_float(w[k][i] & 0xffff0000u);
     }
-    w[0][i] = __builtin_amdgcn_perm(b[1], b[0], 0x07060302);
-    w[1][i] = __builtin_amdgcn_perm(m[1], m[0], 0x07060302);
-    w[2][i] = __builtin_amdgcn_perm(l[1], l[0], 0x07060302);
   }
 #pragma unroll
   for (int k = 0; k < 3; ++k) p[k] = make_uint4(w[k][0], w[k][1], w[k][2], w[k][3]);
@@ -376,8 +373,9 @@ __device__ __forceinline__ void prob_product(f32x4 (&acc)[HDP / 16], const T* ti
 }
 
 // dS of any size: three bf16 planes times bf16 rows, or times the two bf16
-// planes of fp16 rows (the product of the two smallest, 2^-24 of the sum's
-// terms or less, left out).
+// planes of fp16 rows.  The product of the two smallest is left out: 2^-8 of
+// the row element times 2^-17 of dS, at most 2^-25 of the sum's terms (over all
+// fp16 significands and 4 M of fp32; half of what one fp32 product rounds off).
 template <typename T, int HDP>
 __device__ __forceinline__ void grad_product(f32x4 (&acc)[HDP / 16], const T* tile, const T* planes,
                                              const f32x4 (&x)[2], int n, int g) {
