@@ -184,3 +184,85 @@ def test_first_call_on_another_stream(cuda):
         got = m(x)
         torch.cuda.synchronize()
         assert torch.equal(y, want) and torch.equal(got, want)
+
+
+def _replays_equal(step, leaf, again):
+    """Captures step() (outputs: a list of tensors) and compares every output
+    of several replays, eager work and synchronizations between them, with the
+    eager call; then once more with `again` written into leaf."""
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(2):
+            step()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        outs = step()
+    for new in (None, again):
+        if new is not None:
+            with torch.no_grad():
+                leaf.copy_(new)
+        want = [t.clone() for t in step()]
+        for r in range(3):
+            noise = torch.randn(2048, 2048, device=leaf.device).sum()
+            torch.cuda.synchronize()
+            for t in outs:
+                t.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            for i, (a, b) in enumerate(zip(outs, want)):
+                assert torch.equal(a, b), f"replay {r}, output {i} of {len(outs)}"
+            del noise
+    del graph
+
+
+@pytest.mark.parametrize("padded", [False, True])
+def test_layer_training_step(cuda, padded, monkeypatch):
+    monkeypatch.setenv("HYDRA_CCGQA_MASK_SEMANTICS", "key_padding")
+    m, x = _layer(cuda).train(), _input(cuda).requires_grad_()
+    go = torch.randn(x.shape, device=cuda).to(torch.bfloat16)
+    mask = torch.arange(512, device=cuda) < torch.tensor([[512], [300]], device=cuda) if padded else None
+
+    def step():
+        y = m(x, mask=mask)
+        return [y.detach(), *torch.autograd.grad(y, [x, *m.parameters()], go)]
+
+    _replays_equal(step, x, torch.randn_like(x))
+
+
+@pytest.mark.parametrize("n,V", [(3000, 32000), (3000, 4099), (70000, 512)])
+def test_loss_step(cuda, n, V):
+    from hydra_amd.kernels import chunked_cross_entropy
+
+    h = torch.randn(n, 256, device=cuda).to(torch.bfloat16).requires_grad_()
+    w = (torch.randn(V, 256, device=cuda) * 0.05).to(torch.bfloat16).requires_grad_()
+    t = torch.randint(0, V, (n,), device=cuda)
+    t[::7] = -100
+
+    def step():
+        loss = chunked_cross_entropy(h, w, t, chunk_size=2048)
+        return [loss.detach(), *torch.autograd.grad(loss, [h, w])]
+
+    _replays_equal(step, h, torch.randn_like(h))
+
+
+def test_mod_training_step(cuda):
+    from hydra_amd.kernels import fused_rms_norm
+    from hydra_amd.routing import gather_by_indices, mod_topk, weighted_residual_scatter
+
+    B, L, D, k = 4, 1024, 512, 768
+    scores = torch.randn(B, L, device=cuda)
+    x = torch.randn(B, L, D, device=cuda).to(torch.bfloat16).requires_grad_()
+    gain = torch.ones(D, device=cuda, dtype=torch.bfloat16).requires_grad_()
+    weights = torch.rand(B, k, device=cuda).requires_grad_()
+    go = torch.randn(B, L, D, device=cuda).to(torch.bfloat16)
+
+    def step():
+        _, idx, _ = mod_topk(scores, k)
+        y = fused_rms_norm(gather_by_indices(x, idx, distinct=True), gain)
+        out = weighted_residual_scatter(x.clone(), y, idx, weights)
+        return [out.detach(), *torch.autograd.grad(out, [x, gain, weights], go)]
+
+    _replays_equal(step, x, torch.randn_like(x))
