@@ -168,9 +168,11 @@ def _rope_tables(cos: torch.Tensor, sin: torch.Tensor, S: int, bf16_ok: bool):
     kernel widens them itself (bf16_ok; flag CCGQA_ROPE_BF16) -- with whole
     rows one after the other; converted otherwise (an expanded table, a slice
     of a wider one)."""
-    rows = cos.shape[-2] if cos.dim() == 4 else cos.shape[0]
+    rows = min(t.shape[-2] if t.dim() == 4 else t.shape[0] for t in (cos, sin))
     if rows < S:
         raise ValueError(f"ccgqa_prep: RoPE cache covers {rows} positions < S={S}")
+    if cos.shape[-1] != sin.shape[-1]:
+        raise ValueError(f"ccgqa_prep: RoPE tables of {cos.shape[-1]} and {sin.shape[-1]} columns")
     half = bf16_ok and cos.dtype == sin.dtype == torch.bfloat16
     if (half or cos.dtype == sin.dtype == torch.float32) and cos.stride(-1) == sin.stride(-1) == 1 and \
             cos.dim() == sin.dim() and cos.dim() in (2, 4) and \

@@ -41,3 +41,18 @@ def test_tables_that_do_not_cover_the_sequence_are_refused(shape):
 
     with pytest.raises(ValueError, match="RoPE cache"):
         _rope_tables(torch.zeros(shape), torch.zeros(shape), 5, True)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("batched", [False, True])
+def test_sine_tables_apart_from_the_cosines(dtype, batched):
+    """The kernel walks both tables by one row stride: a sine table with too
+    few rows or another width is refused, one with more rows is not."""
+    from hydra_amd.attention.backends.ccgqa.ops import _rope_tables
+
+    tables = [torch.zeros(n, w, dtype=dtype) for n, w in ((6, 8), (4, 8), (6, 4), (9, 8))]
+    cos, short, narrow, longer = (t[None, None] if batched else t for t in tables)
+    for sin in (short, narrow):
+        with pytest.raises(ValueError, match="RoPE"):
+            _rope_tables(cos, sin, 5, True)
+    _rope_tables(cos, longer, 5, True)
