@@ -184,7 +184,8 @@ class CCGQAAttention(nn.Module):
         if tiled:
             flags |= CCGQA_W_TILED  # conv weights in MFMA-fragment order
         with torch.no_grad():
-            packed, packed_o = self._packed(convw, x.dtype, tiled)
+            w_o = self.o_proj.weight
+            packed, packed_o = self._packed(convw, w_o, x.dtype, tiled)
             q, k, v = ccgqa_prep(
                 qkv.detach(), self.n_heads, self.n_kv_heads, self.head_dim, flags, *packed,
                 temperature=self.key_temperature if self.use_qk_norm else None,
@@ -197,7 +198,7 @@ class CCGQAAttention(nn.Module):
                               key_mask=mask, mask_mode=_mask_mode() if mask is not None else 0,
                               out=o_view,
                               bound_temperature=self.key_temperature if self.use_qk_norm else None)
-        out = output_projection(out, self.o_proj.weight, packed_o)
+        out = output_projection(out, w_o, packed_o)
         if self.output_scale != 1.0:
             out = out * self.output_scale
         return out
@@ -225,12 +226,11 @@ class CCGQAAttention(nn.Module):
             out = out * self.output_scale
         return out
 
-    def _packed(self, convw, dtype, tiled):
+    def _packed(self, convw, w_o, dtype, tiled):
         """The four conv weights packed in `dtype` (tap-major, or MFMA-tiled;
         None without convs), and o_proj's weight in hydra_linear_fwd's fragment
         order (None where that kernel does not take it); rebuilt only when a
         weight changes."""
-        w_o = self.o_proj.weight
         o_ok = linear_weight_ok(w_o)
         ws = (*convw, w_o) if o_ok else convw
         if not ws:
@@ -250,10 +250,11 @@ class CCGQAAttention(nn.Module):
         return (packed[:4] if convw else (None,) * 4), (packed[-1] if o_ok else None)
 
     def _packed_conv_weights(self, convw, dtype, tiled=False):
-        return self._packed(convw, dtype, tiled)[0]
+        return self._packed(convw, self.o_proj.weight, dtype, tiled)[0]
 
     def _packed_o_proj(self):
-        return self._packed((), self.o_proj.weight.dtype, False)[1]
+        w_o = self.o_proj.weight
+        return self._packed((), w_o, w_o.dtype, False)[1]
 
     def _load_from_state_dict(self, state_dict, prefix, local_metadata, strict, missing_keys,
                               unexpected_keys, error_msgs):

@@ -4,6 +4,7 @@ here; strides, pointers and the current stream go to the library."""
 from __future__ import annotations
 
 import ctypes
+import operator
 import threading
 import weakref
 from typing import Optional
@@ -59,21 +60,31 @@ def pack_conv_weights_tiled(ws, dtype: torch.dtype, n_heads: int, n_kv_heads: in
     return tuple(packed)
 
 
+_version = operator.attrgetter("_version")
+
+
+def _state(ws):
+    """What tells apart one set of values of the weights ws from another, as
+    long as these objects live."""
+    return (*map(id, ws), *map(_version, ws), *map(torch.Tensor.data_ptr, ws))
+
+
 class _Pack:
-    __slots__ = ("refs", "versions", "ptrs", "tensors", "event", "streams", "captured")
+    __slots__ = ("refs", "state", "tensors", "event", "streams", "captured", "__weakref__")
+
+    def __init__(self, ws, state, tensors):
+        this = weakref.ref(self)
+
+        def gone(_):  # another object may get the id of a weight that is no more
+            p = this()
+            if p is not None:
+                p.state = None
+
+        self.refs, self.state, self.tensors = [weakref.ref(w, gone) for w in ws], state, tensors
+        self.event, self.streams, self.captured = None, set(), False
 
     def same(self, ws) -> bool:
         return len(ws) == len(self.refs) and all(r() is w for r, w in zip(self.refs, ws))
-
-    def holds(self, ws) -> bool:
-        for r, v, a, w in zip(self.refs, self.versions, self.ptrs, ws):
-            if r() is not w or w._version != v or w.data_ptr() != a:
-                return False
-        return True
-
-    def note(self, ws, tensors) -> None:
-        self.versions, self.ptrs = [w._version for w in ws], [w.data_ptr() for w in ws]
-        self.tensors = tensors
 
 
 class PackedWeights:
@@ -106,10 +117,10 @@ class PackedWeights:
     def get(self, ws, tag):
         """The tensors that the weights ws (a tuple) were last packed to, or
         None; `tag` tells apart what ws may be packed to."""
-        p = self._last.get(tag)
-        if p is None or not p.holds(ws):
+        p, state = self._last.get(tag), _state(ws)
+        if p is None or p.state != state:
             p = self._seen(ws, tag)
-            if p is None or not p.holds(ws):
+            if p is None or p.state != state:
                 return None
         if ws[0].is_cuda:
             if torch.cuda.is_current_stream_capturing():
@@ -118,7 +129,10 @@ class PackedWeights:
                     self._captured.append((tag, p))
             elif _lib.stream(ws[0]) not in p.streams:
                 here = torch.cuda.current_stream(ws[0].device)
-                here.wait_event(p.event)
+                if p.event is None:
+                    here.wait_stream(torch.cuda.default_stream(ws[0].device))
+                else:
+                    here.wait_event(p.event)
                 for t in p.tensors:
                     t.record_stream(here)
                 p.streams.add(here.cuda_stream)
@@ -136,16 +150,19 @@ class PackedWeights:
                 for old, new in zip(p.tensors, tensors):
                     old.copy_(new)
                 torch.cuda.synchronize(ws[0].device)  # replays to come read the new values
-                p.note(ws, p.tensors)
+                p.state = _state(ws)
             else:
-                p = _Pack()
-                p.refs, p.captured, p.event, p.streams = [weakref.ref(w) for w in ws], False, None, set()
                 # a layout that is the weight's own: a copy, or a later pack would write to the weight
-                p.note(ws, tuple(t.clone() if t.data_ptr() == w.data_ptr() else t for t, w in zip(tensors, ws)))
+                tensors = tuple(t.clone() if t.data_ptr() == w.data_ptr() else t for t, w in zip(tensors, ws))
+                p = _Pack(ws, _state(ws), tensors)
                 if ws[0].is_cuda:
-                    here = torch.cuda.current_stream(ws[0].device)
-                    p.event = here.record_event()
-                    p.streams.add(here.cuda_stream)
+                    here = _lib.stream(ws[0])
+                    p.streams.add(here)
+                    # The default stream (0) is never captured and always there
+                    # to wait for: no event, which would hold up the launches
+                    # that follow (30 us of a module's first pass).
+                    if here != 0:
+                        p.event = torch.cuda.current_stream(ws[0].device).record_event()
             self._last[tag] = p
         return p.tensors
 
@@ -168,15 +185,17 @@ def _rope_tables(cos: torch.Tensor, sin: torch.Tensor, S: int, bf16_ok: bool):
     kernel widens them itself (bf16_ok; flag CCGQA_ROPE_BF16) -- with whole
     rows one after the other; converted otherwise (an expanded table, a slice
     of a wider one)."""
-    rows = min(t.shape[-2] if t.dim() == 4 else t.shape[0] for t in (cos, sin))
+    rows = cos.shape[-2] if cos.dim() == 4 else cos.shape[0]
+    alike = cos.shape == sin.shape
+    if not alike:
+        rows = min(rows, sin.shape[-2] if sin.dim() == 4 else sin.shape[0])
+        if cos.shape[-1] != sin.shape[-1]:
+            raise ValueError(f"ccgqa_prep: RoPE tables of {cos.shape[-1]} and {sin.shape[-1]} columns")
     if rows < S:
         raise ValueError(f"ccgqa_prep: RoPE cache covers {rows} positions < S={S}")
-    if cos.shape[-1] != sin.shape[-1]:
-        raise ValueError(f"ccgqa_prep: RoPE tables of {cos.shape[-1]} and {sin.shape[-1]} columns")
     half = bf16_ok and cos.dtype == sin.dtype == torch.bfloat16
-    if (half or cos.dtype == sin.dtype == torch.float32) and cos.stride(-1) == sin.stride(-1) == 1 and \
-            cos.dim() == sin.dim() and cos.dim() in (2, 4) and \
-            cos.stride(-2) == sin.stride(-2) == cos.shape[-1] == sin.shape[-1] and cos.shape[-1] % 4 == 0 and \
+    if alike and (half or cos.dtype == sin.dtype == torch.float32) and cos.stride(-1) == sin.stride(-1) == 1 and \
+            cos.dim() in (2, 4) and cos.stride(-2) == sin.stride(-2) == cos.shape[-1] and cos.shape[-1] % 4 == 0 and \
             (cos.data_ptr() | sin.data_ptr()) % 16 == 0:
         return cos, sin, cos.stride(-2), CCGQA_ROPE_BF16 if half else 0
     cos, sin = ((t[0, 0] if t.dim() == 4 else t)[:S].float().contiguous() for t in (cos, sin))
@@ -379,7 +398,7 @@ def output_projection(x: torch.Tensor, weight: torch.Tensor,
     backward for) stay on the library GEMM, as in the reference."""
     N, K = weight.shape
     if (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)) or \
-            x.dtype != torch.bfloat16 or not linear_weight_ok(weight) or x.shape[-1] != K:
+            x.dtype != torch.bfloat16 or not (packed is not None or linear_weight_ok(weight)) or x.shape[-1] != K:
         return F.linear(x, weight)
     _lib.require_gpu("output_projection", x, weight, packed)
     x2 = x.reshape(-1, K)

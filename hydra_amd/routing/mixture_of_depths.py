@@ -28,15 +28,23 @@ def _recording(*tensors) -> bool:
 def _plain(*modules) -> bool:
     """Whether calling these modules is calling their class's forward: no
     hooks, on them or on every module, and no forward set on the instance."""
-    return not _has_any_global_hook() and not any(
-        m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
-        or "forward" in m.__dict__ for m in modules)
+    if _has_any_global_hook():
+        return False
+    for m in modules:
+        if (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                or "forward" in m.__dict__):
+            return False
+    return True
 
 
 def _own(obj: nn.Module, base: type, *methods: str) -> bool:
     """Whether obj's methods are base's: not overridden by its class, not set
     on the instance."""
-    return all(getattr(type(obj), m) is getattr(base, m) and m not in obj.__dict__ for m in methods)
+    same = type(obj) is base
+    for m in methods:
+        if m in obj.__dict__ or not (same or getattr(type(obj), m) is getattr(base, m)):
+            return False
+    return True
 
 
 def _plain_tensor(x: torch.Tensor) -> bool:
