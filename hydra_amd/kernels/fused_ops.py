@@ -401,7 +401,8 @@ def _ce_grad_planes_in_place(logits: torch.Tensor, V: int, targets: torch.Tensor
     with _lib.on_device(logits):
         _lib.call("hydra_ce_grad_planes", logits.data_ptr(), rows, V, pitch, targets.data_ptr(), int(ignore_index),
                   logits.data_ptr(), 2 * pitch, pitch, _lib.ptr(grad_scale), _lib.stream(logits))
-    return logits.view(torch.bfloat16).view(2 * rows, pitch)[:, :V]
+    planes = logits.view(torch.bfloat16).view(2 * rows, pitch)
+    return planes if pitch == V else planes[:, :V]
 
 
 class ChunkedCrossEntropyFunction(torch.autograd.Function):
@@ -452,7 +453,8 @@ class ChunkedCrossEntropyFunction(torch.autograd.Function):
             # Other dtypes keep the fp32 GEMMs: fp32 operands would need three
             # planes each, six products, for no gain worth the name.  So does
             # create_graph, which products with an `out` cannot record.
-            V = weight.shape[0]
+            V, wt = weight.shape[0], weight.t()
+            pitch = (V + 7) // 8 * 8
             in_place = V <= CE_IN_PLACE_VOCAB
             # longer rows: the planes lie beside the logits, of half a chunk each
             step = cs if in_place else max(1, (min(cs, h.shape[0]) + 1) // 2)
@@ -460,19 +462,20 @@ class ChunkedCrossEntropyFunction(torch.autograd.Function):
             for s in range(0, h.shape[0], step):
                 hc = h[s:s + step]
                 n = hc.shape[0]
-                logits = torch.empty((n, (V + 7) // 8 * 8), dtype=torch.float32, device=h.device)
-                torch.mm(hc, weight.t(), out_dtype=torch.float32, out=logits[:, :V])
-                if in_place:
+                if pitch == V:
+                    logits = torch.mm(hc, wt, out_dtype=torch.float32)
+                else:
+                    logits = torch.empty((n, pitch), dtype=torch.float32, device=h.device)
+                    torch.mm(hc, wt, out_dtype=torch.float32, out=logits[:, :V])
+                if in_place:  # a token's two rows, one after the other
                     planes = _ce_grad_planes_in_place(logits, V, t[s:s + step], ctx.ignore_index, scale)
-                    pair = (n, 2)  # a token's two rows, one after the other
+                    first, second, both = slice(0, None, 2), slice(1, None, 2), torch.cat((hc, hc), 1).view(2 * n, dim)
                 else:
                     planes = _ce_grad_planes(logits[:, :V], t[s:s + step], ctx.ignore_index, scale)
-                    pair = (2, n)
+                    first, second, both = slice(0, n), slice(n, None), torch.cat((hc, hc))
                 del logits
-                side = pair.index(2)
-                gh = torch.mm(planes, weight, out_dtype=torch.float32).view(*pair, dim)
-                torch.add(gh.select(side, 0), gh.select(side, 1), out=grad_h[s:s + step])
-                both = hc.unsqueeze(side).expand(*pair, dim).reshape(2 * n, dim)
+                gh = torch.mm(planes, weight, out_dtype=torch.float32)
+                torch.add(gh[first], gh[second], out=grad_h[s:s + step])
                 if grad_w is None:
                     grad_w = torch.mm(planes.t(), both, out_dtype=torch.float32)
                 else:
