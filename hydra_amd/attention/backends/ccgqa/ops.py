@@ -123,11 +123,14 @@ class PackedWeights:
             if p is None or p.state != state:
                 return None
         if ws[0].is_cuda:
-            if torch.cuda.is_current_stream_capturing():
+            raw = _lib.stream(ws[0])
+            if raw == 0 and raw in p.streams:
+                pass  # the default stream is never captured
+            elif torch.cuda.is_current_stream_capturing():
                 if not p.captured:
                     p.captured = True
                     self._captured.append((tag, p))
-            elif _lib.stream(ws[0]) not in p.streams:
+            elif raw not in p.streams:
                 here = torch.cuda.current_stream(ws[0].device)
                 if p.event is None:
                     here.wait_stream(torch.cuda.default_stream(ws[0].device))
@@ -135,7 +138,7 @@ class PackedWeights:
                     here.wait_event(p.event)
                 for t in p.tensors:
                     t.record_stream(here)
-                p.streams.add(here.cuda_stream)
+                p.streams.add(raw)
         return p.tensors
 
     def put(self, ws, tag, tensors):

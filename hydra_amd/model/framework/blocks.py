@@ -33,11 +33,12 @@ def _mlp_residual(mlp: nn.Module, h: torch.Tensor, y: torch.Tensor) -> torch.Ten
     changes or hooks into (also under such a MoD wrapper that does not route
     yet).  h is a fresh tensor of the caller's: its storage may hold the
     result."""
-    if isinstance(mlp, SwiGLUMLPFused) and _plain(mlp):
-        if not _own(mlp, SwiGLUMLPFused, "forward_residual"):
-            return mlp.forward_residual(h, y)
-        if _own(mlp, SwiGLUMLPFused, "forward"):
-            return mlp.forward_residual(h, y, own=True)
+    if isinstance(mlp, SwiGLUMLPFused):
+        if _plain(mlp):
+            if _own(mlp, SwiGLUMLPFused, "forward", "forward_residual"):
+                return mlp.forward_residual(h, y, own=True)
+            if not _own(mlp, SwiGLUMLPFused, "forward_residual"):
+                return mlp.forward_residual(h, y)
     elif (isinstance(mlp, MoDMLPWrapper) and _own(mlp, MoDMLPWrapper, "forward") and mlp._dense()
             and isinstance(mlp.mlp, SwiGLUMLPFused)
             and _own(mlp.mlp, SwiGLUMLPFused, "forward", "forward_residual") and _plain(mlp, mlp.mlp)):

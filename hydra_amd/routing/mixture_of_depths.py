@@ -28,21 +28,20 @@ def _recording(*tensors) -> bool:
 def _plain(*modules) -> bool:
     """Whether calling these modules is calling their class's forward: no
     hooks, on them or on every module, and no forward set on the instance."""
-    if _has_any_global_hook():
-        return False
     for m in modules:
-        if (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
-                or "forward" in m.__dict__):
+        d = m.__dict__
+        if (d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"]
+                or "forward" in d):
             return False
-    return True
+    return not _has_any_global_hook()
 
 
 def _own(obj: nn.Module, base: type, *methods: str) -> bool:
     """Whether obj's methods are base's: not overridden by its class, not set
     on the instance."""
-    same = type(obj) is base
+    d, cls = obj.__dict__, type(obj)
     for m in methods:
-        if m in obj.__dict__ or not (same or getattr(type(obj), m) is getattr(base, m)):
+        if m in d or (cls is not base and getattr(cls, m) is not getattr(base, m)):
             return False
     return True
 
