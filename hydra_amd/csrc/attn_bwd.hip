@@ -44,7 +44,9 @@
 // more MFMA per fragment.  Measured against one thread per row in fp32:
 // B8 4/1 heads x 64, S 777, padded: 101.4 ms -> below 0.1; B2 28/4 heads x
 // 16, S 2048, causal: 60 ms -> below 0.3 (whole layer steps 102.5 -> 1.41
-// and 61.3 -> 1.40 ms, what remains is the rest of the layer).
+// and 61.3 -> 1.40 ms, what remains is the rest of the layer).  Of all these
+// forms only dK/dV of the reference mask at head_dim 64 with two head groups spills to
+// scratch (14 registers, 60 bytes per lane: 512 threads leave it 256).
 // In the same two forms rows that a query does not see stay out of its sums
 // whatever they hold: with an infinity or NaN in a staged row the weight 0 of
 // an unseen one gives NaN, so a wave that ends with a NaN in its accumulators
@@ -990,8 +992,9 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(
 
 // ---------------------------------------------------------------------------
 // Generic path: fp32 math, one thread per query row (dQ) or key row (dK, dV).
-// Rows of up to MAXD elements are accumulated in registers.
-template <typename T, int MAXD, bool CAUSAL, int MASK>
+// Rows of up to kGenericMaxHd elements, held in scratch memory (rolled loops).
+constexpr int kGenericMaxHd = 256;
+template <typename T, bool CAUSAL, int MASK>
 __global__ __launch_bounds__(128) void attn_bwd_generic_dq_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
     const T* __restrict__ dout, const float* __restrict__ dvec, const float* __restrict__ lse2,
@@ -1009,10 +1012,9 @@ __global__ __launch_bounds__(128) void attn_bwd_generic_dq_kernel(
   const int kvh = h / (Hq / Hkv);
   const T* qr = q + b * qs0 + h * qs1 + s * qs2;
   const T* dr = dout + b * ds0 + h * ds1 + s * ds2;
-  constexpr int UNR = MAXD <= 64 ? MAXD : 1;  // longer rows live in scratch anyway
-  float qv[MAXD], ov[MAXD], acc[MAXD];
-#pragma unroll UNR
-  for (int e = 0; e < MAXD; ++e) {
+  float qv[kGenericMaxHd], ov[kGenericMaxHd], acc[kGenericMaxHd];
+#pragma unroll 1
+  for (int e = 0; e < kGenericMaxHd; ++e) {
     qv[e] = e < hd ? to_f32(qr[e]) : 0.f;
     ov[e] = e < hd ? to_f32(dr[e]) : 0.f;
     acc[e] = 0.f;
@@ -1025,25 +1027,25 @@ __global__ __launch_bounds__(128) void attn_bwd_generic_dq_kernel(
     const T* kr = k + b * ks0 + kvh * ks1 + t * ks2;
     const T* vr = v + b * vs0 + kvh * vs1 + t * vs2;
     float sc = 0.f, dpv = 0.f;
-#pragma unroll UNR
-    for (int e = 0; e < MAXD; ++e)
+#pragma unroll 1
+    for (int e = 0; e < kGenericMaxHd; ++e)
       if (e < hd) {
         sc = fmaf(qv[e], to_f32(kr[e]), sc);
         dpv = fmaf(ov[e], to_f32(vr[e]), dpv);
       }
     const float p = exp2f(fmaf(sc, scale_log2, -l2));
     const float ds = p * (dpv - dd);
-#pragma unroll UNR
-    for (int e = 0; e < MAXD; ++e)
+#pragma unroll 1
+    for (int e = 0; e < kGenericMaxHd; ++e)
       if (e < hd) acc[e] = fmaf(ds, to_f32(kr[e]), acc[e]);
   }
   T* orow = dq + b * dqs0 + h * dqs1 + s * dqs2;
-#pragma unroll UNR
-  for (int e = 0; e < MAXD; ++e)
+#pragma unroll 1
+  for (int e = 0; e < kGenericMaxHd; ++e)
     if (e < hd) orow[e] = from_f32<T>(acc[e] * scale);
 }
 
-template <typename T, int MAXD, bool CAUSAL, int MASK>
+template <typename T, bool CAUSAL, int MASK>
 __global__ __launch_bounds__(128) void attn_bwd_generic_dkdv_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
     const T* __restrict__ dout, const float* __restrict__ dvec, const float* __restrict__ lse2,
@@ -1062,10 +1064,9 @@ __global__ __launch_bounds__(128) void attn_bwd_generic_dkdv_kernel(
   const int G = Hq / Hkv;
   const T* kr = k + b * ks0 + kvh * ks1 + t * ks2;
   const T* vr = v + b * vs0 + kvh * vs1 + t * vs2;
-  constexpr int UNR = MAXD <= 64 ? MAXD : 1;  // longer rows live in scratch anyway
-  float kv[MAXD], vv[MAXD], ak[MAXD], av[MAXD];
-#pragma unroll UNR
-  for (int e = 0; e < MAXD; ++e) {
+  float kv[kGenericMaxHd], vv[kGenericMaxHd], ak[kGenericMaxHd], av[kGenericMaxHd];
+#pragma unroll 1
+  for (int e = 0; e < kGenericMaxHd; ++e) {
     kv[e] = e < hd ? to_f32(kr[e]) : 0.f;
     vv[e] = e < hd ? to_f32(vr[e]) : 0.f;
     ak[e] = 0.f;
@@ -1080,16 +1081,16 @@ __global__ __launch_bounds__(128) void attn_bwd_generic_dkdv_kernel(
       const T* qr = q + b * qs0 + h * qs1 + s * qs2;
       const T* dr = dout + b * ds0 + h * ds1 + s * ds2;
       float sc = 0.f, dpv = 0.f;
-#pragma unroll UNR
-      for (int e = 0; e < MAXD; ++e)
+#pragma unroll 1
+      for (int e = 0; e < kGenericMaxHd; ++e)
         if (e < hd) {
           sc = fmaf(to_f32(qr[e]), kv[e], sc);
           dpv = fmaf(to_f32(dr[e]), vv[e], dpv);
         }
       const float p = exp2f(fmaf(sc, scale_log2, -lse2[rb + s]));
       const float ds = p * (dpv - dvec[rb + s]);
-#pragma unroll UNR
-      for (int e = 0; e < MAXD; ++e)
+#pragma unroll 1
+      for (int e = 0; e < kGenericMaxHd; ++e)
         if (e < hd) {
           av[e] = fmaf(p, to_f32(dr[e]), av[e]);
           ak[e] = fmaf(ds, to_f32(qr[e]), ak[e]);
@@ -1098,8 +1099,8 @@ __global__ __launch_bounds__(128) void attn_bwd_generic_dkdv_kernel(
   }
   T* okr = dk + b * dks0 + kvh * dks1 + t * dks2;
   T* ovr = dv + b * dvs0 + kvh * dvs1 + t * dvs2;
-#pragma unroll UNR
-  for (int e = 0; e < MAXD; ++e)
+#pragma unroll 1
+  for (int e = 0; e < kGenericMaxHd; ++e)
     if (e < hd) {
       okr[e] = from_f32<T>(ak[e] * scale);
       ovr[e] = from_f32<T>(av[e]);
@@ -1321,7 +1322,7 @@ int launch_mfma(const BwdArgs& a, const float* dvec, const float* lse2, float* p
   return rc != HYDRA_OK ? rc : rj;
 }
 
-template <typename T, int MAXD, bool CAUSAL, int MASK>
+template <typename T, bool CAUSAL, int MASK>
 int launch_generic(const BwdArgs& a, const float* dvec, const float* lse2) {
   const float sl2 = a.scale * kLog2e;
   const T* q = static_cast<const T*>(a.q);
@@ -1330,14 +1331,14 @@ int launch_generic(const BwdArgs& a, const float* dvec, const float* lse2) {
   const T* d = static_cast<const T*>(a.dout);
   const int64_t qrows = static_cast<int64_t>(a.B) * a.Hq * a.S;
   const int64_t krows = static_cast<int64_t>(a.B) * a.Hkv * a.S;
-  attn_bwd_generic_dkdv_kernel<T, MAXD, CAUSAL, MASK>
+  attn_bwd_generic_dkdv_kernel<T, CAUSAL, MASK>
       <<<dim3(static_cast<unsigned>((krows + 127) / 128)), 128, 0, a.st>>>(
           q, k, v, d, dvec, lse2, a.kmask, static_cast<T*>(a.dk), static_cast<T*>(a.dv), krows, a.Hq,
           a.Hkv, a.S, a.hd, a.qs[0], a.qs[1], a.qs[2], a.ks[0], a.ks[1], a.ks[2], a.vs[0],
           a.vs[1], a.vs[2], a.dos[0], a.dos[1], a.dos[2], a.dks[0], a.dks[1], a.dks[2],
           a.dvs[0], a.dvs[1], a.dvs[2], sl2, a.scale);
   if (int rc = check_launch("attn_bwd: generic dkdv")) return rc;
-  attn_bwd_generic_dq_kernel<T, MAXD, CAUSAL, MASK>
+  attn_bwd_generic_dq_kernel<T, CAUSAL, MASK>
       <<<dim3(static_cast<unsigned>((qrows + 127) / 128)), 128, 0, a.st>>>(
           q, k, v, d, dvec, lse2, a.kmask, static_cast<T*>(a.dq), qrows, a.Hq, a.Hkv, a.S, a.hd,
           a.qs[0], a.qs[1], a.qs[2], a.ks[0], a.ks[1], a.ks[2], a.vs[0], a.vs[1], a.vs[2],
@@ -1353,11 +1354,11 @@ int run_other(const BwdArgs& a, int dtype, float* dvec, float* lse2, float* part
                                     a.mask_mode, a.B, a.Hq, a.Hkv, a.S, a.hd, a.qs, a.ks, a.vs, a.os, a.dos, a.dqs,
                                     a.dks, a.dvs, a.causal, a.scale, dtype, a.st},
                         part, part_bytes);
-  if (a.mask_mode == HYDRA_MASK_REFERENCE_SDPA) return launch_generic<T, 256, true, 2>(a, dvec, lse2);
+  if (a.mask_mode == HYDRA_MASK_REFERENCE_SDPA) return launch_generic<T, true, 2>(a, dvec, lse2);
   if (a.mask_mode == HYDRA_MASK_KEY_PADDING)
-    return a.causal ? launch_generic<T, 256, true, 1>(a, dvec, lse2) : launch_generic<T, 256, false, 1>(a, dvec, lse2);
-  return a.causal ? launch_generic<T, 256, true, 0>(a, dvec, lse2)
-                  : launch_generic<T, 256, false, 0>(a, dvec, lse2);
+    return a.causal ? launch_generic<T, true, 1>(a, dvec, lse2) : launch_generic<T, false, 1>(a, dvec, lse2);
+  return a.causal ? launch_generic<T, true, 0>(a, dvec, lse2)
+                  : launch_generic<T, false, 0>(a, dvec, lse2);
 }
 
 template <int HD>

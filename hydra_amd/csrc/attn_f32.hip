@@ -56,9 +56,9 @@
 // 0.26 ms; fp32 B2 8/2 x 16, S 512, causal 8.7 -> 0.17 ms (launch-bound).
 // Errors against 64 bits: fp32 1.8e-6 -> 5.8e-7, fp16 2.3e-4 (the output's
 // rounding) both.  16-bit planes against the fp32 instruction on the converted
-// rows, fp16: the first of these calls' kernels forward 71 -> 33, dK/dV 115 ->
-// 54, dQ 88 -> 40 us; B8 8/2 x 64, S 2048 1516 -> 616 us; B2 8/2 x 128, S 2048
-// 841 -> 352 us; B4 8/2 x 16, S 2048 270 -> 208 us.
+// rows, fp16: the first of these calls' kernels forward 71 -> 32, dK/dV 115 ->
+// 50, dQ 88 -> 34 us; B8 8/2 x 64, S 2048 1516 -> 596 us; B2 8/2 x 128, S 2048
+// 841 -> 318 us; B4 8/2 x 16, S 2048 270 -> 194 us.
 #include "attn_f32.h"
 
 #include <algorithm>
@@ -1007,8 +1007,10 @@ struct Plan {
   size_t kv_floats, q_floats;
 };
 constexpr int kMinTiles = 6, kRounds = 3;
-// Workgroups of each backward kernel resident on a CU (registers; 142 / 125 at
-// head_dim 64), by head_dim 16, 32, 64, 128.
+// Workgroups of each backward kernel resident on a CU, by head_dim 16, 32, 64,
+// 128: the fp32 kernels' (148 / 137 registers at head_dim 64).  The 16-bit ones
+// (149 / 115) hold one or two fewer at head_dim 16 and one more dQ workgroup at
+// 64: one table serves them, since it only scales how many chunks a walk gives.
 constexpr int kKvPerCu[4] = {6, 5, 3, 2}, kQPerCu[4] = {7, 5, 3, 2};
 
 // split = false: every walk whole (no partials).
