@@ -148,7 +148,8 @@ class PackedWeights:
             return tensors
         with self._lock:
             p = self._seen(ws, tag)
-            if p is not None:
+            if p is not None and all(o.shape == n.shape and o.dtype == n.dtype and o.device == n.device
+                                     for o, n in zip(p.tensors, tensors)):
                 torch.cuda.synchronize(ws[0].device)  # replays that read them are done
                 for old, new in zip(p.tensors, tensors):
                     old.copy_(new)

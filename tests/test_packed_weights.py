@@ -87,3 +87,24 @@ def test_packing_in_one_launch_refuses_host_memory(monkeypatch):
         assert torch.equal(got, pack_conv_weight(w, torch.bfloat16, True))
     with pytest.raises(RuntimeError, match="GPU tensors only"):
         ccgqa_prep(torch.zeros(1, 8, 256, dtype=torch.bfloat16), 2, 1, 64, 1 | 64, *ws)
+
+
+def test_a_captured_pack_of_another_form_is_left_alone():
+    """Weights that moved, or are packed to another shape or type since a
+    capture read them, get tensors of their own."""
+    from hydra_amd.attention.backends.ccgqa.ops import PackedWeights
+
+    packs = PackedWeights()
+    w = nn.Parameter(torch.randn(4))
+    (old,) = packs.put((w,), None, (-w.detach(),))
+    p = packs._last[None]
+    p.captured = True
+    packs._captured.append((None, p))
+    before = old.clone()
+    for data in (torch.randn(6), torch.randn(4, dtype=torch.float64)):
+        w.data = data
+        assert packs.get((w,), None) is None
+        (new,) = packs.put((w,), None, (-w.detach(),))
+        assert torch.equal(new, -w) and new.dtype == w.dtype
+        assert packs.get((w,), None)[0] is new
+        assert torch.equal(old, before)
